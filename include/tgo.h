@@ -212,19 +212,43 @@ int tgo_swiglu_rows(const void * gate_bf16, const void * up_bf16, void * activat
 int tgo_swiglu_backward(const void * gate_bf16, const void * up_bf16, const void * grad_activated_bf16,
                         const void * grad_gate_bf16, void * d_gate_bf16, void * d_up_bf16, int64_t count, void * stream);
 
-/* Routing of a small batch in one launch: the [tokens, top_k] expert choices sorted by expert (stable), as the
- * metadata the grouped entry points take, with one group per expert:
+/* Routing of a batch: the [tokens, top_k] expert choices sorted by expert (stable), as the metadata the grouped entry
+ * points take, with one group per expert:
  *   slot_rows int64 [tokens * top_k]       sorted row of each (token, choice) slot; -1 for an expert outside [0, num_experts)
  *   row_index int64 [tokens * top_k]       token of each sorted row (the gather index of the gathered entry points);
  *                                          -1 behind the last row
  *   expert_indices int64 [num_experts]     0, 1, 2, ...
  *   expert_offsets int32 [num_experts]     rows of experts 0..e
- * At most TGO_ROUTE_SMALL_LIMIT slots and experts (one workgroup sorts them); larger batches are sorted by the caller.
+ * One launch for at most 4096 slots, two above that, which need `workspace` (tgo_route_workspace_bytes, else 0 and NULL).
+ * At most TGO_ROUTE_SLOT_LIMIT slots and TGO_ROUTE_EXPERT_LIMIT experts.
  * No counterpart in the reference, whose callers sort with tensor operations (torch_ggml_ops/grouped_mmq.py:216 takes
- * the sorted metadata); at decode sizes those operations are a dozen launches, more than the layer's own. */
+ * the sorted metadata); those operations are one to two dozen launches. */
+#define TGO_ROUTE_SLOT_LIMIT 4194304
+#define TGO_ROUTE_EXPERT_LIMIT 4096
+int64_t tgo_route_workspace_bytes(int64_t slots, int64_t num_experts);
+int tgo_route(const int64_t * slot_experts, int64_t tokens, int64_t top_k, int64_t num_experts, int64_t * row_index,
+              int64_t * slot_rows, int64_t * expert_indices, int32_t * expert_offsets, void * workspace, void * stream);
+
+/* tgo_route for a batch of one launch, which needs no workspace: at most TGO_ROUTE_SMALL_LIMIT slots and experts. */
 #define TGO_ROUTE_SMALL_LIMIT 4096
 int tgo_route_small(const int64_t * slot_experts, int64_t tokens, int64_t top_k, int64_t num_experts, int64_t * row_index,
                     int64_t * slot_rows, int64_t * expert_indices, int32_t * expert_offsets, void * stream);
+
+/* Backward of the weighted return to tokens (tgo_moe_combine).
+ * tgo_invert_slots: row_token int64 [num_rows], row_weight fp32 [num_rows] = token and weight of the slot whose slot_rows
+ * entry names the row, -1 and 0 for a row that none names (at most one slot may name a row): what
+ * tgo_grouped_mmq_grad_input_weighted takes.
+ * tgo_slot_weight_grad: grad_weights fp32 [tokens, top_k] = dot(rows[slot_rows[t, j], :], grad_tokens[t, :]), fp32 sums of
+ * bf16 products in a fixed order; 0 for a slot outside the rows.  `features` is a multiple of 8.
+ * tgo_clear_uncovered_rows: zeros in the rows of rows_bf16 [num_rows, features] that lie in no valid group, which
+ * tgo_grouped_mmq_grad_input leaves unwritten.
+ * No counterpart in the reference, which leaves the combine and its gradient to the caller. */
+int tgo_invert_slots(const int64_t * slot_rows, const float * slot_weights, int64_t tokens, int64_t top_k, int64_t num_rows,
+                     int64_t * row_token, float * row_weight, void * stream);
+int tgo_slot_weight_grad(const void * rows_bf16, const void * grad_tokens_bf16, const int64_t * slot_rows, float * grad_weights,
+                         int64_t tokens, int64_t top_k, int64_t num_rows, int64_t features, void * stream);
+int tgo_clear_uncovered_rows(void * rows_bf16, int64_t num_rows, int64_t features, const int64_t * expert_indices,
+                             const int32_t * expert_offsets, int64_t num_experts, int64_t num_groups, void * stream);
 
 /* The row gather of the gathered entry points run backwards: the gradients of the sorted rows summed per token,
  *   output[t, :] = bf16( sum of rows[order[i], :] for starts[t] <= i < starts[t + 1] )      (t < tokens)
@@ -241,7 +265,7 @@ int tgo_rows_to_tokens(const void * rows_bf16, const int64_t * order, const int6
 /* Routing-weighted return from expert-sorted rows to tokens:
  *   output[t, :] = sum_j slot_weights[t, j] * rows[slot_rows[t, j], :]      (t < tokens, j < top_k)
  * rows bf16 [num_rows, features], slot_rows int64 [tokens, top_k] (the sorted row of each choice; a value
- * outside [0, num_rows) contributes nothing), slot_weights fp32 [tokens, top_k], output bf16
+ * outside [0, num_rows) contributes nothing), slot_weights fp32 [tokens, top_k] (NULL: ones), output bf16
  * [tokens, features].  Choices are accumulated in index order in fp32 and rounded once, so the result is
  * deterministic (no atomics).  `features` is a multiple of 8.  One pass over the rows replaces the caller-side
  * scale and index_add of a MoE layer.  No counterpart in the reference, which leaves this to the caller

@@ -1,0 +1,91 @@
+"""Kernels around the matrix products of a layer at the sizes where they can go wrong (-m gpu): the
+routing sort in one and in several workgroups, the gradient of the routing weights and the
+clearing of uncovered rows."""
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import f32, nrmse, random_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    import torch_ggml_ops
+    import synth
+
+    assert torch.cuda.is_available()
+    return torch_ggml_ops, synth
+
+
+@pytest.mark.parametrize("slots,experts", ((4096, 256), (4097, 257), (5000, 4096), (65 * 1024 + 3, 1025), (200_001, 255), (70_000, 1)))
+def test_route_in_several_workgroups(ops, slots, experts):
+    """Stable sort by expert with slots whose expert does not exist: those get row -1 and the rows behind the last are -1."""
+    tgo, _ = ops
+    flat = np.random.default_rng(slots).integers(-1, experts + 1, size=slots)
+    row_index, slot_rows, indices, offsets = tgo.route(torch.from_numpy(flat.reshape(slots, 1)).cuda(), experts)
+    valid = (flat >= 0) & (flat < experts)
+    order = np.argsort(np.where(valid, flat, experts), kind="stable")[: valid.sum()]
+    assert np.array_equal(row_index.cpu().numpy()[: order.size], order)
+    assert (row_index[order.size :] == -1).all()
+    expected = np.full(slots, -1)
+    expected[order] = np.arange(order.size)
+    assert np.array_equal(slot_rows.reshape(-1).cpu().numpy(), expected)
+    assert np.array_equal(offsets.cpu().numpy(), np.cumsum(np.bincount(flat[valid], minlength=experts)))
+    assert np.array_equal(indices.cpu().numpy(), np.arange(experts))
+
+
+@pytest.mark.parametrize("tokens,top_k,features", ((1, 1, 8), (5, 3, 520), (33, 8, 2048)))
+def test_routing_weight_gradient_and_inverse(ops, tokens, top_k, features):
+    tgo, _ = ops
+    num_rows = tokens * top_k
+    generator = np.random.default_rng(features)
+    slots = generator.permutation(num_rows + 2)[: tokens * top_k] - 1   # one slot may be -1 and one past the rows
+    slot_rows = torch.from_numpy(slots.reshape(tokens, top_k)).cuda()
+    rows, grad = random_bf16((num_rows, features), seed=1), random_bf16((tokens, features), seed=2)
+    weights = torch.rand(tokens, top_k, device="cuda")
+    actual = torch.ops.torch_ggml_ops.moe_combine_weight_grad.default(rows, grad, slot_rows)
+    present = (slots >= 0) & (slots < num_rows)
+    picked = rows.double()[torch.from_numpy(np.where(present, slots, 0)).cuda()].reshape(tokens, top_k, features)
+    expected = (picked * grad.double().unsqueeze(1)).sum(-1) * torch.from_numpy(present.reshape(tokens, top_k)).cuda()
+    torch.testing.assert_close(actual.double(), expected, rtol=1e-5, atol=1e-4)
+    token, weight = torch.ops.torch_ggml_ops.invert_slots.default(slot_rows, weights, num_rows)
+    expected_token, expected_weight = np.full(num_rows, -1), np.zeros(num_rows, dtype=np.float32)
+    for i in np.flatnonzero(present):
+        expected_token[slots[i]], expected_weight[slots[i]] = i // top_k, weights.cpu().numpy().reshape(-1)[i]
+    assert np.array_equal(token.cpu().numpy(), expected_token) and np.array_equal(weight.cpu().numpy(), expected_weight)
+
+
+@pytest.mark.parametrize("rows,offsets,experts", ((700, (3, 3, 255, 256, 600), (0, 1, 7, 2, 3)), (5, (5,), (0,)), (300, (400, 10), (0, 1))))
+def test_rows_outside_every_group_are_cleared(ops, rows, offsets, experts):
+    """Empty groups, groups of an expert that does not exist and groups that end behind the rows cover nothing."""
+    from torch_ggml_ops import _native
+
+    x = torch.ones(rows, 24, dtype=torch.bfloat16, device="cuda")
+    indices = torch.tensor(experts, dtype=torch.int64, device="cuda")
+    ends = torch.tensor(offsets, dtype=torch.int32, device="cuda")
+    _native.check(_native.lib.tgo_clear_uncovered_rows(
+        x.data_ptr(), rows, 24, indices.data_ptr(), ends.data_ptr(), 5, len(offsets), torch.cuda.current_stream().cuda_stream))
+    covered, begin = np.zeros(rows, dtype=bool), 0
+    for end, expert in zip(offsets, experts):
+        if begin < end <= rows and expert < 5:
+            covered[begin:end] = True
+        begin = end
+    assert np.array_equal(x.float().cpu().numpy(), np.broadcast_to(covered[:, None], (rows, 24)).astype(np.float32))
+
+
+def test_swiglu_with_slot_rows_equals_the_sorted_gradient(ops):
+    tgo, synth = ops
+    tokens, top_k, experts, k, n = 70, 3, 5, 512, 64
+    gate, up = (synth.random_packed_weight(12, (experts, n), k, seed=s).cuda() for s in (1, 2))
+    slot_experts = torch.from_numpy(np.random.default_rng(3).integers(0, experts, size=(tokens, top_k))).cuda()
+    row_index, slot_rows, indices, offsets = tgo.route(slot_experts, experts)
+    grads = []
+    for listed in (None, slot_rows):
+        hidden = random_bf16((tokens, k), seed=4).requires_grad_(True)
+        out = tgo.grouped_mmq_swiglu(hidden, gate, up, indices, offsets, 12, n, row_index, listed)
+        out.backward(random_bf16(out.shape, seed=5))
+        grads.append(hidden.grad)
+    assert nrmse(f32(grads[1]), f32(grads[0])) < 3e-3   # (the order of the fp32 sums of a token's rows)

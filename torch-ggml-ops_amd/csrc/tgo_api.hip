@@ -477,7 +477,7 @@ static int grouped_forward(const void * input_bf16, const int64_t * row_index, i
     const tgo::Q8Workspace view = tgo::q8_workspace_view(workspace, rows, in_features, gemv, operand_kind);
     void * task_base = static_cast<char *>(workspace) + (tgo::q8_workspace_bytes(rows, in_features) + 15) / 16 * 16;
     const int row_tile = gemv ? tgo::GEMV_ROW_TILE : tgo::forward_row_tile(quant_type, view.operand_kind());
-    const auto launch = fused ? tgo::launch_mmq_forward_swiglu : gemv ? tgo::launch_mmq_gemv : tgo::launch_mmq_forward;
+        const auto launch = fused ? tgo::launch_mmq_forward_swiglu : gemv ? tgo::launch_mmq_gemv : tgo::launch_mmq_forward;
     const tgo::TaskList tasks = tgo::task_list_view(task_base, rows, num_groups, row_tile);
 
     // the quantizer writes the tile-task list on the side; the MFMA kernel runs a task of at most 32 rows in
@@ -585,8 +585,8 @@ int tgo_moe_combine(const void * rows_bf16, const int64_t * slot_rows, const flo
     }
     TGO_TRY(check_pointer(rows_bf16, "rows"));
     TGO_TRY(check_pointer(output_bf16, "output"));
-    if (slot_rows == nullptr || slot_weights == nullptr) {
-        return fail(TGO_ERR_INVALID, "slot_rows and slot_weights must not be null");
+    if (slot_rows == nullptr) {
+        return fail(TGO_ERR_INVALID, "slot_rows must not be null");
     }
     return check_hip(tgo::launch_moe_combine(static_cast<const uint16_t *>(rows_bf16), slot_rows, slot_weights,
                                              static_cast<uint16_t *>(output_bf16), static_cast<int>(tokens),
@@ -610,10 +610,90 @@ int tgo_route_small(const int64_t * slot_experts, int64_t tokens, int64_t top_k,
         expert_offsets == nullptr) {
         return fail(TGO_ERR_INVALID, "slot_experts, row_index, slot_rows, expert_indices and expert_offsets must not be null");
     }
-    return check_hip(tgo::launch_route_small(slot_experts, static_cast<int>(tokens * top_k), static_cast<int>(top_k),
-                                             static_cast<int>(num_experts), row_index, slot_rows, expert_indices,
-                                             expert_offsets, static_cast<hipStream_t>(stream)),
-                     "route_small launch");
+    return tgo_route(slot_experts, tokens, top_k, num_experts, row_index, slot_rows, expert_indices, expert_offsets, nullptr, stream);
+}
+
+int64_t tgo_route_workspace_bytes(int64_t slots, int64_t num_experts) {
+    if (slots <= 0 || num_experts <= 0) {
+        return 0;
+    }
+    const int blocks = tgo::route_blocks(slots);
+    return blocks > 1 ? blocks * num_experts * static_cast<int64_t>(sizeof(int32_t)) : 0;
+}
+
+int tgo_route(const int64_t * slot_experts, int64_t tokens, int64_t top_k, int64_t num_experts, int64_t * row_index,
+              int64_t * slot_rows, int64_t * expert_indices, int32_t * expert_offsets, void * workspace, void * stream) {
+    if (tokens <= 0 || top_k <= 0 || num_experts <= 0) {
+        return fail(TGO_ERR_INVALID, "tokens, top_k and num_experts must be positive");
+    }
+    if (tokens > TGO_ROUTE_SLOT_LIMIT || top_k > TGO_ROUTE_SLOT_LIMIT || tokens * top_k > TGO_ROUTE_SLOT_LIMIT ||
+        num_experts > TGO_ROUTE_EXPERT_LIMIT) {
+        return fail(TGO_ERR_INVALID, "tgo_route sorts at most %d slots over at most %d experts; got %lld x %lld over %lld",
+                    TGO_ROUTE_SLOT_LIMIT, TGO_ROUTE_EXPERT_LIMIT, static_cast<long long>(tokens),
+                    static_cast<long long>(top_k), static_cast<long long>(num_experts));
+    }
+    if (slot_experts == nullptr || row_index == nullptr || slot_rows == nullptr || expert_indices == nullptr ||
+        expert_offsets == nullptr) {
+        return fail(TGO_ERR_INVALID, "slot_experts, row_index, slot_rows, expert_indices and expert_offsets must not be null");
+    }
+    if (workspace == nullptr && tgo_route_workspace_bytes(tokens * top_k, num_experts) > 0) {
+        return fail(TGO_ERR_INVALID, "workspace must not be null for this many slots");
+    }
+    return check_hip(tgo::launch_route(slot_experts, tokens * top_k, static_cast<int>(top_k), static_cast<int>(num_experts),
+                                       static_cast<int32_t *>(workspace), row_index, slot_rows, expert_indices, expert_offsets,
+                                       static_cast<hipStream_t>(stream)),
+                     "route launch");
+}
+
+int tgo_invert_slots(const int64_t * slot_rows, const float * slot_weights, int64_t tokens, int64_t top_k, int64_t num_rows,
+                     int64_t * row_token, float * row_weight, void * stream) {
+    if (tokens <= 0 || top_k <= 0 || num_rows <= 0) {
+        return fail(TGO_ERR_INVALID, "tokens, top_k and num_rows must be positive");
+    }
+    if (tokens > INT_LIMIT || top_k > INT_LIMIT || tokens * top_k > INT_LIMIT || num_rows > INT_LIMIT) {
+        return fail(TGO_ERR_INVALID, "a dimension exceeds the kernel limit");
+    }
+    if (slot_rows == nullptr || slot_weights == nullptr || row_token == nullptr || row_weight == nullptr) {
+        return fail(TGO_ERR_INVALID, "slot_rows, slot_weights, row_token and row_weight must not be null");
+    }
+    return check_hip(tgo::launch_invert_slots(slot_rows, slot_weights, tokens * top_k, static_cast<int>(top_k), num_rows,
+                                              row_token, row_weight, static_cast<hipStream_t>(stream)),
+                     "invert_slots launch");
+}
+
+int tgo_slot_weight_grad(const void * rows_bf16, const void * grad_tokens_bf16, const int64_t * slot_rows, float * grad_weights,
+                         int64_t tokens, int64_t top_k, int64_t num_rows, int64_t features, void * stream) {
+    if (tokens <= 0 || top_k <= 0 || num_rows <= 0) {
+        return fail(TGO_ERR_INVALID, "tokens, top_k and num_rows must be positive");
+    }
+    if (features <= 0 || features % 8 != 0) {
+        return fail(TGO_ERR_INVALID, "features must be a positive multiple of 8; got %lld", static_cast<long long>(features));
+    }
+    if (tokens > INT_LIMIT || top_k > INT_LIMIT || tokens * top_k > INT_LIMIT || features > INT_LIMIT || num_rows > INT_LIMIT) {
+        return fail(TGO_ERR_INVALID, "a dimension exceeds the kernel limit");
+    }
+    TGO_TRY(check_pointer(rows_bf16, "rows"));
+    TGO_TRY(check_pointer(grad_tokens_bf16, "grad_tokens"));
+    if (slot_rows == nullptr || grad_weights == nullptr) {
+        return fail(TGO_ERR_INVALID, "slot_rows and grad_weights must not be null");
+    }
+    return check_hip(tgo::launch_slot_weight_grad(static_cast<const uint16_t *>(rows_bf16),
+                                                  static_cast<const uint16_t *>(grad_tokens_bf16), slot_rows, grad_weights,
+                                                  tokens * top_k, static_cast<int>(top_k), num_rows,
+                                                  static_cast<int>(features), static_cast<hipStream_t>(stream)),
+                     "slot_weight_grad launch");
+}
+
+int tgo_clear_uncovered_rows(void * rows_bf16, int64_t num_rows, int64_t features, const int64_t * expert_indices,
+                             const int32_t * expert_offsets, int64_t num_experts, int64_t num_groups, void * stream) {
+    TGO_TRY(check_grouped(num_experts, num_groups, expert_indices, expert_offsets));
+    if (rows_bf16 == nullptr || num_rows <= 0 || features <= 0 || num_rows > INT_LIMIT || features > INT_LIMIT) {
+        return fail(TGO_ERR_INVALID, "rows must not be null and its dimensions positive and below 2^31");
+    }
+    return check_hip(tgo::launch_clear_uncovered(static_cast<uint16_t *>(rows_bf16), num_rows, static_cast<int>(features),
+                                                 expert_indices, expert_offsets, static_cast<int>(num_groups),
+                                                 static_cast<int>(num_experts), static_cast<hipStream_t>(stream)),
+                     "clear_uncovered launch");
 }
 
 int tgo_rows_to_tokens(const void * rows_bf16, const int64_t * order, const int64_t * starts, void * output_bf16,

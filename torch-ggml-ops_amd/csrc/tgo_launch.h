@@ -236,9 +236,26 @@ hipError_t launch_quantize_q8_1(const uint16_t * input, const Q8Workspace & ws, 
 // up_then_activated[i] = swiglu(gate[i], up_then_activated[i]) over `count` bf16 values (timed with the forward kernels).
 hipError_t launch_swiglu_rows(const uint16_t * gate, const uint16_t * up, uint16_t * activated, int64_t count,
                               hipStream_t stream);   // (`activated` may be `up`)
-// The (token, choice) slots of a small batch sorted by expert in one launch (at most 4096 slots and experts).
-hipError_t launch_route_small(const int64_t * slot_experts, int slots, int top_k, int num_experts, int64_t * row_index,
-                              int64_t * slot_rows, int64_t * expert_indices, int32_t * expert_offsets, hipStream_t stream);
+// The (token, choice) slots sorted by expert: one launch up to ROUTE_SINGLE_SLOTS slots, above that two, with room for
+// route_blocks(slots) * num_experts counts in `counts` (nullptr otherwise).
+constexpr int64_t ROUTE_SINGLE_SLOTS = 4096;
+constexpr int ROUTE_MAX_BLOCKS = 64;
+constexpr int ROUTE_EXPERT_LIMIT = 4096;
+constexpr int64_t ROUTE_SLOT_LIMIT = int64_t{1} << 22;   // (a wave counts its slots of one expert in 16 bits)
+int route_blocks(int64_t slots);
+hipError_t launch_route(const int64_t * slot_experts, int64_t slots, int top_k, int num_experts, int32_t * counts,
+                        int64_t * row_index, int64_t * slot_rows, int64_t * expert_indices, int32_t * expert_offsets,
+                        hipStream_t stream);
+// row_token[r], row_weight[r]: token and weight of the slot that names row r (-1 and 0 when none does).
+hipError_t launch_invert_slots(const int64_t * slot_rows, const float * slot_weights, int64_t slots, int top_k,
+                               int64_t num_rows, int64_t * row_token, float * row_weight, hipStream_t stream);
+// grad_weights[slot] = dot(rows[slot_rows[slot], :], grad_tokens[slot / top_k, :]); `features` is a multiple of 8.
+hipError_t launch_slot_weight_grad(const uint16_t * rows, const uint16_t * grad_tokens, const int64_t * slot_rows,
+                                   float * grad_weights, int64_t slots, int top_k, int64_t num_rows, int features,
+                                   hipStream_t stream);
+// Zeros in the rows that lie in no valid group.
+hipError_t launch_clear_uncovered(uint16_t * rows, int64_t num_rows, int features, const int64_t * expert_indices,
+                                  const int32_t * expert_offsets, int num_groups, int num_experts, hipStream_t stream);
 // out[t, :] = sum of rows[order[i], :] over i in [starts[t], starts[t + 1]), in list order (fp32, one rounding).
 hipError_t launch_rows_to_tokens(const uint16_t * rows, const int64_t * order, const int64_t * starts, uint16_t * out,
                                  int tokens, int64_t num_rows, int features, hipStream_t stream);
@@ -253,7 +270,8 @@ hipError_t launch_q8_unpack(const Q8Workspace & ws, int8_t * q, float * d, float
                             int64_t in_features, hipStream_t stream);
 
 // out[t, :] = sum_j slot_weights[t, j] * rows[slot_rows[t, j], :] (bf16 rows, fp32 accumulation in choice order,
-// one rounding); a slot whose row is outside [0, num_rows) contributes nothing.  `features` is a multiple of 8.
+// one rounding); a slot whose row is outside [0, num_rows) contributes nothing.  `features` is a multiple of 8;
+// `slot_weights` may be null: weights of one.
 hipError_t launch_moe_combine(const uint16_t * rows, const int64_t * slot_rows, const float * slot_weights,
                               uint16_t * out, int tokens, int top_k, int64_t num_rows, int features,
                               hipStream_t stream);

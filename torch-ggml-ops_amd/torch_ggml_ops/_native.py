@@ -53,6 +53,12 @@ lib.tgo_grouped_mmq_swiglu.argtypes = [_p, _p, _i64, _p, _p, _p, _p, _p, _p, _p,
 lib.tgo_swiglu_rows.argtypes = [_p, _p, _p, _i64, _p]
 lib.tgo_swiglu_backward.argtypes = [_p, _p, _p, _p, _p, _p, _i64, _p]
 lib.tgo_route_small.argtypes = [_p, _i64, _i64, _i64, _p, _p, _p, _p, _p]
+lib.tgo_route.argtypes = [_p, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p]
+lib.tgo_route_workspace_bytes.argtypes = [_i64, _i64]
+lib.tgo_route_workspace_bytes.restype = _i64
+lib.tgo_invert_slots.argtypes = [_p, _p, _i64, _i64, _i64, _p, _p, _p]
+lib.tgo_slot_weight_grad.argtypes = [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _p]
+lib.tgo_clear_uncovered_rows.argtypes = [_p, _i64, _i64, _p, _p, _i64, _i64, _p]
 lib.tgo_rows_to_tokens.argtypes = [_p, _p, _p, _p, _i64, _i64, _i64, _p]
 lib.tgo_moe_combine.argtypes = [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _p]
 lib.tgo_grouped_mmq_grad_input.argtypes = [_p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _int, _p]
@@ -92,6 +98,11 @@ EXPORTS = (
     "tgo_swiglu_rows",
     "tgo_swiglu_backward",
     "tgo_route_small",
+    "tgo_route",
+    "tgo_route_workspace_bytes",
+    "tgo_invert_slots",
+    "tgo_slot_weight_grad",
+    "tgo_clear_uncovered_rows",
     "tgo_rows_to_tokens",
     "tgo_moe_combine",
     "tgo_grouped_mmq_grad_input",

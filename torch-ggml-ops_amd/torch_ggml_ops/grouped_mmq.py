@@ -99,7 +99,7 @@ def _grad_input(
         if (second[0], second[2], second[3], second[4], second[5]) != (rows, out_features, experts, groups, bytes_per_expert):
             raise RuntimeError("paired grouped MMQ backward tensors must have identical physical geometry")
     with _native.on_device(first_grad.device):
-        grad_input = (first_grad.new_zeros if zero_fill else first_grad.new_empty)((rows, in_features))
+        grad_input = first_grad.new_empty((rows, in_features))
         sources = 2 if second_weight is not None else 1
         workspace = first_grad.new_empty(
             (_native.lib.tgo_grad_workspace_bytes(rows, out_features, groups, sources),), dtype=torch.uint8
@@ -117,6 +117,13 @@ def _grad_input(
                 rows, out_features, in_features, experts, groups, int(quant_type), _stream(first_grad),
             )
         )
+        if zero_fill:
+            _native.check(
+                _native.lib.tgo_clear_uncovered_rows(
+                    grad_input.data_ptr(), rows, in_features, expert_indices.data_ptr(), expert_offsets.data_ptr(), experts,
+                    groups, _stream(first_grad),
+                )
+            )
     return grad_input
 
 

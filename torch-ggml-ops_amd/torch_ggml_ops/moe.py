@@ -75,6 +75,55 @@ def _combine_fake(rows, slot_rows, slot_weights):
     return rows.new_empty((slot_rows.shape[0], rows.shape[1]))
 
 
+torch.library.define(
+    "torch_ggml_ops::moe_combine_weight_grad", "(Tensor rows, Tensor grad_tokens, Tensor slot_rows) -> Tensor"
+)
+torch.library.define(
+    "torch_ggml_ops::invert_slots", "(Tensor slot_rows, Tensor slot_weights, int num_rows) -> (Tensor, Tensor)"
+)
+
+
+@torch.library.impl("torch_ggml_ops::moe_combine_weight_grad", "CUDA")
+def _weight_grad_device(rows, grad_tokens, slot_rows):
+    """Gradient of the routing weights of ``moe_combine``: the dot product of each slot's row with its token's gradient."""
+    tokens, top_k = slot_rows.shape
+    grad_weights = torch.empty((tokens, top_k), dtype=torch.float32, device=rows.device)
+    with _native.on_device(rows.device):
+        _native.check(
+            _native.lib.tgo_slot_weight_grad(
+                rows.data_ptr(), grad_tokens.data_ptr(), slot_rows.data_ptr(), grad_weights.data_ptr(), tokens, top_k,
+                rows.shape[0], rows.shape[1], _native.stream_of(rows.device),
+            )
+        )
+    return grad_weights
+
+
+@torch.library.register_fake("torch_ggml_ops::moe_combine_weight_grad")
+def _weight_grad_fake(rows, grad_tokens, slot_rows):
+    return slot_rows.new_empty(slot_rows.shape, dtype=torch.float32)
+
+
+@torch.library.impl("torch_ggml_ops::invert_slots", "CUDA")
+def _invert_slots_device(slot_rows, slot_weights, num_rows):
+    """Token and routing weight of every expert-sorted row; -1 and 0 for a row that no slot names."""
+    tokens, top_k = slot_rows.shape
+    row_token = torch.empty(num_rows, dtype=torch.int64, device=slot_rows.device)
+    row_weight = torch.empty(num_rows, dtype=torch.float32, device=slot_rows.device)
+    with _native.on_device(slot_rows.device):
+        _native.check(
+            _native.lib.tgo_invert_slots(
+                slot_rows.data_ptr(), slot_weights.data_ptr(), tokens, top_k, num_rows, row_token.data_ptr(),
+                row_weight.data_ptr(), _native.stream_of(slot_rows.device),
+            )
+        )
+    return row_token, row_weight
+
+
+@torch.library.register_fake("torch_ggml_ops::invert_slots")
+def _invert_slots_fake(slot_rows, slot_weights, num_rows):
+    return slot_rows.new_empty((num_rows,)), slot_rows.new_empty((num_rows,), dtype=torch.float32)
+
+
 def _setup_combine_context(ctx, inputs, output) -> None:
     rows, slot_rows, slot_weights = inputs
     ctx.num_rows = rows.shape[0]
@@ -83,20 +132,19 @@ def _setup_combine_context(ctx, inputs, output) -> None:
 
 def _combine_backward(ctx, grad_output):
     rows, slot_rows, slot_weights = ctx.saved_tensors
-    tokens, top_k = slot_rows.shape
-    flat = slot_rows.reshape(-1)
-    present = (flat >= 0) & (flat < ctx.num_rows)
-    safe = flat.clamp(0, ctx.num_rows - 1)
-    grad_per_slot = grad_output.repeat_interleave(top_k, dim=0)
+    _tokens, top_k = slot_rows.shape
     grad_rows = grad_weights = None
     if ctx.needs_input_grad[0]:
+        flat = slot_rows.reshape(-1)
+        present = (flat >= 0) & (flat < ctx.num_rows)
+        safe = flat.clamp(0, ctx.num_rows - 1)
+        grad_per_slot = grad_output.repeat_interleave(top_k, dim=0)
         scaled = (grad_per_slot.float() * (slot_weights.reshape(-1, 1) * present.unsqueeze(1))).to(grad_output.dtype)
         grad_rows = grad_output.new_zeros((ctx.num_rows, grad_output.shape[1]))
         # every row belongs to at most one slot, so this is a plain scatter, not a reduction
         grad_rows.index_add_(0, safe, scaled)
     if ctx.needs_input_grad[2]:
-        products = (rows.index_select(0, safe).float() * grad_per_slot.float()).sum(dim=1)
-        grad_weights = (products * present).reshape(tokens, top_k)
+        grad_weights = torch.ops.torch_ggml_ops.moe_combine_weight_grad.default(rows, grad_output.contiguous(), slot_rows)
     return grad_rows, None, grad_weights
 
 
@@ -191,29 +239,17 @@ def _grouped_combine_backward(ctx, grad_output, grad_rows):
     packed_weight, expert_indices, expert_offsets, slot_rows, slot_weights, rows = ctx.saved_tensors
     if grad_output is None:
         return None, None, None, None, None, None, None, None
-    tokens, top_k = slot_rows.shape
-    flat = slot_rows.reshape(-1)
-    present = (flat >= 0) & (flat < ctx.num_rows)
-    safe = flat.clamp(0, ctx.num_rows - 1)
     grad_output = grad_output.contiguous()
     grad_input = grad_weights = None
     if ctx.needs_input_grad[0]:
         # the inverse of slot_rows: token and routing weight of every expert-sorted row (rows that no slot names
-        # keep token -1, i.e. a zero cotangent); slots outside the rows are sent to a spare entry
-        spare = ctx.num_rows
-        target = torch.where(present, safe, torch.full_like(safe, spare))
-        row_token = torch.full((ctx.num_rows + 1,), -1, dtype=torch.int64, device=flat.device)
-        row_token[target] = torch.arange(tokens, device=flat.device).repeat_interleave(top_k)
-        row_weight = torch.zeros((ctx.num_rows + 1,), dtype=torch.float32, device=flat.device)
-        row_weight[target] = slot_weights.reshape(-1)
+        # have token -1, i.e. a zero cotangent)
+        row_token, row_weight = torch.ops.torch_ggml_ops.invert_slots.default(slot_rows, slot_weights, ctx.num_rows)
         grad_input = torch.ops.torch_ggml_ops.grouped_mmq_grad_input_weighted.default(
-            grad_output, row_token[:spare].contiguous(), row_weight[:spare].contiguous(), packed_weight,
-            expert_indices, expert_offsets, ctx.quant_type, ctx.in_features,
+            grad_output, row_token, row_weight, packed_weight, expert_indices, expert_offsets, ctx.quant_type, ctx.in_features
         )
     if ctx.needs_input_grad[5]:
-        grad_per_slot = grad_output.repeat_interleave(top_k, dim=0)
-        products = (rows.index_select(0, safe).float() * grad_per_slot.float()).sum(dim=1)
-        grad_weights = (products * present).reshape(tokens, top_k)
+        grad_weights = torch.ops.torch_ggml_ops.moe_combine_weight_grad.default(rows, grad_output, slot_rows)
     return grad_input, None, None, None, None, grad_weights, None, None
 
 
@@ -250,19 +286,20 @@ def grouped_mmq_combine(
     return output
 
 
-ROUTE_SMALL_LIMIT = 4096   # TGO_ROUTE_SMALL_LIMIT
+ROUTE_SLOT_LIMIT = 4194304   # TGO_ROUTE_SLOT_LIMIT
+ROUTE_EXPERT_LIMIT = 4096    # TGO_ROUTE_EXPERT_LIMIT
 
 
 torch.library.define(
-    "torch_ggml_ops::route_small",
+    "torch_ggml_ops::route",
     "(Tensor slot_experts, int num_experts) -> (Tensor, Tensor, Tensor, Tensor)",
 )
 
 
-@torch.library.impl("torch_ggml_ops::route_small", "CUDA")
-def _route_small_device(slot_experts, num_experts):
-    """``route`` for a decode-sized batch as one kernel (``tgo_route_small``) instead of a sort and a dozen small
-    tensor operations, which at that size cost more than the layer's own launches.  Same results."""
+@torch.library.impl("torch_ggml_ops::route", "CUDA")
+def _route_device(slot_experts, num_experts):
+    """``route`` as one or two kernels (``tgo_route``) instead of a sort and a dozen tensor operations, which cost more
+    than a layer's own launches at decode sizes and a third of its time in a prefill.  Same results."""
     slot_experts = slot_experts.to(torch.int64).contiguous()
     tokens, top_k = slot_experts.shape
     device = slot_experts.device
@@ -270,18 +307,21 @@ def _route_small_device(slot_experts, num_experts):
     slot_rows = torch.empty((tokens, top_k), dtype=torch.int64, device=device)
     expert_indices = torch.empty(num_experts, dtype=torch.int64, device=device)
     expert_offsets = torch.empty(num_experts, dtype=torch.int32, device=device)
+    workspace_bytes = _native.lib.tgo_route_workspace_bytes(tokens * top_k, num_experts)
+    workspace = torch.empty(workspace_bytes, dtype=torch.uint8, device=device) if workspace_bytes > 0 else None
     with _native.on_device(device):
         _native.check(
-            _native.lib.tgo_route_small(
+            _native.lib.tgo_route(
                 slot_experts.data_ptr(), tokens, top_k, num_experts, row_index.data_ptr(), slot_rows.data_ptr(),
-                expert_indices.data_ptr(), expert_offsets.data_ptr(), _native.stream_of(device),
+                expert_indices.data_ptr(), expert_offsets.data_ptr(), None if workspace is None else workspace.data_ptr(),
+                _native.stream_of(device),
             )
         )
     return row_index, slot_rows, expert_indices, expert_offsets
 
 
-@torch.library.register_fake("torch_ggml_ops::route_small")
-def _route_small_fake(slot_experts, num_experts):
+@torch.library.register_fake("torch_ggml_ops::route")
+def _route_fake(slot_experts, num_experts):
     tokens, top_k = slot_experts.shape
     return (
         slot_experts.new_empty((tokens * top_k,), dtype=torch.int64),
@@ -299,8 +339,8 @@ def route(slot_experts: torch.Tensor, num_experts: int):
     group per expert (experts without rows are empty groups, which the operators skip).
     """
     tokens, top_k = slot_experts.shape
-    if slot_experts.is_cuda and 0 < tokens * top_k <= ROUTE_SMALL_LIMIT and 0 < num_experts <= ROUTE_SMALL_LIMIT:
-        return torch.ops.torch_ggml_ops.route_small.default(slot_experts, int(num_experts))
+    if slot_experts.is_cuda and 0 < tokens * top_k <= ROUTE_SLOT_LIMIT and 0 < num_experts <= ROUTE_EXPERT_LIMIT:
+        return torch.ops.torch_ggml_ops.route.default(slot_experts, int(num_experts))
     flat = slot_experts.reshape(-1)
     order = torch.argsort(flat, stable=True)
     row_index = torch.div(order, top_k, rounding_mode="floor")
@@ -334,7 +374,8 @@ def moe_layer(
     experts = gate_weight.shape[0]
     row_index, slot_rows, expert_indices, expert_offsets = route(slot_experts, experts)
     activated = grouped_mmq_swiglu(
-        hidden, gate_weight, up_weight, expert_indices, expert_offsets, gate_up_type, intermediate_features, row_index
+        hidden, gate_weight, up_weight, expert_indices, expert_offsets, gate_up_type, intermediate_features, row_index,
+        slot_rows,
     )
     return grouped_mmq_combine(
         activated, down_weight, expert_indices, expert_offsets, slot_rows, slot_weights, down_type, hidden.shape[1]

@@ -27,7 +27,7 @@ from .gathered import _rows_grad_input, _scatter_to_tokens
 torch.library.define(
     "torch_ggml_ops::grouped_mmq_swiglu",
     "(Tensor input, Tensor? row_index, Tensor gate_packed_weight, Tensor up_packed_weight, Tensor expert_indices, "
-    "Tensor expert_offsets, int quant_type, int out_features) -> (Tensor, Tensor, Tensor)",
+    "Tensor expert_offsets, int quant_type, int out_features, Tensor? slot_rows=None) -> (Tensor, Tensor, Tensor)",
 )
 
 
@@ -39,9 +39,15 @@ def _keeps_up(quant_type: int, rows: int, out_features: int) -> bool:
 
 @torch.library.impl("torch_ggml_ops::grouped_mmq_swiglu", "CUDA")
 def _swiglu_device(
-    input, row_index, gate_packed_weight, up_packed_weight, expert_indices, expert_offsets, quant_type, out_features
+    input, row_index, gate_packed_weight, up_packed_weight, expert_indices, expert_offsets, quant_type, out_features,
+    slot_rows=None,
 ):
     rows = input.shape[0] if row_index is None else row_index.shape[0]
+    if slot_rows is not None:
+        if row_index is None or slot_rows.dim() != 2 or slot_rows.shape[0] != input.shape[0]:
+            raise RuntimeError("slot_rows goes with row_index and must have shape [tokens, top_k]")
+        if slot_rows.dtype != torch.int64 or slot_rows.device != input.device or not slot_rows.is_contiguous():
+            raise RuntimeError("slot_rows must be a contiguous torch.int64 tensor on the input's device")
     if _keeps_up(quant_type, rows, out_features):
         # what tgo_grouped_mmq_swiglu does for such a call, with the activation written beside the up projection
         # instead of over it
@@ -66,7 +72,8 @@ def _swiglu_device(
 
 @torch.library.register_fake("torch_ggml_ops::grouped_mmq_swiglu")
 def _swiglu_fake(
-    input, row_index, gate_packed_weight, up_packed_weight, expert_indices, expert_offsets, quant_type, out_features
+    input, row_index, gate_packed_weight, up_packed_weight, expert_indices, expert_offsets, quant_type, out_features,
+    slot_rows=None,
 ):
     rows = input.shape[0] if row_index is None else row_index.shape[0]
     kept = rows if _keeps_up(quant_type, rows, out_features) else 0
@@ -91,21 +98,38 @@ def _activation_backward(gate, up, grad_activated, grad_gate):
     return d_gate, d_up
 
 
+def _sum_slots(grad_rows, slot_rows):
+    """``out[t] = sum_j grad_rows[slot_rows[t, j]]``, fp32 sums in choice order, one rounding."""
+    tokens, top_k = slot_rows.shape
+    out = grad_rows.new_empty((tokens, grad_rows.shape[1]))
+    with _native.on_device(grad_rows.device):
+        _native.check(
+            _native.lib.tgo_moe_combine(
+                grad_rows.data_ptr(), slot_rows.data_ptr(), None, out.data_ptr(), tokens, top_k, grad_rows.shape[0],
+                grad_rows.shape[1], _native.stream_of(grad_rows.device),
+            )
+        )
+    return out
+
+
 def _setup_context(ctx, inputs, output) -> None:
-    input, row_index, gate_weight, up_weight, expert_indices, expert_offsets, quant_type, out_features = inputs
+    input, row_index, gate_weight, up_weight, expert_indices, expert_offsets, quant_type, out_features, slot_rows = inputs
+    # (the gate and up outputs rarely get a gradient of their own: without this the engine would hand the backward zero
+    # tensors of their size)
+    ctx.set_materialize_grads(False)
     ctx.quant_type, ctx.out_features = quant_type, out_features
     ctx.tokens, ctx.in_features = input.shape
     ctx.gathered = row_index is not None
     if ctx.needs_input_grad[0]:
         ctx.save_for_backward(
-            input, row_index, gate_weight, up_weight, expert_indices, expert_offsets, output[1], output[2]
+            input, row_index, gate_weight, up_weight, expert_indices, expert_offsets, output[1], output[2], slot_rows
         )
 
 
 def _backward(ctx, grad_activated, grad_gate, grad_up):
     grad_input = None
     if ctx.needs_input_grad[0] and (grad_activated is not None or grad_gate is not None or grad_up is not None):
-        input, row_index, gate_weight, up_weight, expert_indices, expert_offsets, gate, up = ctx.saved_tensors
+        input, row_index, gate_weight, up_weight, expert_indices, expert_offsets, gate, up, slot_rows = ctx.saved_tensors
         d_gate = grad_gate
         d_up = grad_up if up.shape[0] > 0 else None   # (the third output is a placeholder when the up projection is not kept)
         if grad_activated is not None:
@@ -125,8 +149,12 @@ def _backward(ctx, grad_activated, grad_gate, grad_up):
             grad_rows = _rows_grad_input(
                 d_gate, None, gate_weight, None, expert_indices, expert_offsets, ctx.quant_type, ctx.in_features
             )
-        grad_input = _scatter_to_tokens(grad_rows, row_index, ctx.tokens) if ctx.gathered else grad_rows
-    return grad_input, None, None, None, None, None, None, None
+        if slot_rows is not None:
+            # the rows of each token are listed already: their sum is the combine with weights of one
+            grad_input = _sum_slots(grad_rows, slot_rows)
+        else:
+            grad_input = _scatter_to_tokens(grad_rows, row_index, ctx.tokens) if ctx.gathered else grad_rows
+    return grad_input, None, None, None, None, None, None, None, None
 
 
 torch.library.register_autograd("torch_ggml_ops::grouped_mmq_swiglu", _backward, setup_context=_setup_context)
@@ -141,15 +169,18 @@ def grouped_mmq_swiglu(
     quant_type: int,
     out_features: int,
     row_index: Optional[torch.Tensor] = None,
+    slot_rows: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
     """``silu(gate) * up`` of the grouped gate/up pair, ``[rows, out_features]`` bf16.
 
     ``input`` holds expert-sorted rows, or token rows when ``row_index`` (the token of each sorted row) is given.
+    ``slot_rows`` (int64 ``[tokens, top_k]``, as ``route`` returns it with ``row_index``) lists the rows of each token for
+    the gradient, which otherwise sorts ``row_index`` to find them.
     Rows that no valid group covers are left uninitialised, as for ``grouped_mmq``.
     """
     activated, _gate, _up = torch.ops.torch_ggml_ops.grouped_mmq_swiglu.default(
         input, row_index, gate_packed_weight, up_packed_weight, expert_indices, expert_offsets,
-        int(quant_type), int(out_features),
+        int(quant_type), int(out_features), slot_rows,
     )
     return activated
 
