@@ -250,6 +250,21 @@ int tgo_slot_weight_grad(const void * rows_bf16, const void * grad_tokens_bf16, 
 int tgo_clear_uncovered_rows(void * rows_bf16, int64_t num_rows, int64_t features, const int64_t * expert_indices,
                              const int32_t * expert_offsets, int64_t num_experts, int64_t num_groups, void * stream);
 
+/* Mean cross-entropy of the head's logits against `targets` (int64 [rows]) over the rows whose target is not ignore_index,
+ * and with grad_hidden_bf16 [rows, in_features] set the gradient of that mean with respect to hidden_bf16, computed
+ * chunk_rows rows at a time (one chunk of logits exists at a time): the forward product, two passes that form the softmax
+ * statistics and write (softmax - one_hot) / count as the packed cotangent, and the grad-input product.  loss: fp32 [1].
+ * A target outside [0, out_features) that is not ignored makes the loss and its row's gradient NaN.
+ * `workspace`: tgo_lm_head_workspace_bytes (-1 for invalid sizes); `gradient` says whether grad_hidden will be set.
+ * The schedule of the reference's training code (docs/mmq_fwd_optimization.md:293), which has no such function.
+ * tgo_scale_bf16: output[i] = bf16(input[i] * factor[0]), `count` a multiple of 8 (the incoming gradient of the loss). */
+int64_t tgo_lm_head_workspace_bytes(int64_t rows, int64_t in_features, int64_t out_features, int64_t chunk_rows, int quant_type,
+                                    int gradient);
+int tgo_lm_head_loss(const void * hidden_bf16, const void * packed, const int64_t * targets, float * loss, void * grad_hidden_bf16,
+                     void * workspace, int64_t rows, int64_t in_features, int64_t out_features, int64_t chunk_rows,
+                     int64_t ignore_index, int quant_type, void * stream);
+int tgo_scale_bf16(const void * input_bf16, const float * factor, void * output_bf16, int64_t count, void * stream);
+
 /* The row gather of the gathered entry points run backwards: the gradients of the sorted rows summed per token,
  *   output[t, :] = bf16( sum of rows[order[i], :] for starts[t] <= i < starts[t + 1] )      (t < tokens)
  * rows bf16 [num_rows, features]; order int64 [num_rows] lists the sorted rows token by token (a stable sort of the

@@ -1,12 +1,12 @@
-"""Kernels around the matrix products of a layer at the sizes where they can go wrong (-m gpu): the
-routing sort in one and in several workgroups, the gradient of the routing weights and the
-clearing of uncovered rows."""
+"""Kernels around the matrix products of a layer and of the loss at the sizes where they can go wrong (-m gpu): the
+routing sort in one and in several workgroups, the gradient of the routing weights, the clearing of uncovered rows, and
+the loss of a chunk whose vocabulary is no multiple of a piece, a span or a tile."""
 
 import numpy as np
 import pytest
 import torch
 
-from helpers import f32, nrmse, random_bf16
+from helpers import QTYPES, f32, nrmse, random_bf16
 
 pytestmark = pytest.mark.gpu
 
@@ -89,3 +89,25 @@ def test_swiglu_with_slot_rows_equals_the_sorted_gradient(ops):
         out.backward(random_bf16(out.shape, seed=5))
         grads.append(hidden.grad)
     assert nrmse(f32(grads[1]), f32(grads[0])) < 3e-3   # (the order of the fp32 sums of a token's rows)
+
+
+@pytest.mark.parametrize("qname,rows,vocabulary,chunk", (("Q6_K", 70, 8195, 64), ("Q4_K", 33, 1001, 32), ("Q5_K", 3, 40, 256), ("Q6_K", 300, 33000, 256)))
+def test_loss_of_ragged_vocabularies(ops, qname, rows, vocabulary, chunk):
+    tgo, synth = ops
+    qtype, k = QTYPES[qname], 256
+    weight = synth.random_packed_weight(qtype, (vocabulary,), k, seed=qtype, scale_range=(1e-3, 3e-2)).cuda()
+    targets = torch.from_numpy(np.random.default_rng(rows).integers(0, vocabulary, size=rows)).cuda()
+    targets[0], targets[-1] = vocabulary - 1, -100
+    hidden = random_bf16((rows, k), seed=7).requires_grad_(True)
+    loss = tgo.chunked_lm_head_loss(hidden, weight, targets, qtype, vocabulary, chunk_rows=chunk)
+    loss.backward()
+    plain = random_bf16((rows, k), seed=7)
+    logits = torch.cat([tgo.mmq(part.clone(), weight, qtype, vocabulary) for part in plain.split(chunk)]).float().requires_grad_(True)
+    reference = torch.nn.functional.cross_entropy(logits, targets, ignore_index=-100)
+    reference.backward()
+    expected = torch.ops.torch_ggml_ops.mmq_grad_input.default(logits.grad.bfloat16(), weight, qtype, k)
+    torch.testing.assert_close(loss, reference, rtol=1e-5, atol=1e-6)
+    assert nrmse(f32(hidden.grad), f32(expected)) < 5e-3
+    assert not f32(hidden.grad)[-1].any()
+    targets[1] = vocabulary   # neither a column nor ignored
+    assert torch.isnan(tgo.chunked_lm_head_loss(hidden.detach(), weight, targets, qtype, vocabulary, chunk_rows=chunk))

@@ -2,6 +2,7 @@
 // kernel dispatch.  Nothing here allocates or synchronises.
 #include "../../include/tgo.h"
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <mutex>
@@ -348,7 +349,7 @@ int tgo_mmq_forward(const void * input_bf16, const void * packed, void * output_
     return check_hip(launch(static_cast<const uint8_t *>(packed), nullptr, 0, view,
                             static_cast<uint16_t *>(output_bf16), nullptr, nullptr, static_cast<int>(rows),
                             static_cast<int>(in_features),
-                            static_cast<int>(out_features), quant_type, hip_stream),
+                            static_cast<int>(out_features), quant_type, hip_stream, 0),
                      "mmq_forward launch");
 }
 
@@ -384,7 +385,7 @@ int tgo_mmq_forward_prepared_as(const void * workspace, const void * packed, voi
     TGO_TRY(check_hip(launch(static_cast<const uint8_t *>(packed), nullptr, 0, view,
                              static_cast<uint16_t *>(output_bf16), nullptr, nullptr, static_cast<int>(rows),
                              static_cast<int>(in_features), static_cast<int>(out_features), quant_type,
-                             static_cast<hipStream_t>(stream)),
+                             static_cast<hipStream_t>(stream), 0),
                       "mmq_forward_prepared launch"));
     // (the workspace was quantized by an earlier call: were it of another kind than this call was told, its layout
     // would not be the one this launch assumed)
@@ -422,6 +423,117 @@ int tgo_mmq_grad_input(const void * grad_output_bf16, const void * packed, void 
                                                 static_cast<int>(rows), static_cast<int>(out_features),
                                                 static_cast<int>(in_features), quant_type, hip_stream, partial),
                      "mmq_grad_input launch");
+}
+
+// ---- chunked cross-entropy through a packed head --------------------------------------------------------------
+// Workspace of one chunk: q8_1 activations, bf16 logits (rows padded to whole 16-byte pieces), and for the gradient the
+// packed cotangent and the split reduction's scratch; then the statistics, the count and the loss of every row.
+namespace {
+struct HeadWorkspace {
+    int64_t logits, cotangent, partial, stats, count, row_loss, bytes;
+    int64_t pitch;
+};
+HeadWorkspace head_workspace(int64_t rows, int64_t in_features, int64_t out_features, int64_t chunk, int quant_type, bool gradient) {
+    const auto align = [](int64_t bytes) { return (bytes + 255) / 256 * 256; };
+    HeadWorkspace w;
+    w.pitch = (out_features + 7) / 8 * 8;
+    w.logits = align(tgo::q8_workspace_bytes(chunk, in_features));
+    w.cotangent = w.logits + align(chunk * w.pitch * 2);
+    w.partial = w.cotangent + (gradient ? align(tgo::cotangent_workspace_bytes(chunk, out_features)) : 0);
+    // (the last chunk may split its reduction where the full ones do not)
+    const int64_t rest = rows % chunk;
+    int64_t partial = gradient ? tgo::dense_grad_partial_bytes(chunk, out_features, in_features, quant_type) : 0;
+    if (gradient && rest > 0) {
+        partial = std::max(partial, tgo::dense_grad_partial_bytes(rest, out_features, in_features, quant_type));
+    }
+    w.stats = w.partial + align(partial);
+    w.count = w.stats + align(chunk * tgo::loss_spans(out_features) * static_cast<int64_t>(sizeof(float2)));
+    w.row_loss = w.count + 256;
+    w.bytes = w.row_loss + align(rows * static_cast<int64_t>(sizeof(float)));
+    return w;
+}
+constexpr int64_t HEAD_CHUNK_LIMIT = 65535;   // rows of a chunk: a grid dimension of the statistics kernel
+int check_head(int64_t rows, int64_t in_features, int64_t out_features, int64_t chunk_rows, int quant_type) {
+    TGO_TRY(check_matmul_shape(rows, in_features, out_features, quant_type));
+    if (chunk_rows <= 0) {
+        return fail(TGO_ERR_INVALID, "chunk_rows must be positive");
+    }
+    return TGO_OK;
+}
+}  // namespace
+
+int64_t tgo_lm_head_workspace_bytes(int64_t rows, int64_t in_features, int64_t out_features, int64_t chunk_rows, int quant_type,
+                                    int gradient) {
+    if (check_head(rows, in_features, out_features, chunk_rows, quant_type) != TGO_OK) {
+        return -1;
+    }
+    return head_workspace(rows, in_features, out_features, std::min({chunk_rows, rows, HEAD_CHUNK_LIMIT}), quant_type, gradient != 0).bytes;
+}
+
+int tgo_lm_head_loss(const void * hidden_bf16, const void * packed, const int64_t * targets, float * loss, void * grad_hidden_bf16,
+                     void * workspace, int64_t rows, int64_t in_features, int64_t out_features, int64_t chunk_rows,
+                     int64_t ignore_index, int quant_type, void * stream) {
+    TGO_TRY(check_head(rows, in_features, out_features, chunk_rows, quant_type));
+    TGO_TRY(check_pointer(hidden_bf16, "input"));
+    TGO_TRY(check_pointer(packed, "packed_weight"));
+    TGO_TRY(check_pointer(workspace, "workspace"));
+    if (targets == nullptr || loss == nullptr) {
+        return fail(TGO_ERR_INVALID, "targets and loss must not be null");
+    }
+    const bool gradient = grad_hidden_bf16 != nullptr;
+    if (gradient) {
+        TGO_TRY(check_pointer(grad_hidden_bf16, "grad_input"));
+    }
+    hipStream_t hip_stream = static_cast<hipStream_t>(stream);
+    const int64_t chunk_limit = std::min({chunk_rows, rows, HEAD_CHUNK_LIMIT});
+    const HeadWorkspace w = head_workspace(rows, in_features, out_features, chunk_limit, quant_type, gradient);
+    uint8_t * const base = static_cast<uint8_t *>(workspace);
+    uint16_t * const logits = reinterpret_cast<uint16_t *>(base + w.logits);
+    float * const count = reinterpret_cast<float *>(base + w.count);
+    float * const row_loss = reinterpret_cast<float *>(base + w.row_loss);
+    const uint8_t * const weights = static_cast<const uint8_t *>(packed);
+    TGO_TRY(check_hip(tgo::launch_count_targets(targets, rows, ignore_index, count, hip_stream), "count_targets launch"));
+    for (int64_t begin = 0; begin < rows; begin += chunk_limit) {
+        const int64_t chunk = std::min(chunk_limit, rows - begin);
+        const int r = static_cast<int>(chunk), n = static_cast<int>(out_features), k = static_cast<int>(in_features);
+        const bool gemv = tgo::use_gemv(chunk, 0);
+        const tgo::Q8Workspace view =
+            tgo::q8_workspace_view(base, chunk, in_features, gemv, tgo::forward_operand_kind(quant_type, chunk, out_features, 1));
+        TGO_TRY(check_hip(tgo::launch_quantize_q8_1(static_cast<const uint16_t *>(hidden_bf16) + begin * in_features, view, chunk,
+                                                    in_features, hip_stream),
+                          "quantize_q8_1 launch"));
+        const auto multiply = gemv ? tgo::launch_mmq_gemv : tgo::launch_mmq_forward;
+        TGO_TRY(check_hip(multiply(weights, nullptr, 0, view, logits, nullptr, nullptr, r, k, n, quant_type, hip_stream,
+                                   static_cast<int>(w.pitch)),
+                          "mmq_forward launch"));
+        uint8_t * const cotangent = gradient ? base + w.cotangent : nullptr;
+        TGO_TRY(check_hip(tgo::launch_cross_entropy(logits, w.pitch, r, n, reinterpret_cast<float2 *>(base + w.stats),
+                                                    targets + begin, ignore_index, count, row_loss + begin, cotangent, hip_stream),
+                          "cross_entropy launch"));
+        if (gradient) {
+            float * const partial = tgo::dense_grad_partial_bytes(chunk, out_features, in_features, quant_type) > 0
+                ? reinterpret_cast<float *>(base + w.partial) : nullptr;
+            TGO_TRY(check_hip(tgo::launch_mmq_grad_input(cotangent, nullptr, weights, nullptr, 0,
+                                                         static_cast<uint16_t *>(grad_hidden_bf16) + begin * in_features, nullptr,
+                                                         r, n, k, quant_type, hip_stream, partial),
+                              "mmq_grad_input launch"));
+        }
+    }
+    return check_hip(tgo::launch_loss_total(row_loss, rows, count, loss, hip_stream), "loss_total launch");
+}
+
+int tgo_scale_bf16(const void * input_bf16, const float * factor, void * output_bf16, int64_t count, void * stream) {
+    if (count <= 0 || count % 8 != 0) {
+        return fail(TGO_ERR_INVALID, "count must be a positive multiple of 8; got %lld", static_cast<long long>(count));
+    }
+    TGO_TRY(check_pointer(input_bf16, "input"));
+    TGO_TRY(check_pointer(output_bf16, "output"));
+    if (factor == nullptr) {
+        return fail(TGO_ERR_INVALID, "factor must not be null");
+    }
+    return check_hip(tgo::launch_scale_bf16(static_cast<const uint16_t *>(input_bf16), factor, static_cast<uint16_t *>(output_bf16),
+                                            count, static_cast<hipStream_t>(stream)),
+                     "scale launch");
 }
 
 // Shared body of the grouped forward entry points; `row_index` is null for pre-sorted rows.
@@ -477,8 +589,7 @@ static int grouped_forward(const void * input_bf16, const int64_t * row_index, i
     const tgo::Q8Workspace view = tgo::q8_workspace_view(workspace, rows, in_features, gemv, operand_kind);
     void * task_base = static_cast<char *>(workspace) + (tgo::q8_workspace_bytes(rows, in_features) + 15) / 16 * 16;
     const int row_tile = gemv ? tgo::GEMV_ROW_TILE : tgo::forward_row_tile(quant_type, view.operand_kind());
-        const auto launch = fused ? tgo::launch_mmq_forward_swiglu : gemv ? tgo::launch_mmq_gemv : tgo::launch_mmq_forward;
-    const tgo::TaskList tasks = tgo::task_list_view(task_base, rows, num_groups, row_tile);
+        const tgo::TaskList tasks = tgo::task_list_view(task_base, rows, num_groups, row_tile);
 
     // the quantizer writes the tile-task list on the side; the MFMA kernel runs a task of at most 32 rows in
     // about a third of a full task's time, so the groups of that size are listed last and fill the grid's tail
@@ -489,10 +600,13 @@ static int grouped_forward(const void * input_bf16, const int64_t * row_index, i
                                                 hip_stream, row_index, input_rows, &build),
                       "quantize_q8_1 launch"));
     // a pair is one launch: both projections of a task run side by side and share its activations in L2
-    TGO_TRY(check_hip(launch(static_cast<const uint8_t *>(packed_first), static_cast<const uint8_t *>(packed_second),
-                             bytes_per_expert, view, static_cast<uint16_t *>(output_first),
-                             static_cast<uint16_t *>(output_second), &tasks, static_cast<int>(rows),
-                             static_cast<int>(in_features), static_cast<int>(out_features), quant_type, hip_stream),
+    const auto launch = [&](auto function, auto... rest) {
+        return function(static_cast<const uint8_t *>(packed_first), static_cast<const uint8_t *>(packed_second), bytes_per_expert,
+                        view, static_cast<uint16_t *>(output_first), static_cast<uint16_t *>(output_second), &tasks,
+                        static_cast<int>(rows), static_cast<int>(in_features), static_cast<int>(out_features), quant_type,
+                        hip_stream, rest...);
+    };
+    TGO_TRY(check_hip(fused ? launch(tgo::launch_mmq_forward_swiglu) : launch(gemv ? tgo::launch_mmq_gemv : tgo::launch_mmq_forward, 0),
                       "grouped mmq_forward launch"));
     return swiglu && !fused ? finish_swiglu() : TGO_OK;
 }

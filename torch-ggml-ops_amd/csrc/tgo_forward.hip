@@ -470,8 +470,8 @@ TGO_DEVICE void forward_task(const ForwardArgs & a, ForwardLds<TYPE> & lds, int 
         uint16_t * block = reinterpret_cast<uint16_t *>(&wq[0][0]);
         stage_tile_32x32<128>(block, acc[0], wave * 32, lane);
         __syncthreads();
-        const int64_t origin = static_cast<int64_t>(row_start) * a.out_features + n0;
-        store_staged_rows<128>(block, y + origin, a.out_features, row_end - row_start, a.out_features - n0, tid,
+        const int64_t origin = static_cast<int64_t>(row_start) * a.out_stride + n0;
+        store_staged_rows<128>(block, y + origin, a.out_stride, row_end - row_start, a.out_features - n0, tid,
                                THREADS, fuse ? a.y + origin : nullptr);
         return;
     } else {
@@ -487,8 +487,8 @@ TGO_DEVICE void forward_task(const ForwardArgs & a, ForwardLds<TYPE> & lds, int 
 #pragma unroll
     for (int round = 0; round < S::WAVES / 4; ++round) {
         if ((wave >> 2) == round && wave_active) {
-            const int64_t origin = static_cast<int64_t>(wave_row) * a.out_features + n0;
-            store_rows_32x128<STAGE_PITCH, false, TRANSPOSED>(stage, acc, y + origin, a.out_features, row_end - wave_row,
+            const int64_t origin = static_cast<int64_t>(wave_row) * a.out_stride + n0;
+            store_rows_32x128<STAGE_PITCH, false, TRANSPOSED>(stage, acc, y + origin, a.out_stride, row_end - wave_row,
                                                              a.out_features - n0, lane, fuse ? a.y + origin : nullptr);
         }
         if (round + 1 < S::WAVES / 4) {
@@ -582,7 +582,7 @@ static hipError_t launch_forward_typed(const ForwardArgs & args, hipStream_t str
 static hipError_t launch_forward(const uint8_t * packed, const uint8_t * packed_second, int64_t bytes_per_expert,
                                  const Q8Workspace & ws, uint16_t * output, uint16_t * output_second,
                                  const TaskList * tasks, int rows, int in_features, int out_features,
-                                 int quant_type, hipStream_t stream, bool swiglu) {
+                                 int quant_type, hipStream_t stream, bool swiglu, int output_stride) {
     if (ws.by_rows()) {
         return hipErrorInvalidValue;   // this kernel reads the tile-ordered activation layout
     }
@@ -611,6 +611,7 @@ static hipError_t launch_forward(const uint8_t * packed, const uint8_t * packed_
     args.rows_padded = static_cast<int>(ws.rows_padded);
     args.in_features = in_features;
     args.out_features = out_features;
+    args.out_stride = output_stride > 0 ? output_stride : out_features;
     args.n_tiles = (out_features + FWD_TN - 1) / FWD_TN;
     if (tasks != nullptr) {
         args.task_count = tasks->count;
@@ -667,9 +668,9 @@ static hipError_t launch_forward(const uint8_t * packed, const uint8_t * packed_
 hipError_t launch_mmq_forward(const uint8_t * packed, const uint8_t * packed_second, int64_t bytes_per_expert,
                               const Q8Workspace & ws, uint16_t * output, uint16_t * output_second,
                               const TaskList * tasks, int rows, int in_features, int out_features,
-                              int quant_type, hipStream_t stream) {
+                              int quant_type, hipStream_t stream, int output_stride) {
     return launch_forward(packed, packed_second, bytes_per_expert, ws, output, output_second, tasks, rows,
-                          in_features, out_features, quant_type, stream, false);
+                          in_features, out_features, quant_type, stream, false, output_stride);
 }
 
 hipError_t launch_mmq_forward_swiglu(const uint8_t * packed, const uint8_t * packed_second, int64_t bytes_per_expert,
@@ -680,7 +681,7 @@ hipError_t launch_mmq_forward_swiglu(const uint8_t * packed, const uint8_t * pac
         return hipErrorInvalidValue;
     }
     return launch_forward(packed, packed_second, bytes_per_expert, ws, output, output_second, tasks, rows,
-                          in_features, out_features, quant_type, stream, true);
+                          in_features, out_features, quant_type, stream, true, 0);
 }
 
 }  // namespace tgo

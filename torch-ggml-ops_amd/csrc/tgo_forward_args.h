@@ -34,6 +34,7 @@ struct ForwardArgs {
     int rows_padded;
     int in_features;
     int out_features;
+    int out_stride;   // values from one row of y to the next (out_features, or more)
     int n_tiles;
     int projections;   // 1, or 2 for a pair: both share the task's activations, so their tiles run side by side
     int swiglu;        // 1: a workgroup runs gate (-> y) then up and stores swiglu(gate, up) -> y_second

@@ -502,13 +502,13 @@ TGO_DEVICE void forward_half_task(const ForwardArgs & a, HalfLds<TYPE> & lds, in
             stage_tile_32x32<STAGE_PITCH, true>(stage_base, acc[0], wave * 32, lane);
         }
         __syncthreads();
-        const int64_t origin = static_cast<int64_t>(row_start) * a.out_features + n0;
-        store_staged_rows<STAGE_PITCH>(stage_base, y + origin, a.out_features, row_end - row_start, a.out_features - n0, tid,
+        const int64_t origin = static_cast<int64_t>(row_start) * a.out_stride + n0;
+        store_staged_rows<STAGE_PITCH>(stage_base, y + origin, a.out_stride, row_end - row_start, a.out_features - n0, tid,
                                        THREADS, fuse ? a.y + origin : nullptr);
     } else {
         if (wave_active) {
-            const int64_t origin = static_cast<int64_t>(wave_row) * a.out_features + n0;
-            store_rows_32x128<STAGE_PITCH, false, true>(stage_base + wave * (32 * STAGE_PITCH), acc, y + origin, a.out_features,
+            const int64_t origin = static_cast<int64_t>(wave_row) * a.out_stride + n0;
+            store_rows_32x128<STAGE_PITCH, false, true>(stage_base + wave * (32 * STAGE_PITCH), acc, y + origin, a.out_stride,
                                                         row_end - wave_row, a.out_features - n0, lane,
                                                         fuse ? a.y + origin : nullptr);
         }

@@ -576,11 +576,11 @@ TGO_DEVICE void short_group_items(const ForwardArgs & a, ShortLds<TYPE> & lds, c
         for (int v = 0; v < 16; ++v) {
             acc[v] = total[v] * row_power;
         }
-        uint16_t * const y = (second ? a.y_second : a.y) + static_cast<int64_t>(row_start) * a.out_features + n0;
+        uint16_t * const y = (second ? a.y_second : a.y) + static_cast<int64_t>(row_start) * a.out_stride + n0;
         // (recomputing the lane's share here is cheaper than keeping it alive through the loop: kept, it is spilled, and
         // its reload waits for every load in flight)
         const int lane_here = lane_afresh();
-        store_rows_32xn<1>(&acc, y, a.out_features, row_end - row_start, a.out_features - n0, lane_here);
+        store_rows_32xn<1>(&acc, y, a.out_stride, row_end - row_start, a.out_features - n0, lane_here);
     }
     group_barrier();   // (the next item reuses the LDS buffers)
     ++item;
@@ -1227,7 +1227,7 @@ __global__ __launch_bounds__(FSC_THREADS, 3) void mmq_forward_scaled_kernel(cons
                         acc[nt][4 * j + 2] *= row_power * column_power.z;
                         acc[nt][4 * j + 3] *= row_power * column_power.w;
                     }
-                    store_rows_32xn<1>(&acc[nt], y + static_cast<int64_t>(r0) * a.out_features + n0 + 32 * nt, a.out_features,
+                    store_rows_32xn<1>(&acc[nt], y + static_cast<int64_t>(r0) * a.out_stride + n0 + 32 * nt, a.out_stride,
                                        row_end - r0, a.out_features - n0 - 32 * nt, lane_here);
                     __builtin_amdgcn_sched_barrier(0);
                 }

@@ -48,6 +48,7 @@ struct GemvArgs {
     int rows_padded;
     int in_features;
     int out_features;
+    int out_stride;   // values from one row of y to the next (out_features, or more)
     int n_groups;   // workgroups per task and projection: groups of GEMV_GN (long) weight rows
     int projections;   // 1, or 2 for a pair
     int unit_staging;  // 2-byte aligned formats: the tensors may be read in whole aligned 16-byte units (wide_stage_ok)
@@ -650,7 +651,7 @@ TGO_DEVICE void gemv_task(const GemvArgs & a, uint8_t * raw, uint8_t * x_lds, co
         const int sub = FOLD == 1 ? 0 : FOLD == 2 ? s : 2 * s + (lane >> 5);
         const int n = (n0 + wave * GEMV_WAVE_ROWS + i) * FOLD + sub;
         if ((lane & (WIDTH / COUNT - 1)) == 0 && r < nrows && n < a.out_features) {
-            y[static_cast<int64_t>(row_start + r) * a.out_features + n] = to_bf16_bits(total);
+            y[static_cast<int64_t>(row_start + r) * a.out_stride + n] = to_bf16_bits(total);
         }
     }
 }
@@ -886,7 +887,7 @@ TGO_DEVICE void gemv_task_k45(const GemvArgs & a, uint8_t * raw, const uint8_t *
             }
         }
         if (member < nrows && n < a.out_features) {
-            y[static_cast<int64_t>(row_start + member) * a.out_features + n] = to_bf16_bits(mine);
+            y[static_cast<int64_t>(row_start + member) * a.out_stride + n] = to_bf16_bits(mine);
         }
     }
 }
@@ -1015,7 +1016,7 @@ TGO_DEVICE void gemv_task_k45_direct(const GemvArgs & a, const uint8_t * weights
             value += __shfl_xor(value, offset);
         }
         if ((lane & (32 / FOLD - 1)) == 0 && n < a.out_features) {
-            y[static_cast<int64_t>(row_start) * a.out_features + n] = to_bf16_bits(value);
+            y[static_cast<int64_t>(row_start) * a.out_stride + n] = to_bf16_bits(value);
         }
     }
 }
@@ -1277,7 +1278,7 @@ TGO_DEVICE void gemv_task_k45_mfma(const GemvArgs & a, uint8_t * raw, float * sc
             total += partial[(w * 16 + m) * GEMV_GN + n];
         }
         if (m < nrows && n0 + n < a.out_features) {
-            y[static_cast<int64_t>(row_start + m) * a.out_features + n0 + n] = to_bf16_bits(total);
+            y[static_cast<int64_t>(row_start + m) * a.out_stride + n0 + n] = to_bf16_bits(total);
         }
     }
 }
@@ -1580,6 +1581,7 @@ static GemvArgs gemv_common_args(const uint8_t * packed, const uint8_t * packed_
     args.rows = rows;
     args.in_features = in_features;
     args.out_features = out_features;
+    args.out_stride = out_features;
     args.n_groups = (out_features + GEMV_GN - 1) / GEMV_GN;
     // (a dense call has one "expert": the whole weight)
     const int64_t weight_bytes = static_cast<int64_t>(out_features) * args.row_bytes;
@@ -1620,12 +1622,13 @@ hipError_t launch_mmq_gemv_fused(const uint8_t * packed, const uint8_t * packed_
 hipError_t launch_mmq_gemv(const uint8_t * packed, const uint8_t * packed_second, int64_t bytes_per_expert,
                            const Q8Workspace & ws, uint16_t * output, uint16_t * output_second,
                            const TaskList * tasks, int rows, int in_features, int out_features,
-                           int quant_type, hipStream_t stream) {
+                           int quant_type, hipStream_t stream, int output_stride) {
     if (!ws.by_rows()) {
         return hipErrorInvalidValue;   // these kernels read the row-major activation layout
     }
     GemvArgs args = gemv_common_args(packed, packed_second, bytes_per_expert, output, output_second, rows, in_features,
                                      out_features, quant_type);
+    args.out_stride = output_stride > 0 ? output_stride : out_features;
     args.qx = ws.q;
     args.dx = ws.d;
     args.sx = ws.sum;

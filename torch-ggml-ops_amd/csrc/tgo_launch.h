@@ -277,10 +277,11 @@ hipError_t launch_moe_combine(const uint16_t * rows, const int64_t * slot_rows, 
                               hipStream_t stream);
 // Dense when tasks == nullptr (row tiles follow from `rows`), grouped otherwise.  With `packed_second` and
 // `output_second` set, one launch computes both projections of a pair from the same activation workspace.
+// `output_stride`: values from one output row to the next, 0 for out_features.
 hipError_t launch_mmq_forward(const uint8_t * packed, const uint8_t * packed_second, int64_t bytes_per_expert,
                               const Q8Workspace & ws, uint16_t * output, uint16_t * output_second,
                               const TaskList * tasks, int rows, int in_features, int out_features,
-                              int quant_type, hipStream_t stream);
+                              int quant_type, hipStream_t stream, int output_stride = 0);
 // Pair only: `output` receives the first projection (gate) and `output_second` silu(gate) * second projection,
 // both factors rounded to bf16 first, the product rounded once.
 hipError_t launch_mmq_forward_swiglu(const uint8_t * packed, const uint8_t * packed_second, int64_t bytes_per_expert,
@@ -290,7 +291,7 @@ hipError_t launch_mmq_forward_swiglu(const uint8_t * packed, const uint8_t * pac
 hipError_t launch_mmq_gemv(const uint8_t * packed, const uint8_t * packed_second, int64_t bytes_per_expert,
                            const Q8Workspace & ws, uint16_t * output, uint16_t * output_second,
                            const TaskList * tasks, int rows, int in_features, int out_features,
-                           int quant_type, hipStream_t stream);
+                           int quant_type, hipStream_t stream, int output_stride = 0);
 // The same from bf16 activations in one launch: every workgroup quantizes its task's rows itself and, for a grouped
 // call (`expert_offsets` set), finds its task in the group list, so neither a quantizer launch nor a task list
 // exists.  Formats whose decode-regime routines read their activations one 16-value unit per lane.
@@ -313,6 +314,20 @@ hipError_t launch_mmq_gemv_fused(const uint8_t * packed, const uint8_t * packed_
                                  const int64_t * expert_indices, const int32_t * expert_offsets, int num_experts,
                                  int num_groups, uint16_t * output, uint16_t * output_second, int rows, int in_features,
                                  int out_features, int quant_type, hipStream_t stream);
+// ---- cross-entropy of a chunk of logits (tgo_loss.hip) ----
+constexpr int LOSS_SPAN = 8192;   // columns whose statistics one workgroup forms
+static inline int loss_spans(int64_t columns) { return static_cast<int>((columns + LOSS_SPAN - 1) / LOSS_SPAN); }
+// count[0] = max(1, targets that are not ignored); loss[0] = sum(row_loss) / count[0].
+hipError_t launch_count_targets(const int64_t * targets, int64_t rows, int64_t ignore_index, float * count, hipStream_t stream);
+hipError_t launch_loss_total(const float * row_loss, int64_t rows, const float * count, float * loss, hipStream_t stream);
+// Loss of each row, and with `cotangent` set (softmax - one_hot) / count as launch_pack_cotangent would pack it.
+// `logits`: bf16 rows `pitch` values apart (a multiple of 8, the buffer whole); `stats`: rows * loss_spans(columns).
+hipError_t launch_cross_entropy(const uint16_t * logits, int64_t pitch, int rows, int columns, float2 * stats,
+                                const int64_t * targets, int64_t ignore_index, const float * count, float * row_loss,
+                                uint8_t * cotangent, hipStream_t stream);
+// out[i] = bf16(in[i] * factor[0]); `count` is a multiple of 8.
+hipError_t launch_scale_bf16(const uint16_t * in, const float * factor, uint16_t * out, int64_t count, hipStream_t stream);
+
 // Cotangent in MFMA fragment order: [rows_padded/32][chunks] slabs of 1 KiB (32 rows x 16 columns), zero
 // padded; the column count is rounded up to 64 so that kernels can walk it four chunks at a time.
 static inline int cotangent_chunks(int64_t out_features) { return static_cast<int>((out_features + 63) / 64 * 4); }

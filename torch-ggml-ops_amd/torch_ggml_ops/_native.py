@@ -59,6 +59,10 @@ lib.tgo_route_workspace_bytes.restype = _i64
 lib.tgo_invert_slots.argtypes = [_p, _p, _i64, _i64, _i64, _p, _p, _p]
 lib.tgo_slot_weight_grad.argtypes = [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _p]
 lib.tgo_clear_uncovered_rows.argtypes = [_p, _i64, _i64, _p, _p, _i64, _i64, _p]
+lib.tgo_lm_head_workspace_bytes.argtypes = [_i64, _i64, _i64, _i64, _int, _int]
+lib.tgo_lm_head_workspace_bytes.restype = _i64
+lib.tgo_lm_head_loss.argtypes = [_p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _int, _p]
+lib.tgo_scale_bf16.argtypes = [_p, _p, _p, _i64, _p]
 lib.tgo_rows_to_tokens.argtypes = [_p, _p, _p, _p, _i64, _i64, _i64, _p]
 lib.tgo_moe_combine.argtypes = [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _p]
 lib.tgo_grouped_mmq_grad_input.argtypes = [_p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _int, _p]
@@ -103,6 +107,9 @@ EXPORTS = (
     "tgo_invert_slots",
     "tgo_slot_weight_grad",
     "tgo_clear_uncovered_rows",
+    "tgo_lm_head_workspace_bytes",
+    "tgo_lm_head_loss",
+    "tgo_scale_bf16",
     "tgo_rows_to_tokens",
     "tgo_moe_combine",
     "tgo_grouped_mmq_grad_input",

@@ -5,59 +5,103 @@ reference is tuned on); keeping them for the backward pass of the loss costs mor
 the rest of the step.  The reference's production schedule therefore walks the rows in chunks of
 256 (its measured best; 128 and 64 are its lower-memory fallbacks,
 docs/mmq_fwd_optimization.md:293) and runs forward and backward of each chunk back to back:
-``mmq`` for the chunk's logits, the loss and its gradient with respect to the logits, and
-``mmq_grad_input`` for the chunk's share of the hidden-state gradient.  Only one chunk of logits
-exists at a time.  That loop lives in the reference's training code, not in its package; this
-module is the same schedule on top of this package's operators.
+the forward product for the chunk's logits, the loss and its gradient with respect to the logits, and
+the grad-input product for the chunk's share of the hidden-state gradient.  Only one chunk of logits
+exists at a time.  That loop lives in the reference's training code, not in its package; here it is one
+call into the library, whose loss kernels write the logits' gradient as the operand the grad-input kernels
+read.
 """
 
 from __future__ import annotations
 
 import torch
 
+from . import _native, _validate
+
 DEFAULT_CHUNK_ROWS = 256   # the reference's production chunk
+
+
+torch.library.define(
+    "torch_ggml_ops::lm_head_loss",
+    "(Tensor hidden, Tensor packed_weight, Tensor targets, int quant_type, int out_features, int chunk_rows, "
+    "int ignore_index, bool gradient) -> (Tensor, Tensor)",
+)
+
+
+@torch.library.impl("torch_ggml_ops::lm_head_loss", "CUDA")
+def _lm_head_loss_device(hidden, packed_weight, targets, quant_type, out_features, chunk_rows, ignore_index, gradient):
+    """(mean loss, its gradient with respect to ``hidden`` or an empty tensor): every launch of every chunk is issued by
+    one call into the library (``tgo_lm_head_loss``)."""
+    if hidden.shape[0] > chunk_rows and (not hidden.is_contiguous() or hidden.storage_offset() != 0):
+        hidden = hidden.clone(memory_format=torch.contiguous_format)   # (such rows were always accepted chunk by chunk)
+    rows, in_features, out_features = _validate.dense(hidden, packed_weight, quant_type, out_features, backward=False)
+    targets = targets.contiguous()
+    if targets.device != hidden.device:
+        raise RuntimeError("hidden and targets must be on the same device")
+    with _native.on_device(hidden.device):
+        loss = torch.empty((), dtype=torch.float32, device=hidden.device)
+        grad_hidden = torch.empty_like(hidden) if gradient else hidden.new_empty((0, in_features))
+        workspace_bytes = _native.lib.tgo_lm_head_workspace_bytes(
+            rows, in_features, out_features, chunk_rows, int(quant_type), int(gradient)
+        )
+        workspace = torch.empty(max(workspace_bytes, 0), dtype=torch.uint8, device=hidden.device)
+        _native.check(
+            _native.lib.tgo_lm_head_loss(
+                hidden.data_ptr(), packed_weight.data_ptr(), targets.data_ptr(), loss.data_ptr(),
+                grad_hidden.data_ptr() if gradient else None, workspace.data_ptr(), rows, in_features, out_features,
+                chunk_rows, ignore_index, int(quant_type), _native.stream_of(hidden.device),
+            )
+        )
+    return loss, grad_hidden
+
+
+@torch.library.register_fake("torch_ggml_ops::lm_head_loss")
+def _lm_head_loss_fake(hidden, packed_weight, targets, quant_type, out_features, chunk_rows, ignore_index, gradient):
+    return (
+        hidden.new_empty((), dtype=torch.float32), hidden.new_empty(hidden.shape if gradient else (0, hidden.shape[1]))
+    )
+
+
+torch.library.define("torch_ggml_ops::scale_bf16", "(Tensor input, Tensor factor) -> Tensor")
+
+
+@torch.library.impl("torch_ggml_ops::scale_bf16", "CUDA")
+def _scale_device(input, factor):
+    """``(input.float() * factor).to(bfloat16)`` for a contiguous bf16 tensor and an fp32 scalar on its device."""
+    out = torch.empty_like(input)
+    with _native.on_device(input.device):
+        _native.check(
+            _native.lib.tgo_scale_bf16(
+                input.data_ptr(), factor.data_ptr(), out.data_ptr(), input.numel(), _native.stream_of(input.device)
+            )
+        )
+    return out
+
+
+@torch.library.register_fake("torch_ggml_ops::scale_bf16")
+def _scale_fake(input, factor):
+    return input.new_empty(input.shape)
 
 
 class _ChunkedLoss(torch.autograd.Function):
     @staticmethod
     def forward(ctx, hidden, packed_weight, targets, quant_type, out_features, chunk_rows, ignore_index):
-        ops = torch.ops.torch_ggml_ops
-        rows, in_features = hidden.shape
-        counted = targets != ignore_index
-        # (a tensor: no host synchronisation; the loss of a batch without any counted row is 0 / 1)
-        count = counted.sum().clamp(min=1).to(torch.float32)
-        total = torch.zeros((), dtype=torch.float32, device=hidden.device)
-        need_grad = ctx.needs_input_grad[0]
-        grad_hidden = torch.empty_like(hidden) if need_grad else None
-        for begin in range(0, rows, chunk_rows):
-            end = min(rows, begin + chunk_rows)
-            # (the operators take tensors at storage offset zero only: a chunk is copied out, a few hundred rows)
-            chunk = hidden if begin == 0 and end == rows else hidden[begin:end].clone()
-            logits = ops.mmq.default(chunk, packed_weight, quant_type, out_features).float()
-            log_probabilities = torch.log_softmax(logits, dim=-1)
-            chunk_targets = targets[begin:end]
-            chunk_counted = counted[begin:end]
-            safe_targets = torch.where(chunk_counted, chunk_targets, torch.zeros_like(chunk_targets))
-            picked = log_probabilities.gather(1, safe_targets.unsqueeze(1)).squeeze(1)
-            total = total - (picked * chunk_counted).sum()
-            if need_grad:
-                # d(mean loss)/d(logits) = (softmax - one_hot) / count on counted rows, 0 elsewhere
-                grad_logits = torch.exp(log_probabilities)
-                grad_logits.scatter_add_(1, safe_targets.unsqueeze(1), -torch.ones_like(picked).unsqueeze(1))
-                grad_logits = grad_logits * (chunk_counted.unsqueeze(1) / count)
-                grad_hidden[begin:end] = ops.mmq_grad_input.default(
-                    grad_logits.to(hidden.dtype), packed_weight, quant_type, in_features
-                )
-        if need_grad:
+        loss, grad_hidden = torch.ops.torch_ggml_ops.lm_head_loss.default(
+            hidden, packed_weight, targets, quant_type, out_features, chunk_rows, ignore_index, ctx.needs_input_grad[0]
+        )
+        if ctx.needs_input_grad[0]:
             ctx.save_for_backward(grad_hidden)
-        return total / count
+        return loss
 
     @staticmethod
     def backward(ctx, grad_loss):
         grad_hidden = None
         if ctx.needs_input_grad[0]:
             (saved,) = ctx.saved_tensors
-            grad_hidden = (saved.float() * grad_loss).to(saved.dtype)
+            if grad_loss.requires_grad:   # (a gradient of the gradient: tensor operations, which autograd can follow)
+                grad_hidden = (saved.float() * grad_loss).to(saved.dtype)
+            else:
+                grad_hidden = torch.ops.torch_ggml_ops.scale_bf16.default(saved, grad_loss)
         return grad_hidden, None, None, None, None, None, None
 
 
@@ -75,7 +119,7 @@ def chunked_lm_head_loss(
 
     ``hidden`` bf16 ``[rows, in_features]`` (contiguous), ``targets`` int64 ``[rows]``.  Differentiable with
     respect to ``hidden``: the gradient is computed chunk by chunk during the forward pass (each chunk's logits
-    are dropped as soon as its ``mmq_grad_input`` has run) and scaled by the incoming gradient in backward.
+    are dropped as soon as its grad-input product has run) and scaled by the incoming gradient in backward.
     Equals ``cross_entropy(mmq(hidden, ...).float(), targets)`` up to the bf16 rounding of the logit gradients.
     """
     if hidden.dim() != 2:
