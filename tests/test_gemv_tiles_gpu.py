@@ -1,0 +1,57 @@
+"""GPU parity of the decode-regime kernel for tasks of several rows against the CPU oracle (-m gpu): its edges are the
+16 rows of a task, the 16 weight rows of a tile (a last workgroup with tiles missing, one and several waves per
+tile), the two, four or fewer shares of K, and weight blocks at every address modulo 16 up to the tensor's last."""
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import QTYPES, assert_matches_f32_reference, bits, random_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    import torch_ggml_ops
+    import synth
+
+    assert torch.cuda.is_available()
+    return torch_ggml_ops, synth
+
+
+@pytest.mark.parametrize("qname", tuple(QTYPES))
+@pytest.mark.parametrize("rows,n,k", [(17, 16400, 256), (32, 5472, 768), (5, 3280, 1280), (20, 1840, 2304), (9, 2064, 16384)])
+def test_dense(ops, oracle, qname, rows, n, k):
+    tgo, synth = ops
+    qtype = QTYPES[qname]
+    host = synth.random_packed_weight(qtype, (n,), k, seed=700 + qtype + rows)
+    x = random_bf16((rows, k), seed=rows)
+    assert_matches_f32_reference(tgo.mmq(x, host.cuda(), qtype, n), oracle.mmq_forward(qtype, bits(x), host.numpy(), n, k))
+
+
+@pytest.mark.parametrize("qname", tuple(QTYPES))
+@pytest.mark.parametrize("n,k", [(2048, 512), (816, 256), (208, 1024), (96, 2304)])
+def test_grouped(ops, oracle, qname, n, k):
+    """Groups of 1 to 33 rows (up to three tasks), empty ones, an expert that does not exist."""
+    tgo, synth = ops
+    qtype, experts = QTYPES[qname], 24
+    host = [synth.random_packed_weight(qtype, (experts, n), k, seed=seed + qtype) for seed in (800, 900)]
+    sizes = [1, 16, 0, 2, 33, 0, 5, 1, 17, 3, 0, 1, 1, 4, 1, 2, 0, 1, 1, 0, 3]
+    chosen = np.random.default_rng(5).permutation(experts)[: len(sizes)].tolist()
+    chosen[3] = experts
+    offsets = np.cumsum(sizes).tolist()
+    x = random_bf16((offsets[-1], k), seed=31)
+    indices = torch.tensor(chosen, dtype=torch.int64, device="cuda")
+    ends = torch.tensor(offsets, dtype=torch.int32, device="cuda")
+    outputs = tgo.grouped_mmq_pair(x, host[0].cuda(), host[1].cuda(), indices, ends, qtype, n)
+    exact = [oracle.grouped(oracle.mmq_forward, qtype, bits(x), h.numpy(), chosen, offsets, n, k, n) for h in host]
+    covered = ~np.isnan(exact[0][:, 0])
+    assert covered.sum() == offsets[-1] - 2
+    on_device = torch.from_numpy(covered).cuda()
+    for actual, expected in zip(outputs, exact):
+        assert_matches_f32_reference(actual[on_device], expected[covered])
+    activated = tgo.grouped_mmq_swiglu(x, host[0].cuda(), host[1].cuda(), indices, ends, qtype, n)
+    gate, up = (o.float() for o in outputs)
+    expected = (torch.nn.functional.silu(gate) * up)[on_device]
+    assert ((activated.float()[on_device] - expected).abs() <= 2.0**-7 * expected.abs() + 1e-6).all()

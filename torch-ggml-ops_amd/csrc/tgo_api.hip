@@ -331,7 +331,7 @@ int tgo_mmq_forward(const void * input_bf16, const void * packed, void * output_
     TGO_TRY(check_pointer(output_bf16, "output"));
     TGO_TRY(check_pointer(workspace, "workspace"));
     hipStream_t hip_stream = static_cast<hipStream_t>(stream);
-    if (tgo::gemv_fuses(quant_type, rows, 0)) {
+    if (tgo::gemv_fuses(quant_type, rows, 0) && !tgo::gemv_takes_tiles(packed, nullptr, rows, 0, in_features, out_features, quant_type)) {
         // one launch: the decode-regime kernels of these formats quantize their activations themselves
         return check_hip(tgo::launch_mmq_gemv_fused(static_cast<const uint8_t *>(packed), nullptr, 0,
                                                     static_cast<const uint16_t *>(input_bf16), nullptr, rows, nullptr,
@@ -568,7 +568,8 @@ static int grouped_forward(const void * input_bf16, const int64_t * row_index, i
                          "swiglu launch");
     };
     const bool gemv = tgo::use_gemv(rows, num_groups);
-    if (gemv && tgo::gemv_fuses(quant_type, rows, num_groups)) {
+    const bool tiles = tgo::gemv_takes_tiles(packed_first, packed_second, rows, num_groups, in_features, out_features, quant_type);
+    if (gemv && !tiles && tgo::gemv_fuses(quant_type, rows, num_groups)) {
         // one launch: the decode-regime kernels of these formats quantize their activations and find their tasks
         // themselves
         TGO_TRY(check_hip(tgo::launch_mmq_gemv_fused(
@@ -588,8 +589,8 @@ static int grouped_forward(const void * input_bf16, const int64_t * row_index, i
     const bool fused = swiglu && !gemv && operand_kind != tgo::OPERAND_SCALED;
     const tgo::Q8Workspace view = tgo::q8_workspace_view(workspace, rows, in_features, gemv, operand_kind);
     void * task_base = static_cast<char *>(workspace) + (tgo::q8_workspace_bytes(rows, in_features) + 15) / 16 * 16;
-    const int row_tile = gemv ? tgo::GEMV_ROW_TILE : tgo::forward_row_tile(quant_type, view.operand_kind());
-        const tgo::TaskList tasks = tgo::task_list_view(task_base, rows, num_groups, row_tile);
+    const int row_tile = tiles ? tgo::GEMV_TILES_ROWS : gemv ? tgo::GEMV_ROW_TILE : tgo::forward_row_tile(quant_type, view.operand_kind());
+    const tgo::TaskList tasks = tgo::task_list_view(task_base, rows, num_groups, row_tile);
 
     // the quantizer writes the tile-task list on the side; the MFMA kernel runs a task of at most 32 rows in
     // about a third of a full task's time, so the groups of that size are listed last and fill the grid's tail
@@ -606,6 +607,14 @@ static int grouped_forward(const void * input_bf16, const int64_t * row_index, i
                         static_cast<int>(rows), static_cast<int>(in_features), static_cast<int>(out_features), quant_type,
                         hip_stream, rest...);
     };
+    if (tiles) {
+        return check_hip(tgo::launch_mmq_gemv_tiles(
+                             static_cast<const uint8_t *>(packed_first), static_cast<const uint8_t *>(packed_second), bytes_per_expert,
+                             view, static_cast<uint16_t *>(output_first), static_cast<uint16_t *>(output_second), &tasks,
+                             static_cast<int>(rows), static_cast<int>(in_features), static_cast<int>(out_features), quant_type,
+                             swiglu, hip_stream),
+                         "grouped mmq_forward launch");
+    }
     TGO_TRY(check_hip(fused ? launch(tgo::launch_mmq_forward_swiglu) : launch(gemv ? tgo::launch_mmq_gemv : tgo::launch_mmq_forward, 0),
                       "grouped mmq_forward launch"));
     return swiglu && !fused ? finish_swiglu() : TGO_OK;

@@ -101,6 +101,49 @@ static inline bool use_gemv(int64_t rows, int64_t groups) {
     return groups <= 0 ? rows <= GEMV_DENSE_ROWS : rows <= 4 * groups;
 }
 
+// Decode-regime calls that take the kernel for tasks of several rows (tgo_gemv_tiles.hip), which unpacks every weight once
+// per task, instead of those of tgo_gemv.hip, whose dot products cost the same again for every row.  It needs whole tiles of
+// 16 weight rows and 16-byte aligned weights.  The lines lie where the two measured equal (2048 x 512 and 4096 x 1024 experts
+// and their down projections, 1 to 124 tokens; dense 4096 x 2048 and 28672 x 8192, 1 to 32 rows):
+//  - grouped: Q5_K always (1 token 17 -> 12 us), Q4_K too unless K is long enough for the other kernel's own matrix
+//    instructions to pay; Q3_K from 16 rows.  Q6_K and IQ2_S, whose unpacking is the longest, when the rows are half as many as
+//    the groups if K is short (the other kernel idles there), else three and one and a half (long K: two and a half)
+//    times as many.
+//  - calls of fewer than four million weights never: their time is their launches and latencies, and most of them are one
+//    launch of the other kernel.
+//  - dense: Q3_K, Q6_K and IQ2_S from five rows (the others have eight at most in registers, and two launches' worth of rows
+//    reads the weights twice); Q4_K and Q5_K beyond 16 rows, or on matrices that fill the chip, from nine and three.
+constexpr int GEMV_TILES_ROWS = 16;              // rows of its tasks
+constexpr int64_t GEMV_TILES_WORKGROUPS = 384;   // workgroups that a launch should have for a wave to take four tiles of 16 weight rows instead of two
+static inline bool gemv_takes_tiles(const void * packed, const void * packed_second, int64_t rows, int64_t groups, int64_t in_features,
+                                    int64_t out_features, int quant_type) {
+    if (!use_gemv(rows, groups) || out_features % 16 != 0 ||
+        (reinterpret_cast<uintptr_t>(packed) | reinterpret_cast<uintptr_t>(packed_second)) % 16 != 0 ||
+        in_features > (INT64_C(1) << 22) || rows > (1 << 24)) {   // (the kernel's offsets within a tile have 32 bits)
+        return false;
+    }
+    const int64_t matrices = groups <= 0 ? 1 : rows < groups ? rows : groups;
+    if (matrices * out_features * in_features < (INT64_C(1) << 22)) {
+        return false;
+    }
+    const int64_t super_blocks = in_features / 256;
+    if (groups <= 0) {
+        const bool large = out_features * in_features >= (INT64_C(1) << 25);
+        switch (quant_type) {
+            case 12: return rows > 16 || (large && rows > 8);
+            case 13: return rows > 16 || (large && rows > 2);
+            default: return rows > 4;
+        }
+    }
+    switch (quant_type) {
+        case 11: return rows >= 16;
+        case 12: return super_blocks <= 8;
+        case 13: return true;
+        case 14: return super_blocks <= 4 ? 2 * rows >= groups : rows >= 3 * groups;
+        default: return super_blocks <= 4 ? 2 * rows >= groups : 2 * rows >= (super_blocks <= 8 ? 3 : 5) * groups;
+    }
+}
+
 // q8_1 workspace: quantized values, then fp32 scales, then fp32 sums, in one of four layouts over the same bytes.
 // The MFMA kernels want 32-row tiles in fragment order: int8, fp16 numbers holding the same integers, or (scaled)
 // the dequantized values d * q * 2^-e as fp16 with e chosen per row and super-block; the GEMV family reads a few
@@ -292,6 +335,10 @@ hipError_t launch_mmq_gemv(const uint8_t * packed, const uint8_t * packed_second
                            const Q8Workspace & ws, uint16_t * output, uint16_t * output_second,
                            const TaskList * tasks, int rows, int in_features, int out_features,
                            int quant_type, hipStream_t stream, int output_stride = 0);
+hipError_t launch_mmq_gemv_tiles(const uint8_t * packed, const uint8_t * packed_second, int64_t bytes_per_expert,
+                                 const Q8Workspace & ws, uint16_t * output, uint16_t * output_second,
+                                 const TaskList * tasks, int rows, int in_features, int out_features,
+                                 int quant_type, bool swiglu, hipStream_t stream, int output_stride = 0);
 // The same from bf16 activations in one launch: every workgroup quantizes its task's rows itself and, for a grouped
 // call (`expert_offsets` set), finds its task in the group list, so neither a quantizer launch nor a task list
 // exists.  Formats whose decode-regime routines read their activations one 16-value unit per lane.
