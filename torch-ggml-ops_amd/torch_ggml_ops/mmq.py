@@ -10,7 +10,7 @@ from __future__ import annotations
 
 import torch
 
-from . import _native, _validate
+from . import _direct, _native, _validate
 
 torch.library.define(
     "torch_ggml_ops::mmq",
@@ -103,6 +103,10 @@ torch.library.register_autograd("torch_ggml_ops::mmq_grad_input", _mmq_grad_inpu
 
 def mmq(input: torch.Tensor, packed_weight: torch.Tensor, quant_type: int, out_features: int) -> torch.Tensor:
     """``input @ W.T`` for a packed GGUF weight ``[out_features, row_bytes]``; bf16 in, bf16 out."""
+    if not torch.compiler.is_compiling():
+        output = _direct.mmq(input, packed_weight, quant_type, out_features)   # (None: not a plain call)
+        if output is not None:
+            return output
     return torch.ops.torch_ggml_ops.mmq.default(input, packed_weight, int(quant_type), int(out_features))
 
 

@@ -16,7 +16,7 @@ from __future__ import annotations
 
 import torch
 
-from . import _native, _validate
+from . import _direct, _native, _validate
 from .grouped_mmq import _forward as _grouped_forward
 from .swiglu import grouped_mmq_swiglu
 
@@ -371,6 +371,13 @@ def moe_layer(
     ``down_weight`` packed ``[experts, features, ...]``.  Differentiable with respect to ``hidden`` and
     ``slot_weights``.
     """
+    if not torch.compiler.is_compiling():
+        output = _direct.moe_layer(
+            hidden, slot_experts, slot_weights, gate_weight, up_weight, down_weight, gate_up_type, down_type,
+            intermediate_features,
+        )   # (None: not a plain call)
+        if output is not None:
+            return output
     experts = gate_weight.shape[0]
     row_index, slot_rows, expert_indices, expert_offsets = route(slot_experts, experts)
     activated = grouped_mmq_swiglu(
