@@ -258,7 +258,7 @@ int64_t tgo_dense_grad_workspace_bytes(int64_t rows, int64_t out_features, int64
         return -1;
     }
     return (tgo::cotangent_workspace_bytes(rows, out_features) + 15) / 16 * 16 +
-           tgo::dense_grad_partial_bytes(rows, out_features, in_features, quant_type);
+           tgo::dense_grad_partial_bytes(rows, out_features, in_features);
 }
 
 int64_t tgo_grad_workspace_bytes(int64_t rows, int64_t out_features, int64_t num_groups, int sources) {
@@ -415,7 +415,7 @@ int tgo_mmq_grad_input(const void * grad_output_bf16, const void * packed, void 
                                                  hip_stream),
                       "pack_cotangent launch"));
     // scratch for the split reduction of small calls follows the packed cotangent
-    float * partial = tgo::dense_grad_partial_bytes(rows, out_features, in_features, quant_type) > 0
+    float * partial = tgo::dense_grad_partial_bytes(rows, out_features, in_features) > 0
         ? reinterpret_cast<float *>(cotangent + (tgo::cotangent_workspace_bytes(rows, out_features) + 15) / 16 * 16)
         : nullptr;
     return check_hip(tgo::launch_mmq_grad_input(cotangent, nullptr, static_cast<const uint8_t *>(packed), nullptr, 0,
@@ -442,9 +442,9 @@ HeadWorkspace head_workspace(int64_t rows, int64_t in_features, int64_t out_feat
     w.partial = w.cotangent + (gradient ? align(tgo::cotangent_workspace_bytes(chunk, out_features)) : 0);
     // (the last chunk may split its reduction where the full ones do not)
     const int64_t rest = rows % chunk;
-    int64_t partial = gradient ? tgo::dense_grad_partial_bytes(chunk, out_features, in_features, quant_type) : 0;
+    int64_t partial = gradient ? tgo::dense_grad_partial_bytes(chunk, out_features, in_features) : 0;
     if (gradient && rest > 0) {
-        partial = std::max(partial, tgo::dense_grad_partial_bytes(rest, out_features, in_features, quant_type));
+        partial = std::max(partial, tgo::dense_grad_partial_bytes(rest, out_features, in_features));
     }
     w.stats = w.partial + align(partial);
     w.count = w.stats + align(chunk * tgo::loss_spans(out_features) * static_cast<int64_t>(sizeof(float2)));
@@ -511,7 +511,7 @@ int tgo_lm_head_loss(const void * hidden_bf16, const void * packed, const int64_
                                                     targets + begin, ignore_index, count, row_loss + begin, cotangent, hip_stream),
                           "cross_entropy launch"));
         if (gradient) {
-            float * const partial = tgo::dense_grad_partial_bytes(chunk, out_features, in_features, quant_type) > 0
+            float * const partial = tgo::dense_grad_partial_bytes(chunk, out_features, in_features) > 0
                 ? reinterpret_cast<float *>(base + w.partial) : nullptr;
             TGO_TRY(check_hip(tgo::launch_mmq_grad_input(cotangent, nullptr, weights, nullptr, 0,
                                                          static_cast<uint16_t *>(grad_hidden_bf16) + begin * in_features, nullptr,

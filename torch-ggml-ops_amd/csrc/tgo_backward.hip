@@ -7,15 +7,15 @@
 // is the A operand of one v_mfma_f32_32x32x16_bf16, so the main kernels fetch it with one fully coalesced
 // 16-byte-per-lane load (a row-major cotangent would cost 32 cache lines per wave load).
 //
-// mmq_grad_input_kernel (every format): a workgroup (4 waves) owns 256 rows x 128 values of K (half a
-// super-block column) and walks the reduction dimension N in steps of 64 weight rows.  Per step the 64 packed
-// blocks are copied to LDS, dequantized once to bf16 (bit-exact with the scalar reference decoder) into a
-// transposed tile [k][n] whose rows are what a lane needs as its B operand, and shared by the four waves; wave
-// w owns rows [64w, 64w+64) and all 128 columns: 2 x 4 MFMA tiles, 32 MFMAs per step.  The tile is double
-// buffered and the loop is software pipelined.
+// mmq_grad_input_split_kernel: a workgroup owns 256 rows x 128 values of K (half a super-block column) and walks the
+// reduction dimension N in steps of 64 weight rows.  Per step the 64 packed blocks are copied to LDS, dequantized once to bf16
+// (bit-exact with the scalar reference decoder) into a transposed tile [k][n] whose rows are what a lane needs as its B
+// operand; half of the waves dequantize, half multiply.  Dense calls whose tiles do not fill the chip cut N into ranges.
 //
-// mmq_grad_input_split_kernel (Q4_K and Q5_K, what the launcher picks for them): the same tile, with the waves
-// of a workgroup specialised into multipliers and decoders; described where it is defined.
+// mmq_grad_input_short_kernel: tasks of a few rows of a grouped call; described where it is defined.
+//
+// mmq_grad_input_kernel: the same tile as the split kernel's by four waves that all dequantize and multiply, for calls
+// beyond the 32-bit offsets of the two others (a cotangent of 4 GiB).
 //
 // The pair variant of both walks a second (dY, W) in the same loop with one fp32 accumulator, so the sum of
 // both Jacobian products is rounded to bf16 once.
@@ -197,6 +197,22 @@ TGO_DEVICE void decode_k45_octet(const uint8_t * raw, const float2 * scale_min, 
         const uint4 packed = make_uint4(pack_bf16x2(w[e][0], w[e][1]), pack_bf16x2(w[e][2], w[e][3]),
                                         pack_bf16x2(w[e][4], w[e][5]), pack_bf16x2(w[e][6], w[e][7]));
         *reinterpret_cast<uint4 *>(&wb[(k_local + e) * BWD_PITCH + 8 * octet]) = packed;
+    }
+}
+
+// fp32 partial sums of range `split` straight from the accumulators (operands swapped): a lane holds row `row` of its tile
+// and, as elements 4 j .. 4 j + 3, the four columns from 8 j + 4 half on: 16-byte stores
+TGO_DEVICE void store_partial_32x128(const BackwardArgs & a, const v16f (&acc)[4], int split, int row, int row_end, int k_tile, int half) {
+    if (row < row_end) {
+        float * const out = a.partial + (static_cast<int64_t>(split) * a.rows + row) * a.in_features + k_tile * BWD_TK + 4 * half;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                *reinterpret_cast<float4 *>(out + kt * 32 + 8 * j) =
+                    make_float4(acc[kt][4 * j], acc[kt][4 * j + 1], acc[kt][4 * j + 2], acc[kt][4 * j + 3]);
+            }
+        }
     }
 }
 
@@ -758,21 +774,9 @@ __global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_ker
         return;
     }
     if (a.n_splits > 1) {
-        // fp32 partial sums straight from the accumulators (operands swapped): a lane holds row l32 of its tile
-        // and, as elements 4 j .. 4 j + 3, the four columns from 8 j + 4 half on: 16-byte stores
-        float * out = a.partial + (static_cast<int64_t>(split) * a.rows + wave_row + l32) * a.in_features + k_tile * BWD_TK + 4 * half;
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt) {
-            if (wave_row + rt * 32 + l32 < row_end) {
-#pragma unroll
-                for (int kt = 0; kt < 4; ++kt) {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        *reinterpret_cast<float4 *>(out + static_cast<int64_t>(rt * 32) * a.in_features + kt * 32 + 8 * j) =
-                            make_float4(acc[rt][kt][4 * j], acc[rt][kt][4 * j + 1], acc[rt][kt][4 * j + 2], acc[rt][kt][4 * j + 3]);
-                    }
-                }
-            }
+            store_partial_32x128(a, acc[rt], split, wave_row + rt * 32 + l32, row_end, k_tile, half);
         }
         return;
     }
@@ -788,9 +792,9 @@ __global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_ker
     }
 }
 
-// ---- role-split variant (Q4_K / Q5_K) ------------------------------------------------------------------------
-// Same tile as above (256 rows x 128 values of K, reduction steps of 64 weight rows, double-buffered bf16
-// tile), but the eight waves of a workgroup are specialised: waves 0-3 only multiply (64 rows each), waves
+// ---- role-split variant --------------------------------------------------------------------------------------
+// 256 rows x 128 values of K, reduction steps of 64 weight rows, double-buffered bf16
+// tile; the eight waves of a workgroup are specialised: waves 0-3 only multiply (64 rows each), waves
 // 4-7 only dequantize.  Each SIMD then holds one wave that keeps the matrix pipe busy and one that keeps the
 // vector ALU busy, and the two kinds of work overlap instead of alternating; one barrier per step hands the
 // finished tile over.
@@ -804,11 +808,16 @@ __global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_ker
 // has the blocks of steps g+4..g+7 in flight in registers, so no stage waits for the one before it.  A
 // multiplier wave keeps the cotangent fragments of the next step in flight (two steps were measured: no faster, and
 // the registers serve the weight-fragment look-ahead better).
+//
+// Measured, 256 rows of a 248320 x 2048 head (16 ranges): Q4_K 955 -> 316 us, Q6_K 655 -> 356, IQ2_S 527 -> 333 (820 TFLOP/s)
+// against the general kernel, whose waves dequantize and multiply in turn; the matrix pipe is busy for
+// a third of the time at the clock the card then holds, the decoder waves' LDS traffic and arithmetic for the rest.
 constexpr int BSP_THREADS = 512;
 constexpr int BSP_ROWS_PER_DECODER = BWD_NS / 4;   // weight rows a decoder wave owns per step
 constexpr int BSP_RAW_DEPTH = 4;                   // steps of packed blocks in flight per decoder wave
 constexpr int BSP_COT_DEPTH = 2;                   // cotangent fragment sets per multiplier wave (1 in use)
 constexpr int BSP_SM_PITCH = BSP_ROWS_PER_DECODER + 1;
+constexpr int BSP_OCTET_PITCH = BSP_ROWS_PER_DECODER + 4;
 constexpr int BSP_MAX_ITEMS = 64;                  // items per workgroup (one wave builds the table)
 constexpr int BSP_GRID = 256;                      // one workgroup per CU
 
@@ -822,6 +831,14 @@ constexpr int BSP_GRID = 256;                      // one workgroup per CU
 template <int IMMEDIATE = 0>
 TGO_DEVICE void async_load16(u32x4 & destination, const void * base, uint32_t offset) {
     asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(destination) : "v"(offset), "s"(base), "n"(IMMEDIATE));
+}
+template <int YOUNGER>
+TGO_DEVICE void await_loads(u32x4 (&r)[2]) {
+    asm volatile("s_waitcnt vmcnt(%2)" : "+v"(r[0]), "+v"(r[1]) : "n"(YOUNGER));
+}
+template <int YOUNGER>
+TGO_DEVICE void await_loads(u32x4 (&r)[4]) {
+    asm volatile("s_waitcnt vmcnt(%4)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]) : "n"(YOUNGER));
 }
 template <int YOUNGER>
 TGO_DEVICE void await_loads(u32x4 (&r)[3]) {
@@ -840,6 +857,31 @@ struct SplitItem {
     int row_start;
     int row_end;
     int k_tile;
+    int step_begin;   // its range of reduction steps
+    int step_end;
+    int split;        // which range that is
+};
+
+// How the decoder waves fetch and hold a format's packed blocks: UNITS pieces of 16 bytes, parked side by side, PITCH bytes from
+// row to row.  Q4_K / Q5_K consist of such pieces.  Blocks of the others start on any even address, and so do their pieces
+// (memory takes that; LDS does not: a misaligned 16-byte write stalls it for 50 cycles, which fetching aligned units
+// and shifting them in the write cost, half of a Q6_K step).  None reaches over the ends of the block; the fields land at
+//   Q3_K   bytes 0 .. 95 where they are, the last piece is bytes 94 .. 109: scales from 98, d at 110
+//   Q6_K   bytes 0 .. 207 where they are, the last piece is bytes 194 .. 209: d at 222
+//   IQ2_S  bytes 2 .. 81 first (indices from 0, signs 32, upper index bits 64, scales 72), then bytes 0 .. 15: d at 80
+template <int TYPE>
+struct SplitBlock {
+    static constexpr int BLOCK = Format<TYPE>::BLOCK_BYTES;
+    static constexpr bool ALIGNED = BLOCK % 16 == 0;
+    static constexpr int UNITS = (BLOCK + 15) / 16;
+    static constexpr int piece_offset(int unit) {   // of a piece in the block
+        return TYPE == IQ2_S ? (unit == UNITS - 1 ? 0 : 2 + 16 * unit) : unit == UNITS - 1 ? BLOCK - 16 : 16 * unit;
+    }
+    static constexpr int PITCH = ALIGNED || UNITS % 2 == 1 ? 16 * UNITS : 16 * UNITS + 16;   // rows spread over the banks
+    static constexpr int SLOT_BYTES = BSP_ROWS_PER_DECODER * PITCH;
+    static constexpr int REGS = (BSP_ROWS_PER_DECODER * UNITS + 63) / 64;
+    static constexpr int SCALE_GROUPS = ALIGNED ? 4 : 8;   // scales in half a super-block
+    static constexpr int BIAS = TYPE == Q3_K ? 4 : TYPE == Q6_K ? 32 : TYPE == IQ2_S ? 128 : 0;   // of the quants as unsigned bytes
 };
 
 // Position in a workgroup's stream of reduction steps, with the item's description cached in scalars.
@@ -851,28 +893,29 @@ struct SplitCursor {
     int row_start;
     int row_end;
     int k_tile;
+    int step_begin;
+    int step_end;
     const uint8_t * base;   // where this step's loads start (meaning depends on the stage that owns the cursor)
 };
 
 template <int TYPE>
 __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(const BackwardArgs a,
                                                                               const int total_items) {
-    using F = Format<TYPE>;
-    static_assert(TYPE == Q4_K || TYPE == Q5_K, "16-byte aligned blocks only");
-    constexpr int RAW_UNITS = F::BLOCK_BYTES / 16;
-    // LDS pitch of a parked block: the block itself (a multiple of 16 bytes for these formats), so a wave's units
-    // land back to back with 16-byte writes; its readers address 16 rows at a time, which 36 or 44 words per row
-    // still spread over distinct banks
-    constexpr int BSP_RAW_PITCH = F::BLOCK_BYTES;
-    constexpr int RAW_REGS = (BSP_ROWS_PER_DECODER * RAW_UNITS + 63) / 64;
-    static_assert(RAW_REGS == 3, "await_loads takes three registers per step");
+    using B = SplitBlock<TYPE>;
+    constexpr bool K45 = TYPE == Q4_K || TYPE == Q5_K;
+    constexpr int RAW_UNITS = B::UNITS;
+    constexpr int BSP_RAW_PITCH = B::PITCH;
+    constexpr int RAW_REGS = B::REGS;
     constexpr int QS = TYPE == Q4_K ? 16 : 48;
     __shared__ __attribute__((aligned(16))) uint16_t wb[2][BWD_TK * BWD_PITCH];
-    __shared__ __attribute__((aligned(16))) uint8_t raw_all[4][3][BSP_ROWS_PER_DECODER * BSP_RAW_PITCH];
-    __shared__ float2 scale_min_all[4][2][4 * BSP_SM_PITCH];
+    __shared__ __attribute__((aligned(16))) uint8_t raw_all[4][3][B::SLOT_BYTES];
+    __shared__ float2 scale_min_all[4][2][B::SCALE_GROUPS * BSP_SM_PITCH];
+    // IQ2_S: codebook, and per decoder wave and step the (codebook index, signs) of each eight values and weight row
+    __shared__ uint2 grid[TYPE == IQ2_S ? TGO_IQ2S_GRID_ENTRIES : 1];
+    __shared__ __attribute__((aligned(16))) uint32_t octets_all[TYPE == IQ2_S ? 4 : 1][2][TYPE == IQ2_S ? 16 * BSP_OCTET_PITCH : 4];
     __shared__ __attribute__((aligned(16))) uint16_t stage_all[4][32 * (BWD_TK + 8)];
     __shared__ SplitItem items[BSP_MAX_ITEMS];
-    __shared__ int item_count;
+    __shared__ int item_count, step_count;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -882,13 +925,29 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
 
     // item table: slot i of this workgroup is linear item blockIdx.x + i * gridDim.x; empty slots (padding of
     // the task list) are squeezed out
+    const int n_total = a.out_features;
+    const int steps_per_source = (n_total + BWD_NS - 1) / BWD_NS;
+    if constexpr (TYPE == IQ2_S) {
+        expand_iq2s_grid(grid, tid, BSP_THREADS);
+    }
     if (wave == 0) {
-        SplitItem item = {0, 0, 0, -1};
+        SplitItem item = {0, 0, 0, -1, 0, steps_per_source, 0};
         const int64_t linear = blockIdx.x + static_cast<int64_t>(lane) * gridDim.x;
         if (linear < total_items) {
             int k_tile, task, first_task = 0, ordinary = 0;
             int tasks = (a.rows + BWD_TR - 1) / BWD_TR;
-            if (a.task_count != nullptr) {
+            if (a.n_splits > 1) {
+                // the two column tiles of a super-block side by side on an XCD: they read the same packed blocks
+                const int pairs = a.k_tiles / 2;
+                const int pair = static_cast<int>(linear) / (2 * XCDS) * XCDS + static_cast<int>(linear) % XCDS;
+                const int rest = pair / pairs;
+                k_tile = 2 * (pair - rest * pairs) + (static_cast<int>(linear) / XCDS) % 2;
+                task = rest % tasks;
+                item.split = rest / tasks;
+                item.step_begin = static_cast<int>(static_cast<int64_t>(steps_per_source) * item.split / a.n_splits);
+                item.step_end = static_cast<int>(static_cast<int64_t>(steps_per_source) * (item.split + 1) / a.n_splits);
+                task = item.split < a.n_splits ? task : tasks;
+            } else if (a.task_count != nullptr) {
                 task_segment(a, first_task, tasks, ordinary);   // (never the short segment: first_task is 0)
                 xcd_chunk(static_cast<int>(linear), a.k_tiles, tasks, ordinary, k_tile, task);
             } else {
@@ -912,8 +971,14 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
         if (valid) {
             items[__popcll(mask & ((1ull << lane) - 1ull))] = item;
         }
+        int steps = valid ? (item.step_end - item.step_begin) * a.sources : 0;
+#pragma unroll
+        for (int offset = 32; offset > 0; offset >>= 1) {
+            steps += __shfl_xor(steps, offset);
+        }
         if (lane == 0) {
             item_count = __popcll(mask);
+            step_count = steps;
         }
     }
     __syncthreads();
@@ -921,9 +986,7 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
     if (n_items == 0) {
         return;
     }
-    const int n_total = a.out_features;
-    const int steps_per_source = (n_total + BWD_NS - 1) / BWD_NS;
-    const int total_steps = n_items * steps_per_source * a.sources;
+    const int total_steps = step_count;
 
     auto item_field = [&](int item, int field) {
         return __builtin_amdgcn_readfirstlane(reinterpret_cast<const int *>(&items[item])[field]);
@@ -934,13 +997,15 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
         c.row_start = item_field(item, 1);
         c.row_end = item_field(item, 2);
         c.k_tile = item_field(item, 3);
+        c.step_begin = item_field(item, 4);
+        c.step_end = item_field(item, 5);
+        c.n_step = c.step_begin;
+        c.source = 0;
     };
-    // `rebase(cursor)` sets cursor.base for step 0 of the cursor's (item, source); within a source the base
+    // `rebase(cursor)` sets cursor.base for the first step of the cursor's (item, source); within a source the base
     // moves by `step_bytes` per step.
     auto first_step = [&](auto && rebase) {
         SplitCursor c;
-        c.source = 0;
-        c.n_step = 0;
         open_item(c, 0);
         rebase(c);
         return c;
@@ -948,20 +1013,18 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
     // A cursor at the last step stays there: stages that look past the end repeat it (harmless re-reads
     // instead of branches).  Returns true when the cursor moved to another item.
     auto advance = [&](SplitCursor & c, auto && rebase, int64_t step_bytes) {
-        if (c.n_step + 1 < steps_per_source) {
+        if (c.n_step + 1 < c.step_end) {
             ++c.n_step;
             c.base += step_bytes;
             return false;
         }
         if (c.source + 1 < a.sources) {
-            c.n_step = 0;
+            c.n_step = c.step_begin;
             ++c.source;
             rebase(c);
             return false;
         }
         if (c.item + 1 < n_items) {
-            c.n_step = 0;
-            c.source = 0;
             open_item(c, c.item + 1);
             rebase(c);
             return true;
@@ -983,19 +1046,20 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
         // row; the last step of a source clamps rows past the end of the matrix to its last row.
         const int tail_rows = n_total - (steps_per_source - 1) * BWD_NS;
         uint32_t unit_offset[RAW_REGS], unit_offset_tail[RAW_REGS];
+        const auto lane_row = [&](int i) { return min(lane + 64 * i, BSP_ROWS_PER_DECODER * RAW_UNITS - 1) / RAW_UNITS; };
+        const auto lane_unit = [&](int i) { return min(lane + 64 * i, BSP_ROWS_PER_DECODER * RAW_UNITS - 1) % RAW_UNITS; };
 #pragma unroll
         for (int i = 0; i < RAW_REGS; ++i) {
-            const int id = min(lane + 64 * i, BSP_ROWS_PER_DECODER * RAW_UNITS - 1);
-            const int row = dw * BSP_ROWS_PER_DECODER + id / RAW_UNITS;
-            const int unit = id % RAW_UNITS;
-            unit_offset[i] = static_cast<uint32_t>(row * a.row_bytes + unit * 16);
-            unit_offset_tail[i] = static_cast<uint32_t>(min(row, tail_rows - 1) * a.row_bytes + unit * 16);
+            const int row = dw * BSP_ROWS_PER_DECODER + lane_row(i);
+            const int piece = B::piece_offset(lane_unit(i));
+            unit_offset[i] = static_cast<uint32_t>(row * a.row_bytes + piece);
+            unit_offset_tail[i] = static_cast<uint32_t>(min(row, tail_rows - 1) * a.row_bytes + piece);
         }
+        const int64_t step_bytes = BWD_NS * a.row_bytes;
         auto rebase = [&](SplitCursor & c) {
             c.base = (c.source == 0 ? packed_of[0] : packed_of[1]) + static_cast<int64_t>(c.expert) * a.bytes_per_expert +
-                     static_cast<int64_t>(c.k_tile >> 1) * F::BLOCK_BYTES;
+                     static_cast<int64_t>(c.k_tile >> 1) * B::BLOCK + c.step_begin * step_bytes;
         };
-        const int64_t step_bytes = BWD_NS * a.row_bytes;
         auto load_raw = [&](const SplitCursor & c, u32x4 (&regs)[RAW_REGS]) {
             const bool tail = c.n_step == steps_per_source - 1;
 #pragma unroll
@@ -1008,11 +1072,7 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
             await_loads<RAW_YOUNGER>(regs);
 #pragma unroll
             for (int i = 0; i < RAW_REGS; ++i) {
-                const int id = min(lane + 64 * i, BSP_ROWS_PER_DECODER * RAW_UNITS - 1);
-                const int row = id / RAW_UNITS;
-                const int unit = id - row * RAW_UNITS;
-                static_assert(BSP_RAW_PITCH == RAW_UNITS * 16, "consecutive lanes write consecutive 16-byte units");
-                *reinterpret_cast<u32x4 *>(raw + row * BSP_RAW_PITCH + unit * 16) = regs[i];
+                *reinterpret_cast<u32x4 *>(raw + lane_row(i) * BSP_RAW_PITCH + 16 * lane_unit(i)) = regs[i];
             }
         };
         // Stages 2 and 3 are each split into the LDS reads and the arithmetic on what was read, so that the
@@ -1021,36 +1081,82 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
         //
         // stage 2: (d * sc, dmin * m) of this lane's (row, 32-value group); rows past the end of the weight
         // matrix get (0, 0) and therefore decode to exact zeros
+        // The other formats have a scale per 16 values and a constant bias of the quants instead: (s, bias * s), and the
+        // lane's two groups.  IQ2_S: also the codebook indices and signs of the lane's four octets of values.
         struct ScaleInputs {
-            uint32_t d_dmin, low, mid, high;   // the 16-byte block header: two halves, then 12 bytes of 6-bit fields
+            uint32_t d_dmin, low, mid, high;   // Q4_K / Q5_K: the 16-byte block header: two halves, then 12 bytes of 6-bit fields
         };
-        auto scales_fetch = [&](const uint8_t * raw) {
+        auto scales_fetch = [&](int info, const uint8_t * raw) {
             const uint8_t * blk = raw + (lane & 15) * BSP_RAW_PITCH;
-            ScaleInputs in;
-            in.d_dmin = lds_u32(blk);
-            in.low = lds_u32(blk + 4);
-            in.mid = lds_u32(blk + 8);
-            in.high = lds_u32(blk + 12);
+            const int pair = lane >> 4;
+            const int half_block = info & 1;
+            ScaleInputs in = {0, 0, 0, 0};
+            if constexpr (K45) {
+                in.d_dmin = lds_u32(blk);
+                in.low = lds_u32(blk + 4);
+                in.mid = lds_u32(blk + 8);
+                in.high = lds_u32(blk + 12);
+            } else if constexpr (TYPE == Q3_K) {
+                in.d_dmin = lds_u16(blk + 110);
+                in.low = lds_u16(blk + 98 + 2 * pair);
+                in.mid = lds_u16(blk + 106 + 2 * (pair & 1));
+            } else if constexpr (TYPE == Q6_K) {
+                in.d_dmin = lds_u16(blk + 222);
+                in.low = lds_u16(blk + 192 + 8 * half_block + 2 * pair);
+            } else {
+                in.d_dmin = lds_u16(blk + 80) | (static_cast<uint32_t>(blk[72 + 4 * half_block + pair]) << 16);
+                in.low = lds_u32(blk + 16 * half_block + 4 * pair);        // codebook indices of four octets, eight bits each
+                in.mid = lds_u32(blk + 32 + 16 * half_block + 4 * pair);   // their signs
+                in.high = blk[64 + 4 * half_block + pair];                 // the indices' upper two bits
+            }
             return in;
         };
-        auto scales_finish = [&](int info, const ScaleInputs & in, float2 * scale_min) {
+        auto scales_finish = [&](int info, const ScaleInputs & in, float2 * scale_min, uint32_t * octets) {
             const int n = lane & 15;
-            const int group_local = lane >> 4;
-            const int shift = 8 * group_local;
-            const uint32_t b0 = (in.low >> shift) & 0xffu, b1 = (in.mid >> shift) & 0xffu, b2 = (in.high >> shift) & 0xffu;
-            uint32_t sc, mn;
-            if ((info & 1) == 0) {   // groups 0..3 of the super-block: plain 6-bit fields
-                sc = b0 & 63u;
-                mn = b1 & 63u;
-            } else {                 // groups 4..7: low nibbles in the third word, top two bits above the first eight
-                sc = (b2 & 15u) | ((b0 >> 6) << 4);
-                mn = (b2 >> 4) | ((b1 >> 6) << 4);
-            }
             const bool valid = (info >> 1) * BWD_NS + dw * BSP_ROWS_PER_DECODER + n < n_total;
-            scale_min[group_local * BSP_SM_PITCH + n] =
-                valid ? make_float2(half_bits_to_float(in.d_dmin & 0xffffu) * static_cast<float>(sc),
-                                    half_bits_to_float(in.d_dmin >> 16) * static_cast<float>(mn))
-                      : make_float2(0.0f, 0.0f);
+            if constexpr (K45) {
+                const int group_local = lane >> 4;
+                const int shift = 8 * group_local;
+                const uint32_t b0 = (in.low >> shift) & 0xffu, b1 = (in.mid >> shift) & 0xffu, b2 = (in.high >> shift) & 0xffu;
+                uint32_t sc, mn;
+                if ((info & 1) == 0) {   // groups 0..3 of the super-block: plain 6-bit fields
+                    sc = b0 & 63u;
+                    mn = b1 & 63u;
+                } else {                 // groups 4..7: low nibbles in the third word, top two bits above the first eight
+                    sc = (b2 & 15u) | ((b0 >> 6) << 4);
+                    mn = (b2 >> 4) | ((b1 >> 6) << 4);
+                }
+                scale_min[group_local * BSP_SM_PITCH + n] =
+                    valid ? make_float2(half_bits_to_float(in.d_dmin & 0xffffu) * static_cast<float>(sc),
+                                        half_bits_to_float(in.d_dmin >> 16) * static_cast<float>(mn))
+                          : make_float2(0.0f, 0.0f);
+            } else {
+                const int pair = lane >> 4;
+                const float d = half_bits_to_float(in.d_dmin & 0xffffu);
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    float scale;
+                    if constexpr (TYPE == Q3_K) {
+                        const uint32_t low = (in.low >> (8 * g + 4 * (info & 1))) & 15u;
+                        const uint32_t high = (in.mid >> (8 * g + 4 * (info & 1) + 2 * (pair >> 1))) & 3u;
+                        scale = d * static_cast<float>(static_cast<int>(low | (high << 4)) - 32);
+                    } else if constexpr (TYPE == Q6_K) {
+                        scale = d * static_cast<float>(static_cast<int>(in.low << (24 - 8 * g)) >> 24);
+                    } else {
+                        scale = d * 0.125f * static_cast<float>(((in.d_dmin >> (16 + 4 * g)) & 15u) * 2 + 1);
+                    }
+                    // (products of an 11-bit and an at most 8-bit number: exact, and so is the bias, a power of two)
+                    scale = valid ? scale : 0.0f;
+                    scale_min[(2 * pair + g) * BSP_SM_PITCH + n] = make_float2(scale, scale * B::BIAS);
+                }
+                if constexpr (TYPE == IQ2_S) {
+#pragma unroll
+                    for (int o = 0; o < 4; ++o) {
+                        const uint32_t index = ((in.low >> (8 * o)) & 0xffu) | (((in.high >> (2 * o)) & 3u) << 8);
+                        octets[(4 * pair + o) * BSP_OCTET_PITCH + n] = index | (((in.mid >> (8 * o)) & 0xffu) << 16);
+                    }
+                }
+            }
         };
         // stage 3: a lane decodes 8 weight rows x 4 consecutive K positions and stores each K position's
         // eight bf16 values with one 16-byte write
@@ -1062,17 +1168,37 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
         const int word = (lane >> 1) & 15;
         const int nibble = lane >> 5;
         const int position = (word & 7) * 4;
-        const int group_local = 2 * (word >> 3) + nibble;
-        auto decode_fetch = [&](int info, const uint8_t * raw, const float2 * scale_min) {
+        // Q4_K / Q5_K: two lanes share a word, a nibble each.  The others: 4 * (lane >> 1) is the lane's position in the half.
+        const int group_local = K45 ? 2 * (word >> 3) + nibble : lane >> 4;                  // 32-value group inside the half block
+        const int scale_group = K45 ? group_local : lane >> 3;
+        auto decode_fetch = [&](int info, const uint8_t * raw, const float2 * scale_min, const uint32_t * octets) {
             const int half_block = info & 1;
             DecodeInputs in;
+            if constexpr (TYPE == IQ2_S) {
+                const uint32_t * mine = octets + (lane >> 2) * BSP_OCTET_PITCH + 8 * octet;
+                const uint4 low = *reinterpret_cast<const uint4 *>(mine), high = *reinterpret_cast<const uint4 *>(mine + 4);
+                const uint32_t records[8] = {low.x, low.y, low.z, low.w, high.x, high.y, high.z, high.w};
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    in.qs[i] = reinterpret_cast<const uint32_t *>(grid)[2 * (records[i] & 0x3ffu) + ((lane >> 1) & 1)];
+                    in.qh[i] = records[i] >> 16;
+                }
+            }
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const int n = 8 * octet + i;
                 const uint8_t * blk = raw + n * BSP_RAW_PITCH;
-                in.qs[i] = lds_u32(blk + QS + 64 * half_block + 4 * word);
-                in.qh[i] = TYPE == Q5_K ? lds_u32(blk + 16 + position) : 0u;
-                in.sm[i] = scale_min[group_local * BSP_SM_PITCH + n];
+                if constexpr (K45) {
+                    in.qs[i] = lds_u32(blk + QS + 64 * half_block + 4 * word);
+                    in.qh[i] = TYPE == Q5_K ? lds_u32(blk + 16 + position) : 0u;
+                } else if constexpr (TYPE == Q3_K) {
+                    in.qs[i] = lds_u32(blk + 32 + 32 * half_block + 4 * ((lane >> 1) & 7));
+                    in.qh[i] = lds_u32(blk + 4 * ((lane >> 1) & 7));
+                } else if constexpr (TYPE == Q6_K) {
+                    in.qs[i] = lds_u32(blk + 64 * half_block + 4 * ((lane >> 1) & 15));
+                    in.qh[i] = lds_u32(blk + 128 + 32 * half_block + 4 * ((lane >> 1) & 7));
+                }
+                in.sm[i] = scale_min[scale_group * BSP_SM_PITCH + n];
             }
             return in;
         };
@@ -1081,16 +1207,27 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
             float w[4][8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                uint32_t q = (in.qs[i] >> (4 * nibble)) & 0x0f0f0f0fu;
-                if constexpr (TYPE == Q5_K) {
-                    q |= ((in.qh[i] >> group) & 0x01010101u) << 4;
+                uint32_t q;   // four quants as unsigned bytes, above their true values by the bias
+                if constexpr (K45) {
+                    q = (in.qs[i] >> (4 * nibble)) & 0x0f0f0f0fu;
+                    if constexpr (TYPE == Q5_K) {
+                        q |= ((in.qh[i] >> group) & 0x01010101u) << 4;
+                    }
+                } else if constexpr (TYPE == Q3_K) {
+                    q = ((in.qs[i] >> (2 * group_local)) & 0x03030303u) | (((in.qh[i] >> group) & 0x01010101u) << 2);
+                } else if constexpr (TYPE == Q6_K) {
+                    q = ((in.qs[i] >> (4 * nibble)) & 0x0f0f0f0fu) | (((in.qh[i] >> (2 * group_local)) & 0x03030303u) << 4);
+                } else {
+                    // the four signs spread to a bit per byte; a negative magnitude is its complement plus one
+                    const uint32_t negative = (((in.qh[i] >> (4 * ((lane >> 1) & 1))) & 15u) * 0x00204081u) & 0x01010101u;
+                    q = ((in.qs[i] ^ (negative * 0xffu)) + negative) ^ 0x80808080u;
                 }
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     w[e][i] = in.sm[i].x * static_cast<float>((q >> (8 * e)) & 0xffu) - in.sm[i].y;
                 }
             }
-            const int k_local = 32 * group_local + position;
+            const int k_local = K45 ? 32 * group_local + position : 4 * (lane >> 1);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const uint4 packed = make_uint4(pack_bf16x2(w[e][0], w[e][1]), pack_bf16x2(w[e][2], w[e][3]),
@@ -1105,6 +1242,7 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
         };
         auto raw_slot = [&](int slot) { return raw_all[dw][slot]; };
         auto sm_slot = [&](int slot) { return scale_min_all[dw][slot]; };
+        auto octet_slot = [&](int slot) { return octets_all[TYPE == IQ2_S ? dw : 0][slot]; };
 
         // Step t uses raw slot t % 3, scale slot t & 1, tile t & 1 and register set t % 4.  Only the load
         // stage walks the item list; what the later stages need to know about a step (which half of the
@@ -1130,11 +1268,11 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
             request(ring[t]);
         }
         wave_sync();
-        scales_finish(info[6], scales_fetch(raw_slot(0)), sm_slot(0));
-        scales_finish(info[5], scales_fetch(raw_slot(1)), sm_slot(1));
+        scales_finish(info[6], scales_fetch(info[6], raw_slot(0)), sm_slot(0), octet_slot(0));
+        scales_finish(info[5], scales_fetch(info[5], raw_slot(1)), sm_slot(1), octet_slot(1));
         wave_sync();
-        decode_finish(info[6], decode_fetch(info[6], raw_slot(0), sm_slot(0)), wb[0]);
-        DecodeInputs pending = decode_fetch(info[5], raw_slot(1), sm_slot(1));   // step 1
+        decode_finish(info[6], decode_fetch(info[6], raw_slot(0), sm_slot(0), octet_slot(0)), wb[0]);
+        DecodeInputs pending = decode_fetch(info[5], raw_slot(1), sm_slot(1), octet_slot(1));   // step 1
         __syncthreads();
         // While the multipliers consume step g: finish decoding g + 1 (its inputs were read from LDS during
         // the previous round), scales of g + 2 (inputs read first thing, used after the decode), park g + 3,
@@ -1150,13 +1288,13 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
                 if (g < total_steps) {
                     const int g3_plus1 = g3 == 2 ? 0 : g3 + 1;
                     const int g3_plus2 = g3_plus1 == 2 ? 0 : g3_plus1 + 1;
-                    const ScaleInputs scale_inputs = scales_fetch(raw_slot(g3_plus2));
+                    const ScaleInputs scale_inputs = scales_fetch(info[4], raw_slot(g3_plus2));
                     __builtin_amdgcn_sched_barrier(0);
                     decode_finish(info[5], pending, wb[(g + 1) & 1]);
-                    scales_finish(info[4], scale_inputs, sm_slot(g & 1));
+                    scales_finish(info[4], scale_inputs, sm_slot(g & 1), octet_slot(g & 1));
                     park(ring[(u + 3) % BSP_RAW_DEPTH], raw_slot(g3));
                     wave_sync();
-                    pending = decode_fetch(info[4], raw_slot(g3_plus2), sm_slot(g & 1));
+                    pending = decode_fetch(info[4], raw_slot(g3_plus2), sm_slot(g & 1), octet_slot(g & 1));
                     request(ring[(u + 3) % BSP_RAW_DEPTH]);
                     __builtin_amdgcn_sched_barrier(0);
                     g3 = g3_plus1;
@@ -1194,7 +1332,9 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
             async_load16<3072>(regs[rt][3], c.base, fetch_offset[rt]);
         }
     };
-    auto rebase_fetch = [&](SplitCursor & c) { c.base = c.source == 0 ? cotangent_of[0] : cotangent_of[1]; };
+    auto rebase_fetch = [&](SplitCursor & c) {
+        c.base = (c.source == 0 ? cotangent_of[0] : cotangent_of[1]) + static_cast<int64_t>(c.step_begin) * ((BWD_NS / 16) * 1024);
+    };
     auto rebase_none = [&](SplitCursor &) {};
 
     v16f acc[2][4];
@@ -1265,7 +1405,7 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
                         }
                         __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);   // MFMAs
                     }
-                    if (c_now.source == a.sources - 1 && c_now.n_step == steps_per_source - 1) {
+                    if (c_now.source == a.sources - 1 && c_now.n_step == c_now.step_end - 1) {
                         // last step of the item: transpose the results through this wave's staging area
                         // and write whole rows, then start the next item from zero
                         const int k_tile = c_now.k_tile;
@@ -1276,7 +1416,10 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
 #pragma unroll
                         for (int rt = 0; rt < 2; ++rt) {
                             const int r0 = wave_row + rt * 32;
-                            if (r0 < row_end) {
+                            if (a.n_splits > 1) {
+                                store_partial_32x128(a, acc[rt], item_field(c_now.item, 6), r0 + (lane_here & 31), row_end, k_tile,
+                                                     lane_here >> 5);
+                            } else if (r0 < row_end) {
                                 store_rows_32x128<BWD_TK + 8, true, true>(
                                     stage_all[wave], acc[rt],
                                     a.dx + static_cast<int64_t>(r0) * a.in_features + k_tile * BWD_TK, a.in_features,
@@ -1716,30 +1859,25 @@ static hipError_t launch_backward_typed(const BackwardArgs & args, hipStream_t s
             return status;
         }
     }
-    if (args.n_splits > 1) {
-        // (every format takes the general kernel here: what this path needs is many short workgroups)
-        const dim3 grid(static_cast<unsigned>(total), static_cast<unsigned>(args.n_splits));
-        general(std::false_type{}, grid, args);
+    // the role-split kernel addresses the packed cotangent and a step's weight rows with 32-bit lane offsets
+    const bool role_split = cotangent_workspace_bytes(args.rows, args.out_features) < (int64_t{1} << 32) &&
+                      args.row_bytes * 2 * BWD_NS < (int64_t{1} << 32);
+    const bool splits = args.n_splits > 1;
+    if (role_split) {
+        // one persistent workgroup per CU, more only when a workgroup's item table would overflow
+        const int tasks = (args.rows + BWD_TR - 1) / BWD_TR;
+        const int64_t items = splits ? (static_cast<int64_t>(args.k_tiles / 2) * tasks * args.n_splits + XCDS - 1) / XCDS * XCDS * 2 : total;
+        const int64_t needed = (items + BSP_MAX_ITEMS - 1) / BSP_MAX_ITEMS;
+        const int64_t grid = (std::max<int64_t>(std::min<int64_t>(items, BSP_GRID), needed) + XCDS - 1) / XCDS * XCDS;
+        mmq_grad_input_split_kernel<TYPE><<<static_cast<unsigned>(grid), BSP_THREADS, 0, stream>>>(args, static_cast<int>(items));
+    } else {
+        general(std::false_type{}, dim3(static_cast<unsigned>(total), static_cast<unsigned>(args.n_splits)), args);
+    }
+    if (splits) {
         const int64_t count = static_cast<int64_t>(args.rows) * args.in_features;
         reduce_partials_kernel<<<static_cast<unsigned>((count / 8 + 255) / 256), 256, 0, stream>>>(
             args.partial, args.dx, count, args.n_splits);
-        return hipGetLastError();
     }
-    // the role-split kernel addresses the packed cotangent and a step's weight rows with 32-bit lane offsets
-    const bool small_offsets = cotangent_workspace_bytes(args.rows, args.out_features) < (int64_t{1} << 32) &&
-                               args.row_bytes * 2 * BWD_NS < (int64_t{1} << 32);
-    if constexpr (TYPE == Q4_K || TYPE == Q5_K) {
-        if (small_offsets) {
-            // one persistent workgroup per CU, more only when a workgroup's item table would overflow
-            const int64_t needed = (total + BSP_MAX_ITEMS - 1) / BSP_MAX_ITEMS;
-            const int64_t grid =
-                (std::max<int64_t>(std::min<int64_t>(total, BSP_GRID), needed) + XCDS - 1) / XCDS * XCDS;
-            mmq_grad_input_split_kernel<TYPE><<<static_cast<unsigned>(grid), BSP_THREADS, 0, stream>>>(
-                args, static_cast<int>(total));
-            return hipGetLastError();
-        }
-    }
-    general(std::false_type{}, dim3(static_cast<unsigned>(total)), args);
     return hipGetLastError();
 }
 
@@ -1752,7 +1890,7 @@ hipError_t launch_mmq_grad_input(const uint8_t * cotangent_first, const uint8_t 
     // `partial` (dense calls only): room for dense_grad_splits() fp32 copies of the result, or nullptr
     args.partial = partial;
     args.n_splits = tasks == nullptr && partial != nullptr
-        ? dense_grad_splits(rows, out_features, in_features, has_role_split(quant_type)) : 1;
+        ? dense_grad_splits(rows, out_features, in_features) : 1;
     args.cotangent[0] = cotangent_first;
     args.cotangent[1] = cotangent_second;
     args.packed[0] = packed_first;

@@ -72,26 +72,23 @@ constexpr int GEMV_DENSE_ROWS = 32;
 // rows, 64 per step) alone, so a call of a few hundred rows keeps K / 128 workgroups busy and takes as long as one
 // of them needs for N / 64 dependent steps.  Such calls cut the reduction into this many ranges, one workgroup each,
 // which leave fp32 partial results that a second kernel adds up in a fixed order.  1: no split.
-// `role_split`: the format has the role-split kernel (Q4_K, Q5_K), which loses to this scheme only up to 32
-// items; the general kernel of the other formats gains from a second workgroup per CU up to 256 items.
-static inline int dense_grad_splits(int64_t rows, int64_t out_features, int64_t in_features, bool role_split) {
+// The line lies at half the CUs: 4096 x 2048 Q4_K, 1024 rows (64 items, four ranges) 62 -> 41 us, 2048 rows (128, two) 70 -> 61.
+// Short reductions (fewer than 32 steps) gain from it up to an eighth of the CUs only: 1024 x 4096, 512 rows 24 -> 30 us.
+constexpr int BACKWARD_WORKGROUPS = 256;   // one per CU
+static inline int dense_grad_splits(int64_t rows, int64_t out_features, int64_t in_features) {
     const int64_t items = (rows + BACKWARD_ROW_TILE - 1) / BACKWARD_ROW_TILE * (in_features / 128);
     const int64_t steps = (out_features + 63) / 64;
-    if (items > (role_split ? 32 : 256)) {
+    if (items > (steps < 32 ? 32 : 128)) {
         return 1;
     }
-    // about one workgroup per CU for a single row tile, two beyond (measured: with one row tile a second
-    // workgroup per CU only lengthens everyone's first loads)
-    int64_t splits = (rows <= BACKWARD_ROW_TILE ? 256 : 512) / items;
+    int64_t splits = BACKWARD_WORKGROUPS / items;
     splits = splits < steps / 2 ? splits : steps / 2;   // at least two steps each
     splits = splits < 16 ? splits : 16;
     return splits < 2 ? 1 : static_cast<int>(splits);
 }
-// Q4_K (12) and Q5_K (13) have the role-split kernel.
-static inline bool has_role_split(int quant_type) { return quant_type == 12 || quant_type == 13; }
-// fp32 scratch of the split reduction for a dense call of this format: the same decision as the launcher's
-static inline int64_t dense_grad_partial_bytes(int64_t rows, int64_t out_features, int64_t in_features, int quant_type) {
-    const int splits = dense_grad_splits(rows, out_features, in_features, has_role_split(quant_type));
+// fp32 scratch of the split reduction for a dense call: the same decision as the launcher's
+static inline int64_t dense_grad_partial_bytes(int64_t rows, int64_t out_features, int64_t in_features) {
+    const int splits = dense_grad_splits(rows, out_features, in_features);
     return splits > 1 ? splits * rows * in_features * 4 : 0;
 }
 
