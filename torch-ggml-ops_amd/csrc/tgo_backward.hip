@@ -862,25 +862,13 @@ struct SplitItem {
     int split;        // which range that is
 };
 
-// How the decoder waves fetch and hold a format's packed blocks: UNITS pieces of 16 bytes, parked side by side, PITCH bytes from
-// row to row.  Q4_K / Q5_K consist of such pieces.  Blocks of the others start on any even address, and so do their pieces
-// (memory takes that; LDS does not: a misaligned 16-byte write stalls it for 50 cycles, which fetching aligned units
-// and shifting them in the write cost, half of a Q6_K step).  None reaches over the ends of the block; the fields land at
-//   Q3_K   bytes 0 .. 95 where they are, the last piece is bytes 94 .. 109: scales from 98, d at 110
-//   Q6_K   bytes 0 .. 207 where they are, the last piece is bytes 194 .. 209: d at 222
-//   IQ2_S  bytes 2 .. 81 first (indices from 0, signs 32, upper index bits 64, scales 72), then bytes 0 .. 15: d at 80
+// How the decoder waves hold a format's packed blocks.
 template <int TYPE>
-struct SplitBlock {
-    static constexpr int BLOCK = Format<TYPE>::BLOCK_BYTES;
-    static constexpr bool ALIGNED = BLOCK % 16 == 0;
-    static constexpr int UNITS = (BLOCK + 15) / 16;
-    static constexpr int piece_offset(int unit) {   // of a piece in the block
-        return TYPE == IQ2_S ? (unit == UNITS - 1 ? 0 : 2 + 16 * unit) : unit == UNITS - 1 ? BLOCK - 16 : 16 * unit;
-    }
-    static constexpr int PITCH = ALIGNED || UNITS % 2 == 1 ? 16 * UNITS : 16 * UNITS + 16;   // rows spread over the banks
-    static constexpr int SLOT_BYTES = BSP_ROWS_PER_DECODER * PITCH;
-    static constexpr int REGS = (BSP_ROWS_PER_DECODER * UNITS + 63) / 64;
-    static constexpr int SCALE_GROUPS = ALIGNED ? 4 : 8;   // scales in half a super-block
+struct SplitBlock : BlockPieces<TYPE> {
+    using P = BlockPieces<TYPE>;
+    static constexpr int SLOT_BYTES = BSP_ROWS_PER_DECODER * P::PITCH;
+    static constexpr int REGS = (BSP_ROWS_PER_DECODER * P::UNITS + 63) / 64;
+    static constexpr int SCALE_GROUPS = P::ALIGNED ? 4 : 8;   // scales in half a super-block
     static constexpr int BIAS = TYPE == Q3_K ? 4 : TYPE == Q6_K ? 32 : TYPE == IQ2_S ? 128 : 0;   // of the quants as unsigned bytes
 };
 
@@ -1051,7 +1039,7 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
 #pragma unroll
         for (int i = 0; i < RAW_REGS; ++i) {
             const int row = dw * BSP_ROWS_PER_DECODER + lane_row(i);
-            const int piece = B::piece_offset(lane_unit(i));
+            const int piece = B::offset(lane_unit(i));
             unit_offset[i] = static_cast<uint32_t>(row * a.row_bytes + piece);
             unit_offset_tail[i] = static_cast<uint32_t>(min(row, tail_rows - 1) * a.row_bytes + piece);
         }

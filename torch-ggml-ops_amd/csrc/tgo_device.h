@@ -368,6 +368,25 @@ static __host__ __device__ inline bool wide_stage_ok(const void * packed, int64_
     return (reinterpret_cast<uintptr_t>(packed) & 15) == 0 && (bytes_per_expert & 15) == 0;
 }
 
+// ---- packed blocks as 16-byte pieces at their own addresses ------------------------------------------------------
+// UNITS pieces of 16 bytes, parked side by side in LDS, PITCH bytes from row to row.  Q4_K / Q5_K consist of such pieces.
+// Blocks of the others start on any even address, and so do their pieces (memory takes that; LDS does not: a misaligned
+// 16-byte write stalls it for 50 cycles, which fetching aligned units and shifting them in the write cost).  None reaches over
+// the ends of its block, and in LDS every field that is read as words is aligned, except Q3_K's scales:
+//   Q3_K   bytes 0 .. 95 where they are, the last piece is bytes 94 .. 109: scales from 98, d at 110
+//   Q6_K   bytes 0 .. 207 where they are, the last piece is bytes 194 .. 209: d at 222
+//   IQ2_S  bytes 2 .. 81 first (indices from 0, signs 32, upper index bits 64, scales 72), then bytes 0 .. 15: d at 80
+template <int TYPE>
+struct BlockPieces {
+    static constexpr int BLOCK = Format<TYPE>::BLOCK_BYTES;
+    static constexpr bool ALIGNED = BLOCK % 16 == 0;
+    static constexpr int UNITS = (BLOCK + 15) / 16;
+    static constexpr int offset(int unit) {   // of a piece in the block
+        return TYPE == IQ2_S ? (unit == UNITS - 1 ? 0 : 2 + 16 * unit) : unit == UNITS - 1 ? BLOCK - 16 : 16 * unit;
+    }
+    static constexpr int PITCH = UNITS % 2 == 1 ? 16 * UNITS : 16 * UNITS + 16;   // (4 * odd words: rows spread over the banks)
+};
+
 template <int REGS>
 struct WideRegs {
     u32x4_t unit[REGS];

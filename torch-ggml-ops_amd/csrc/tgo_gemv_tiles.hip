@@ -14,7 +14,7 @@
 // weight row col.  Its B operand is 32 values of K x 16 activation rows: lane (col, part) holds the same values of row col.
 // Neighbouring lanes therefore hold different rows, and a load from memory in that arrangement costs the address unit a
 // cycle per lane (measured: the kernel then waits for that unit alone, at 2 TB/s).  So a wave fetches the packed
-// blocks of its 16 weight rows as 16-byte units, neighbouring lanes neighbouring units, two steps ahead into registers,
+// blocks of its 16 weight rows as 16-byte pieces, neighbouring lanes neighbouring pieces, two steps ahead into registers,
 // parks them in LDS of its own, and reads each lane's bytes from there; the activations go the same way, once per
 // super-block.  LDS executes a wave's accesses in order, so no barrier is needed anywhere in the loop.
 // A wave walks a range of super-blocks (the four waves of a workgroup split K, up to four ways) and, for each, its R tiles of
@@ -24,9 +24,9 @@
 // 52 % of the vector units' time), however many rows a task has, beside LDS (27 %) and the packed bytes (28672 x 8192 Q4_K:
 // 39 us, 3.4 TB/s); a fetch ring of four steps or a third workgroup per CU changed nothing.  The kernels of tgo_gemv.hip
 // pay four v_dot4 plus scaling per 16 weights and activation row instead and need no whole tiles: better for one to three
-// rows.  Measured against them, gate and up of 256 experts (2048 x 512) for 97 tokens of eight choices: Q3_K 174 -> 81 us, Q5_K
-// 133 -> 92, IQ2_S 137 -> 108; down (512 x 2048): Q4_K 105 -> 46, Q6_K 89 -> 80; dense 28672 x 8192, 16 rows: Q3_K 230 -> 52,
-// Q4_K 65 -> 46, Q6_K 160 -> 81.
+// rows.  Measured against them, gate and up of 256 experts (2048 x 512) for 97 tokens of eight choices: Q3_K 174 -> 75 us, Q5_K
+// 133 -> 92, IQ2_S 137 -> 87; down (512 x 2048): Q4_K 105 -> 45, Q6_K 89 -> 73; dense 28672 x 8192, 16 rows: Q3_K 230 -> 44,
+// Q4_K 65 -> 46, Q6_K 160 -> 69.
 #include <algorithm>
 #include <type_traits>
 
@@ -67,7 +67,6 @@ struct TilesArgs {
 };
 
 // ---- a lane's share of a super-block --------------------------------------------------------------------------------
-// (In LDS a block's fields are aligned, whatever its address in memory: TileSlot.)
 // Eight values (8 part .. + 7) of each of the super-block's eight 32-value blocks, packed, and the scales.
 template <int TYPE> struct LaneBlock;
 template <> struct LaneBlock<Q4_K> { uint4 header; uint2 q[4]; };
@@ -76,7 +75,7 @@ template <> struct LaneBlock<Q3_K> { uint2 q[2], high; uint4 scales; };
 template <> struct LaneBlock<Q6_K> { uint2 low[4], high[2]; uint4 scales; uint16_t d; };
 template <> struct LaneBlock<IQ2_S> { uint4 index[2], sign[2]; uint2 high, scales; uint16_t d; };
 
-// `row`: the lane's block in LDS (IQ2_S: 14 bytes before a multiple of 16, others: at one); `mine`: row + 8 * part.
+// `row`: the lane's block in LDS as BlockPieces lays it out; `mine`: row + 8 * part.
 template <int TYPE>
 TGO_DEVICE void lane_load(LaneBlock<TYPE> & r, const uint8_t * row, const uint8_t * mine) {
     if constexpr (TYPE == Q4_K || TYPE == Q5_K) {
@@ -92,7 +91,10 @@ TGO_DEVICE void lane_load(LaneBlock<TYPE> & r, const uint8_t * row, const uint8_
         r.q[0] = *reinterpret_cast<const uint2 *>(mine + 32);
         r.q[1] = *reinterpret_cast<const uint2 *>(mine + 64);
         r.high = *reinterpret_cast<const uint2 *>(mine);
-        r.scales = *reinterpret_cast<const uint4 *>(row + 96);   // (and d)
+        // (two bytes of quants, the scales, d)
+        const uint4 tail = *reinterpret_cast<const uint4 *>(row + 96);
+        r.scales = make_uint4(__builtin_amdgcn_alignbyte(tail.y, tail.x, 2), __builtin_amdgcn_alignbyte(tail.z, tail.y, 2),
+                              __builtin_amdgcn_alignbyte(tail.w, tail.z, 2), tail.w >> 16);
     } else if constexpr (TYPE == Q6_K) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -101,38 +103,19 @@ TGO_DEVICE void lane_load(LaneBlock<TYPE> & r, const uint8_t * row, const uint8_
         r.high[0] = *reinterpret_cast<const uint2 *>(mine + 128);
         r.high[1] = *reinterpret_cast<const uint2 *>(mine + 160);
         r.scales = *reinterpret_cast<const uint4 *>(row + 192);
-        r.d = *reinterpret_cast<const uint16_t *>(row + 208);
+        r.d = *reinterpret_cast<const uint16_t *>(row + 222);
     } else {
         // (a lane's eight values of a block are one codebook index byte, one sign byte and two index bits: it takes the
         // words that hold those of all four lanes of its row)
-        r.d = *reinterpret_cast<const uint16_t *>(row);
-        r.index[0] = *reinterpret_cast<const uint4 *>(row + 2);
-        r.index[1] = *reinterpret_cast<const uint4 *>(row + 18);
-        r.sign[0] = *reinterpret_cast<const uint4 *>(row + 34);
-        r.sign[1] = *reinterpret_cast<const uint4 *>(row + 50);
-        r.high = *reinterpret_cast<const uint2 *>(row + 66);
-        r.scales = *reinterpret_cast<const uint2 *>(row + 74);
+        r.d = *reinterpret_cast<const uint16_t *>(row + 80);
+        r.index[0] = *reinterpret_cast<const uint4 *>(row);
+        r.index[1] = *reinterpret_cast<const uint4 *>(row + 16);
+        r.sign[0] = *reinterpret_cast<const uint4 *>(row + 32);
+        r.sign[1] = *reinterpret_cast<const uint4 *>(row + 48);
+        r.high = *reinterpret_cast<const uint2 *>(row + 64);
+        r.scales = *reinterpret_cast<const uint2 *>(row + 72);
     }
 }
-
-// The packed blocks of 16 weight rows in LDS, PITCH bytes from row to row (4 * odd words: the lanes of a read, which differ
-// in the row, spread over the banks).  They travel as the aligned 16-byte units of memory that cover them, but a unit is
-// stored at the place of its bytes in the block, so the blocks, and with them the words that the lanes read, are aligned in
-// LDS: Q3_K, Q6_K and IQ2_S blocks start on any even address in memory, and an unaligned LDS access takes more than twice as
-// long (there are two to four such writes per step instead of four to seven such reads).  IQ2_S blocks start SHIFT bytes in,
-// which aligns everything behind their scale.  The bytes of the neighbouring blocks that come along land in the padding.
-template <int TYPE>
-struct TileSlot {
-    static constexpr int BLOCK = Format<TYPE>::BLOCK_BYTES;
-    static constexpr bool ALIGNED = BLOCK % 16 == 0;
-    static constexpr int UNITS = ALIGNED ? BLOCK / 16 : (BLOCK + 14 + 15) / 16;
-    static constexpr bool SPARE_UNIT = !ALIGNED && 16 * (UNITS - 1) >= BLOCK;   // some alignments do not reach the last unit
-    static constexpr int SHIFT = TYPE == IQ2_S ? 14 : 0;
-    static constexpr int PITCH = UNITS % 2 == 1 ? 16 * UNITS : 16 * UNITS + 16;
-    static_assert(PITCH >= 16 * UNITS && (ALIGNED || PITCH >= BLOCK + 14), "what comes along with a row's block touches no other row's");
-    static constexpr int FRONT = ALIGNED ? 0 : 16;   // bytes before the first row
-    static constexpr int REGS = (16 * UNITS + 63) / 64;
-};
 
 // Sub-scales of the lane's values in the eight blocks, one byte each, and the super-block's scale(s).
 struct LaneScales {
@@ -302,7 +285,7 @@ constexpr int TILES_XS_PITCH = 20;   // floats: eight scales, eight sums, paddin
 
 template <int TYPE>
 struct TileWaveLds {
-    alignas(16) uint8_t raw[TileSlot<TYPE>::FRONT + 16 * TileSlot<TYPE>::PITCH];
+    alignas(16) uint8_t raw[16 * BlockPieces<TYPE>::PITCH];
     alignas(16) uint8_t x[GEMV_TILES_ROWS * TILES_X_PITCH];
     alignas(16) float scales[GEMV_TILES_ROWS * TILES_XS_PITCH];
 };
@@ -312,7 +295,8 @@ struct TileWaveLds {
 // silu(gate) * up, both rounded to bf16 first, and the gate.
 template <int TYPE, int R, bool SWIGLU>
 __global__ __launch_bounds__(TILES_THREADS, 2) void mmq_gemv_tiles_kernel(const TilesArgs a) {
-    using S = TileSlot<TYPE>;
+    using S = BlockPieces<TYPE>;
+    constexpr int REGS = (16 * S::UNITS + 63) / 64;
     constexpr bool K45 = TYPE == Q4_K || TYPE == Q5_K;
     constexpr int SIDES = SWIGLU ? 2 : 1;
     static_assert(R % SIDES == 0, "as many gate as up tiles");
@@ -370,65 +354,44 @@ __global__ __launch_bounds__(TILES_THREADS, 2) void mmq_gemv_tiles_kernel(const 
         (second ? a.packed_second : a.packed) + static_cast<int64_t>(expert) * a.bytes_per_expert,
         SWIGLU ? a.packed_second + static_cast<int64_t>(expert) * a.bytes_per_expert : nullptr};
 
-    // A tile's units of a super-block, neighbouring lanes neighbouring units of a row (lanes past the tile repeat its last
-    // unit, tiles past the matrix its last tile).
+    // A tile's pieces of a super-block, neighbouring lanes neighbouring pieces of a row (lanes past the tile repeat its last
+    // piece, tiles past the matrix its last tile).
+    struct __attribute__((packed, aligned(2))) Piece { u32x4_t value; };
     struct Units {
-        u32x4_t value[S::REGS];
+        u32x4_t value[REGS];
     };
     auto tile_base = [&](int sb, int r) __attribute__((always_inline)) {
         const int n = min(n0 + (tile0 + r % COLUMN_TILES) * 16, a.out_features - 16);
         return side_weights[SWIGLU ? r / COLUMN_TILES : 0] + static_cast<int64_t>(n) * a.row_bytes + static_cast<int64_t>(sb) * S::BLOCK;
     };
-    uint32_t unit_row[S::REGS], unit_parked[S::REGS];   // bytes from the tile's first block to the lane's row; where its unit is parked
-    int unit_first[S::REGS];                            // 16 * unit
+    uint32_t piece_from[REGS], piece_to[REGS];   // bytes from the tile's first block; place in `raw`
 #pragma unroll
-    for (int i = 0; i < S::REGS; ++i) {
+    for (int i = 0; i < REGS; ++i) {
         const int id = min(lane + 64 * i, 16 * S::UNITS - 1);
-        const int row = id / S::UNITS;
-        unit_first[i] = 16 * (id - row * S::UNITS);
-        unit_row[i] = static_cast<uint32_t>(row) * a.row_bytes + (S::ALIGNED ? unit_first[i] : 0);
-        unit_parked[i] = S::FRONT + S::SHIFT + row * S::PITCH + unit_first[i];
+        const int row = id / S::UNITS, unit = id - row * S::UNITS;
+        piece_from[i] = static_cast<uint32_t>(row) * a.row_bytes + S::offset(unit);
+        piece_to[i] = row * S::PITCH + 16 * unit;
     }
     auto fetch = [&](Units & units, int sb, int r) __attribute__((always_inline)) {
         const uint8_t * const base = tile_base(sb, r);
-        if constexpr (S::ALIGNED) {
 #pragma unroll
-            for (int i = 0; i < S::REGS; ++i) {
-                units.value[i] = *reinterpret_cast<const u32x4_t *>(base + unit_row[i]);
-            }
-        } else {
-            const uint32_t ahead = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(base)) & 15u;
-            const uint8_t * const aligned = base - ahead;
-#pragma unroll
-            for (int i = 0; i < S::REGS; ++i) {
-                const uint32_t first = ahead + unit_row[i];
-                uint32_t unit = unit_first[i];
-                if constexpr (S::SPARE_UNIT) {   // (a unit that lies entirely behind the block may lie behind the tensor)
-                    unit = unit < (first & 15u) + S::BLOCK ? unit : 0u;
-                }
-                units.value[i] = *reinterpret_cast<const u32x4_t *>(aligned + ((first & ~15u) + unit));
+        for (int i = 0; i < REGS; ++i) {
+            if constexpr (S::ALIGNED) {
+                units.value[i] = *reinterpret_cast<const u32x4_t *>(base + piece_from[i]);
+            } else {
+                units.value[i] = reinterpret_cast<const Piece *>(base + piece_from[i])->value;
             }
         }
     };
-    auto park = [&](const Units & units, int sb, int r) __attribute__((always_inline)) {
-        asm volatile("" ::: "memory");   // (written as units, read as other types: the compiler must keep the order)
-        if constexpr (S::ALIGNED) {
+    auto park = [&](const Units & units) __attribute__((always_inline)) {
+        asm volatile("" ::: "memory");   // (written as pieces, read as other types: the compiler must keep the order)
 #pragma unroll
-            for (int i = 0; i < S::REGS; ++i) {
-                *reinterpret_cast<u32x4_t *>(mine.raw + unit_parked[i]) = units.value[i];
-            }
-        } else {
-            struct __attribute__((packed, aligned(2))) Unaligned { u32x4_t value; };
-            const uint32_t ahead = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(tile_base(sb, r))) & 15u;
-#pragma unroll
-            for (int i = 0; i < S::REGS; ++i) {
-                // (a spare unit's place is taken by padding)
-                reinterpret_cast<Unaligned *>(mine.raw + (unit_parked[i] - ((ahead + unit_row[i]) & 15u)))->value = units.value[i];
-            }
+        for (int i = 0; i < REGS; ++i) {
+            *reinterpret_cast<u32x4_t *>(mine.raw + piece_to[i]) = units.value[i];
         }
         asm volatile("" ::: "memory");
     };
-    const uint8_t * const my_block = mine.raw + S::FRONT + S::SHIFT + col * S::PITCH;
+    const uint8_t * const my_block = mine.raw + col * S::PITCH;
     Units ring[TILES_RING];
 #pragma unroll
     for (int i = 0; i < TILES_RING; ++i) {
@@ -568,7 +531,7 @@ __global__ __launch_bounds__(TILES_THREADS, 2) void mmq_gemv_tiles_kernel(const 
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 Units & units = ring[(u * R + r) % TILES_RING];
-                park(units, sb, r);
+                park(units);
                 LaneBlock<TYPE> block;
                 lane_load<TYPE>(block, my_block, my_block + 8 * part);
                 fetch(units, min(sb + (r + TILES_RING) / R, sb_end - 1), (r + TILES_RING) % R);

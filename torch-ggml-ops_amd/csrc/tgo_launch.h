@@ -103,13 +103,13 @@ static inline bool use_gemv(int64_t rows, int64_t groups) {
 // 16 weight rows and 16-byte aligned weights.  The lines lie where the two measured equal (2048 x 512 and 4096 x 1024 experts
 // and their down projections, 1 to 124 tokens; dense 4096 x 2048 and 28672 x 8192, 1 to 32 rows):
 //  - grouped: Q5_K always (1 token 17 -> 12 us), Q4_K too unless K is long enough for the other kernel's own matrix
-//    instructions to pay; Q3_K from 16 rows.  Q6_K and IQ2_S, whose unpacking is the longest, when the rows are half as many as
-//    the groups if K is short (the other kernel idles there), else three and one and a half (long K: two and a half)
-//    times as many.
+//    instructions to pay; Q3_K and IQ2_S from 16 and 24 rows.  Q6_K, whose unpacking is the longest: from 16 rows if K is three or
+//    four super-blocks, from half as many rows as groups below that (the other kernel folds rows there), from one and a half
+//    times as many above.
 //  - calls of fewer than four million weights never: their time is their launches and latencies, and most of them are one
 //    launch of the other kernel.
-//  - dense: Q3_K, Q6_K and IQ2_S from five rows (the others have eight at most in registers, and two launches' worth of rows
-//    reads the weights twice); Q4_K and Q5_K beyond 16 rows, or on matrices that fill the chip, from nine and three.
+//  - dense matrices that fill the chip: Q3_K always (28672 x 8192, one row: 54 -> 41 us), Q5_K, Q6_K and IQ2_S from three rows (80 ->
+//    65 us for Q6_K), Q4_K from four.  Smaller ones: Q3_K and IQ2_S from five rows, Q6_K from nine, Q4_K and Q5_K beyond 16.
 constexpr int GEMV_TILES_ROWS = 16;              // rows of its tasks
 constexpr int64_t GEMV_TILES_WORKGROUPS = 384;   // workgroups that a launch should have for a wave to take four tiles of 16 weight rows instead of two
 static inline bool gemv_takes_tiles(const void * packed, const void * packed_second, int64_t rows, int64_t groups, int64_t in_features,
@@ -127,17 +127,19 @@ static inline bool gemv_takes_tiles(const void * packed, const void * packed_sec
     if (groups <= 0) {
         const bool large = out_features * in_features >= (INT64_C(1) << 25);
         switch (quant_type) {
-            case 12: return rows > 16 || (large && rows > 8);
-            case 13: return rows > 16 || (large && rows > 2);
-            default: return rows > 4;
+            case 11: return rows > (large ? 0 : 4);
+            case 12: return rows > (large ? 3 : 16);
+            case 13: return rows > (large ? 2 : 16);
+            case 14: return rows > (large ? 2 : 8);
+            default: return rows > (large ? 2 : 4);
         }
     }
     switch (quant_type) {
         case 11: return rows >= 16;
         case 12: return super_blocks <= 8;
         case 13: return true;
-        case 14: return super_blocks <= 4 ? 2 * rows >= groups : rows >= 3 * groups;
-        default: return super_blocks <= 4 ? 2 * rows >= groups : 2 * rows >= (super_blocks <= 8 ? 3 : 5) * groups;
+        case 14: return super_blocks <= 2 ? 2 * rows >= groups : super_blocks <= 4 ? rows >= 16 : 2 * rows >= 3 * groups;
+        default: return rows >= 24;
     }
 }
 
