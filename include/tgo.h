@@ -88,6 +88,16 @@ int tgo_mmq_forward(const void * input_bf16, const void * packed, void * output_
                     void * workspace, int64_t rows, int64_t in_features, int64_t out_features,
                     int quant_type, void * stream);
 
+/* tgo_mmq_forward and tgo_mmq_forward_prepared_as with tgo_forward_scratch_bytes() bytes of `scratch` (0: NULL is as good): dense
+ * calls of more rows than the decode kernels take, whose tiles would not fill the chip, then cut K into ranges that run side by
+ * side and leave fp32 sums there, which a second kernel adds up in a fixed order.  No counterpart in
+ * the reference. */
+int64_t tgo_forward_scratch_bytes(int64_t rows, int64_t in_features, int64_t out_features, int quant_type);
+int tgo_mmq_forward_scratch(const void * input_bf16, const void * packed, void * output_bf16, void * workspace, void * scratch,
+                            int64_t rows, int64_t in_features, int64_t out_features, int quant_type, void * stream);
+int tgo_mmq_forward_prepared_scratch(const void * workspace, const void * packed, void * output_bf16, void * scratch, int64_t rows,
+                                     int64_t in_features, int64_t out_features, int quant_type, int operand, void * stream);
+
 /* tgo_mmq_forward without a workspace argument and without any allocation: the q8_1 activation
  * workspace is a fixed array inside the library's code object (one copy per GPU, held until the
  * process ends), TGO_STATIC_WORKSPACE_BYTES large.  Calls whose

@@ -323,8 +323,34 @@ int tgo_q8_workspace_unpack(const void * workspace, void * q_int8, void * d_f32,
                      "q8_unpack launch");
 }
 
+int64_t tgo_forward_scratch_bytes(int64_t rows, int64_t in_features, int64_t out_features, int quant_type) {
+    if (rows <= 0 || in_features <= 0 || out_features <= 0 || tgo::use_gemv(rows, 0)) {
+        return 0;
+    }
+    // (a prepared workspace may hold either kind of exact operands)
+    return std::max(tgo::forward_partial_bytes(rows, in_features, out_features, quant_type, tgo::OPERAND_INT8),
+                    tgo::forward_partial_bytes(rows, in_features, out_features, quant_type, tgo::OPERAND_HALF));
+}
+
 int tgo_mmq_forward(const void * input_bf16, const void * packed, void * output_bf16, void * workspace,
                     int64_t rows, int64_t in_features, int64_t out_features, int quant_type, void * stream) {
+    return tgo_mmq_forward_scratch(input_bf16, packed, output_bf16, workspace, nullptr, rows, in_features, out_features, quant_type,
+                                   stream);
+}
+
+// The matmul half of a dense call of the kernel family that `view` was quantized for.
+static hipError_t launch_dense(const void * packed, const tgo::Q8Workspace & view, void * output_bf16, void * scratch, int64_t rows,
+                               int64_t in_features, int64_t out_features, int quant_type, hipStream_t stream) {
+    const uint8_t * const weights = static_cast<const uint8_t *>(packed);
+    uint16_t * const output = static_cast<uint16_t *>(output_bf16);
+    const int r = static_cast<int>(rows), k = static_cast<int>(in_features), n = static_cast<int>(out_features);
+    return view.by_rows() ? tgo::launch_mmq_gemv(weights, nullptr, 0, view, output, nullptr, nullptr, r, k, n, quant_type, stream, 0)
+                          : tgo::launch_mmq_forward(weights, nullptr, 0, view, output, nullptr, nullptr, r, k, n, quant_type, stream, 0,
+                                                    static_cast<float *>(scratch));
+}
+
+int tgo_mmq_forward_scratch(const void * input_bf16, const void * packed, void * output_bf16, void * workspace, void * scratch,
+                            int64_t rows, int64_t in_features, int64_t out_features, int quant_type, void * stream) {
     TGO_TRY(check_matmul_shape(rows, in_features, out_features, quant_type));
     TGO_TRY(check_pointer(input_bf16, "input"));
     TGO_TRY(check_pointer(packed, "packed_weight"));
@@ -345,11 +371,7 @@ int tgo_mmq_forward(const void * input_bf16, const void * packed, void * output_
     TGO_TRY(check_hip(tgo::launch_quantize_q8_1(static_cast<const uint16_t *>(input_bf16), view, rows, in_features,
                                                 hip_stream),
                       "quantize_q8_1 launch"));
-    const auto launch = tgo::use_gemv(rows, 0) ? tgo::launch_mmq_gemv : tgo::launch_mmq_forward;
-    return check_hip(launch(static_cast<const uint8_t *>(packed), nullptr, 0, view,
-                            static_cast<uint16_t *>(output_bf16), nullptr, nullptr, static_cast<int>(rows),
-                            static_cast<int>(in_features),
-                            static_cast<int>(out_features), quant_type, hip_stream, 0),
+    return check_hip(launch_dense(packed, view, output_bf16, scratch, rows, in_features, out_features, quant_type, hip_stream),
                      "mmq_forward launch");
 }
 
@@ -374,6 +396,11 @@ int tgo_mmq_forward_static(const void * input_bf16, const void * packed, void * 
 
 int tgo_mmq_forward_prepared_as(const void * workspace, const void * packed, void * output_bf16, int64_t rows,
                                 int64_t in_features, int64_t out_features, int quant_type, int operand, void * stream) {
+    return tgo_mmq_forward_prepared_scratch(workspace, packed, output_bf16, nullptr, rows, in_features, out_features, quant_type,
+                                            operand, stream);
+}
+int tgo_mmq_forward_prepared_scratch(const void * workspace, const void * packed, void * output_bf16, void * scratch, int64_t rows,
+                                     int64_t in_features, int64_t out_features, int quant_type, int operand, void * stream) {
     TGO_TRY(check_matmul_shape(rows, in_features, out_features, quant_type));
     TGO_TRY(check_pointer(workspace, "workspace"));
     TGO_TRY(check_pointer(packed, "packed_weight"));
@@ -381,11 +408,8 @@ int tgo_mmq_forward_prepared_as(const void * workspace, const void * packed, voi
     TGO_TRY(check_workspace_operand(operand));
     const tgo::Q8Workspace view =
         tgo::q8_workspace_view(const_cast<void *>(workspace), rows, in_features, tgo::use_gemv(rows, 0), operand);
-    const auto launch = tgo::use_gemv(rows, 0) ? tgo::launch_mmq_gemv : tgo::launch_mmq_forward;
-    TGO_TRY(check_hip(launch(static_cast<const uint8_t *>(packed), nullptr, 0, view,
-                             static_cast<uint16_t *>(output_bf16), nullptr, nullptr, static_cast<int>(rows),
-                             static_cast<int>(in_features), static_cast<int>(out_features), quant_type,
-                             static_cast<hipStream_t>(stream), 0),
+    TGO_TRY(check_hip(launch_dense(packed, view, output_bf16, scratch, rows, in_features, out_features, quant_type,
+                                   static_cast<hipStream_t>(stream)),
                       "mmq_forward_prepared launch"));
     // (the workspace was quantized by an earlier call: were it of another kind than this call was told, its layout
     // would not be the one this launch assumed)
@@ -502,9 +526,9 @@ int tgo_lm_head_loss(const void * hidden_bf16, const void * packed, const int64_
         TGO_TRY(check_hip(tgo::launch_quantize_q8_1(static_cast<const uint16_t *>(hidden_bf16) + begin * in_features, view, chunk,
                                                     in_features, hip_stream),
                           "quantize_q8_1 launch"));
-        const auto multiply = gemv ? tgo::launch_mmq_gemv : tgo::launch_mmq_forward;
-        TGO_TRY(check_hip(multiply(weights, nullptr, 0, view, logits, nullptr, nullptr, r, k, n, quant_type, hip_stream,
-                                   static_cast<int>(w.pitch)),
+        const int pitch = static_cast<int>(w.pitch);
+        TGO_TRY(check_hip(gemv ? tgo::launch_mmq_gemv(weights, nullptr, 0, view, logits, nullptr, nullptr, r, k, n, quant_type, hip_stream, pitch)
+                               : tgo::launch_mmq_forward(weights, nullptr, 0, view, logits, nullptr, nullptr, r, k, n, quant_type, hip_stream, pitch),
                           "mmq_forward launch"));
         uint8_t * const cotangent = gradient ? base + w.cotangent : nullptr;
         TGO_TRY(check_hip(tgo::launch_cross_entropy(logits, w.pitch, r, n, reinterpret_cast<float2 *>(base + w.stats),
@@ -615,7 +639,7 @@ static int grouped_forward(const void * input_bf16, const int64_t * row_index, i
                              swiglu, hip_stream),
                          "grouped mmq_forward launch");
     }
-    TGO_TRY(check_hip(fused ? launch(tgo::launch_mmq_forward_swiglu) : launch(gemv ? tgo::launch_mmq_gemv : tgo::launch_mmq_forward, 0),
+    TGO_TRY(check_hip(fused ? launch(tgo::launch_mmq_forward_swiglu) : gemv ? launch(tgo::launch_mmq_gemv, 0) : launch(tgo::launch_mmq_forward, 0, nullptr),
                       "grouped mmq_forward launch"));
     return swiglu && !fused ? finish_swiglu() : TGO_OK;
 }

@@ -105,9 +105,13 @@ PyObject * direct_mmq(PyObject *, PyObject * const * args, Py_ssize_t count) {
         c10::SmallVector<int64_t, 5> shape(input.sizes().begin(), input.sizes().end());
         shape.back() = out_features;
         output = at::detail::empty_cuda(shape, at::kBFloat16, input.device(), std::nullopt);
-        const c10::DataPtr workspace = c10::GetAllocator(c10::kCUDA)->allocate(tgo_q8_workspace_bytes(rows, in_features));
-        status = tgo_mmq_forward(input.data_ptr(), weight.data_ptr(), output.data_ptr(), workspace.get(), rows, in_features,
-                                 out_features, static_cast<int>(quant_type), c10::hip::getCurrentHIPStream(device).stream());
+        const int64_t workspace_bytes = (tgo_q8_workspace_bytes(rows, in_features) + 255) / 256 * 256;
+        const int64_t scratch_bytes = tgo_forward_scratch_bytes(rows, in_features, out_features, static_cast<int>(quant_type));
+        const c10::DataPtr workspace = c10::GetAllocator(c10::kCUDA)->allocate(workspace_bytes + scratch_bytes);
+        void * const scratch = scratch_bytes > 0 ? static_cast<uint8_t *>(workspace.get()) + workspace_bytes : nullptr;
+        status = tgo_mmq_forward_scratch(input.data_ptr(), weight.data_ptr(), output.data_ptr(), workspace.get(), scratch, rows,
+                                         in_features, out_features, static_cast<int>(quant_type),
+                                         c10::hip::getCurrentHIPStream(device).stream());
     }
     return finished(status, output);
     END_HANDLE_TH_ERRORS

@@ -58,7 +58,7 @@ struct ForwardLds {
 
 // WIDE (formats whose blocks are not multiples of 16 bytes): the packed blocks are prefetched into registers as
 // aligned units like those of Q4_K / Q5_K (wide_fetch) instead of being copied two bytes at a time when needed.
-template <int TYPE, bool NARROW, bool WIDE>
+template <int TYPE, bool NARROW, bool WIDE, bool RANGES>
 TGO_DEVICE void forward_task(const ForwardArgs & a, ForwardLds<TYPE> & lds, int n_tile, bool second, int expert,
                              int row_start, int row_end) {
     using F = Format<TYPE>;
@@ -85,7 +85,8 @@ TGO_DEVICE void forward_task(const ForwardArgs & a, ForwardLds<TYPE> & lds, int 
     const bool fuse = a.swiglu != 0 && second;   // the gate tile of this workgroup's first pass is in a.y
     const int n0 = n_tile * FWD_TN;
     const int blocks_per_row = a.in_features / 32;
-    const int super_blocks = a.in_features / QK_K;
+    int kb_begin, kb_end;
+    forward_k_range<RANGES>(a, kb_begin, kb_end);
 
     if constexpr (TYPE == IQ2_S) {
         expand_iq2s_grid(grid, tid, THREADS);
@@ -179,9 +180,9 @@ TGO_DEVICE void forward_task(const ForwardArgs & a, ForwardLds<TYPE> & lds, int 
     constexpr int X_AHEAD = PLANES == 1 ? 4 : 8;
     v4i x[X_AHEAD];
     float sum_next[4];
-    auto load_x = [&](int block) {
+    auto load_x = [&](int block, int slot) {   // (slot: block % X_AHEAD)
         const int clamped = block < blocks_per_row ? block : blocks_per_row - 1;
-        x[block % X_AHEAD] = *reinterpret_cast<const v4i *>(qx_task + static_cast<int64_t>(clamped) * 1024 + x_lane_offset);
+        x[slot] = *reinterpret_cast<const v4i *>(qx_task + static_cast<int64_t>(clamped) * 1024 + x_lane_offset);
     };
     auto load_sums = [&](int kb) {
         if constexpr (F::HAS_MIN) {
@@ -193,13 +194,13 @@ TGO_DEVICE void forward_task(const ForwardArgs & a, ForwardLds<TYPE> & lds, int 
         }
     };
 
-    load_raw(0, tid);
-    load_dx(0, tid);
+    load_raw(kb_begin, tid);
+    load_dx(kb_begin, tid);
     if (wave_active) {
-        load_sums(0);
+        load_sums(kb_begin);
 #pragma unroll
         for (int b = 0; b < X_AHEAD; ++b) {
-            load_x(b);
+            load_x(kb_begin * 8 + b, b);
         }
     }
 
@@ -228,7 +229,7 @@ TGO_DEVICE void forward_task(const ForwardArgs & a, ForwardLds<TYPE> & lds, int 
     constexpr int TILES = MODE == 2 ? 1 : FWD_NT;
     auto tile_of = [&](int index) { return MODE == 2 ? wave : index; };
 #pragma unroll 1
-    for (int kb = 0; kb < super_blocks; ++kb) {
+    for (int kb = kb_begin; kb < kb_end; ++kb) {
         // Two barriers per super-block.  `raw` is rewritten here while no wave can still be unpacking it
         // (all passed the second barrier of the previous round); the activation scales alternate between
         // two copies because slower waves may still be reading the previous one.
@@ -245,7 +246,7 @@ TGO_DEVICE void forward_task(const ForwardArgs & a, ForwardLds<TYPE> & lds, int 
         __builtin_amdgcn_s_setprio(3);
 
         // the last round re-fetches its own super-block instead of branching around the prefetch
-        const int kb_next = kb + 1 < super_blocks ? kb + 1 : kb;
+        const int kb_next = kb + 1 < kb_end ? kb + 1 : kb;
         load_raw(kb_next, t);
         load_dx(kb_next, t);
 
@@ -378,7 +379,7 @@ TGO_DEVICE void forward_task(const ForwardArgs & a, ForwardLds<TYPE> & lds, int 
                     if (t % TILES == TILES - 1) {
                         // block t / TILES is done (its last MFMA has been issued): its registers take the
                         // block X_AHEAD further on
-                        load_x(block0 + t / TILES + X_AHEAD);
+                        load_x(block0 + t / TILES + X_AHEAD, (t / TILES) % X_AHEAD);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -449,7 +450,7 @@ TGO_DEVICE void forward_task(const ForwardArgs & a, ForwardLds<TYPE> & lds, int 
                 // the super-block is done: fetch the next one's activation fragments
 #pragma unroll
                 for (int b = 0; b < 8; ++b) {
-                    load_x(kb * 8 + b + X_AHEAD);
+                    load_x(kb * 8 + b + X_AHEAD, b % X_AHEAD);
                 }
             }
         }
@@ -463,6 +464,16 @@ TGO_DEVICE void forward_task(const ForwardArgs & a, ForwardLds<TYPE> & lds, int 
         } else {
             main_loop(std::integral_constant<int, 0>{});
         }
+    }
+    if constexpr (RANGES) {
+        if (wave_active) {
+            constexpr int TILES = narrow ? 1 : FWD_NT;
+#pragma unroll
+            for (int nt = 0; nt < TILES; ++nt) {
+                store_partial_32x32<PLANES == 2>(a, acc[nt], wave_row, row_end, n0 + 32 * (narrow ? wave : nt), lane);
+            }
+        }
+        return;
     }
     __syncthreads();
     if constexpr (narrow) {
@@ -502,7 +513,7 @@ TGO_DEVICE void forward_task(const ForwardArgs & a, ForwardLds<TYPE> & lds, int 
 // rows).  Such tasks are common under skewed routing, so for them the four waves of a single-plane
 // workgroup take one of the four 32-row weight tiles each instead.  The variants are separate
 // instantiations of the task body so that neither's registers weigh on the other.
-template <int TYPE>
+template <int TYPE, bool RANGES = false>
 TGO_DEVICE void forward_any_task(const ForwardArgs & a, ForwardLds<TYPE> & lds, int n_tile, bool second, int expert,
                                  int row_start, int row_end) {
     constexpr bool SINGLE = Format<TYPE>::PLANES == 1;
@@ -510,21 +521,21 @@ TGO_DEVICE void forward_any_task(const ForwardArgs & a, ForwardLds<TYPE> & lds, 
     if constexpr (Format<TYPE>::BLOCK_BYTES % 16 != 0) {
         if (a.wide != 0) {
             if (narrow) {
-                forward_task<TYPE, SINGLE, true>(a, lds, n_tile, second, expert, row_start, row_end);
+                forward_task<TYPE, SINGLE, true, RANGES>(a, lds, n_tile, second, expert, row_start, row_end);
             } else {
-                forward_task<TYPE, false, true>(a, lds, n_tile, second, expert, row_start, row_end);
+                forward_task<TYPE, false, true, RANGES>(a, lds, n_tile, second, expert, row_start, row_end);
             }
             return;
         }
     }
     if (narrow) {
-        forward_task<TYPE, SINGLE, false>(a, lds, n_tile, second, expert, row_start, row_end);
+        forward_task<TYPE, SINGLE, false, RANGES>(a, lds, n_tile, second, expert, row_start, row_end);
     } else {
-        forward_task<TYPE, false, false>(a, lds, n_tile, second, expert, row_start, row_end);
+        forward_task<TYPE, false, false, RANGES>(a, lds, n_tile, second, expert, row_start, row_end);
     }
 }
 
-template <int TYPE>
+template <int TYPE, bool RANGES>
 __global__ __launch_bounds__(ForwardShape<TYPE>::THREADS, 2) void mmq_forward_kernel(const ForwardArgs a) {
     using F = Format<TYPE>;
     using S = ForwardShape<TYPE>;
@@ -537,7 +548,7 @@ __global__ __launch_bounds__(ForwardShape<TYPE>::THREADS, 2) void mmq_forward_ke
     if (!forward_pick(a, n_tile, second, expert, row_start, row_end)) {
         return;
     }
-    forward_any_task<TYPE>(a, lds, n_tile, second, expert, row_start, row_end);
+    forward_any_task<TYPE, RANGES>(a, lds, n_tile, second, expert, row_start, row_end);
 }
 
 // Fused SwiGLU, its own kernel so that the plain forward's register allocation is untouched.  The gate tile
@@ -571,18 +582,51 @@ static hipError_t launch_forward_typed(const ForwardArgs & args, hipStream_t str
         return hipErrorInvalidValue;
     }
     const ProfileScope scope(2, stream);
-    if (args.swiglu != 0) {
+    if (args.partial != nullptr) {
+        mmq_forward_kernel<TYPE, true><<<dim3(static_cast<unsigned>(total), static_cast<unsigned>(args.k_splits)), ForwardShape<TYPE>::THREADS, 0, stream>>>(args);
+    } else if (args.swiglu != 0) {
         mmq_forward_swiglu_kernel<TYPE><<<static_cast<unsigned>(total), ForwardShape<TYPE>::THREADS, 0, stream>>>(args);
     } else {
-        mmq_forward_kernel<TYPE><<<static_cast<unsigned>(total), ForwardShape<TYPE>::THREADS, 0, stream>>>(args);
+        mmq_forward_kernel<TYPE, false><<<static_cast<unsigned>(total), ForwardShape<TYPE>::THREADS, 0, stream>>>(args);
     }
     return hipGetLastError();
+}
+
+// y = bf16(the ranges' sums, added in order): eight columns per thread.
+__global__ __launch_bounds__(256) void forward_reduce_kernel(const ForwardArgs a) {
+    const int groups = a.n_tiles * (FWD_TN / 8);
+    const int64_t id = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    const int64_t row = id / groups;
+    const int n = static_cast<int>(id - row * groups) * 8;
+    if (row >= a.rows || n >= a.out_features) {
+        return;
+    }
+    const int64_t pitch = a.n_tiles * FWD_TN;
+    float sum[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s = 0; s < a.k_splits; ++s) {
+        const float * const from = a.partial + (static_cast<int64_t>(s) * a.rows + row) * pitch + n;
+        const float4 low = *reinterpret_cast<const float4 *>(from), high = *reinterpret_cast<const float4 *>(from + 4);
+        sum[0] += low.x; sum[1] += low.y; sum[2] += low.z; sum[3] += low.w;
+        sum[4] += high.x; sum[5] += high.y; sum[6] += high.z; sum[7] += high.w;
+    }
+    uint16_t * const to = a.y + row * a.out_stride + n;
+    if (a.out_stride % 8 == 0 && n + 8 <= a.out_features) {
+        *reinterpret_cast<uint4 *>(to) = make_uint4(pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3]),
+                                                    pack_bf16x2(sum[4], sum[5]), pack_bf16x2(sum[6], sum[7]));
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            if (n + e < a.out_features) {
+                to[e] = to_bf16_bits(sum[e]);
+            }
+        }
+    }
 }
 
 static hipError_t launch_forward(const uint8_t * packed, const uint8_t * packed_second, int64_t bytes_per_expert,
                                  const Q8Workspace & ws, uint16_t * output, uint16_t * output_second,
                                  const TaskList * tasks, int rows, int in_features, int out_features,
-                                 int quant_type, hipStream_t stream, bool swiglu, int output_stride) {
+                                 int quant_type, hipStream_t stream, bool swiglu, int output_stride, float * partial) {
     if (ws.by_rows()) {
         return hipErrorInvalidValue;   // this kernel reads the tile-ordered activation layout
     }
@@ -613,6 +657,7 @@ static hipError_t launch_forward(const uint8_t * packed, const uint8_t * packed_
     args.out_features = out_features;
     args.out_stride = output_stride > 0 ? output_stride : out_features;
     args.n_tiles = (out_features + FWD_TN - 1) / FWD_TN;
+    args.k_splits = 1;
     if (tasks != nullptr) {
         args.task_count = tasks->count;
         args.task_early = tasks->early;
@@ -629,48 +674,43 @@ static hipError_t launch_forward(const uint8_t * packed, const uint8_t * packed_
         args.task_expert = nullptr;
         args.task_row_start = nullptr;
         args.task_row_end = nullptr;
-        // A dense call whose full tiles would not even give every second CU a workgroup runs as smaller tiles.
-        // Single-plane formats: 32 rows, i.e. the kernel's narrow variant, whose four waves split the weight rows
-        // (four times the workgroups, each about a third as long).  The two-plane formats have no narrow variant,
-        // but their eight waves own 32 rows each: with tiles of 128, 64 or 32 rows only 4, 2 or 1 of them multiply
-        // (the others still help to unpack), the vector work of a tile no longer queues two waves deep on every
-        // SIMD, and there are 2, 4 or 8 times the workgroups; the largest tile that yields 128 workgroups is taken.
-        int row_tile = forward_row_tile(quant_type, ws.operand_kind());
-        const auto tiles = [&](int tile) { return static_cast<int64_t>(args.n_tiles) * ((rows + tile - 1) / tile); };
-        if (row_tile == 128) {
-            if (tiles(128) <= 128) {
-                row_tile = 32;
-            }
-        } else {
-            while (row_tile > 32 && tiles(row_tile) < 128) {
-                row_tile /= 2;
-            }
-        }
-        args.dense_row_tile = row_tile;
-        args.task_slots = (rows + row_tile - 1) / row_tile;
+        const ForwardSplit split = forward_split(rows, in_features, out_features, quant_type, ws.operand_kind(), partial != nullptr);
+        args.dense_row_tile = split.row_tile;
+        args.task_slots = (rows + split.row_tile - 1) / split.row_tile;
+        args.k_splits = split.k_splits;
+        args.partial = split.k_splits > 1 ? partial : nullptr;
     }
     if (ws.scaled_tiles()) {
         return launch_forward_scaled(args, quant_type, stream);
     }
-    if (ws.half_tiles()) {
-        return launch_forward_half(args, quant_type, stream);
+    const auto launch = [&]() {
+        if (ws.half_tiles()) {
+            return launch_forward_half(args, quant_type, stream);
+        }
+        switch (quant_type) {
+            case Q3_K: return launch_forward_typed<Q3_K>(args, stream);
+            case Q4_K: return launch_forward_typed<Q4_K>(args, stream);
+            case Q5_K: return launch_forward_typed<Q5_K>(args, stream);
+            case Q6_K: return launch_forward_typed<Q6_K>(args, stream);
+            case IQ2_S: return launch_forward_typed<IQ2_S>(args, stream);
+            default: return hipErrorInvalidValue;
+        }
+    };
+    const hipError_t status = launch();
+    if (status != hipSuccess || args.partial == nullptr) {
+        return status;
     }
-    switch (quant_type) {
-        case Q3_K: return launch_forward_typed<Q3_K>(args, stream);
-        case Q4_K: return launch_forward_typed<Q4_K>(args, stream);
-        case Q5_K: return launch_forward_typed<Q5_K>(args, stream);
-        case Q6_K: return launch_forward_typed<Q6_K>(args, stream);
-        case IQ2_S: return launch_forward_typed<IQ2_S>(args, stream);
-        default: return hipErrorInvalidValue;
-    }
+    const int64_t threads = static_cast<int64_t>(rows) * args.n_tiles * (FWD_TN / 8);
+    forward_reduce_kernel<<<static_cast<unsigned>((threads + 255) / 256), 256, 0, stream>>>(args);
+    return hipGetLastError();
 }
 
 hipError_t launch_mmq_forward(const uint8_t * packed, const uint8_t * packed_second, int64_t bytes_per_expert,
                               const Q8Workspace & ws, uint16_t * output, uint16_t * output_second,
                               const TaskList * tasks, int rows, int in_features, int out_features,
-                              int quant_type, hipStream_t stream, int output_stride) {
+                              int quant_type, hipStream_t stream, int output_stride, float * partial) {
     return launch_forward(packed, packed_second, bytes_per_expert, ws, output, output_second, tasks, rows,
-                          in_features, out_features, quant_type, stream, false, output_stride);
+                          in_features, out_features, quant_type, stream, false, output_stride, partial);
 }
 
 hipError_t launch_mmq_forward_swiglu(const uint8_t * packed, const uint8_t * packed_second, int64_t bytes_per_expert,
@@ -681,7 +721,7 @@ hipError_t launch_mmq_forward_swiglu(const uint8_t * packed, const uint8_t * pac
         return hipErrorInvalidValue;
     }
     return launch_forward(packed, packed_second, bytes_per_expert, ws, output, output_second, tasks, rows,
-                          in_features, out_features, quant_type, stream, true, 0);
+                          in_features, out_features, quant_type, stream, true, 0, nullptr);
 }
 
 }  // namespace tgo

@@ -41,6 +41,8 @@ struct ForwardArgs {
     int task_slots;
     int dense_row_tile;   // dense calls: rows per workgroup (the format's row tile, or 32 when that fills the chip better)
     int wide;             // 2-byte aligned formats: the weights may be fetched as aligned 16-byte units (wide_stage_ok)
+    float * partial;      // dense calls too small to fill the chip: fp32 sums of each range of K, [range][row][n_tiles * 128], or nullptr
+    int k_splits;         // how many ranges (blockIdx.y picks one); 1 when partial is nullptr
     int early_only;       // grouped calls: 1 = this launch runs the tasks listed before the short ones, another kernel the rest
 };
 
@@ -75,6 +77,41 @@ TGO_DEVICE bool forward_pick_linear(const ForwardArgs & a, int linear, int & n_t
         row_end = min(a.rows, row_start + a.dense_row_tile);
     }
     return true;
+}
+
+// Super-blocks [begin, end) of K that this workgroup multiplies.  RANGES: the kernel variants for k_splits > 1 (instantiations of
+// their own: the branch at the end of the loop alone made the plain ones spill).
+template <bool RANGES>
+TGO_DEVICE void forward_k_range(const ForwardArgs & a, int & begin, int & end) {
+    const int super_blocks = a.in_features / QK_K;
+    begin = RANGES ? super_blocks * static_cast<int>(blockIdx.y) / a.k_splits : 0;
+    end = RANGES ? super_blocks * (static_cast<int>(blockIdx.y) + 1) / a.k_splits : super_blocks;
+}
+
+// A range's sums of a 32 x 32 tile straight from the accumulators.  TRANSPOSED: the lane holds row l32 of the tile and, as
+// elements 4 j .. 4 j + 3, columns 8 j + 4 half ..; otherwise column l32 and those rows.
+template <bool TRANSPOSED, typename V16>
+TGO_DEVICE void store_partial_32x32(const ForwardArgs & a, const V16 & acc, int row0, int row_end, int n0, int lane) {
+    const int l32 = lane & 31, half = lane >> 5;
+    const int pitch = a.n_tiles * FWD_TN;
+    float * const out = a.partial + (static_cast<int64_t>(blockIdx.y) * a.rows + row0) * pitch + n0;
+    if constexpr (TRANSPOSED) {
+        if (row0 + l32 < row_end) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                *reinterpret_cast<float4 *>(out + static_cast<int64_t>(l32) * pitch + 8 * j + 4 * half) =
+                    make_float4(acc[4 * j], acc[4 * j + 1], acc[4 * j + 2], acc[4 * j + 3]);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const int row = 8 * (v / 4) + 4 * half + v % 4;
+            if (row0 + row < row_end) {
+                out[static_cast<int64_t>(row) * pitch + l32] = acc[v];
+            }
+        }
+    }
 }
 
 TGO_DEVICE bool forward_pick(const ForwardArgs & a, int & n_tile, bool & second, int & expert, int & row_start,

@@ -61,7 +61,7 @@ struct HalfLds {
 };
 
 // NARROW: a task of at most 32 rows; every wave takes the same 32 activation rows and weight tile number `wave`.
-template <int TYPE, bool NARROW, bool WIDE>
+template <int TYPE, bool NARROW, bool WIDE, bool RANGES>
 TGO_DEVICE void forward_half_task(const ForwardArgs & a, HalfLds<TYPE> & lds, int n_tile, bool second, int expert,
                                   int row_start, int row_end) {
     using F = Format<TYPE>;
@@ -90,7 +90,8 @@ TGO_DEVICE void forward_half_task(const ForwardArgs & a, HalfLds<TYPE> & lds, in
     const bool fuse = a.swiglu != 0 && second;   // the gate tile of this workgroup's first pass is in a.y
     const int n0 = n_tile * FWD_TN;
     const int blocks_per_row = a.in_features / 32;
-    const int super_blocks = a.in_features / QK_K;
+    int kb_begin, kb_end;
+    forward_k_range<RANGES>(a, kb_begin, kb_end);
 
     if constexpr (TYPE == IQ2_S) {
         expand_iq2s_selectors(lds.codebook, tid, THREADS);
@@ -185,9 +186,9 @@ TGO_DEVICE void forward_half_task(const ForwardArgs & a, HalfLds<TYPE> & lds, in
         }
     };
 
-    load_raw(0, tid);
+    load_raw(kb_begin, tid);
     if (wave_active) {
-        load_stage(0);
+        load_stage(kb_begin * 8);
     }
 
     constexpr int CT = NARROW ? 1 : FWD_NT;   // weight tiles per wave
@@ -410,12 +411,12 @@ TGO_DEVICE void forward_half_task(const ForwardArgs & a, HalfLds<TYPE> & lds, in
         constexpr bool ACTIVE = decltype(mode_tag)::value != 0;
         if constexpr (!PIPE) {
 #pragma unroll 1
-            for (int kb = 0; kb < super_blocks; ++kb) {
+            for (int kb = kb_begin; kb < kb_end; ++kb) {
                 int t = tid;
                 asm volatile("" : "+v"(t));
                 // (every wave has left the previous round's last unpack phase, the last reader of `raw`)
                 park_raw(kb, t, 0);
-                const int kb_next = kb + 1 < super_blocks ? kb + 1 : kb;   // the last round re-fetches its own blocks
+                const int kb_next = kb + 1 < kb_end ? kb + 1 : kb;   // the last round re-fetches its own blocks
                 auto stage = [&](auto stage_tag) {
                     constexpr int s = decltype(stage_tag)::value;
                     __syncthreads();   // the blocks are parked; nobody still reads the previous stage's operand tile
@@ -443,17 +444,17 @@ TGO_DEVICE void forward_half_task(const ForwardArgs & a, HalfLds<TYPE> & lds, in
             {
                 int t = tid;
                 asm volatile("" : "+v"(t));
-                park_raw(0, t, 0);
+                park_raw(kb_begin, t, 0);
                 __syncthreads();
                 unpack(std::integral_constant<int, 0>{}, t, 0, 0);
                 __syncthreads();
             }
 #pragma unroll 1
-            for (int kb = 0; kb < super_blocks; ++kb) {
+            for (int kb = kb_begin; kb < kb_end; ++kb) {
                 int t = tid;
                 asm volatile("" : "+v"(t));
-                const int parity = kb & 1;
-                const int kb_next = kb + 1 < super_blocks ? kb + 1 : kb;   // the last round re-fetches its own blocks
+                const int parity = (kb - kb_begin) & 1;
+                const int kb_next = kb + 1 < kb_end ? kb + 1 : kb;   // the last round re-fetches its own blocks
                 auto stage = [&](auto stage_tag) {
                     constexpr int s = decltype(stage_tag)::value;
                     if constexpr (s == STAGES - 2) {
@@ -489,6 +490,15 @@ TGO_DEVICE void forward_half_task(const ForwardArgs & a, HalfLds<TYPE> & lds, in
     } else {
         main_loop(std::integral_constant<int, 0>{});
     }
+    if constexpr (RANGES) {
+        if (wave_active) {
+#pragma unroll
+            for (int nt = 0; nt < CT; ++nt) {
+                store_partial_32x32<true>(a, acc[nt], wave_row, row_end, n0 + 32 * tile_of(nt), lane);
+            }
+        }
+        return;
+    }
     __syncthreads();
 
     // The LDS of the packed blocks and the operand tile is free now: the results, which the swapped operands left
@@ -515,28 +525,28 @@ TGO_DEVICE void forward_half_task(const ForwardArgs & a, HalfLds<TYPE> & lds, in
     }
 }
 
-template <int TYPE>
+template <int TYPE, bool RANGES = false>
 TGO_DEVICE void forward_half_any_task(const ForwardArgs & a, HalfLds<TYPE> & lds, int n_tile, bool second, int expert,
                                       int row_start, int row_end) {
     const bool narrow = row_end - row_start <= 32;
     if constexpr (Format<TYPE>::BLOCK_BYTES % 16 != 0) {
         if (a.wide != 0) {
             if (narrow) {
-                forward_half_task<TYPE, true, true>(a, lds, n_tile, second, expert, row_start, row_end);
+                forward_half_task<TYPE, true, true, RANGES>(a, lds, n_tile, second, expert, row_start, row_end);
             } else {
-                forward_half_task<TYPE, false, true>(a, lds, n_tile, second, expert, row_start, row_end);
+                forward_half_task<TYPE, false, true, RANGES>(a, lds, n_tile, second, expert, row_start, row_end);
             }
             return;
         }
     }
     if (narrow) {
-        forward_half_task<TYPE, true, false>(a, lds, n_tile, second, expert, row_start, row_end);
+        forward_half_task<TYPE, true, false, RANGES>(a, lds, n_tile, second, expert, row_start, row_end);
     } else {
-        forward_half_task<TYPE, false, false>(a, lds, n_tile, second, expert, row_start, row_end);
+        forward_half_task<TYPE, false, false, RANGES>(a, lds, n_tile, second, expert, row_start, row_end);
     }
 }
 
-template <int TYPE>
+template <int TYPE, bool RANGES>
 __global__ __launch_bounds__(HalfShape<TYPE>::THREADS, 2) void mmq_forward_half_kernel(const ForwardArgs a) {
     __shared__ HalfLds<TYPE> lds;
     int n_tile, expert, row_start, row_end;
@@ -544,7 +554,7 @@ __global__ __launch_bounds__(HalfShape<TYPE>::THREADS, 2) void mmq_forward_half_
     if (!forward_pick(a, n_tile, second, expert, row_start, row_end)) {
         return;
     }
-    forward_half_any_task<TYPE>(a, lds, n_tile, second, expert, row_start, row_end);
+    forward_half_any_task<TYPE, RANGES>(a, lds, n_tile, second, expert, row_start, row_end);
 }
 
 // Fused SwiGLU: the gate tile goes to a.y as usual; the up pass of the same workgroup reads it back in its epilogue,
@@ -575,10 +585,12 @@ static hipError_t launch_forward_half_typed(const ForwardArgs & args, hipStream_
         return hipErrorInvalidValue;
     }
     const ProfileScope scope(2, stream);
-    if (args.swiglu != 0) {
+    if (args.partial != nullptr) {
+        mmq_forward_half_kernel<TYPE, true><<<dim3(static_cast<unsigned>(total), static_cast<unsigned>(args.k_splits)), HalfShape<TYPE>::THREADS, 0, stream>>>(args);
+    } else if (args.swiglu != 0) {
         mmq_forward_half_swiglu_kernel<TYPE><<<static_cast<unsigned>(total), HalfShape<TYPE>::THREADS, 0, stream>>>(args);
     } else {
-        mmq_forward_half_kernel<TYPE><<<static_cast<unsigned>(total), HalfShape<TYPE>::THREADS, 0, stream>>>(args);
+        mmq_forward_half_kernel<TYPE, false><<<static_cast<unsigned>(total), HalfShape<TYPE>::THREADS, 0, stream>>>(args);
     }
     return hipGetLastError();
 }

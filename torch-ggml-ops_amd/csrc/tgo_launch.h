@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <algorithm>
 
 namespace tgo {
 
@@ -67,6 +68,76 @@ constexpr int GEMV_ROW_TILE = 8;
 // Dense calls of up to this many rows take it too, GEMV_ROW_TILE rows at a time: the MFMA kernel's 128-row
 // column tiles leave most of the chip idle on a matrix of a few thousand rows, and its latency per tile is long.
 constexpr int GEMV_DENSE_ROWS = 32;
+
+// Dense forward calls: rows per workgroup, and, with exact operands, the ranges that K is cut into (each workgroup then leaves
+// fp32 sums that a second kernel adds up in a fixed order; needs forward_partial_bytes() of scratch).
+// A workgroup takes 2 to 6 us per super-block of K however few rows it has, so a call of a few tiles is as slow as its K is
+// long: one row tile of 1024 x 4096 Q6_K 102 us on 8 CUs.  The ranges were chosen from a sweep of tiles x ranges over 1024 x 4096,
+// 4096 x 2048, 5003 x 4096 and 4096 x 8192, 64 to 1024 rows:
+//  - 128-row tiles (two workgroups per CU): 32-row tiles while those are at most 256, up to 640 workgroups, ranges of four
+//    super-blocks, of two where even that leaves CUs idle; short K (fewer than 16) only below 128 tiles.
+//    4096 x 8192 Q5_K, 64 rows: 71 -> 37 us, 517 rows 142 -> 99; 1024 x 4096 Q3_K, 64 rows: 50 -> 21.
+//  - 256-row int8 tiles (one workgroup per CU; weights of two planes, the longest to unpack): up to 256 workgroups, ranges of two
+//    super-blocks.  1024 x 4096 Q6_K, 64 rows: 102 -> 33 us; 5003 x 4096, 517 rows: 124 -> 98.
+//  - 256-row fp16 tiles: the narrow variant up to 128 tiles, else the largest tile that yields 128 workgroups; ranges of four
+//    super-blocks (a narrow workgroup's start costs as much as one).  4096 x 8192 IQ2_S, 64 rows: 77 -> 44 us.
+// Matrices of fewer than four million weights keep one range: the second launch takes most of what ranges gain there, and their
+// sums stay those of the grouped calls bit for bit.
+struct ForwardSplit {
+    int row_tile;
+    int k_splits;
+};
+static inline ForwardSplit forward_split(int64_t rows, int64_t in_features, int64_t out_features, int quant_type, int operand_kind,
+                                         bool scratch) {
+    const int64_t n_tiles = (out_features + 127) / 128;
+    const int64_t super_blocks = in_features / 256;
+    const int full_tile = forward_row_tile(quant_type, operand_kind);
+    const auto tiles = [&](int tile) { return n_tiles * ((rows + tile - 1) / tile); };
+    if (scratch && operand_kind != OPERAND_SCALED && out_features * in_features >= (INT64_C(1) << 22)) {
+        int tile = full_tile;
+        int64_t most;   // ranges
+        if (full_tile == 128) {
+            tile = tiles(32) <= 256 ? 32 : 128;
+            const int64_t wanted = tiles(tile) * (super_blocks / 4) < 256 ? super_blocks / 2 : super_blocks / 4;
+            most = tiles(tile) > 128 && super_blocks < 16 ? 1 : std::min(640 / tiles(tile), wanted);
+        } else if (operand_kind == OPERAND_INT8) {
+            most = std::min(256 / tiles(tile), super_blocks / 2);
+        } else {
+            most = super_blocks / 4;
+            if (tiles(32) <= 128) {
+                tile = 32;
+            }
+            while (tile > 64 && tiles(tile) * most < 128) {
+                tile /= 2;
+            }
+            most = std::min(256 / tiles(tile), most);
+        }
+        if (most >= 2) {
+            return {tile, most >= 8 ? 8 : most >= 4 ? 4 : 2};
+        }
+    }
+    // One range.  Full tiles that would not even give every second CU a workgroup become smaller ones.
+    // Single-plane formats: 32 rows, i.e. the kernel's narrow variant, whose four waves split the weight rows
+    // (four times the workgroups, each about a third as long).  The two-plane formats have no narrow variant,
+    // but their eight waves own 32 rows each: with tiles of 128, 64 or 32 rows only 4, 2 or 1 of them multiply
+    // (the others still help to unpack), the vector work of a tile no longer queues two waves deep on every
+    // SIMD, and there are 2, 4 or 8 times the workgroups; the largest tile that yields 128 workgroups is taken.
+    int row_tile = full_tile;
+    if (row_tile == 128) {
+        if (tiles(128) <= 128) {
+            row_tile = 32;
+        }
+    } else {
+        while (row_tile > 32 && tiles(row_tile) < 128) {
+            row_tile /= 2;
+        }
+    }
+    return {row_tile, 1};
+}
+static inline int64_t forward_partial_bytes(int64_t rows, int64_t in_features, int64_t out_features, int quant_type, int operand_kind) {
+    const int splits = forward_split(rows, in_features, out_features, quant_type, operand_kind, true).k_splits;
+    return splits > 1 ? splits * rows * ((out_features + 127) / 128 * 128) * 4 : 0;
+}
 
 // Dense grad-input: a workgroup owns 256 rows x 128 columns of the result and walks the whole reduction (N weight
 // rows, 64 per step) alone, so a call of a few hundred rows keeps K / 128 workgroups busy and takes as long as one
@@ -323,7 +394,7 @@ hipError_t launch_moe_combine(const uint16_t * rows, const int64_t * slot_rows, 
 hipError_t launch_mmq_forward(const uint8_t * packed, const uint8_t * packed_second, int64_t bytes_per_expert,
                               const Q8Workspace & ws, uint16_t * output, uint16_t * output_second,
                               const TaskList * tasks, int rows, int in_features, int out_features,
-                              int quant_type, hipStream_t stream, int output_stride = 0);
+                              int quant_type, hipStream_t stream, int output_stride = 0, float * partial = nullptr);
 // Pair only: `output` receives the first projection (gate) and `output_second` silu(gate) * second projection,
 // both factors rounded to bf16 first, the product rounded once.
 hipError_t launch_mmq_forward_swiglu(const uint8_t * packed, const uint8_t * packed_second, int64_t bytes_per_expert,

@@ -38,6 +38,10 @@ lib.tgo_dequant_bf16.argtypes = [_p, _p, _i64, _i64, _int, _p]
 lib.tgo_quantize_q8_1.argtypes = [_p, _p, _i64, _i64, _p]
 lib.tgo_q8_workspace_unpack.argtypes = [_p, _p, _p, _p, _i64, _i64, _p]
 lib.tgo_mmq_forward.argtypes = [_p, _p, _p, _p, _i64, _i64, _i64, _int, _p]
+lib.tgo_forward_scratch_bytes.argtypes = [_i64, _i64, _i64, _int]
+lib.tgo_forward_scratch_bytes.restype = _i64
+lib.tgo_mmq_forward_scratch.argtypes = [_p, _p, _p, _p, _p, _i64, _i64, _i64, _int, _p]
+lib.tgo_mmq_forward_prepared_scratch.argtypes = [_p, _p, _p, _p, _i64, _i64, _i64, _int, _int, _p]
 lib.tgo_mmq_forward_static.argtypes = [_p, _p, _p, _i64, _i64, _i64, _int, _p]
 lib.tgo_mmq_forward_prepared.argtypes = [_p, _p, _p, _i64, _i64, _i64, _int, _p]
 lib.tgo_quantize_q8_1_as.argtypes = [_p, _p, _i64, _i64, _int, _p]
@@ -91,6 +95,9 @@ EXPORTS = (
     "tgo_quantize_q8_1",
     "tgo_q8_workspace_unpack",
     "tgo_mmq_forward",
+    "tgo_forward_scratch_bytes",
+    "tgo_mmq_forward_scratch",
+    "tgo_mmq_forward_prepared_scratch",
     "tgo_mmq_forward_static",
     "tgo_mmq_forward_prepared",
     "tgo_quantize_q8_1_as",
@@ -160,6 +167,15 @@ def stream_of(device: torch.device) -> int:
     if _raw_stream is not None and device.index is not None:
         return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
+
+
+def forward_scratch(tensor: torch.Tensor, rows: int, in_features: int, out_features: int, quant_type: int):
+    """(tensor that keeps it, pointer) of the scratch memory of a dense forward call; (None, None) when it needs none."""
+    size = lib.tgo_forward_scratch_bytes(rows, in_features, out_features, int(quant_type))
+    if size == 0:
+        return None, None
+    scratch = tensor.new_empty((size,), dtype=torch.uint8)
+    return scratch, scratch.data_ptr()
 
 
 def on_device(device: torch.device):

@@ -93,9 +93,10 @@ def _mmq_prepared_device(
         )
     with _native.on_device(workspace.device):
         output = workspace.new_empty((rows, out_features), dtype=torch.bfloat16)
+        _scratch, scratch = _native.forward_scratch(workspace, rows, in_features, out_features, quant_type)
         _native.check(
-            _native.lib.tgo_mmq_forward_prepared_as(
-                workspace.data_ptr(), packed_weight.data_ptr(), output.data_ptr(),
+            _native.lib.tgo_mmq_forward_prepared_scratch(
+                workspace.data_ptr(), packed_weight.data_ptr(), output.data_ptr(), scratch,
                 rows, in_features, out_features, int(quant_type), kind, _stream(workspace),
             )
         )
