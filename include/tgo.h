@@ -98,6 +98,19 @@ int tgo_mmq_forward_scratch(const void * input_bf16, const void * packed, void *
 int tgo_mmq_forward_prepared_scratch(const void * workspace, const void * packed, void * output_bf16, void * scratch, int64_t rows,
                                      int64_t in_features, int64_t out_features, int quant_type, int operand, void * stream);
 
+/* Several dense projections of one input: the activations are quantized once, as `operand` (TGO_OPERAND_INT8, _HALF or _SCALED), into
+ * `workspace` (tgo_q8_workspace_bytes), and multiplied with each packed weight; `scratch`: the largest
+ * tgo_forward_scratch_bytes() of the projections, or NULL.  The arrays have `count` entries and lie in host memory.
+ * tgo_mmq_pair_grad_input: the gradient of the input of two projections of one shape and format, summed in fp32 and rounded
+ * once; `workspace` holds tgo_pair_grad_workspace_bytes() bytes.  No counterparts in the reference. */
+int tgo_mmq_multi_forward(const void * input_bf16, int count, const void * const * packed, void * const * outputs_bf16,
+                          const int64_t * out_features, const int * quant_types, void * workspace, void * scratch, int64_t rows,
+                          int64_t in_features, int operand, void * stream);
+int64_t tgo_pair_grad_workspace_bytes(int64_t rows, int64_t out_features, int64_t in_features, int quant_type);
+int tgo_mmq_pair_grad_input(const void * grad_output_first, const void * grad_output_second, const void * packed_first,
+                            const void * packed_second, void * grad_input_bf16, void * workspace, int64_t rows, int64_t out_features,
+                            int64_t in_features, int quant_type, void * stream);
+
 /* tgo_mmq_forward without a workspace argument and without any allocation: the q8_1 activation
  * workspace is a fixed array inside the library's code object (one copy per GPU, held until the
  * process ends), TGO_STATIC_WORKSPACE_BYTES large.  Calls whose

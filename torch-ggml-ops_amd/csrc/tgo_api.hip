@@ -424,6 +424,46 @@ int tgo_mmq_forward_prepared(const void * workspace, const void * packed, void *
                                        tgo::forward_operand_kind(0), stream);
 }
 
+int tgo_mmq_multi_forward(const void * input_bf16, int count, const void * const * packed, void * const * outputs_bf16,
+                          const int64_t * out_features, const int * quant_types, void * workspace, void * scratch, int64_t rows,
+                          int64_t in_features, int operand, void * stream) {
+    TGO_TRY(check_pointer(input_bf16, "input"));
+    TGO_TRY(check_pointer(workspace, "workspace"));
+    TGO_TRY(check_workspace_operand(operand));
+    if (count <= 0) {
+        return fail(TGO_ERR_INVALID, "at least one projection is required; got %d", count);
+    }
+    for (int i = 0; i < count; ++i) {
+        TGO_TRY(check_matmul_shape(rows, in_features, out_features[i], quant_types[i]));
+        TGO_TRY(check_pointer(packed[i], "packed_weight"));
+        TGO_TRY(check_pointer(outputs_bf16[i], "output"));
+    }
+    hipStream_t hip_stream = static_cast<hipStream_t>(stream);
+    const tgo::Q8Workspace view = tgo::q8_workspace_view(workspace, rows, in_features, tgo::use_gemv(rows, 0), operand);
+    TGO_TRY(check_hip(tgo::launch_quantize_q8_1(static_cast<const uint16_t *>(input_bf16), view, rows, in_features, hip_stream),
+                      "quantize_q8_1 launch"));
+    for (int i = 0; i < count; ++i) {
+        // two projections of one shape and format (key and value) side by side in one launch: alone, either leaves most of the
+        // chip idle (2048 rows of 1024 x 4096: 39 us each, 43 us together); calls that take ranges of K fill it by themselves
+        const bool pair = i + 1 < count && !view.by_rows() && quant_types[i] == quant_types[i + 1] && out_features[i] == out_features[i + 1] &&
+                          tgo::forward_partial_bytes(rows, in_features, out_features[i], quant_types[i], view.operand_kind()) == 0;
+        if (pair) {
+            TGO_TRY(check_hip(tgo::launch_mmq_forward(static_cast<const uint8_t *>(packed[i]), static_cast<const uint8_t *>(packed[i + 1]), 0,
+                                                      view, static_cast<uint16_t *>(outputs_bf16[i]),
+                                                      static_cast<uint16_t *>(outputs_bf16[i + 1]), nullptr, static_cast<int>(rows),
+                                                      static_cast<int>(in_features), static_cast<int>(out_features[i]), quant_types[i],
+                                                      hip_stream),
+                              "mmq_multi_forward launch"));
+            ++i;
+        } else {
+            TGO_TRY(check_hip(launch_dense(packed[i], view, outputs_bf16[i], scratch, rows, in_features, out_features[i], quant_types[i],
+                                           hip_stream),
+                              "mmq_multi_forward launch"));
+        }
+    }
+    return TGO_OK;
+}
+
 int tgo_mmq_grad_input(const void * grad_output_bf16, const void * packed, void * grad_input_bf16,
                        void * workspace, int64_t rows, int64_t out_features, int64_t in_features,
                        int quant_type, void * stream) {
@@ -447,6 +487,39 @@ int tgo_mmq_grad_input(const void * grad_output_bf16, const void * packed, void 
                                                 static_cast<int>(rows), static_cast<int>(out_features),
                                                 static_cast<int>(in_features), quant_type, hip_stream, partial),
                      "mmq_grad_input launch");
+}
+
+int64_t tgo_pair_grad_workspace_bytes(int64_t rows, int64_t out_features, int64_t in_features, int quant_type) {
+    const int64_t single = tgo_dense_grad_workspace_bytes(rows, out_features, in_features, quant_type);
+    return single < 0 ? single : single + (tgo::cotangent_workspace_bytes(rows, out_features) + 15) / 16 * 16;
+}
+
+int tgo_mmq_pair_grad_input(const void * grad_output_first, const void * grad_output_second, const void * packed_first,
+                            const void * packed_second, void * grad_input_bf16, void * workspace, int64_t rows, int64_t out_features,
+                            int64_t in_features, int quant_type, void * stream) {
+    TGO_TRY(check_matmul_shape(rows, in_features, out_features, quant_type));
+    TGO_TRY(check_pointer(grad_output_first, "grad_output"));
+    TGO_TRY(check_pointer(grad_output_second, "grad_output"));
+    TGO_TRY(check_pointer(packed_first, "packed_weight"));
+    TGO_TRY(check_pointer(packed_second, "packed_weight"));
+    TGO_TRY(check_pointer(grad_input_bf16, "grad_input"));
+    TGO_TRY(check_pointer(workspace, "workspace"));
+    hipStream_t hip_stream = static_cast<hipStream_t>(stream);
+    const int64_t cotangent_bytes = (tgo::cotangent_workspace_bytes(rows, out_features) + 15) / 16 * 16;
+    uint8_t * const cotangent = static_cast<uint8_t *>(workspace);
+    TGO_TRY(check_hip(tgo::launch_pack_cotangent(static_cast<const uint16_t *>(grad_output_first),
+                                                 static_cast<const uint16_t *>(grad_output_second), cotangent,
+                                                 cotangent + cotangent_bytes, static_cast<int>(rows), static_cast<int>(out_features),
+                                                 hip_stream),
+                      "pack_cotangent launch"));
+    float * const partial = tgo::dense_grad_partial_bytes(rows, out_features, in_features) > 0
+        ? reinterpret_cast<float *>(cotangent + 2 * cotangent_bytes)
+        : nullptr;
+    return check_hip(tgo::launch_mmq_grad_input(cotangent, cotangent + cotangent_bytes, static_cast<const uint8_t *>(packed_first),
+                                                static_cast<const uint8_t *>(packed_second), 0, static_cast<uint16_t *>(grad_input_bf16),
+                                                nullptr, static_cast<int>(rows), static_cast<int>(out_features),
+                                                static_cast<int>(in_features), quant_type, hip_stream, partial),
+                     "mmq_pair_grad_input launch");
 }
 
 // ---- chunked cross-entropy through a packed head --------------------------------------------------------------

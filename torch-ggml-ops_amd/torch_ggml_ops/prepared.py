@@ -17,11 +17,13 @@ sequence run on the scaled kernels like one large ``mmq``.
 The reference has no such operator; it lists this reuse as its next optimisation
 (docs/mmq_fwd_optimization.md:299-307).  ``mmq_multi`` is the convenience wrapper with autograd
 (gradient with respect to the input only, as for ``mmq``: the sum of the projections'
-``mmq_grad_input``).
+``mmq_grad_input``, that of two neighbours of one shape and format taken in fp32); its forward is one call into the
+library, which quantizes and multiplies.
 """
 
 from __future__ import annotations
 
+import ctypes
 from typing import Sequence
 
 import torch
@@ -108,33 +110,109 @@ def _mmq_prepared_fake(workspace, packed_weight, rows, in_features, quant_type, 
     return workspace.new_empty((rows, out_features), dtype=torch.bfloat16)
 
 
+torch.library.define(
+    "torch_ggml_ops::mmq_multi_forward",
+    "(Tensor input, Tensor[] packed_weights, int[] quant_types, int[] out_features, str operand) -> Tensor[]",
+)
+torch.library.define(
+    "torch_ggml_ops::mmq_pair_grad_input",
+    "(Tensor first_grad_output, Tensor second_grad_output, Tensor first_packed_weight, Tensor second_packed_weight, "
+    "int quant_type, int in_features) -> Tensor",
+)
+
+
+@torch.library.impl("torch_ggml_ops::mmq_multi_forward", "CUDA")
+def _multi_device(input, packed_weights, quant_types, out_features, operand):
+    rows, in_features = _activation_shape(input)
+    kind = _workspace_kind(operand)
+    with _native.on_device(input.device):
+        workspace = input.new_empty((_native.lib.tgo_q8_workspace_bytes(rows, in_features),), dtype=torch.uint8)
+        for weight, quant_type, features in zip(packed_weights, quant_types, out_features):
+            _validate.prepared(workspace, weight, rows, in_features, quant_type, features)
+        outputs = [input.new_empty((*input.shape[:-1], features)) for features in out_features]
+        scratch_bytes = max(
+            _native.lib.tgo_forward_scratch_bytes(rows, in_features, features, quant_type)
+            for quant_type, features in zip(quant_types, out_features)
+        )
+        scratch = input.new_empty((scratch_bytes,), dtype=torch.uint8) if scratch_bytes > 0 else None
+        count = len(outputs)
+        pointers = ctypes.c_void_p * count
+        _native.check(
+            _native.lib.tgo_mmq_multi_forward(
+                input.data_ptr(), count, pointers(*(w.data_ptr() for w in packed_weights)),
+                pointers(*(o.data_ptr() for o in outputs)), (ctypes.c_int64 * count)(*out_features),
+                (ctypes.c_int * count)(*quant_types), workspace.data_ptr(), None if scratch is None else scratch.data_ptr(),
+                rows, in_features, kind, _stream(input),
+            )
+        )
+    return outputs
+
+
+@torch.library.register_fake("torch_ggml_ops::mmq_multi_forward")
+def _multi_fake(input, packed_weights, quant_types, out_features, operand):
+    return [input.new_empty((*input.shape[:-1], features)) for features in out_features]
+
+
+@torch.library.impl("torch_ggml_ops::mmq_pair_grad_input", "CUDA")
+def _pair_grad_input_device(first_grad, second_grad, first_weight, second_weight, quant_type, in_features):
+    rows, in_features, out_features = _validate.dense(first_grad, first_weight, quant_type, in_features, backward=True)
+    if _validate.dense(second_grad, second_weight, quant_type, in_features, backward=True) != (rows, in_features, out_features):
+        raise RuntimeError("the two projections of a pair must have the same shape")
+    if second_grad.device != first_grad.device:
+        raise RuntimeError("all tensors of a pair must be on the same device")
+    with _native.on_device(first_grad.device):
+        grad_input = first_grad.new_empty((*first_grad.shape[:-1], in_features))
+        workspace = first_grad.new_empty(
+            (_native.lib.tgo_pair_grad_workspace_bytes(rows, out_features, in_features, quant_type),), dtype=torch.uint8
+        )
+        _native.check(
+            _native.lib.tgo_mmq_pair_grad_input(
+                first_grad.data_ptr(), second_grad.data_ptr(), first_weight.data_ptr(), second_weight.data_ptr(),
+                grad_input.data_ptr(), workspace.data_ptr(), rows, out_features, in_features, int(quant_type), _stream(first_grad),
+            )
+        )
+    return grad_input
+
+
+@torch.library.register_fake("torch_ggml_ops::mmq_pair_grad_input")
+def _pair_grad_input_fake(first_grad, second_grad, first_weight, second_weight, quant_type, in_features):
+    return first_grad.new_empty((*first_grad.shape[:-1], in_features))
+
+
 class _MultiProjection(torch.autograd.Function):
     @staticmethod
     def forward(ctx, input, quant_types, out_features, *packed_weights):
         rows, in_features = _activation_shape(input)
+        quant_types, out_features = [int(q) for q in quant_types], [int(n) for n in out_features]
         operand = multi_operand(quant_types, rows, out_features)
-        workspace = torch.ops.torch_ggml_ops.quantize_q8_1.default(input, operand)
-        outputs = tuple(
-            torch.ops.torch_ggml_ops.mmq_prepared.default(
-                workspace, weight, rows, in_features, int(quant_type), int(features), operand
-            ).view(*input.shape[:-1], int(features))
-            for weight, quant_type, features in zip(packed_weights, quant_types, out_features)
-        )
-        ctx.quant_types = tuple(int(q) for q in quant_types)
+        outputs = torch.ops.torch_ggml_ops.mmq_multi_forward.default(input, packed_weights, quant_types, out_features, operand)
+        ctx.quant_types, ctx.out_features = quant_types, out_features
         ctx.in_features = in_features
         ctx.save_for_backward(*packed_weights)
-        return outputs
+        return tuple(outputs)
 
     @staticmethod
     def backward(ctx, *grad_outputs):
         grad_input = None
         if ctx.needs_input_grad[0]:
-            for grad, weight, quant_type in zip(grad_outputs, ctx.saved_tensors, ctx.quant_types):
+            weights = ctx.saved_tensors
+            i = 0
+            while i < len(weights):
+                grad, weight, quant_type = grad_outputs[i], weights[i], ctx.quant_types[i]
+                i += 1
                 if grad is None:
                     continue
-                term = torch.ops.torch_ggml_ops.mmq_grad_input.default(
-                    grad.contiguous(), weight, quant_type, ctx.in_features
-                )
+                # two neighbours of one shape and format (key and value): one kernel, summed in fp32
+                if (
+                    i < len(weights) and grad_outputs[i] is not None and ctx.quant_types[i] == quant_type
+                    and ctx.out_features[i] == ctx.out_features[i - 1]
+                ):
+                    term = torch.ops.torch_ggml_ops.mmq_pair_grad_input.default(
+                        grad.contiguous(), grad_outputs[i].contiguous(), weight, weights[i], quant_type, ctx.in_features
+                    )
+                    i += 1
+                else:
+                    term = torch.ops.torch_ggml_ops.mmq_grad_input.default(grad.contiguous(), weight, quant_type, ctx.in_features)
                 grad_input = term if grad_input is None else grad_input + term
         return (grad_input, None, None) + (None,) * len(ctx.saved_tensors)
 
