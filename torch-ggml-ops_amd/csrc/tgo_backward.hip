@@ -825,7 +825,9 @@ constexpr int BSP_GRID = 256;                      // one workgroup per CU
 // persistent loop (it drains the queue once per round, which exposes a full memory latency every few steps),
 // so the prefetches of the role-split kernel are issued and awaited by hand.  Global loads return in order:
 // waiting until at most N of them are outstanding completes everything but the N youngest.  The wait names
-// the awaited registers as read-write operands so that no use of them can be scheduled ahead of it.
+// the awaited registers as read-write operands so that no use of them can be scheduled ahead of it.  What that cannot forbid
+// -- a copy, a spill or a reuse of a register between its load and its wait -- check_loads_in_flight.py looks for on every
+// path of the assembly, and the build fails if there is one.
 
 // `base` must be wave-uniform (it travels in scalar registers); `offset` is this lane's byte offset.
 template <int IMMEDIATE = 0>
@@ -975,6 +977,11 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
         return;
     }
     const int total_steps = step_count;
+    // Both roles walk whole rounds of the decoders' ring.  Steps behind the last one repeat its loads and are not multiplied (at
+    // most three, none where the matrix has a multiple of 256 rows): so no branch leads around a load or its wait, and every
+    // path through the loops is one that can be taken, which is what the build's proof (check_loads_in_flight.py) follows.
+    const int walked_steps = (total_steps + BSP_RAW_DEPTH - 1) / BSP_RAW_DEPTH * BSP_RAW_DEPTH;
+    static_assert(BSP_RAW_DEPTH % BSP_COT_DEPTH == 0, "the multipliers' rounds fill the decoders'");
 
     auto item_field = [&](int item, int field) {
         return __builtin_amdgcn_readfirstlane(reinterpret_cast<const int *>(&items[item])[field]);
@@ -1269,25 +1276,23 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
         // wrote without waiting; the fences only keep the compiler from reordering them.
         int g3 = 0;   // g % 3
 #pragma unroll 1
-        for (int base = 0; base < total_steps; base += BSP_RAW_DEPTH) {
+        for (int base = 0; base < walked_steps; base += BSP_RAW_DEPTH) {
 #pragma unroll
             for (int u = 0; u < BSP_RAW_DEPTH; ++u) {
                 const int g = base + u;
-                if (g < total_steps) {
-                    const int g3_plus1 = g3 == 2 ? 0 : g3 + 1;
-                    const int g3_plus2 = g3_plus1 == 2 ? 0 : g3_plus1 + 1;
-                    const ScaleInputs scale_inputs = scales_fetch(info[4], raw_slot(g3_plus2));
-                    __builtin_amdgcn_sched_barrier(0);
-                    decode_finish(info[5], pending, wb[(g + 1) & 1]);
-                    scales_finish(info[4], scale_inputs, sm_slot(g & 1), octet_slot(g & 1));
-                    park(ring[(u + 3) % BSP_RAW_DEPTH], raw_slot(g3));
-                    wave_sync();
-                    pending = decode_fetch(info[4], raw_slot(g3_plus2), sm_slot(g & 1), octet_slot(g & 1));
-                    request(ring[(u + 3) % BSP_RAW_DEPTH]);
-                    __builtin_amdgcn_sched_barrier(0);
-                    g3 = g3_plus1;
-                    __syncthreads();
-                }
+                const int g3_plus1 = g3 == 2 ? 0 : g3 + 1;
+                const int g3_plus2 = g3_plus1 == 2 ? 0 : g3_plus1 + 1;
+                const ScaleInputs scale_inputs = scales_fetch(info[4], raw_slot(g3_plus2));
+                __builtin_amdgcn_sched_barrier(0);
+                decode_finish(info[5], pending, wb[(g + 1) & 1]);
+                scales_finish(info[4], scale_inputs, sm_slot(g & 1), octet_slot(g & 1));
+                park(ring[(u + 3) % BSP_RAW_DEPTH], raw_slot(g3));
+                wave_sync();
+                pending = decode_fetch(info[4], raw_slot(g3_plus2), sm_slot(g & 1), octet_slot(g & 1));
+                request(ring[(u + 3) % BSP_RAW_DEPTH]);
+                __builtin_amdgcn_sched_barrier(0);
+                g3 = g3_plus1;
+                __syncthreads();
             }
         }
         return;
@@ -1347,82 +1352,80 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
     }
     __syncthreads();
 #pragma unroll 1
-    for (int base = 0; base < total_steps; base += BSP_COT_DEPTH) {
+    for (int base = 0; base < walked_steps; base += BSP_COT_DEPTH) {
 #pragma unroll
         for (int u = 0; u < BSP_COT_DEPTH; ++u) {
             const int g = base + u;
-            if (g < total_steps) {
-                load_cotangent(c_fetch, cot[(u + BSP_COT_DEPTH - 1) % BSP_COT_DEPTH]);
-                fetch_next();
-                await_loads<COT_YOUNGER>(cot[u]);
-                const int wave_row = c_now.row_start + wave * 64;
-                const int row_end = c_now.row_end;
-                if (wave_row < row_end) {
-                    // 16 weight fragments (4 chunks x 4 column tiles), two MFMAs each.  An LDS read takes
-                    // longer than the two MFMAs it feeds, so fragment j + AHEAD is requested before fragment j
-                    // is used; the scheduling groups below pin that interleaving.
-                    const uint16_t * tile = wb[g & 1] + l32 * BWD_PITCH + 8 * half;
-                    auto read_fragment = [&](int j) {
-                        return *reinterpret_cast<const uint4 *>(&tile[(j & 3) * 32 * BWD_PITCH + 16 * (j >> 2)]);
-                    };
-                    constexpr int AHEAD = 6;
-                    uint4 fragment[16];
+            load_cotangent(c_fetch, cot[(u + BSP_COT_DEPTH - 1) % BSP_COT_DEPTH]);
+            fetch_next();
+            await_loads<COT_YOUNGER>(cot[u]);
+            const int wave_row = c_now.row_start + wave * 64;
+            const int row_end = c_now.row_end;
+            if (wave_row < row_end && g < total_steps) {
+                // 16 weight fragments (4 chunks x 4 column tiles), two MFMAs each.  An LDS read takes
+                // longer than the two MFMAs it feeds, so fragment j + AHEAD is requested before fragment j
+                // is used; the scheduling groups below pin that interleaving.
+                const uint16_t * tile = wb[g & 1] + l32 * BWD_PITCH + 8 * half;
+                auto read_fragment = [&](int j) {
+                    return *reinterpret_cast<const uint4 *>(&tile[(j & 3) * 32 * BWD_PITCH + 16 * (j >> 2)]);
+                };
+                constexpr int AHEAD = 6;
+                uint4 fragment[16];
 #pragma unroll
-                    for (int j = 0; j < AHEAD; ++j) {
-                        fragment[j] = read_fragment(j);
+                for (int j = 0; j < AHEAD; ++j) {
+                    fragment[j] = read_fragment(j);
+                }
+#pragma unroll
+                for (int j = 0; j < 16; ++j) {
+                    if (j + AHEAD < 16) {
+                        fragment[j + AHEAD] = read_fragment(j + AHEAD);
                     }
 #pragma unroll
-                    for (int j = 0; j < 16; ++j) {
-                        if (j + AHEAD < 16) {
-                            fragment[j + AHEAD] = read_fragment(j + AHEAD);
-                        }
-#pragma unroll
-                        for (int rt = 0; rt < 2; ++rt) {
-                            // (operands swapped: the lane ends up with one task row and runs of four neighbouring
-                            // columns, which the epilogue stages with 8-byte LDS writes instead of 2-byte ones)
-                            acc[rt][j & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                                __builtin_bit_cast(v8bf, fragment[j]), __builtin_bit_cast(v8bf, cot[u][rt][j >> 2]),
-                                acc[rt][j & 3], 0, 0, 0);
-                        }
-                    }
-                    __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);   // LDS reads
-#pragma unroll
-                    for (int j = 0; j < 16; ++j) {
-                        if (j + AHEAD < 16) {
-                            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                        }
-                        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);   // MFMAs
-                    }
-                    if (c_now.source == a.sources - 1 && c_now.n_step == c_now.step_end - 1) {
-                        // last step of the item: transpose the results through this wave's staging area
-                        // and write whole rows, then start the next item from zero
-                        const int k_tile = c_now.k_tile;
-                        // recomputing the per-lane store offsets here is cheaper than keeping them alive
-                        // (spilled) through the loop, which is what happens if they can be hoisted
-                        int lane_here = lane;
-                        asm volatile("" : "+v"(lane_here));
-#pragma unroll
-                        for (int rt = 0; rt < 2; ++rt) {
-                            const int r0 = wave_row + rt * 32;
-                            if (a.n_splits > 1) {
-                                store_partial_32x128(a, acc[rt], item_field(c_now.item, 6), r0 + (lane_here & 31), row_end, k_tile,
-                                                     lane_here >> 5);
-                            } else if (r0 < row_end) {
-                                store_rows_32x128<BWD_TK + 8, true, true>(
-                                    stage_all[wave], acc[rt],
-                                    a.dx + static_cast<int64_t>(r0) * a.in_features + k_tile * BWD_TK, a.in_features,
-                                    row_end - r0, BWD_TK, lane_here);
-                            }
-#pragma unroll
-                            for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-                                for (int v = 0; v < 16; ++v) acc[rt][kt][v] = 0.0f;
-                        }
+                    for (int rt = 0; rt < 2; ++rt) {
+                        // (operands swapped: the lane ends up with one task row and runs of four neighbouring
+                        // columns, which the epilogue stages with 8-byte LDS writes instead of 2-byte ones)
+                        acc[rt][j & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            __builtin_bit_cast(v8bf, fragment[j]), __builtin_bit_cast(v8bf, cot[u][rt][j >> 2]),
+                            acc[rt][j & 3], 0, 0, 0);
                     }
                 }
-                advance(c_now, rebase_none, 0);
-                __syncthreads();
+                __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);   // LDS reads
+#pragma unroll
+                for (int j = 0; j < 16; ++j) {
+                    if (j + AHEAD < 16) {
+                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    }
+                    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);   // MFMAs
+                }
+                if (c_now.source == a.sources - 1 && c_now.n_step == c_now.step_end - 1) {
+                    // last step of the item: transpose the results through this wave's staging area
+                    // and write whole rows, then start the next item from zero
+                    const int k_tile = c_now.k_tile;
+                    // recomputing the per-lane store offsets here is cheaper than keeping them alive
+                    // (spilled) through the loop, which is what happens if they can be hoisted
+                    int lane_here = lane;
+                    asm volatile("" : "+v"(lane_here));
+#pragma unroll
+                    for (int rt = 0; rt < 2; ++rt) {
+                        const int r0 = wave_row + rt * 32;
+                        if (a.n_splits > 1) {
+                            store_partial_32x128(a, acc[rt], item_field(c_now.item, 6), r0 + (lane_here & 31), row_end, k_tile,
+                                                 lane_here >> 5);
+                        } else if (r0 < row_end) {
+                            store_rows_32x128<BWD_TK + 8, true, true>(
+                                stage_all[wave], acc[rt],
+                                a.dx + static_cast<int64_t>(r0) * a.in_features + k_tile * BWD_TK, a.in_features,
+                                row_end - r0, BWD_TK, lane_here);
+                        }
+#pragma unroll
+                        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+                            for (int v = 0; v < 16; ++v) acc[rt][kt][v] = 0.0f;
+                    }
+                }
             }
+            advance(c_now, rebase_none, 0);
+            __syncthreads();
         }
     }
 }
