@@ -58,6 +58,28 @@ def test_routing_weight_gradient_and_inverse(ops, tokens, top_k, features):
     assert np.array_equal(token.cpu().numpy(), expected_token) and np.array_equal(weight.cpu().numpy(), expected_weight)
 
 
+def test_gradients_of_the_routing_weight_gradient(ops):
+    tgo, _ = ops
+    tokens, top_k, features = 33, 4, 72
+    slot_rows = torch.randperm(tokens * top_k, generator=torch.Generator().manual_seed(1)).reshape(tokens, top_k).cuda()
+    slot_rows[0, 1], slot_rows[5, 0] = -1, tokens * top_k
+    results = []
+    for dtype in (torch.bfloat16, torch.float64):
+        rows = random_bf16((tokens * top_k, features), seed=2).to(dtype).requires_grad_()
+        cotangent = random_bf16((tokens, features), seed=3).to(dtype).requires_grad_()
+        weights = torch.ones(tokens, top_k, device="cuda", requires_grad=True)
+        if dtype == torch.bfloat16:
+            out = tgo.moe_combine(rows, slot_rows, weights)
+        else:
+            present = (slot_rows >= 0) & (slot_rows < tokens * top_k)
+            out = (rows[slot_rows.clamp(0, tokens * top_k - 1)] * (weights * present).unsqueeze(-1)).sum(1)
+        (grad_weights,) = torch.autograd.grad(out, weights, cotangent, create_graph=True)
+        results.append(torch.autograd.grad(grad_weights.square().sum(), (rows, cotangent)))
+    for actual, expected in zip(*results):
+        # (each result is rounded to bf16 once)
+        torch.testing.assert_close(actual.double(), expected, rtol=2**-8, atol=1e-4 * expected.abs().max().item())
+
+
 @pytest.mark.parametrize("rows,offsets,experts", ((700, (3, 3, 255, 256, 600), (0, 1, 7, 2, 3)), (5, (5,), (0,)), (300, (400, 10), (0, 1))))
 def test_rows_outside_every_group_are_cleared(ops, rows, offsets, experts):
     """Empty groups, groups of an expert that does not exist and groups that end behind the rows cover nothing."""

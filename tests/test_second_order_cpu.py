@@ -1,0 +1,80 @@
+"""Gradients of gradients, with tensor operations on the CPU standing in for the kernels: what the formulas give must be what
+differentiating the plain computation twice gives, and what they do not cover must be an error rather than zero."""
+
+import pytest
+import torch
+
+import torch_ggml_ops as tgo
+from torch_ggml_ops import _validate
+
+
+def plain_combine(rows, slot_rows, slot_weights):
+    present = (slot_rows >= 0) & (slot_rows < rows.shape[0])
+    picked = rows[slot_rows.clamp(0, rows.shape[0] - 1)]
+    return (picked * (slot_weights * present).unsqueeze(-1)).sum(1)
+
+
+def plain_weight_grad(rows, grad_tokens, slot_rows):
+    present = (slot_rows >= 0) & (slot_rows < rows.shape[0])
+    return (rows[slot_rows.clamp(0, rows.shape[0] - 1)] * grad_tokens.unsqueeze(1)).sum(-1) * present
+
+
+@pytest.fixture
+def stand_ins():
+    """Registers CPU implementations of the named operators for the time of a test."""
+    library = torch.library.Library("torch_ggml_ops", "IMPL")
+
+    def register(**implementations):
+        for name, implementation in implementations.items():
+            library.impl(name, torch.no_grad()(implementation), "CPU")   # (like a kernel: autograd sees nothing of it)
+
+    yield register
+    library._destroy()
+
+
+@pytest.fixture
+def combine_on_cpu(stand_ins):
+    stand_ins(moe_combine=plain_combine, moe_combine_weight_grad=plain_weight_grad)
+
+
+# (one slot past the rows, one before them, a row that no slot names)
+SLOT_ROWS = torch.tensor([[0, 4], [7, 2], [3, -1]])
+
+
+def combine_inputs():
+    generator = torch.Generator().manual_seed(1)
+    rows = torch.randn(6, 8, generator=generator).requires_grad_()
+    weights = torch.rand(3, 2, generator=generator).requires_grad_()
+    return rows, weights, torch.randn(3, 8, generator=generator).requires_grad_(), torch.randn(3, 2, generator=generator)
+
+
+def test_gradients_of_the_routing_weights_gradient(combine_on_cpu):
+    results = []
+    for combine in (tgo.moe_combine, plain_combine):
+        rows, weights, cotangent, direction = combine_inputs()
+        (grad_weights,) = torch.autograd.grad(combine(rows, SLOT_ROWS, weights), weights, cotangent, create_graph=True)
+        penalty = (grad_weights.square() * direction).sum()
+        grad_rows, grad_cotangent = torch.autograd.grad(penalty, (rows, cotangent), create_graph=True)
+        third = torch.autograd.grad(grad_rows.square().sum() + grad_cotangent.square().sum(), (rows, cotangent))
+        results.append((grad_weights, grad_rows, grad_cotangent, *third))
+    for actual, expected in zip(*results):
+        assert expected.norm() > 0
+        torch.testing.assert_close(actual, expected)   # (fp32 on both sides)
+
+
+def test_gradient_through_the_expert_sorted_rows_is_refused(stand_ins, combine_on_cpu):
+    """``grouped_mmq_combine`` has no gradient for what flows back through the sorted rows that its weights' gradient is
+    made of: an error, not a part that is missing."""
+
+    def product(input, packed, indices, offsets, slot_rows, slot_weights, quant_type, out_features):
+        rows = input @ packed.float()
+        return plain_combine(rows, slot_rows, slot_weights), rows
+
+    stand_ins(grouped_mmq_combine=product)
+    rows, weights, cotangent, _ = combine_inputs()
+    packed = torch.randint(0, 3, (8, 8), generator=torch.Generator().manual_seed(2), dtype=torch.uint8)
+    none = torch.zeros(1, dtype=torch.int64)
+    out = tgo.grouped_mmq_combine(rows.detach(), packed, none, none, SLOT_ROWS, weights, 12, 8)
+    (grad_weights,) = torch.autograd.grad(out, weights, cotangent, create_graph=True)
+    with pytest.raises(RuntimeError, match="auxiliary output without a gradient"):
+        grad_weights.sum().backward()

@@ -124,6 +124,43 @@ def _invert_slots_fake(slot_rows, slot_weights, num_rows):
     return slot_rows.new_empty((num_rows,)), slot_rows.new_empty((num_rows,), dtype=torch.float32)
 
 
+def _slots_to_rows(grad_tokens, slot_rows, slot_weights, num_rows):
+    """``out[slot_rows[t, j]] = slot_weights[t, j] * grad_tokens[t]``, zeros in the rows that no slot names."""
+    flat = slot_rows.reshape(-1)
+    present = (flat >= 0) & (flat < num_rows)
+    per_slot = grad_tokens.repeat_interleave(slot_rows.shape[1], dim=0)
+    scaled = (per_slot.float() * (slot_weights.reshape(-1, 1) * present.unsqueeze(1))).to(grad_tokens.dtype)
+    out = grad_tokens.new_zeros((num_rows, grad_tokens.shape[1]))
+    # every row belongs to at most one slot, so this is a plain scatter, not a reduction
+    out.index_add_(0, flat.clamp(0, num_rows - 1), scaled)
+    return out
+
+
+def _setup_weight_grad_context(ctx, inputs, output) -> None:
+    rows, grad_tokens, slot_rows = inputs
+    ctx.num_rows = rows.shape[0]
+    ctx.save_for_backward(
+        rows if ctx.needs_input_grad[1] else None, grad_tokens if ctx.needs_input_grad[0] else None, slot_rows
+    )
+
+
+def _weight_grad_backward(ctx, grad):
+    """The product is bilinear: the one factor's gradient is the combine with ``grad`` as its weights, the other's the
+    combine's own backward."""
+    rows, grad_tokens, slot_rows = ctx.saved_tensors
+    grad_rows = grad_grad_tokens = None
+    if ctx.needs_input_grad[0]:
+        grad_rows = _slots_to_rows(grad_tokens, slot_rows, grad, ctx.num_rows)
+    if ctx.needs_input_grad[1]:
+        grad_grad_tokens = torch.ops.torch_ggml_ops.moe_combine.default(rows, slot_rows, grad.contiguous())
+    return grad_rows, grad_grad_tokens, None
+
+
+torch.library.register_autograd(
+    "torch_ggml_ops::moe_combine_weight_grad", _weight_grad_backward, setup_context=_setup_weight_grad_context
+)
+
+
 def _setup_combine_context(ctx, inputs, output) -> None:
     rows, slot_rows, slot_weights = inputs
     ctx.num_rows = rows.shape[0]
@@ -132,17 +169,9 @@ def _setup_combine_context(ctx, inputs, output) -> None:
 
 def _combine_backward(ctx, grad_output):
     rows, slot_rows, slot_weights = ctx.saved_tensors
-    _tokens, top_k = slot_rows.shape
     grad_rows = grad_weights = None
     if ctx.needs_input_grad[0]:
-        flat = slot_rows.reshape(-1)
-        present = (flat >= 0) & (flat < ctx.num_rows)
-        safe = flat.clamp(0, ctx.num_rows - 1)
-        grad_per_slot = grad_output.repeat_interleave(top_k, dim=0)
-        scaled = (grad_per_slot.float() * (slot_weights.reshape(-1, 1) * present.unsqueeze(1))).to(grad_output.dtype)
-        grad_rows = grad_output.new_zeros((ctx.num_rows, grad_output.shape[1]))
-        # every row belongs to at most one slot, so this is a plain scatter, not a reduction
-        grad_rows.index_add_(0, safe, scaled)
+        grad_rows = _slots_to_rows(grad_output, slot_rows, slot_weights, ctx.num_rows)
     if ctx.needs_input_grad[2]:
         grad_weights = torch.ops.torch_ggml_ops.moe_combine_weight_grad.default(rows, grad_output.contiguous(), slot_rows)
     return grad_rows, None, grad_weights
