@@ -78,3 +78,28 @@ def test_gradient_through_the_expert_sorted_rows_is_refused(stand_ins, combine_o
     (grad_weights,) = torch.autograd.grad(out, weights, cotangent, create_graph=True)
     with pytest.raises(RuntimeError, match="auxiliary output without a gradient"):
         grad_weights.sum().backward()
+
+
+@pytest.mark.parametrize("widths", ((3, 5), (3, 3), (5, 3, 3)))
+def test_projections_of_one_input_refuse_a_second_gradient(stand_ins, monkeypatch, widths):
+    """Two neighbours of one shape and format share a grad-input kernel, the others have one each: both refuse alike."""
+    monkeypatch.setattr(_validate, "REQUIRE_DEVICE", False)
+
+    def product(grad, packed, quant_type, in_features):
+        return (grad.float() @ packed.float()).to(grad.dtype)
+
+    stand_ins(
+        mmq_multi_forward=lambda input, weights, *rest: [(input.float() @ w.float().t()).to(input.dtype) for w in weights],
+        mmq_grad_input=product,
+        mmq_pair_grad_input=lambda g1, g2, w1, w2, *rest: product(g1, w1, *rest) + product(g2, w2, *rest),
+    )
+    generator = torch.Generator().manual_seed(3)
+    x = torch.randn(4, 256, generator=generator).bfloat16().requires_grad_()
+    weights = [torch.randint(0, 3, (n, 256), generator=generator, dtype=torch.uint8) for n in widths]
+    outputs = tgo.mmq_multi(x, weights, [12] * len(widths), widths)
+    cotangents = [torch.randn(o.shape, generator=generator).bfloat16().requires_grad_() for o in outputs]
+    (grad,) = torch.autograd.grad(outputs, x, cotangents, create_graph=True)
+    expected = sum(c.double() @ w.double() for c, w in zip(cotangents, weights))
+    torch.testing.assert_close(grad.double(), expected, rtol=2**-6, atol=2**-6 * expected.abs().max().item())
+    with pytest.raises(RuntimeError, match="does not support higher-order gradients"):
+        torch.autograd.grad(grad.float().sum(), cotangents)

@@ -179,6 +179,13 @@ def _pair_grad_input_fake(first_grad, second_grad, first_weight, second_weight, 
     return first_grad.new_empty((*first_grad.shape[:-1], in_features))
 
 
+def _pair_grad_input_backward(ctx, grad_grad_input):
+    raise RuntimeError("torch_ggml_ops::mmq_pair_grad_input does not support higher-order gradients")
+
+
+torch.library.register_autograd("torch_ggml_ops::mmq_pair_grad_input", _pair_grad_input_backward)
+
+
 class _MultiProjection(torch.autograd.Function):
     @staticmethod
     def forward(ctx, input, quant_types, out_features, *packed_weights):
