@@ -103,3 +103,51 @@ def test_projections_of_one_input_refuse_a_second_gradient(stand_ins, monkeypatc
     torch.testing.assert_close(grad.double(), expected, rtol=2**-6, atol=2**-6 * expected.abs().max().item())
     with pytest.raises(RuntimeError, match="does not support higher-order gradients"):
         torch.autograd.grad(grad.float().sum(), cotangents)
+
+
+def _opaque(shape):
+    return lambda *args, **kwargs: torch.ones(shape, dtype=torch.bfloat16)
+
+
+@pytest.mark.parametrize("which", ("gathered", "pair_gathered", "swiglu", "swiglu_slots", "combine"))
+def test_backward_made_of_kernels_refuses_a_second_gradient(stand_ins, combine_on_cpu, monkeypatch, which):
+    """Backward formulas that call kernels directly: autograd sees a constant there, so what flows through it has to raise."""
+    from torch_ggml_ops import gathered, swiglu
+
+    rows, tokens, k, n = 6, 3, 256, 8
+    generator = torch.Generator().manual_seed(4)
+    hidden = torch.randn(tokens, k, generator=generator).bfloat16().requires_grad_()
+    slot_weights = torch.rand(tokens, 2, generator=generator).requires_grad_()
+    slot_rows = torch.arange(rows).reshape(tokens, 2)
+    row_index = torch.arange(rows) // 2
+    packed, ids = torch.zeros(1, n, 144, dtype=torch.uint8), torch.zeros(1, dtype=torch.int64)
+    for module in (gathered, swiglu):
+        monkeypatch.setattr(module, "_rows_grad_input", _opaque((rows, k)))
+        monkeypatch.setattr(module, "_scatter_to_tokens", _opaque((tokens, k)))
+    monkeypatch.setattr(swiglu, "_sum_slots", _opaque((tokens, k)))
+    monkeypatch.setattr(swiglu, "_activation_backward", lambda *args: (torch.ones(rows, n, dtype=torch.bfloat16),) * 2)
+    one = _opaque((rows, n))
+    stand_ins(
+        grouped_mmq_gathered=one,
+        grouped_mmq_pair_gathered=lambda *args: (one(), one()),
+        grouped_mmq_swiglu=lambda *args: (one(), one(), one()),
+        grouped_mmq_combine=lambda *args: (torch.ones(tokens, n, dtype=torch.bfloat16), one()),
+        invert_slots=lambda slot_rows, slot_weights, num_rows: (row_index.clone(), slot_weights.reshape(-1).clone()),
+        grouped_mmq_grad_input_weighted=_opaque((tokens, k)),
+    )
+    if which == "gathered":
+        outputs = (tgo.grouped_mmq_gathered(hidden, row_index, packed, ids, ids, 12, n),)
+    elif which == "pair_gathered":
+        outputs = tgo.grouped_mmq_pair_gathered(hidden, row_index, packed, packed, ids, ids, 12, n)
+    elif which == "combine":
+        outputs = (tgo.grouped_mmq_combine(hidden, packed, ids, ids, slot_rows, slot_weights, 12, n),)
+    else:
+        listed = slot_rows if which == "swiglu_slots" else None
+        outputs = (tgo.grouped_mmq_swiglu(hidden, packed, packed, ids, ids, 12, n, row_index, listed),)
+    cotangents = [torch.ones_like(o) for o in outputs]
+    assert not torch.autograd.grad(outputs, hidden, cotangents, retain_graph=True)[0].requires_grad
+    cotangents = [c.requires_grad_() for c in cotangents]
+    (grad,) = torch.autograd.grad(outputs, hidden, cotangents, create_graph=True)
+    penalty = grad.float().square().sum() + sum(c.float().sum() for c in cotangents)
+    with pytest.raises(RuntimeError, match="does not support higher-order gradients"):
+        torch.autograd.grad(penalty, cotangents)

@@ -18,6 +18,7 @@ from __future__ import annotations
 import torch
 
 from . import _native
+from .grouped_mmq import _first_order
 from .grouped_mmq import _forward as _grouped_forward
 from .grouped_mmq import _grad_input as _grouped_grad_input
 
@@ -117,7 +118,9 @@ def _gathered_backward(ctx, grad_output):
         grad_rows = _rows_grad_input(
             grad_output, None, packed_weight, None, expert_indices, expert_offsets, ctx.quant_type, ctx.in_features
         )
-        grad_input = _scatter_to_tokens(grad_rows, row_index, ctx.tokens)
+        grad_input = _first_order(
+            "grouped_mmq_gathered", _scatter_to_tokens(grad_rows, row_index, ctx.tokens), grad_output
+        )
     return grad_input, None, None, None, None, None, None
 
 
@@ -153,7 +156,10 @@ def _pair_gathered_backward(ctx, first_grad_output, second_grad_output):
                 second_grad_output, None, second_weight, None, expert_indices, expert_offsets, ctx.quant_type, ctx.in_features
             )
         if grad_rows is not None:
-            grad_input = _scatter_to_tokens(grad_rows, row_index, ctx.tokens)
+            grad_input = _first_order(
+                "grouped_mmq_pair_gathered", _scatter_to_tokens(grad_rows, row_index, ctx.tokens),
+                first_grad_output, second_grad_output,
+            )
     return grad_input, None, None, None, None, None, None, None
 
 

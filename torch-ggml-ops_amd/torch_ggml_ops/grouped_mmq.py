@@ -217,6 +217,25 @@ def _no_double_backward(name: str):
     return backward
 
 
+class _FirstOrder(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, name, result, *sources):
+        ctx.name = name
+        return result.view_as(result)
+
+    @staticmethod
+    def backward(ctx, grad):
+        raise RuntimeError(f"torch_ggml_ops::{ctx.name} does not support higher-order gradients")
+
+
+def _first_order(name: str, result: torch.Tensor, *sources):
+    """``result`` of a backward formula that calls kernels directly, which autograd takes for a constant: under
+    ``create_graph``, differentiating it with respect to what it was made of raises instead of giving nothing."""
+    if torch.is_grad_enabled() and any(source is not None and source.requires_grad for source in sources):
+        return _FirstOrder.apply(name, result, *sources)
+    return result
+
+
 torch.library.register_autograd(
     "torch_ggml_ops::grouped_mmq_grad_input", _no_double_backward("grouped_mmq_grad_input")
 )

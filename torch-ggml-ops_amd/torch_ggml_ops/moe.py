@@ -18,6 +18,7 @@ import torch
 
 from . import _direct, _native, _validate
 from .grouped_mmq import _forward as _grouped_forward
+from .grouped_mmq import _no_double_backward
 from .swiglu import grouped_mmq_swiglu
 
 torch.library.define(
@@ -232,6 +233,11 @@ def _grad_input_weighted_fake(
     grad_tokens, row_token, row_weight, packed_weight, expert_indices, expert_offsets, quant_type, in_features
 ):
     return grad_tokens.new_empty((row_token.shape[0], in_features))
+
+
+torch.library.register_autograd(
+    "torch_ggml_ops::grouped_mmq_grad_input_weighted", _no_double_backward("grouped_mmq_grad_input_weighted")
+)
 
 
 @torch.library.impl("torch_ggml_ops::grouped_mmq_combine", "CUDA")

@@ -21,6 +21,7 @@ from typing import Optional
 import torch
 
 from . import _native
+from .grouped_mmq import _first_order
 from .grouped_mmq import _forward as _grouped_forward
 from .gathered import _rows_grad_input, _scatter_to_tokens
 
@@ -154,6 +155,7 @@ def _backward(ctx, grad_activated, grad_gate, grad_up):
             grad_input = _sum_slots(grad_rows, slot_rows)
         else:
             grad_input = _scatter_to_tokens(grad_rows, row_index, ctx.tokens) if ctx.gathered else grad_rows
+        grad_input = _first_order("grouped_mmq_swiglu", grad_input, input, grad_activated, grad_gate, grad_up)
     return grad_input, None, None, None, None, None, None, None, None
 
 
