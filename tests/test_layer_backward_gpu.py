@@ -133,3 +133,34 @@ def test_loss_of_ragged_vocabularies(ops, qname, rows, vocabulary, chunk):
     assert not f32(hidden.grad)[-1].any()
     targets[1] = vocabulary   # neither a column nor ignored
     assert torch.isnan(tgo.chunked_lm_head_loss(hidden.detach(), weight, targets, qtype, vocabulary, chunk_rows=chunk))
+
+
+@pytest.mark.parametrize("rows", (5, 40))
+@pytest.mark.parametrize("columns", ({}, {8192: "nan"}, {8192: "-inf"}, {8192: "nan", 8193: "-inf"}, {8192: "+inf"}, {3: "-inf", 8193: "nan"}))
+def test_loss_of_logits_that_are_not_finite(ops, columns, rows):
+    """The second span of the vocabulary holds two columns: a NaN there is the row's loss also when nothing finite stands
+    beside it, and a span of -inf adds nothing."""
+    tgo, synth = ops
+    qtype, k, vocabulary = QTYPES["Q4_K"], 256, 8194
+    packed = synth.random_packed_weight(qtype, (vocabulary,), k, seed=1, scale_range=(1e-3, 3e-2))
+    if columns:
+        for column in (8192, 8193):
+            columns = {column: next(iter(columns.values())), **columns}
+    for column, kind in columns.items():
+        # a block of one scale and no minimum: every weight is d * 9 * 1, so that logits are d * 9 * sum(x)
+        block = packed.reshape(vocabulary, -1)[column]
+        block[:] = torch.tensor([0, 0, 0, 0] + [9] * 4 + [0] * 4 + [9] * 4 + [17] * 128, dtype=torch.uint8)
+        block[:2] = torch.tensor({"nan": [0, 0x7E], "-inf": [0, 0x7C], "+inf": [0, 0xFC]}[kind], dtype=torch.uint8)
+    weight = packed.cuda()
+    hidden = -random_bf16((rows, k), seed=2).abs()   # (a negative sum)
+    targets = torch.arange(rows, device="cuda") + 10
+    logits = tgo.mmq(hidden, weight, qtype, vocabulary)
+    for column, kind in columns.items():
+        # (the matrix-core kernels of larger calls make a NaN of an infinite scale, which is the case of the loss then)
+        expected = torch.full((rows,), float(kind) if rows == 5 else float("nan"), device="cuda", dtype=torch.bfloat16)
+        torch.testing.assert_close(logits[:, column], expected, equal_nan=True)
+    reference = torch.nn.functional.cross_entropy(logits.float(), targets)
+    assert reference.isnan() == any(kind != "-inf" or rows != 5 for kind in columns.values())
+    for gradient in (False, True):
+        loss = tgo.chunked_lm_head_loss(hidden.clone().requires_grad_(gradient), weight, targets, qtype, vocabulary)
+        torch.testing.assert_close(loss.detach(), reference, rtol=1e-5, atol=1e-6, equal_nan=True)

@@ -65,7 +65,8 @@ __global__ __launch_bounds__(1024) void loss_total_kernel(const float * __restri
 }
 
 // ---- statistics of a row's spans ------------------------------------------------------------------------------
-// stats[row][span] = (m, sum of exp(x - m)) over LOSS_SPAN columns.  A thread holds four pieces of eight values, all
+// stats[row][span] = (m, sum of exp(x - m)) over LOSS_SPAN columns, m the largest value that is a number; where that is -inf,
+// (-inf, sum of exp(x)): 0 of nothing but -inf, NaN with a NaN among them.  A NaN or +inf makes the sum NaN.  A thread holds four pieces of eight values, all
 // requested before the first is used; enough workgroups for any row count (31 spans for a vocabulary of 248320).
 __global__ __launch_bounds__(256) void loss_stats_kernel(const uint16_t * __restrict__ logits, int64_t pitch, int columns,
                                                          float2 * __restrict__ stats) {
@@ -102,12 +103,13 @@ __global__ __launch_bounds__(256) void loss_stats_kernel(const uint16_t * __rest
     }
     __syncthreads();
     largest = fmaxf(fmaxf(wave_value[0][0], wave_value[0][1]), fmaxf(wave_value[0][2], wave_value[0][3]));
+    const float above = largest == -INFINITY ? 0.0f : largest;   // (-inf - -inf would make a NaN of a span without one)
     float sum = 0.0f;
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            sum += __expf(value[p][e] - largest);
+            sum += __expf(value[p][e] - above);
         }
     }
 #pragma unroll
@@ -149,20 +151,21 @@ __global__ __launch_bounds__(256) void loss_grad_kernel(const uint16_t * __restr
     const bool known = target >= 0 && target < columns;
     // the row's largest value and its sum of exponentials: eight lanes of a row take every eighth span each
     float largest = -INFINITY, sum = 0.0f;
+    const auto join = [&](float other_largest, float other_sum) {
+        const float joined = fmaxf(largest, other_largest);
+        // (a part without a finite maximum keeps its sum: 0, or NaN)
+        sum = (largest == -INFINITY ? sum : sum * __expf(largest - joined)) +
+              (other_largest == -INFINITY ? other_sum : other_sum * __expf(other_largest - joined));
+        largest = joined;
+    };
     for (int s = c; s < spans; s += 8) {
         const float2 part = stats[static_cast<int64_t>(row_read) * spans + s];
-        const float joined = fmaxf(largest, part.x);
-        // (a span whose values are all -inf has no finite maximum: it adds nothing)
-        sum = (largest == -INFINITY ? 0.0f : sum * __expf(largest - joined)) + (part.x == -INFINITY ? 0.0f : part.y * __expf(part.x - joined));
-        largest = joined;
+        join(part.x, part.y);
     }
 #pragma unroll
     for (int offset = 1; offset < 8; offset <<= 1) {
         const float other_largest = __shfl_xor(largest, offset), other_sum = __shfl_xor(sum, offset);
-        const float joined = fmaxf(largest, other_largest);
-        sum = (largest == -INFINITY ? 0.0f : sum * __expf(largest - joined)) +
-              (other_largest == -INFINITY ? 0.0f : other_sum * __expf(other_largest - joined));
-        largest = joined;
+        join(other_largest, other_sum);
     }
     const float log_sum = largest + __logf(sum);
     if (blockIdx.x == 0 && c == 0 && present) {
