@@ -8,6 +8,14 @@
 //                       cotangent ever exists.
 // Both are bound by memory: 256 rows of 248320 logits are 127 MB, read twice and written once; the two passes take
 // 21 + 47 us for what took 465 us and another 43 us to pack.
+//
+// Exponentials and logarithms are the short forms (__expf, __logf; the full ones cost another 11 + 5 us a chunk).  With x <= 0 the
+// product x * log2(e) is rounded once and the hardware's 2^t is good to 2^-23, so that e^x is off by at most
+// (|x| + 2) * 2^-24 + |x| * 2^-26 of itself: 7e-6 at |x| = 88, where it underflows, against the 2^-9 that rounding the cotangent to bf16
+// costs; in a row's sum the terms weigh |x| by e^x, which leaves (log(columns) + 2) * 2^-24 or less, 1e-6.  Measured against
+// 64 bits on vocabularies of 1001 to 151936 and logits of rms 0.5 to 11: loss 4e-8 to 9e-8 of itself, the same figures with
+// the full functions and with tensor operations; gradient 1e-5 to 5e-5 of its norm away from that of the exactly
+// rounded cotangent, with any of the three.
 #include "tgo_device.h"
 #include "tgo_launch.h"
 
