@@ -236,3 +236,16 @@ def test_token_runs_drop_rows_outside_the_input(package):
         if 0 <= token < 4:
             expected[token] += grad_rows[row].float()
     torch.testing.assert_close(result, expected, rtol=0, atol=0)
+
+
+def test_loss_of_no_rows_is_zero(package):
+    """No row, no chunk: the mean over at least one row of nothing, and an empty gradient.  (No kernel is involved.)"""
+    tgo, _, _, synth = package
+    weight = synth.random_packed_weight(synth.Q4_K, (64,), 256, seed=1)
+    hidden = torch.zeros(0, 256, dtype=torch.bfloat16, requires_grad=True)
+    targets = torch.zeros(0, dtype=torch.int64)
+    loss = tgo.chunked_lm_head_loss(hidden, weight, targets, synth.Q4_K, 64)
+    assert loss.shape == () and loss.dtype == torch.float32 and loss.item() == 0.0
+    (loss * 2).backward()
+    assert hidden.grad.shape == (0, 256) and hidden.grad.dtype == torch.bfloat16
+    assert not tgo.chunked_lm_head_loss(hidden.detach(), weight, targets, synth.Q4_K, 64).requires_grad

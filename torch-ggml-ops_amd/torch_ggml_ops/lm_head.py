@@ -86,6 +86,10 @@ def _scale_fake(input, factor):
 class _ChunkedLoss(torch.autograd.Function):
     @staticmethod
     def forward(ctx, hidden, packed_weight, targets, quant_type, out_features, chunk_rows, ignore_index):
+        if hidden.shape[0] == 0:   # (no chunk, no launch: the loss of a batch without any counted row)
+            if ctx.needs_input_grad[0]:
+                ctx.save_for_backward(torch.empty_like(hidden))
+            return torch.zeros((), dtype=torch.float32, device=hidden.device)
         loss, grad_hidden = torch.ops.torch_ggml_ops.lm_head_loss.default(
             hidden, packed_weight, targets, quant_type, out_features, chunk_rows, ignore_index, ctx.needs_input_grad[0]
         )
@@ -98,7 +102,8 @@ class _ChunkedLoss(torch.autograd.Function):
         grad_hidden = None
         if ctx.needs_input_grad[0]:
             (saved,) = ctx.saved_tensors
-            if grad_loss.requires_grad:   # (a gradient of the gradient: tensor operations, which autograd can follow)
+            # (a gradient of the gradient: tensor operations, which autograd can follow; no rows: nothing to launch)
+            if grad_loss.requires_grad or saved.shape[0] == 0:
                 grad_hidden = (saved.float() * grad_loss).to(saved.dtype)
             else:
                 grad_hidden = torch.ops.torch_ggml_ops.scale_bf16.default(saved, grad_loss)
