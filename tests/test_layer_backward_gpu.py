@@ -58,6 +58,25 @@ def test_routing_weight_gradient_and_inverse(ops, tokens, top_k, features):
     assert np.array_equal(token.cpu().numpy(), expected_token) and np.array_equal(weight.cpu().numpy(), expected_weight)
 
 
+@pytest.mark.parametrize("offset", (0, 1, 8))
+def test_routing_weight_gradient_of_a_view_at_any_address(ops, offset):
+    """The gradient of a part of a concatenation is a view into the whole, at whatever address that part has."""
+    tgo, _ = ops
+    tokens, top_k, features = 5, 2, 24
+    rows = random_bf16((tokens * top_k, features), seed=1).requires_grad_()
+    slot_rows = torch.arange(tokens * top_k, device="cuda").reshape(tokens, top_k)
+    weights = torch.rand(tokens, top_k, device="cuda").requires_grad_()
+    ahead = torch.zeros(offset, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    cotangent = random_bf16((offset + tokens * features,), seed=2)
+    joined = torch.cat((ahead, tgo.moe_combine(rows, slot_rows, weights).flatten()))
+    grad_rows, grad_weights = torch.autograd.grad(joined, (rows, weights), cotangent)
+    mine = cotangent[offset:].reshape(tokens, 1, features).double()
+    expected = (rows.detach().double().reshape(tokens, top_k, features) * mine).sum(-1)
+    torch.testing.assert_close(grad_weights.double(), expected, rtol=1e-5, atol=1e-4)
+    expected = (mine * weights.detach().double().unsqueeze(-1)).reshape(-1, features)
+    torch.testing.assert_close(grad_rows.double(), expected, rtol=2**-8, atol=1e-6)
+
+
 def test_gradients_of_the_routing_weight_gradient(ops):
     tgo, _ = ops
     tokens, top_k, features = 33, 4, 72

@@ -87,6 +87,8 @@ torch.library.define(
 @torch.library.impl("torch_ggml_ops::moe_combine_weight_grad", "CUDA")
 def _weight_grad_device(rows, grad_tokens, slot_rows):
     """Gradient of the routing weights of ``moe_combine``: the dot product of each slot's row with its token's gradient."""
+    if grad_tokens.data_ptr() % 16 != 0:   # (a view into a larger gradient: autograd hands over whatever address that has)
+        grad_tokens = grad_tokens.clone()
     tokens, top_k = slot_rows.shape
     grad_weights = torch.empty((tokens, top_k), dtype=torch.float32, device=rows.device)
     with _native.on_device(rows.device):
