@@ -37,6 +37,17 @@ def test_route_in_several_workgroups(ops, slots, experts):
     assert np.array_equal(indices.cpu().numpy(), np.arange(experts))
 
 
+@pytest.mark.parametrize("tokens,top_k,experts", ((1, 8, 256), (512, 8, 4096)))
+def test_route_of_one_launch(ops, tokens, top_k, experts):
+    tgo, _ = ops
+    chosen = torch.randint(-1, experts + 1, (tokens, top_k), generator=torch.Generator().manual_seed(tokens)).cuda()
+    small = torch.ops.torch_ggml_ops.route_small.default(chosen, experts)
+    for actual, expected in zip(small, tgo.route(chosen, experts), strict=True):
+        assert actual.dtype == expected.dtype and torch.equal(actual, expected)
+    with pytest.raises(RuntimeError, match="at most 4096 slots"):
+        torch.ops.torch_ggml_ops.route_small.default(chosen.repeat(4097, 1), experts)
+
+
 @pytest.mark.parametrize("tokens,top_k,features", ((1, 1, 8), (5, 3, 520), (33, 8, 2048)))
 def test_routing_weight_gradient_and_inverse(ops, tokens, top_k, features):
     tgo, _ = ops

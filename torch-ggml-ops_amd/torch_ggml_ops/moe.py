@@ -327,10 +327,20 @@ ROUTE_SLOT_LIMIT = 4194304   # TGO_ROUTE_SLOT_LIMIT
 ROUTE_EXPERT_LIMIT = 4096    # TGO_ROUTE_EXPERT_LIMIT
 
 
-torch.library.define(
-    "torch_ggml_ops::route",
-    "(Tensor slot_experts, int num_experts) -> (Tensor, Tensor, Tensor, Tensor)",
-)
+for _name in ("route", "route_small"):
+    torch.library.define(
+        f"torch_ggml_ops::{_name}", "(Tensor slot_experts, int num_experts) -> (Tensor, Tensor, Tensor, Tensor)"
+    )
+
+
+def _route_outputs(slot_experts, num_experts):
+    tokens, top_k = slot_experts.shape
+    return (
+        slot_experts.new_empty((tokens * top_k,), dtype=torch.int64),
+        slot_experts.new_empty((tokens, top_k), dtype=torch.int64),
+        slot_experts.new_empty((num_experts,), dtype=torch.int64),
+        slot_experts.new_empty((num_experts,), dtype=torch.int32),
+    )
 
 
 @torch.library.impl("torch_ggml_ops::route", "CUDA")
@@ -340,32 +350,37 @@ def _route_device(slot_experts, num_experts):
     slot_experts = slot_experts.to(torch.int64).contiguous()
     tokens, top_k = slot_experts.shape
     device = slot_experts.device
-    row_index = torch.empty(tokens * top_k, dtype=torch.int64, device=device)
-    slot_rows = torch.empty((tokens, top_k), dtype=torch.int64, device=device)
-    expert_indices = torch.empty(num_experts, dtype=torch.int64, device=device)
-    expert_offsets = torch.empty(num_experts, dtype=torch.int32, device=device)
+    outputs = _route_outputs(slot_experts, num_experts)
     workspace_bytes = _native.lib.tgo_route_workspace_bytes(tokens * top_k, num_experts)
     workspace = torch.empty(workspace_bytes, dtype=torch.uint8, device=device) if workspace_bytes > 0 else None
     with _native.on_device(device):
         _native.check(
             _native.lib.tgo_route(
-                slot_experts.data_ptr(), tokens, top_k, num_experts, row_index.data_ptr(), slot_rows.data_ptr(),
-                expert_indices.data_ptr(), expert_offsets.data_ptr(), None if workspace is None else workspace.data_ptr(),
-                _native.stream_of(device),
+                slot_experts.data_ptr(), tokens, top_k, num_experts, *(output.data_ptr() for output in outputs),
+                None if workspace is None else workspace.data_ptr(), _native.stream_of(device),
             )
         )
-    return row_index, slot_rows, expert_indices, expert_offsets
+    return outputs
 
 
-@torch.library.register_fake("torch_ggml_ops::route")
-def _route_fake(slot_experts, num_experts):
+@torch.library.impl("torch_ggml_ops::route_small", "CUDA")
+def _route_small_device(slot_experts, num_experts):
+    """``route`` for a batch of one launch, which needs no workspace (at most 4096 slots and experts)."""
+    slot_experts = slot_experts.to(torch.int64).contiguous()
     tokens, top_k = slot_experts.shape
-    return (
-        slot_experts.new_empty((tokens * top_k,), dtype=torch.int64),
-        slot_experts.new_empty((tokens, top_k), dtype=torch.int64),
-        slot_experts.new_empty((num_experts,), dtype=torch.int64),
-        slot_experts.new_empty((num_experts,), dtype=torch.int32),
-    )
+    outputs = _route_outputs(slot_experts, num_experts)
+    with _native.on_device(slot_experts.device):
+        _native.check(
+            _native.lib.tgo_route_small(
+                slot_experts.data_ptr(), tokens, top_k, num_experts, *(output.data_ptr() for output in outputs),
+                _native.stream_of(slot_experts.device),
+            )
+        )
+    return outputs
+
+
+for _name in ("route", "route_small"):
+    torch.library.register_fake(f"torch_ggml_ops::{_name}")(_route_outputs)
 
 
 def route(slot_experts: torch.Tensor, num_experts: int):
