@@ -249,3 +249,37 @@ def test_loss_of_no_rows_is_zero(package):
     (loss * 2).backward()
     assert hidden.grad.shape == (0, 256) and hidden.grad.dtype == torch.bfloat16
     assert not tgo.chunked_lm_head_loss(hidden.detach(), weight, targets, synth.Q4_K, 64).requires_grad
+
+
+@pytest.mark.parametrize("case", ("here", "missing", "another torch"))
+def test_package_loads_without_the_direct_calls(case, tmp_path):
+    """_direct.so belongs to one torch and one Python: without it, or with another torch, the package says so and sends every
+    call through the registered operators."""
+    import shutil
+    import subprocess
+    import sys
+
+    package = tmp_path / "torch_ggml_ops"
+    shutil.copytree(ROOT / "torch-ggml-ops_amd" / "torch_ggml_ops", package)
+    if case == "missing":
+        (package / "_direct.so").unlink()
+    program = (
+        "import torch, warnings\n"
+        + ("torch.__version__ = '9.9.0'\n" if case == "another torch" else "")
+        + "with warnings.catch_warnings(record=True) as seen:\n"
+        "    warnings.simplefilter('always')\n"
+        "    import torch_ggml_ops as tgo\n"
+        "from torch_ggml_ops import _native\n"
+        f"assert tgo.__file__.startswith({str(tmp_path)!r})\n"
+        "messages = [str(w.message) for w in seen if 'torch_ggml_ops' in str(w.message)]\n"
+        f"assert (_native.direct is not None) == (not messages) == {case == 'here'}, (_native.direct, messages)\n"
+        "x, w = torch.zeros(2, 256, dtype=torch.bfloat16), torch.zeros(3, 144, dtype=torch.uint8)\n"
+        "try:\n"
+        "    tgo.mmq(x, w, 12, 3)\n"
+        "except NotImplementedError as error:\n"
+        "    assert 'torch_ggml_ops::mmq' in str(error)\n"
+        "else:\n"
+        "    raise AssertionError('a call on the CPU went through')\n"
+    )
+    done = subprocess.run([sys.executable, "-c", program], cwd=tmp_path, capture_output=True, text=True, timeout=100)
+    assert done.returncode == 0, done.stderr

@@ -19,6 +19,9 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <cstdio>
+#include <cstring>
+
 #include "../../include/tgo.h"
 
 namespace {
@@ -219,6 +222,27 @@ PyMethodDef methods[] = {
 };
 PyModuleDef module_definition = {PyModuleDef_HEAD_INIT, "_direct", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
+// Whether the running Python and torch are those that this file was compiled against: it reaches into their structures, so with
+// any other the package does without it.  (Asked through functions that every version has.)
+bool built_for_this_process() {
+    char python[16];
+    snprintf(python, sizeof(python), "%d.%d.", PY_MAJOR_VERSION, PY_MINOR_VERSION);
+    if (strncmp(Py_GetVersion(), python, strlen(python)) != 0) {
+        PyErr_Format(PyExc_ImportError, "_direct.so was built for Python %s*", python);
+        return false;
+    }
+    PyObject * const torch = PyImport_ImportModule("torch");
+    PyObject * const version = torch != nullptr ? PyObject_GetAttrString(torch, "__version__") : nullptr;
+    const char * const running = version != nullptr ? PyUnicode_AsUTF8(version) : nullptr;
+    const bool same = running != nullptr && strcmp(running, TGO_TORCH_VERSION) == 0;
+    if (running != nullptr && !same) {
+        PyErr_Format(PyExc_ImportError, "_direct.so was built for torch %s, this is %s", TGO_TORCH_VERSION, running);
+    }
+    Py_XDECREF(version);
+    Py_XDECREF(torch);
+    return same;
+}
+
 }  // namespace
 
-PyMODINIT_FUNC PyInit__direct() { return PyModule_Create(&module_definition); }
+PyMODINIT_FUNC PyInit__direct() { return built_for_this_process() ? PyModule_Create(&module_definition) : nullptr; }

@@ -1,13 +1,14 @@
 """ctypes binding of libtgo_hip.so (the C ABI declared in include/tgo.h).
 
 The library is built in-tree by ``torch-ggml-ops_amd/csrc/Makefile``.  There is no
-fallback: if it is missing, importing the package fails.
+fallback: if it is missing, importing the package fails.  ``_direct.so`` beside it is a shortcut into it that may be missing.
 """
 
 from __future__ import annotations
 
 import contextlib
 import ctypes
+import warnings
 from pathlib import Path
 
 import torch
@@ -21,6 +22,19 @@ if not _LIB_PATH.exists():
     )
 
 lib = ctypes.CDLL(str(_LIB_PATH))
+
+# Calls without a gradient straight from Python: host code for the torch and Python that it was compiled against.  Without it
+# every call takes the registered operators, which launch the same kernels at a higher cost per call.
+try:
+    from . import _direct as direct
+except ImportError as error:
+    direct = None
+    warnings.warn(
+        f"torch_ggml_ops: small calls take longer than they need to ({error}); "
+        "`make -C torch-ggml-ops_amd/csrc` builds _direct.so for this torch and Python",
+        RuntimeWarning,
+        stacklevel=2,
+    )
 
 _p, _i64, _int = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int
 

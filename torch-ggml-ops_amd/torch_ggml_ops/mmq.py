@@ -10,7 +10,8 @@ from __future__ import annotations
 
 import torch
 
-from . import _direct, _native, _validate
+from . import _native, _validate
+from ._native import direct as _direct
 
 torch.library.define(
     "torch_ggml_ops::mmq",
@@ -104,7 +105,7 @@ torch.library.register_autograd("torch_ggml_ops::mmq_grad_input", _mmq_grad_inpu
 
 def mmq(input: torch.Tensor, packed_weight: torch.Tensor, quant_type: int, out_features: int) -> torch.Tensor:
     """``input @ W.T`` for a packed GGUF weight ``[out_features, row_bytes]``; bf16 in, bf16 out."""
-    if not torch.compiler.is_compiling():
+    if _direct is not None and not torch.compiler.is_compiling():
         output = _direct.mmq(input, packed_weight, quant_type, out_features)   # (None: not a plain call)
         if output is not None:
             return output

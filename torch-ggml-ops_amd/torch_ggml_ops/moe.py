@@ -16,7 +16,8 @@ from __future__ import annotations
 
 import torch
 
-from . import _direct, _native, _validate
+from . import _native, _validate
+from ._native import direct as _direct
 from .grouped_mmq import _forward as _grouped_forward
 from .grouped_mmq import _no_double_backward
 from .swiglu import grouped_mmq_swiglu
@@ -423,7 +424,7 @@ def moe_layer(
     ``down_weight`` packed ``[experts, features, ...]``.  Differentiable with respect to ``hidden`` and
     ``slot_weights``.
     """
-    if not torch.compiler.is_compiling():
+    if _direct is not None and not torch.compiler.is_compiling():
         output = _direct.moe_layer(
             hidden, slot_experts, slot_weights, gate_weight, up_weight, down_weight, gate_up_type, down_type,
             intermediate_features,
