@@ -283,3 +283,15 @@ def test_package_loads_without_the_direct_calls(case, tmp_path):
     )
     done = subprocess.run([sys.executable, "-c", program], cwd=tmp_path, capture_output=True, text=True, timeout=100)
     assert done.returncode == 0, done.stderr
+
+
+def test_multi_forward_rejects_missing_arrays(package):
+    _, native, _, _ = package
+    lib, fake = native.lib, 0x10000
+    one = dict(packed=(ctypes.c_void_p * 1)(fake), out=(ctypes.c_void_p * 1)(fake), n=(ctypes.c_int64 * 1)(8), q=(ctypes.c_int * 1)(12))
+    for missing in one:
+        given = {**one, missing: None}
+        status = lib.tgo_mmq_multi_forward(
+            fake, 1, given["packed"], given["out"], given["n"], given["q"], fake, None, 4, 256, 0, None
+        )
+        assert status == 1 and b"must not be null" in lib.tgo_last_error()

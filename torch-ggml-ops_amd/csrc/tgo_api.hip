@@ -433,6 +433,9 @@ int tgo_mmq_multi_forward(const void * input_bf16, int count, const void * const
     if (count <= 0) {
         return fail(TGO_ERR_INVALID, "at least one projection is required; got %d", count);
     }
+    if (packed == nullptr || outputs_bf16 == nullptr || out_features == nullptr || quant_types == nullptr) {
+        return fail(TGO_ERR_INVALID, "packed, outputs_bf16, out_features and quant_types must not be null");
+    }
     for (int i = 0; i < count; ++i) {
         TGO_TRY(check_matmul_shape(rows, in_features, out_features[i], quant_types[i]));
         TGO_TRY(check_pointer(packed[i], "packed_weight"));
