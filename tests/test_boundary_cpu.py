@@ -295,3 +295,18 @@ def test_multi_forward_rejects_missing_arrays(package):
             fake, 1, given["packed"], given["out"], given["n"], given["q"], fake, None, 4, 256, 0, None
         )
         assert status == 1 and b"must not be null" in lib.tgo_last_error()
+
+
+def test_scratch_of_split_calls_has_to_be_aligned(package):
+    """The kernels store 16 bytes at a time into it.  (Calls that need none may be given any pointer.)"""
+    _, native, _, _ = package
+    lib, fake = native.lib, 0x10000
+    rows, k, n, qtype = 64, 4096, 1024, 13
+    assert lib.tgo_forward_scratch_bytes(rows, k, n, qtype) > 0
+    out, sizes, types = (ctypes.c_void_p * 1)(fake), (ctypes.c_int64 * 1)(n), (ctypes.c_int * 1)(qtype)
+    for status in (
+        lib.tgo_mmq_forward_scratch(fake, fake, fake, fake, fake + 8, rows, k, n, qtype, None),
+        lib.tgo_mmq_forward_prepared_scratch(fake, fake, fake, fake + 8, rows, k, n, qtype, 0, None),
+        lib.tgo_mmq_multi_forward(fake, 1, out, out, sizes, types, fake, fake + 8, rows, k, 0, None),
+    ):
+        assert status == 1 and b"scratch data pointer must be 16-byte aligned" in lib.tgo_last_error()

@@ -349,6 +349,14 @@ static hipError_t launch_dense(const void * packed, const tgo::Q8Workspace & vie
                                                     static_cast<float *>(scratch));
 }
 
+// `scratch` of a dense call that cuts K into ranges (tgo_forward_scratch_bytes); any pointer will do where nothing is cut.
+static int check_scratch(const void * scratch, int64_t rows, int64_t in_features, int64_t out_features, int quant_type) {
+    if (scratch != nullptr && tgo_forward_scratch_bytes(rows, in_features, out_features, quant_type) > 0) {
+        return check_pointer(scratch, "scratch");
+    }
+    return TGO_OK;
+}
+
 int tgo_mmq_forward_scratch(const void * input_bf16, const void * packed, void * output_bf16, void * workspace, void * scratch,
                             int64_t rows, int64_t in_features, int64_t out_features, int quant_type, void * stream) {
     TGO_TRY(check_matmul_shape(rows, in_features, out_features, quant_type));
@@ -356,6 +364,7 @@ int tgo_mmq_forward_scratch(const void * input_bf16, const void * packed, void *
     TGO_TRY(check_pointer(packed, "packed_weight"));
     TGO_TRY(check_pointer(output_bf16, "output"));
     TGO_TRY(check_pointer(workspace, "workspace"));
+    TGO_TRY(check_scratch(scratch, rows, in_features, out_features, quant_type));
     hipStream_t hip_stream = static_cast<hipStream_t>(stream);
     if (tgo::gemv_fuses(quant_type, rows, 0) && !tgo::gemv_takes_tiles(packed, nullptr, rows, 0, in_features, out_features, quant_type)) {
         // one launch: the decode-regime kernels of these formats quantize their activations themselves
@@ -406,6 +415,7 @@ int tgo_mmq_forward_prepared_scratch(const void * workspace, const void * packed
     TGO_TRY(check_pointer(packed, "packed_weight"));
     TGO_TRY(check_pointer(output_bf16, "output"));
     TGO_TRY(check_workspace_operand(operand));
+    TGO_TRY(check_scratch(scratch, rows, in_features, out_features, quant_type));
     const tgo::Q8Workspace view =
         tgo::q8_workspace_view(const_cast<void *>(workspace), rows, in_features, tgo::use_gemv(rows, 0), operand);
     TGO_TRY(check_hip(launch_dense(packed, view, output_bf16, scratch, rows, in_features, out_features, quant_type,
@@ -440,6 +450,7 @@ int tgo_mmq_multi_forward(const void * input_bf16, int count, const void * const
         TGO_TRY(check_matmul_shape(rows, in_features, out_features[i], quant_types[i]));
         TGO_TRY(check_pointer(packed[i], "packed_weight"));
         TGO_TRY(check_pointer(outputs_bf16[i], "output"));
+        TGO_TRY(check_scratch(scratch, rows, in_features, out_features[i], quant_types[i]));
     }
     hipStream_t hip_stream = static_cast<hipStream_t>(stream);
     const tgo::Q8Workspace view = tgo::q8_workspace_view(workspace, rows, in_features, tgo::use_gemv(rows, 0), operand);
