@@ -310,3 +310,62 @@ def test_scratch_of_split_calls_has_to_be_aligned(package):
         lib.tgo_mmq_multi_forward(fake, 1, out, out, sizes, types, fake, fake + 8, rows, k, 0, None),
     ):
         assert status == 1 and b"scratch data pointer must be 16-byte aligned" in lib.tgo_last_error()
+
+
+def test_helper_operators_check_what_they_are_given(package, monkeypatch):
+    """The registered operators behind the backward passes and the loss, called as a user may call them: a tensor of another
+    type, shape, device or layout never reaches a kernel."""
+    _, _, validate, synth = package
+    from torch_ggml_ops import lm_head, moe, prepared
+
+    monkeypatch.setattr(validate, "REQUIRE_DEVICE", False)
+    rows, grad = torch.zeros(6, 16, dtype=torch.bfloat16), torch.zeros(3, 16, dtype=torch.bfloat16)
+    slots, weights = torch.zeros(3, 2, dtype=torch.int64), torch.zeros(3, 2)
+    hidden, targets = torch.zeros(4, 256, dtype=torch.bfloat16), torch.zeros(4, dtype=torch.int64)
+    packed = synth.random_packed_weight(synth.Q4_K, (8,), 256, seed=1)
+    elsewhere = torch.zeros(3, 2, dtype=torch.int64, device="meta")
+
+    def refused(function, *arguments, match):
+        with pytest.raises(RuntimeError, match=match):
+            function(*arguments)
+
+    for arguments, match in (
+        ((rows.float(), grad, slots), "rows must have dtype torch.bfloat16"),
+        ((rows, grad.float(), slots), "grad_tokens must have dtype torch.bfloat16"),
+        ((rows, grad, slots.int()), "slot_rows must have dtype torch.int64"),
+        ((rows, grad, elsewhere), "same device"),
+        ((rows, grad[:2], slots), "grad_tokens must have shape"),
+        ((rows, grad[:, :8].contiguous(), slots), "grad_tokens must have shape"),
+        ((rows, grad, slots[:, 0].contiguous()), "slot_rows must have shape"),
+        ((rows[0], grad, slots), "rows must have shape"),
+        ((rows.t().contiguous().t(), grad, slots), "rows must be contiguous"),
+        ((rows, grad.t().contiguous().t(), slots), "grad_tokens must be contiguous"),
+        ((rows, grad, slots.t().contiguous().t()), "slot_rows must be contiguous"),
+        ((rows[:, :12].contiguous(), grad[:, :12].contiguous(), slots), "multiple of 8"),
+    ):
+        refused(moe._check_weight_grad, *arguments, match=match)
+    for arguments, match in (
+        ((slots.int(), weights, 6), "slot_rows must have dtype torch.int64"),
+        ((slots, weights.double(), 6), "slot_weights must have dtype torch.float32"),
+        ((slots, weights[:2], 6), "must both have shape"),
+        ((slots[0], weights[0], 6), "must both have shape"),
+        ((slots, weights.t().contiguous().t(), 6), "slot_weights must be contiguous"),
+        ((elsewhere, weights, 6), "same device"),
+        ((slots, weights, 0), "num_rows must be positive"),
+    ):
+        refused(moe._check_inverse, *arguments, match=match)
+    for bad, match in ((targets[:3], "one entry per row"), (targets.int(), "one entry per row"), (targets.reshape(2, 2), "one entry per row")):
+        refused(lm_head._check_loss, hidden, bad, 256, match=match)
+    refused(lm_head._check_loss, hidden, targets, 0, match="chunk_rows")
+    one = torch.ones(())
+    for arguments, match in (
+        ((hidden.float(), one), "input must have dtype torch.bfloat16"),
+        ((hidden, one.double()), "factor must have dtype torch.float32"),
+        ((hidden, torch.ones(2)), "factor must have one element"),
+        ((hidden.t().contiguous().t(), one), "input must be contiguous"),
+        ((hidden, one.to("meta")), "same device"),
+    ):
+        refused(lm_head._check_scale, *arguments, match=match)
+    for arguments in (([packed], [12, 12], [8]), ([packed], [12], [8, 8]), ([packed, packed], [12], [8]), ([], [], [])):
+        with pytest.raises(ValueError, match="equal length"):
+            prepared._check_projections(*arguments)

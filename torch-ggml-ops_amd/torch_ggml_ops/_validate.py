@@ -223,6 +223,15 @@ def same_weight_geometry(first: torch.Tensor, second: torch.Tensor) -> bool:
     )
 
 
+def operand(tensor: torch.Tensor, name: str, dtype: torch.dtype, device: torch.device) -> None:
+    """Checks of a plain operand of the helper operators: type, device and layout."""
+    _check_tensor(tensor, name, dtype, str(dtype))
+    if tensor.device != device:
+        _fail(f"{name} must be on the same device as the other tensors")
+    if not tensor.is_contiguous():
+        _fail(f"{name} must be contiguous; torch_ggml_ops will not insert a hidden copy")
+
+
 def activation(tensor: torch.Tensor, name: str) -> None:
     """Checks of a bf16 activation tensor that is quantized on its own (quantize_q8_1)."""
     _check_tensor(tensor, name, torch.bfloat16, "torch.bfloat16")

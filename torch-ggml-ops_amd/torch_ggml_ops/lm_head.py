@@ -28,10 +28,20 @@ torch.library.define(
 )
 
 
+def _check_loss(hidden, targets, chunk_rows) -> None:
+    if hidden.dim() != 2:
+        raise RuntimeError("hidden must have shape [rows, in_features]")
+    if targets.dim() != 1 or targets.shape[0] != hidden.shape[0] or targets.dtype != torch.int64:
+        raise RuntimeError("targets must be an int64 tensor with one entry per row of hidden")
+    if chunk_rows <= 0:
+        raise RuntimeError("chunk_rows must be positive")
+
+
 @torch.library.impl("torch_ggml_ops::lm_head_loss", "CUDA")
 def _lm_head_loss_device(hidden, packed_weight, targets, quant_type, out_features, chunk_rows, ignore_index, gradient):
     """(mean loss, its gradient with respect to ``hidden`` or an empty tensor): every launch of every chunk is issued by
     one call into the library (``tgo_lm_head_loss``)."""
+    _check_loss(hidden, targets, chunk_rows)
     if hidden.shape[0] > chunk_rows and (not hidden.is_contiguous() or hidden.storage_offset() != 0):
         hidden = hidden.clone(memory_format=torch.contiguous_format)   # (such rows were always accepted chunk by chunk)
     rows, in_features, out_features = _validate.dense(hidden, packed_weight, quant_type, out_features, backward=False)
@@ -65,9 +75,17 @@ def _lm_head_loss_fake(hidden, packed_weight, targets, quant_type, out_features,
 torch.library.define("torch_ggml_ops::scale_bf16", "(Tensor input, Tensor factor) -> Tensor")
 
 
+def _check_scale(input, factor) -> None:
+    _validate.operand(input, "input", torch.bfloat16, input.device)
+    _validate.operand(factor, "factor", torch.float32, input.device)
+    if factor.numel() != 1:
+        raise RuntimeError("factor must have one element")
+
+
 @torch.library.impl("torch_ggml_ops::scale_bf16", "CUDA")
 def _scale_device(input, factor):
     """``(input.float() * factor).to(bfloat16)`` for a contiguous bf16 tensor and an fp32 scalar on its device."""
+    _check_scale(input, factor)
     out = torch.empty_like(input)
     with _native.on_device(input.device):
         _native.check(
@@ -127,12 +145,7 @@ def chunked_lm_head_loss(
     are dropped as soon as its grad-input product has run) and scaled by the incoming gradient in backward.
     Equals ``cross_entropy(mmq(hidden, ...).float(), targets)`` up to the bf16 rounding of the logit gradients.
     """
-    if hidden.dim() != 2:
-        raise RuntimeError("hidden must have shape [rows, in_features]")
-    if targets.dim() != 1 or targets.shape[0] != hidden.shape[0] or targets.dtype != torch.int64:
-        raise RuntimeError("targets must be an int64 tensor with one entry per row of hidden")
-    if chunk_rows <= 0:
-        raise RuntimeError("chunk_rows must be positive")
+    _check_loss(hidden, targets, chunk_rows)
     return _ChunkedLoss.apply(
         hidden, packed_weight, targets, int(quant_type), int(out_features), int(chunk_rows), int(ignore_index)
     )

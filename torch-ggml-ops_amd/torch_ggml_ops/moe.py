@@ -85,9 +85,24 @@ torch.library.define(
 )
 
 
+def _check_weight_grad(rows, grad_tokens, slot_rows) -> None:
+    _validate.operand(rows, "rows", torch.bfloat16, rows.device)
+    _validate.operand(grad_tokens, "grad_tokens", torch.bfloat16, rows.device)
+    _validate.operand(slot_rows, "slot_rows", torch.int64, rows.device)
+    if rows.dim() != 2 or rows.shape[0] <= 0:
+        _fail("rows must have shape [rows, features] with at least one row")
+    if slot_rows.dim() != 2 or slot_rows.numel() <= 0:
+        _fail("slot_rows must have shape [tokens, top_k]")
+    if grad_tokens.shape != (slot_rows.shape[0], rows.shape[1]):
+        _fail("grad_tokens must have shape [tokens, features]")
+    if rows.shape[1] <= 0 or rows.shape[1] % 8 != 0:
+        _fail(f"features must be a positive multiple of 8; got {rows.shape[1]}")
+
+
 @torch.library.impl("torch_ggml_ops::moe_combine_weight_grad", "CUDA")
 def _weight_grad_device(rows, grad_tokens, slot_rows):
     """Gradient of the routing weights of ``moe_combine``: the dot product of each slot's row with its token's gradient."""
+    _check_weight_grad(rows, grad_tokens, slot_rows)
     if grad_tokens.data_ptr() % 16 != 0:   # (a view into a larger gradient: autograd hands over whatever address that has)
         grad_tokens = grad_tokens.clone()
     tokens, top_k = slot_rows.shape
@@ -107,9 +122,19 @@ def _weight_grad_fake(rows, grad_tokens, slot_rows):
     return slot_rows.new_empty(slot_rows.shape, dtype=torch.float32)
 
 
+def _check_inverse(slot_rows, slot_weights, num_rows) -> None:
+    _validate.operand(slot_rows, "slot_rows", torch.int64, slot_weights.device)
+    _validate.operand(slot_weights, "slot_weights", torch.float32, slot_weights.device)
+    if slot_rows.dim() != 2 or slot_rows.shape != slot_weights.shape or slot_rows.numel() <= 0:
+        _fail("slot_rows and slot_weights must both have shape [tokens, top_k]")
+    if num_rows <= 0:
+        _fail(f"num_rows must be positive; got {num_rows}")
+
+
 @torch.library.impl("torch_ggml_ops::invert_slots", "CUDA")
 def _invert_slots_device(slot_rows, slot_weights, num_rows):
     """Token and routing weight of every expert-sorted row; -1 and 0 for a row that no slot names."""
+    _check_inverse(slot_rows, slot_weights, num_rows)
     tokens, top_k = slot_rows.shape
     row_token = torch.empty(num_rows, dtype=torch.int64, device=slot_rows.device)
     row_weight = torch.empty(num_rows, dtype=torch.float32, device=slot_rows.device)

@@ -121,10 +121,16 @@ torch.library.define(
 )
 
 
+def _check_projections(packed_weights, quant_types, out_features) -> None:
+    if not (len(packed_weights) == len(quant_types) == len(out_features)) or not packed_weights:
+        raise ValueError("packed_weights, quant_types and out_features must be non-empty and of equal length")
+
+
 @torch.library.impl("torch_ggml_ops::mmq_multi_forward", "CUDA")
 def _multi_device(input, packed_weights, quant_types, out_features, operand):
     rows, in_features = _activation_shape(input)
     kind = _workspace_kind(operand)
+    _check_projections(packed_weights, quant_types, out_features)
     with _native.on_device(input.device):
         workspace = input.new_empty((_native.lib.tgo_q8_workspace_bytes(rows, in_features),), dtype=torch.uint8)
         for weight, quant_type, features in zip(packed_weights, quant_types, out_features):
@@ -264,8 +270,7 @@ def mmq_multi(
     out_features: Sequence[int],
 ) -> tuple[torch.Tensor, ...]:
     """``tuple(mmq(input, w, q, n) for ...)`` with the activations quantized once."""
-    if not (len(packed_weights) == len(quant_types) == len(out_features)) or not packed_weights:
-        raise ValueError("packed_weights, quant_types and out_features must be non-empty and of equal length")
+    _check_projections(packed_weights, quant_types, out_features)
     return _MultiProjection.apply(input, tuple(quant_types), tuple(out_features), *packed_weights)
 
 
