@@ -36,7 +36,9 @@ extern "C" {
 #define TGO_TYPE_Q6_K 14
 #define TGO_TYPE_IQ2_S 22
 
-/* Library version (major*10000 + minor*100 + patch). */
+/* Library version (major*10000 + minor*100 + patch): TGO_VERSION of the header that the library was built with.  It grows with
+ * every change of this file that a caller can see. */
+#define TGO_VERSION 113
 int tgo_version(void);
 
 /* Message of the last failure on the calling thread ("" if none). Host pointer. */

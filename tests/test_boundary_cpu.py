@@ -369,3 +369,13 @@ def test_helper_operators_check_what_they_are_given(package, monkeypatch):
     for arguments in (([packed], [12, 12], [8]), ([packed], [12], [8, 8]), ([packed, packed], [12], [8]), ([], [], [])):
         with pytest.raises(ValueError, match="equal length"):
             prepared._check_projections(*arguments)
+
+
+def test_version_is_the_headers(package):
+    """And the header's has grown past 112, the last one without the entry points that the list below begins with."""
+    _, native, _, _ = package
+    header = (ROOT / "include" / "tgo.h").read_text()
+    version = int(re.search(r"#define TGO_VERSION (\d+)", header).group(1))
+    assert native.lib.tgo_version() == version >= 113
+    for name in ("tgo_forward_scratch_bytes", "tgo_mmq_multi_forward", "tgo_mmq_pair_grad_input", "tgo_route", "tgo_lm_head_loss"):
+        assert f"{name}(" in header

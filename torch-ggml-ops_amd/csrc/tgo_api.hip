@@ -191,7 +191,7 @@ ProfileScope::~ProfileScope() {
 
 extern "C" {
 
-int tgo_version(void) { return 112; }
+int tgo_version(void) { return TGO_VERSION; }
 
 int tgo_profile_enable(int enabled) {
     std::lock_guard<std::mutex> lock(g_profile_mutex);

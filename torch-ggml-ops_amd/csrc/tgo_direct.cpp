@@ -222,9 +222,14 @@ PyMethodDef methods[] = {
 };
 PyModuleDef module_definition = {PyModuleDef_HEAD_INIT, "_direct", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
-// Whether the running Python and torch are those that this file was compiled against: it reaches into their structures, so with
-// any other the package does without it.  (Asked through functions that every version has.)
+// Whether the running Python and torch are those that this file was compiled against, and the library the one whose header it
+// read: it reaches into their structures, so with any other the package does without it.  (Asked through functions that every
+// version has.)
 bool built_for_this_process() {
+    if (tgo_version() != TGO_VERSION) {
+        PyErr_Format(PyExc_ImportError, "_direct.so was built for version %d of the library, this is %d", TGO_VERSION, tgo_version());
+        return false;
+    }
     char python[16];
     snprintf(python, sizeof(python), "%d.%d.", PY_MAJOR_VERSION, PY_MINOR_VERSION);
     if (strncmp(Py_GetVersion(), python, strlen(python)) != 0) {
