@@ -20,13 +20,14 @@
 // A wave walks a range of super-blocks (the four waves of a workgroup split K, up to four ways) and, for each, its R tiles of
 // 16 weight rows.  The waves' sums meet in LDS at the end and are added in a fixed order.
 //
-// What bounds it: the unpacking, about a vector instruction per weight of a lane (Q4_K: 217 per 256 x 16 weights and wave,
-// 52 % of the vector units' time), however many rows a task has, beside LDS (27 %) and the packed bytes (28672 x 8192 Q4_K:
-// 39 us, 3.4 TB/s); a fetch ring of four steps or a third workgroup per CU changed nothing.  The kernels of tgo_gemv.hip
+// What it takes: a vector instruction per weight of a lane for the unpacking (Q4_K: 217 per 256 x 16 weights and wave), however many
+// rows a task has.  No unit is full (28672 x 8192 Q4_K, five rows, 37 us: vector units busy 44 % of the time, LDS 35 %, matrix
+// cores 11 %, 3.5 TB/s of packed bytes); what is left is each wave's own chain of fetch, park, read back, unpack and multiply at two workgroups per CU,
+// and a fetch ring of four steps or a third workgroup changed nothing.  The kernels of tgo_gemv.hip
 // pay four v_dot4 plus scaling per 16 weights and activation row instead and need no whole tiles: better for one to three
-// rows.  Measured against them, gate and up of 256 experts (2048 x 512) for 97 tokens of eight choices: Q3_K 174 -> 75 us, Q5_K
-// 133 -> 92, IQ2_S 137 -> 87; down (512 x 2048): Q4_K 105 -> 45, Q6_K 89 -> 73; dense 28672 x 8192, 16 rows: Q3_K 230 -> 44,
-// Q4_K 65 -> 46, Q6_K 160 -> 69.
+// rows.  Measured against them in a layer of 97 tokens of eight choices among 256 experts (kernel time, the fused SwiGLU on top of it
+// not counted): gate and up (2048 x 512) Q3_K 179 -> 75 us, Q5_K 135 -> 92, IQ2_S 140 -> 91; down (512 x 2048) Q4_K 100 -> 42, Q6_K
+// 91 -> 84.  Dense 28672 x 8192, 16 rows: Q3_K 230 -> 44, Q4_K 65 -> 46, Q6_K 160 -> 69.
 #include <algorithm>
 #include <type_traits>
 
