@@ -90,3 +90,39 @@ def test_quantizer_forms_the_activation_halves_exactly():
     assert np.array_equal(halves.astype(np.float64), magnitudes)
     negative = (halves.view(np.uint16) | np.uint16(0x8000)).view(np.float16)   # the sign bit copied from the input
     assert np.array_equal(negative.astype(np.float64)[1:], -magnitudes[1:].astype(np.float64))
+
+
+# ---- operands that carry the super-block's scale (decode16_scaled) ----
+# every fp16 mantissa, brought to where the kernels' normalisation leaves h = 2^-S * d: the row's largest weight, v * h with
+# |v| up to 4096 (Q6_K), lies between 2^4 and 2^9, so its h between 2^-8 and 2^-3; super-blocks of the row down to h = 2^-14 are
+# covered here (below that the rest's own last bit, 2^-24, cuts in: 2^-20 of the row's largest weight at most)
+MANTISSAS = (1.0 + np.arange(1024) / 1024.0).astype(np.float64)
+
+
+def test_scaled_q3_k_operand_is_one_rounding_of_the_exact_product():
+    sub = np.arange(-32, 32, dtype=np.float16)[:, None]
+    biased = np.float16(32) + np.arange(8, dtype=np.float16)[None, :]
+    # (a fused multiply-add of halves: the exact value, rounded once)
+    integer = (biased.astype(np.float64) * sub.astype(np.float64) - 36.0 * sub.astype(np.float64)).astype(np.float16)
+    assert _exact_in_half(36.0 * sub.astype(np.float64))
+    exact = np.multiply.outer(np.arange(-32, 32), np.arange(-4, 4)).astype(np.float64)
+    assert np.array_equal(integer.astype(np.float64), exact)
+
+
+def test_scaled_q6_k_operand_rounds_at_half_an_ulp():
+    sub = np.arange(-128, 128, dtype=np.float64)[:, None, None]
+    quant = np.arange(-32, 32, dtype=np.float64)[None, None, :]
+    for exponent in range(-14, -2):
+        h = MANTISSAS[None, :, None] * 2.0**exponent
+        product = sub * h
+        assert np.array_equal(product.astype(np.float32).astype(np.float64), product)
+        head = product.astype(np.float16).astype(np.float64)
+        rest = (product - head).astype(np.float16).astype(np.float64)
+        assert np.array_equal(head + rest, product)   # the split is exact
+        low = (quant * rest).astype(np.float16).astype(np.float64)
+        operand = (quant * head + low).astype(np.float16).astype(np.float64)
+        exact = quant * product
+        # half an ulp of the result, and what the rounding of the small part adds before it
+        _, power = np.frexp(exact)
+        ulp = np.maximum(np.ldexp(1.0, power - 11), 2.0**-24)
+        assert (np.abs(operand - exact) <= ulp * (0.5 + 2.0**-9)).all(), exponent

@@ -46,10 +46,9 @@
 #include "tgo_device.h"
 #include "tgo_forward_args.h"
 #include "tgo_launch.h"
+#include "tgo_scaled_operand.h"
 
 namespace tgo {
-
-typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int FSC_MULTIPLIERS = 8;                         // multiplying waves, 32 activation rows each
 constexpr int FSC_THREADS = 64 * (FSC_MULTIPLIERS + 4);
@@ -71,11 +70,7 @@ struct ScaledItem {
 template <int TYPE>
 struct ScaledLds {
     static constexpr bool K45 = TYPE == Q4_K || TYPE == Q5_K;
-    // slot of one packed block: Q4_K/Q5_K blocks are whole 16-byte units and lie back to back (16-byte reads of 32
-    // consecutive rows then cover all banks); the other formats take the larger of their two staging pitches
-    static constexpr int RAW_SLOT = K45 ? Format<TYPE>::BLOCK_BYTES
-                                        : (Format<TYPE>::RAW_PITCH > WideStage<TYPE>::PITCH ? Format<TYPE>::RAW_PITCH
-                                                                                             : WideStage<TYPE>::PITCH);
+    static constexpr int RAW_SLOT = ScaledSlot<TYPE>::BYTES;
     alignas(16) uint8_t wq[FSC_BUFFERS][FSC_TILE_BYTES];       // ring of operand tiles, one stage each
     alignas(16) uint8_t raw[4][2][32 * RAW_SLOT];              // per unpacking wave: packed blocks of two super-blocks
     // fp16(-dmin * m * 2^-S): [tile][32 rows][8 blocks], beside the operand tile of the super-block's first stage
@@ -89,89 +84,6 @@ struct ScaledLds {
     int item_count;
     std::conditional_t<TYPE == IQ2_S, Iq2sSelectors, uint2> codebook;
 };
-
-// 6-bit scale and minimum of 32-value group G of a Q4_K/Q5_K block from its 12 scale bytes (three words)
-template <int G>
-TGO_DEVICE void k45_group_scale_min(uint32_t w1, uint32_t w2, uint32_t w3, int & sc, int & mn) {
-    if constexpr (G < 4) {
-        sc = static_cast<int>((w1 >> (8 * G)) & 63u);
-        mn = static_cast<int>((w2 >> (8 * G)) & 63u);
-    } else {
-        constexpr int J = G - 4;
-        sc = static_cast<int>(((w3 >> (8 * J)) & 15u) | (((w1 >> (8 * J + 6)) & 3u) << 4));
-        mn = static_cast<int>(((w3 >> (8 * J + 4)) & 15u) | (((w2 >> (8 * J + 6)) & 3u) << 4));
-    }
-}
-
-// (1024 + byte) pairs times an fp16 multiplier h, minus the bias: fma(1024 + b, h, -1024 h) is evaluated with one
-// rounding and -1024 h is a power-of-two multiple of h, so the result is fp16(b * h).
-TGO_DEVICE HalfScale half_scale_of(float value) {
-    const _Float16 h = static_cast<_Float16>(value);
-    const _Float16 offset = static_cast<_Float16>(-1024.0f) * h;
-    return HalfScale{half2_t{h, h}, half2_t{offset, offset}};
-}
-
-// Largest magnitude a weight of the format can take per unit of its super-block scale d.
-template <int TYPE>
-constexpr float weight_reach() {
-    return TYPE == Q4_K ? 63.0f * 15.0f : TYPE == Q5_K ? 63.0f * 31.0f : TYPE == Q3_K ? 32.0f * 4.0f
-           : TYPE == Q6_K ? 128.0f * 32.0f : 31.0f * 43.0f / 8.0f;
-}
-
-// Byte offset of the fp16 super-block scale d inside a block (Q4_K/Q5_K: d, then dmin).
-template <int TYPE>
-constexpr int scale_offset() { return TYPE == Q3_K ? 108 : TYPE == Q6_K ? 208 : 0; }
-
-
-// Stores the wave's 32 rows x (32 * TILES) columns of results, which the matrix instructions left transposed (weights as the
-// A operand: the lane holds row l32 and, as element v of tile t, column 32 t + 8 (v / 4) + 4 (lane / 32) + v % 4), as
-// bf16.  The two half-waves exchange runs of four columns, after which a lane holds eight neighbouring columns and
-// stores 16 bytes; a row gets 32 contiguous bytes per instruction.  `dst` points at row 0, column 0; rows >=
-// valid_rows and columns >= valid_cols are skipped.  The 16-byte path needs row_stride % 8 == 0 (dst is then 16-byte
-// aligned: the tensor is, and column tiles start at multiples of 128).
-// The lane's number computed from nothing, and opaque: what is derived from it is derived where it is used instead of
-// being kept in a register through a loop (where such a register is spilled, its reload waits for every load in flight).
-TGO_DEVICE int lane_afresh() {
-    int lane = static_cast<int>(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
-    asm volatile("" : "+v"(lane));
-    return lane;
-}
-
-template <int TILES>
-TGO_DEVICE void store_rows_32xn(const v16f * tiles, uint16_t * dst, int64_t row_stride, int valid_rows, int valid_cols, int lane) {
-    const int l32 = lane & 31;
-    const int half = lane >> 5;
-    const bool wide = (row_stride & 7) == 0;
-    uint16_t * const row = dst + l32 * row_stride;
-#pragma unroll
-    for (int t = 0; t < TILES; ++t) {
-#pragma unroll
-        for (int m = 0; m < 2; ++m) {
-            // runs 2m and 2m + 1 of the tile: the lower half-wave keeps its run 2m and takes the upper one's,
-            // the upper half-wave keeps its run 2m + 1 and takes the lower one's
-            const uint32_t p0 = pack_bf16x2(tiles[t][8 * m + 0], tiles[t][8 * m + 1]);
-            const uint32_t p1 = pack_bf16x2(tiles[t][8 * m + 2], tiles[t][8 * m + 3]);
-            const uint32_t q0 = pack_bf16x2(tiles[t][8 * m + 4], tiles[t][8 * m + 5]);
-            const uint32_t q1 = pack_bf16x2(tiles[t][8 * m + 6], tiles[t][8 * m + 7]);
-            const auto s0 = __builtin_amdgcn_permlane32_swap(p0, q0, false, false);
-            const auto s1 = __builtin_amdgcn_permlane32_swap(p1, q1, false, false);
-            const uint32_t words[4] = {s0[0], s1[0], s0[1], s1[1]};
-            const int c = 32 * t + 16 * m + 8 * half;
-            if (l32 < valid_rows && c < valid_cols) {
-                if (wide && c + 8 <= valid_cols) {
-                    *reinterpret_cast<uint4 *>(row + c) = make_uint4(words[0], words[1], words[2], words[3]);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        if (c + e < valid_cols) {
-                            row[c + e] = static_cast<uint16_t>(words[e >> 1] >> (16 * (e & 1)));
-                        }
-                    }
-                }
-            }
-        }
-    }
-}
 
 // ---- groups of at most 32 rows ---------------------------------------------------------------------------------
 // A task of a few rows costs the role-split workgroups below what a full one costs their unpacking waves, while seven of
@@ -534,20 +446,11 @@ TGO_DEVICE void short_group_items(const ForwardArgs & a, ShortLds<TYPE> & lds, c
             const auto * const grid = &lds.codebook;
             float shrink;
             block_power(fabsf(half_bits_to_float(lds_u16(blk + scale_offset<TYPE>()))) * weight_reach<TYPE>(), shrink);
-            const _Float16 h = static_cast<_Float16>(half_weight_scale<TYPE>(blk) * shrink);
-            const half2_t scale = {h, h};
+            const float scale = half_weight_scale<TYPE>(blk) * shrink;
 #pragma unroll
             for (int b = 0; b < 8; ++b) {
-                uint32_t first[8], fine[8];
-                decode16_half<TYPE>(blk, 2 * b + half, grid, first, fine);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    if constexpr (TYPE == Q6_K) {
-                        first[i] = half2_fma(first[i], scale, __builtin_bit_cast(half2_t, half2_mul(fine[i], scale)));
-                    } else {
-                        first[i] = half2_mul(first[i], scale);
-                    }
-                }
+                uint32_t first[8];
+                decode16_scaled<TYPE>(blk, 2 * b + half, grid, scale, first);
                 multiply_block(first, 2 * b, ratio, fragments);
             }
         }
@@ -935,21 +838,11 @@ __global__ __launch_bounds__(FSC_THREADS, 3) void mmq_forward_scaled_kernel(cons
                 const uint8_t * blk = block_of(parity);
                 uint8_t * const out = &lds.wq[target][0] + out_lane;
                 const auto * const grid = &lds.codebook;
-                const _Float16 h = static_cast<_Float16>(half_weight_scale<TYPE>(blk) * shrink);
-                const half2_t scale = {h, h};
+                const float scale = half_weight_scale<TYPE>(blk) * shrink;
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
-                    const int unit = 2 * (4 * S + b) + half;
-                    uint32_t first[8], fine[8];
-                    decode16_half<TYPE>(blk, unit, grid, first, fine);
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        if constexpr (TYPE == Q6_K) {   // sc * q in two parts that share the sign of sc
-                            first[i] = half2_fma(first[i], scale, __builtin_bit_cast(half2_t, half2_mul(fine[i], scale)));
-                        } else {
-                            first[i] = half2_mul(first[i], scale);
-                        }
-                    }
+                    uint32_t first[8];
+                    decode16_scaled<TYPE>(blk, 2 * (4 * S + b) + half, grid, scale, first);
                     uint8_t * dst = out + (2 * b) * 1024;
                     *reinterpret_cast<uint4 *>(dst) = make_uint4(first[0], first[1], first[2], first[3]);
                     *reinterpret_cast<uint4 *>(dst + 512) = make_uint4(first[4], first[5], first[6], first[7]);
