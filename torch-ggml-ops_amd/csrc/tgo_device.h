@@ -135,91 +135,101 @@ static inline int pad_task_slots(int slots, int run = 1) { return (slots + XCDS 
 // One workgroup of 256 threads (all of them call this) scans the groups 256 at a time, so any group count works
 // and no host round trip is needed.  The kernels that consume the list run later in the same stream.
 TGO_DEVICE void build_tasks(const TaskBuild & b, int tid) {
-    __shared__ int scan[256], scan_late[256];
-    __shared__ int running, running_late;
-    // Tasks of at most b.late_rows rows (a group's remainder) cost their workgroups a fraction of a full
-    // task's time; they go behind all the others so that the grid's last wave of workgroups is made of the
-    // short ones.  First sweep: how many tasks come before them.
+    __shared__ int of_wave[4][4];   // [wave][class]
+    // Tasks of at most b.late_rows rows (a group's remainder) cost their workgroups a fraction of a full task's time; they go behind
+    // all the others, those of at most b.last_rows rows last, so that the grid's last wave of workgroups is made of the short ones.
     // (late_whole_groups: only when that remainder is the whole group; the remainder of a larger group then stays
     // behind the group's other tasks, where xcd_chunk keeps it on the XCD that already holds the expert's weights)
-    const auto listed_late = [&](int size) {
-        const int rest = size % b.row_tile;
-        return rest > 0 && rest <= b.late_rows && (b.late_whole_groups == 0 || size <= b.late_rows) ? 1 : 0;
+    // Classes of tasks: 0 ordinary, 1 late, 2 last.
+    struct Group {
+        int row_begin, expert, size, count, rest_class;   // of `count` tasks the last one is of rest_class, the others of class 0
     };
-    int early_total = 0;
-    if (b.late_rows > 0) {
-        int mine = 0;
-        for (int group = tid; group < b.num_groups; group += 256) {
+    const auto group_of = [&](int group) {
+        Group g = {0, -1, 0, 0, 0};
+        if (group < b.num_groups) {
             const int row_begin = group == 0 ? 0 : b.expert_offsets[group - 1];
             const int row_end = b.expert_offsets[group];
             const int64_t expert64 = b.expert_indices[group];
             if (expert64 >= 0 && expert64 < b.num_experts && row_begin >= 0 && row_end > row_begin && row_end <= b.rows) {
-                const int size = row_end - row_begin;
-                mine += (size + b.row_tile - 1) / b.row_tile - listed_late(size);
+                const int size = row_end - row_begin, rest = size % b.row_tile;
+                const bool late = rest > 0 && rest <= b.late_rows && (b.late_whole_groups == 0 || size <= b.late_rows);
+                g = Group{row_begin, static_cast<int>(expert64), size, (size + b.row_tile - 1) / b.row_tile,
+                          !late ? 0 : rest <= b.last_rows ? 2 : 1};
             }
         }
-        scan[tid] = mine;
-        __syncthreads();
-        for (int offset = 128; offset > 0; offset >>= 1) {
-            if (tid < offset) {
-                scan[tid] += scan[tid + offset];
-            }
-            __syncthreads();
+        return g;
+    };
+    const int lane = tid & 63, wave = tid >> 6;
+    // First sweep: where the classes start.
+    bool late_apart = true;
+    int late_first = 0, last_first = 0;   // (0 without late tasks: nothing is listed there then)
+    if (b.late_rows > 0) {
+        int ordinary = 0, late = 0;
+        for (int group = tid; group < b.num_groups; group += 256) {
+            const Group g = group_of(group);
+            ordinary += g.count - (g.rest_class != 0 ? 1 : 0);
+            late += g.rest_class == 1 ? 1 : 0;
         }
-        early_total = scan[0];
+        for (int offset = 32; offset > 0; offset >>= 1) {
+            ordinary += __shfl_xor(ordinary, offset);
+            late += __shfl_xor(late, offset);
+        }
+        if (lane == 0) {
+            of_wave[wave][0] = ordinary;
+            of_wave[wave][1] = late;
+        }
         __syncthreads();
+        ordinary = of_wave[0][0] + of_wave[1][0] + of_wave[2][0] + of_wave[3][0];
+        late = of_wave[0][1] + of_wave[1][1] + of_wave[2][1] + of_wave[3][1];
+        __syncthreads();
+        // (fewer late tasks than ordinary ones: they stay among these, see FORWARD_LATE_ROWS)
+        late_apart = b.last_rows == 0 || late >= ordinary;
+        last_first = ordinary + late;
+        late_first = late_apart ? ordinary : last_first;
     }
-    if (tid == 0) {
-        running = 0;
-        running_late = 0;
-    }
-    __syncthreads();
+    int listed[3] = {0, 0, 0};   // tasks of each class so far
     for (int base = 0; base < b.num_groups; base += 256) {
-        const int group = base + tid;
-        int row_begin = 0, row_end = 0, expert = -1, count = 0, late = 0;
-        if (group < b.num_groups) {
-            row_begin = group == 0 ? 0 : b.expert_offsets[group - 1];
-            row_end = b.expert_offsets[group];
-            const int64_t expert64 = b.expert_indices[group];
-            if (expert64 >= 0 && expert64 < b.num_experts && row_begin >= 0 && row_end > row_begin && row_end <= b.rows) {
-                expert = static_cast<int>(expert64);
-                const int size = row_end - row_begin;
-                count = (size + b.row_tile - 1) / b.row_tile;
-                late = listed_late(size);
+        Group g = group_of(base + tid);
+        if (g.rest_class == 1 && !late_apart) {
+            g.rest_class = 0;
+        }
+        const int ordinary = g.count - (g.rest_class != 0 ? 1 : 0);
+        int up_to = ordinary;   // inclusive sums over the wave
+        for (int offset = 1; offset < 64; offset <<= 1) {
+            const int add = __shfl_up(up_to, offset);
+            up_to += lane >= offset ? add : 0;
+        }
+        const unsigned long long late = __ballot(g.rest_class == 1), last = __ballot(g.rest_class == 2);
+        if (lane == 63) {
+            of_wave[wave][0] = up_to;
+            of_wave[wave][1] = __popcll(late);
+            of_wave[wave][2] = __popcll(last);
+        }
+        __syncthreads();
+        const unsigned long long below = (1ull << lane) - 1ull;
+        int before[3] = {listed[0] + up_to - ordinary, listed[1] + static_cast<int>(__popcll(late & below)),
+                         listed[2] + static_cast<int>(__popcll(last & below))};
+        for (int w = 0; w < 4; ++w) {
+            for (int c = 0; c < 3; ++c) {
+                before[c] += w < wave ? of_wave[w][c] : 0;
+                listed[c] += of_wave[w][c];
             }
         }
-        scan[tid] = count - late;
-        scan_late[tid] = late;
-        __syncthreads();
-        for (int offset = 1; offset < 256; offset <<= 1) {
-            const int add = tid >= offset ? scan[tid - offset] : 0;
-            const int add_late = tid >= offset ? scan_late[tid - offset] : 0;
-            __syncthreads();
-            scan[tid] += add;
-            scan_late[tid] += add_late;
-            __syncthreads();
-        }
-        const int first = running + scan[tid] - (count - late);
-        const int first_late = early_total + running_late + scan_late[tid] - late;
-        for (int t = 0; t < count; ++t) {
-            const int index = t == count - 1 && late ? first_late : first + t;
+        const int rest_index = g.rest_class == 1 ? late_first + before[1] : last_first + before[2];
+        for (int t = 0; t < g.count; ++t) {
+            const int index = t == g.count - 1 && g.rest_class != 0 ? rest_index : before[0] + t;
             if (index < b.tasks.max_tasks) {
-                const int start = row_begin + t * b.row_tile;
-                b.tasks.expert[index] = expert;
+                const int start = g.row_begin + t * b.row_tile;
+                b.tasks.expert[index] = g.expert;
                 b.tasks.row_start[index] = start;
-                b.tasks.row_end[index] = min(start + b.row_tile, row_end);
+                b.tasks.row_end[index] = min(start + b.row_tile, g.row_begin + g.size);
             }
-        }
-        __syncthreads();
-        if (tid == 255) {
-            running += scan[255];
-            running_late += scan_late[255];
         }
         __syncthreads();
     }
     if (tid == 0) {
-        b.tasks.count[0] = min(running + running_late, b.tasks.max_tasks);
-        b.tasks.early[0] = min(running, b.tasks.max_tasks);
+        b.tasks.count[0] = min(listed[0] + listed[1] + listed[2], b.tasks.max_tasks);
+        b.tasks.early[0] = min(listed[0], b.tasks.max_tasks);
     }
     if (tid < TASK_CURSORS) {
         b.tasks.cursor[tid * TASK_CURSOR_STRIDE] = 0;

@@ -59,6 +59,17 @@ static constexpr int forward_row_tile(int quant_type, int operand_kind) {
            : operand_kind == OPERAND_HALF ? 32 * half_forward_waves(quant_type)
                                           : (quant_type == 14 || quant_type == 22 ? 256 : 128);
 }
+// Grouped calls with scaled operands: whole groups of at most FORWARD_LATE_ROWS rows are listed behind the other tasks and run by
+// groups of four waves that all unpack and multiply (tgo_forward_groups.h), where the role-split workgroups with their 256-row tasks
+// wait for four unpacking waves; groups of at most FORWARD_LAST_ROWS rows are listed last.  Uniform groups, 256 experts of 2048 x 512,
+// gate and up with quantizing, us role-split -> this: Q4_K 16 rows 136 -> 123, 32 rows 151 -> 135, 64 rows 250 -> 184, 128 rows
+// 308 -> 286; IQ2_S 64 rows 260 -> 186, 128 rows 318 -> 288; Q6_K 64 rows 339 -> 246, 128 rows 396 -> 324.  192 rows cut in two:
+// a loss (Q4_K 396 -> 405).
+// Fewer groups of 33 to 128 rows than larger tasks, and the former stay with the role-split workgroups: they are then too few to
+// fill the chip, and four waves alone on a CU take longer over a task than twelve (128 experts of 2048 x 768 Q4_K, 700 tokens with
+// power-law 1.1 routing: layer 222 us, 241 with them apart).
+constexpr int FORWARD_LATE_ROWS = 128;
+constexpr int FORWARD_LAST_ROWS = 32;
 constexpr int BACKWARD_ROW_TILE = 256;
 // Grad-input tasks of at most this many rows (a group's remainder) are listed behind the others and run by a
 // kernel variant whose waves split the K columns of the tile instead of its rows.
@@ -322,6 +333,8 @@ struct TaskBuild {
     TaskList tasks;
     int num_experts, num_groups, rows, row_tile;
     int late_rows;  // tasks of at most this many rows are listed after all the others; 0: group order throughout
+    int last_rows;  // > 0: of these, those of at most this many rows last, the others apart only if they are as many as the ordinary
+                    // tasks
     int late_whole_groups;   // 1: only groups of at most late_rows rows are listed late, not the remainders of larger ones
 };
 
