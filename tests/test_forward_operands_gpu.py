@@ -303,6 +303,22 @@ def test_more_tiles_than_one_table_per_cu_holds(ops, grouped):
         assert bool(((a - b).abs() <= b.abs() * 2.0**-7 + OPERAND_NOISE["scaled"] * peak).all())
 
 
+@pytest.mark.parametrize("rows", (1, 256, 300, 1792))
+def test_wide_matrix_and_few_row_tasks(ops, oracle, rows):
+    """Fewer row tasks than XCDs: the items are dealt out in plain order without empty slots, several to a workgroup."""
+    tgo, native, synth = ops
+    qtype, n, k = QTYPES["Q4_K"], 33024 + 5, 256
+    host = synth.random_packed_weight(qtype, (n,), k, seed=79)
+    x = random_bf16((rows + 32, k), seed=80)   # (more than 32 rows: the matrix-core kernels)
+    native.set_forward_operand("scaled")
+    try:
+        actual = tgo.mmq(x, host.cuda(), qtype, n)
+    finally:
+        native.set_forward_operand("auto")
+    pick = slice(0, None) if rows < 300 else slice(rows - 40, None)   # (the oracle's time)
+    assert_matches_f32_reference(actual[pick], oracle.mmq_forward(qtype, bits(x[pick]), host.numpy(), n, k), OPERAND_NOISE["scaled"])
+
+
 @pytest.mark.parametrize("k", (512, 1024))
 @pytest.mark.parametrize("sizes", ([1, 5, 32, 17, 31, 2], [40, 300, 33], [7, 0, 290, 32, 0, 64]))
 def test_only_short_groups_only_long_groups_and_both(ops, oracle, k, sizes):

@@ -725,8 +725,12 @@ __global__ __launch_bounds__(FSC_THREADS, 3) void mmq_forward_scaled_kernel(cons
 template <int TYPE>
 static hipError_t launch_forward_scaled_typed(const ForwardArgs & call, hipStream_t stream) {
     ForwardArgs args = call;
-    const int64_t total = static_cast<int64_t>(args.n_tiles) * args.projections *
-                          (args.task_count != nullptr ? xcd_chunk_slots(args.task_slots) : pad_task_slots(args.task_slots, FWD_XCD_RUN));
+    // (a dense call of fewer row tasks than XCDs is dealt out in plain order, see xcd_tile, and has no empty slots: with those of a
+    // padded list, a wide matrix would need more workgroups than the chip has CUs to hold them in its tables, each with a prologue
+    // and an epilogue that nothing overlaps.  256 rows x 248320 x 2048 Q6_K: 976 workgroups 377 us, 256 workgroups 348.)
+    const int64_t slots = args.task_count != nullptr ? xcd_chunk_slots(args.task_slots)
+                          : args.task_slots < XCDS ? args.task_slots : pad_task_slots(args.task_slots, FWD_XCD_RUN);
+    const int64_t total = static_cast<int64_t>(args.n_tiles) * args.projections * slots;
     // grouped calls: tasks of at most FGR_ROWS rows are listed behind the others and go to workgroups of their own (one per CU, whose
     // groups take column tiles until none is left)
     const int64_t late_chunks = args.task_count != nullptr ? static_cast<int64_t>(args.task_slots) * args.n_tiles * args.projections : 0;
