@@ -105,3 +105,38 @@ def test_q4k_32_rows_square_against_the_oracle_everywhere(ops, oracle):
     dy = torch.randn(m, n, device="cuda", generator=generator).to(torch.bfloat16)
     _check_forward(tgo, oracle, qtype, x, packed_host, packed, n, list(range(m)))
     _check_grad_input(oracle, qtype, dy, packed_host, packed, n, list(range(m)))
+
+
+@pytest.mark.parametrize("rows,n", [(2100, 640), (2305, 2560), (1300, 5000), (704, 11008)])
+def test_row_tiles_chosen_by_rounds_give_every_result(rows, n):
+    """Dense calls with scaled operands whose row tile follows from the rounds of items, nine and ten row tasks over eight XCDs among
+    them: forward and grad-input against the same rows called a few at a time (whose tiles are others)."""
+    import synth
+    import torch_ggml_ops as tgo
+    from torch_ggml_ops import _native
+
+    qtype, k = 13, 512
+    weight = synth.random_packed_weight(qtype, (n,), k, seed=n).cuda()
+    generator = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.randn(rows, k, device="cuda", generator=generator).to(torch.bfloat16)
+    _native.set_forward_operand("scaled")
+    try:
+        whole = tgo.mmq(x, weight, qtype, n)
+        for begin in range(0, rows - 32, 352):   # (parts of more than 32 rows, the matrix-core kernels)
+            part = tgo.mmq(x[begin : begin + 352].clone(), weight, qtype, n)
+            torch.testing.assert_close(whole[begin : begin + 352], part, rtol=0, atol=0)
+    finally:
+        _native.set_forward_operand("auto")
+    x.requires_grad_()
+    grad = torch.randn(rows, n, device="cuda", generator=generator).to(torch.bfloat16)
+    (dx,) = torch.autograd.grad(tgo.mmq(x, weight, qtype, n), x, grad)
+    reference = grad.float() @ tgo_dequantized(weight, qtype, n, k)
+    assert float((dx.float() - reference).norm() / reference.norm()) < 4e-3   # (bf16 weights and results)
+
+
+def tgo_dequantized(weight, qtype, n, k):
+    from torch_ggml_ops import _native
+
+    out = torch.empty(n, k, dtype=torch.bfloat16, device="cuda")
+    _native.check(_native.lib.tgo_dequant_bf16(weight.data_ptr(), out.data_ptr(), n, k, qtype, None))
+    return out.float()

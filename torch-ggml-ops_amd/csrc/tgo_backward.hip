@@ -35,7 +35,6 @@ constexpr int BWD_TK = 128;                // K columns per workgroup
 constexpr int BWD_NS = 64;                 // weight rows per reduction step
 constexpr int BWD_PITCH = BWD_NS + 8;      // bf16 per k-row of the tile: +8 keeps 16-byte reads conflict free
 constexpr int BWD_THREADS = 256;
-constexpr int BWD_XCD_RUN = 4;             // dense calls: consecutive row tasks that share an XCD (grouped calls: xcd_chunk)
 static_assert(BWD_TR == 64 * BWD_THREADS / 64, "64 rows per wave");
 
 // ---- cotangent packing ---------------------------------------------------------------------------------
@@ -271,11 +270,10 @@ __global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_ker
     if (a.task_count != nullptr) {
         task_segment(a, first_task, tasks, ordinary);
     }
-    // (short tasks are remainders of different experts: nothing to gain from keeping neighbours on one XCD)
     if (!SHORT && a.task_count != nullptr) {
         xcd_chunk(blockIdx.x, a.k_tiles, tasks, ordinary, k_tile, task);
     } else {
-        xcd_tile<SHORT ? 1 : BWD_XCD_RUN>(blockIdx.x, a.k_tiles, tasks, k_tile, task);
+        xcd_tile(blockIdx.x, a.k_tiles, tasks, k_tile, task);
     }
     const int kb = k_tile >> 1;          // super-block column
     const int half_block = k_tile & 1;   // which 128 values of it
@@ -941,7 +939,7 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
                 task_segment(a, first_task, tasks, ordinary);   // (never the short segment: first_task is 0)
                 xcd_chunk(static_cast<int>(linear), a.k_tiles, tasks, ordinary, k_tile, task);
             } else {
-                xcd_tile<BWD_XCD_RUN>(static_cast<int>(linear), a.k_tiles, tasks, k_tile, task);
+                xcd_tile(static_cast<int>(linear), a.k_tiles, tasks, k_tile, task);
             }
             if (a.task_count != nullptr) {
                 if (task < tasks) {
@@ -1472,7 +1470,7 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
 
     int k_tile, task, first_task, tasks;
     task_segment(a, first_task, tasks);
-    xcd_tile<1>(blockIdx.x, a.k_tiles, tasks, k_tile, task);
+    xcd_tile(blockIdx.x, a.k_tiles, tasks, k_tile, task);
     if (task >= tasks) {
         return;
     }
@@ -1801,9 +1799,8 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(const float * __re
 
 template <int TYPE>
 static hipError_t launch_backward_typed(const BackwardArgs & args, hipStream_t stream) {
-    const int64_t total = static_cast<int64_t>(args.k_tiles) *
-                          (args.task_count != nullptr ? xcd_chunk_slots(args.task_slots) : pad_task_slots(args.task_slots, BWD_XCD_RUN));
-    const int64_t total_short = static_cast<int64_t>(args.k_tiles) * pad_task_slots(args.short_slots);
+    const int64_t total = xcd_slots(static_cast<int64_t>(args.k_tiles) * (args.task_count != nullptr ? xcd_chunk_slots(args.task_slots) : args.task_slots));
+    const int64_t total_short = xcd_slots(static_cast<int64_t>(args.k_tiles) * args.short_slots);
     if (total <= 0 || total > 0x7fffffffLL || total_short > 0x7fffffffLL) {
         return hipErrorInvalidValue;
     }

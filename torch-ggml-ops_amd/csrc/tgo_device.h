@@ -70,40 +70,17 @@ TGO_DEVICE float bf16_bits_to_float(uint32_t bits16) {
     return __uint_as_float(bits16 << 16);
 }
 
-// Hardware workgroups are dealt round-robin to the 8 XCDs (each with its own L2) by linear id.  The
-// workgroups of one task (its `inner` column tiles, which share activation rows) are therefore given
-// linear ids that are 8 apart, so they run on one XCD, while eight consecutive tasks spread over the
-// eight XCDs.  The grid holds inner * task_slots workgroups with task_slots a multiple of 8.
+// Hardware workgroups are dealt round-robin to the 8 XCDs (each with its own L2) by linear id.  A launch consists of items: the `inner`
+// column tiles of task 0, which share activation rows, then those of task 1 and so on.
 constexpr int XCDS = 8;
-
-// With fewer tasks than XCDs that grouping would leave whole XCDs idle (a dense call of up to one row tile would
-// run on an eighth of the chip), so then the tiles of a task are dealt out in plain order, i.e. across the XCDs.
-// RUN: consecutive tasks that share an XCD.  (Dense calls and the short tasks of the grad-input; grouped launches,
-// where consecutive tasks are row tiles of the same expert, i.e. of the same weights, take xcd_chunk below.)
-template <int RUN = 1>
-TGO_DEVICE void xcd_tile(int linear, int inner, int tasks, int & inner_id, int & task) {
-    if (tasks < XCDS) {
-        task = linear / inner;
-        inner_id = linear - task * inner;
-        return;
-    }
-    // (with only a few runs' worth of tasks, whole runs per XCD would leave XCDs idle: single tasks then)
-    const int run = tasks >= 2 * XCDS * RUN ? RUN : 1;
-    const int span = XCDS * inner * run;
-    const int group = linear / span;
-    const int within = linear - group * span;
-    const int slot = within / XCDS;        // position on this XCD: `run` tasks of `inner` tiles each, task by task
-    const int run_task = slot / inner;
-    task = (group * XCDS + (within % XCDS)) * run + run_task;
-    inner_id = slot - run_task * inner;
-}
 
 // Grouped launches: consecutive tasks of the list are row tiles of the same expert, i.e. of the same weights, so
 // XCD x takes the x-th eighth of the list as one contiguous chunk and an expert's weights are fetched into one L2
 // (two where a chunk boundary cuts through it).  The chunks differ by at most one task.  A list may put cheap
 // tasks behind the others (`early` = number of ordinary ones): both parts are dealt out that way, so every XCD gets
 // its share of either kind and ends with the cheap ones.  The grid holds inner * xcd_chunk_slots(task slots)
-// workgroups; a slot past its XCD's chunks returns task = tasks.
+// workgroups; a slot past its XCD's chunks returns task = tasks.  (Chunks of items that cut through a task: 1 % slower.)
+// Fewer tasks than XCDs are dealt out in plain order, neighbouring tiles to neighbouring XCDs.
 TGO_DEVICE void xcd_chunk(int linear, int inner, int tasks, int early, int & inner_id, int & task) {
     if (tasks < XCDS) {
         task = linear / inner;
@@ -125,9 +102,27 @@ TGO_DEVICE void xcd_chunk(int linear, int inner, int tasks, int early, int & inn
     task = t < late_end - late_first ? early + late_first + t : tasks;
 }
 
-static inline int xcd_chunk_slots(int slots) { return ((slots + XCDS - 1) / XCDS + 1) * XCDS; }
+// Dense launches and the short tasks of the grad-input: XCD x takes the x-th eighth of the items, to within one item.  (Whole tasks
+// per XCD, or runs of four of them, gave one XCD twice the work of the others where a call has nine row tasks: 2600 rows x 5000 x 3072
+// Q5_K 172 -> 127 us.)  At most eight tasks in plain order: every XCD then has its share of the weights for all tasks (1700 rows x
+// 4096 x 4096 Q5_K: 98 us with an XCD per task, 88 in plain order).  The grid holds xcd_slots(inner * tasks) workgroups; a slot past its
+// XCD's items returns task = tasks.
+TGO_DEVICE void xcd_tile(int linear, int inner, int tasks, int & inner_id, int & task) {
+    if (tasks <= XCDS) {
+        task = linear / inner;
+        inner_id = linear - task * inner;
+        return;
+    }
+    const int xcd = linear % XCDS;
+    const int64_t items = static_cast<int64_t>(tasks) * inner;
+    const int64_t first = xcd * items / XCDS, end = (xcd + 1) * items / XCDS;
+    const int64_t item = first + linear / XCDS < end ? first + linear / XCDS : items;
+    task = static_cast<int>(static_cast<uint32_t>(item) / static_cast<uint32_t>(inner));   // (launches have fewer than 2^31 items)
+    inner_id = static_cast<int>(item) - task * inner;
+}
 
-static inline int pad_task_slots(int slots, int run = 1) { return (slots + XCDS * run - 1) / (XCDS * run) * (XCDS * run); }
+static inline int xcd_chunk_slots(int slots) { return ((slots + XCDS - 1) / XCDS + 1) * XCDS; }
+static inline int64_t xcd_slots(int64_t items) { return (items + XCDS - 1) / XCDS * XCDS; }
 
 // Tile tasks of the grouped operators.  Group g covers rows [offsets[g-1], offsets[g]) of expert indices[g].
 // Every valid group is cut into tasks of at most `row_tile` rows; groups with an out-of-range expert, no rows

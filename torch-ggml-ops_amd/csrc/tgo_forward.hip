@@ -576,8 +576,8 @@ __global__ __launch_bounds__(ForwardShape<TYPE>::THREADS, 2) void mmq_forward_sw
 
 template <int TYPE>
 static hipError_t launch_forward_typed(const ForwardArgs & args, hipStream_t stream) {
-    const int64_t total = static_cast<int64_t>(args.n_tiles) * args.projections *
-                          (args.task_count != nullptr ? xcd_chunk_slots(args.task_slots) : pad_task_slots(args.task_slots, FWD_XCD_RUN));
+    const int64_t total = xcd_slots(static_cast<int64_t>(args.n_tiles) * args.projections *
+                                    (args.task_count != nullptr ? xcd_chunk_slots(args.task_slots) : args.task_slots));
     if (total <= 0 || total > 0x7fffffffLL) {
         return hipErrorInvalidValue;
     }
@@ -674,7 +674,8 @@ static hipError_t launch_forward(const uint8_t * packed, const uint8_t * packed_
         args.task_expert = nullptr;
         args.task_row_start = nullptr;
         args.task_row_end = nullptr;
-        const ForwardSplit split = forward_split(rows, in_features, out_features, quant_type, ws.operand_kind(), partial != nullptr);
+        const ForwardSplit split = forward_split(rows, in_features, out_features, quant_type, ws.operand_kind(), partial != nullptr,
+                                                  args.projections);
         args.dense_row_tile = split.row_tile;
         args.task_slots = (rows + split.row_tile - 1) / split.row_tile;
         args.k_splits = split.k_splits;

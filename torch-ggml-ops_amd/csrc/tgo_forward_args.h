@@ -8,7 +8,6 @@
 namespace tgo {
 
 constexpr int FWD_TN = 128;          // weight rows per workgroup
-constexpr int FWD_XCD_RUN = 4;       // dense calls: consecutive row tasks that share an XCD (grouped calls: xcd_chunk)
 constexpr int FWD_NT = FWD_TN / 32;  // 32-row weight tiles per workgroup
 
 struct ForwardArgs {
@@ -39,7 +38,7 @@ struct ForwardArgs {
     int projections;   // 1, or 2 for a pair: both share the task's activations, so their tiles run side by side
     int swiglu;        // 1: a workgroup runs gate (-> y) then up and stores swiglu(gate, up) -> y_second
     int task_slots;
-    int dense_row_tile;   // dense calls: rows per workgroup (the format's row tile, or 32 when that fills the chip better)
+    int dense_row_tile;   // dense calls: rows per workgroup (forward_split)
     int wide;             // 2-byte aligned formats: the weights may be fetched as aligned 16-byte units (wide_stage_ok)
     float * partial;      // dense calls too small to fill the chip: fp32 sums of each range of K, [range][row][n_tiles * 128], or nullptr
     int k_splits;         // how many ranges (blockIdx.y picks one); 1 when partial is nullptr
@@ -57,7 +56,7 @@ TGO_DEVICE bool forward_pick_linear(const ForwardArgs & a, int linear, int & n_t
         tasks = a.early_only != 0 ? early : tasks;
         xcd_chunk(linear, a.n_tiles * a.projections, tasks, early, n_tile, task);
     } else {
-        xcd_tile<FWD_XCD_RUN>(linear, a.n_tiles * a.projections, tasks, n_tile, task);
+        xcd_tile(linear, a.n_tiles * a.projections, tasks, n_tile, task);
     }
     second = n_tile >= a.n_tiles;
     n_tile -= second ? a.n_tiles : 0;

@@ -60,7 +60,7 @@ static_assert(FSC_ROWS == forward_row_tile(12, OPERAND_SCALED), "task rows match
 constexpr int FSC_W_AHEAD = 1;                               // reduction steps a weight fragment is read ahead of its matrix instructions
 
 constexpr int FSC_MAX_ITEMS = 64;      // items per workgroup (one wave builds the table)
-constexpr int FSC_GRID = 256;          // one workgroup per CU
+constexpr int FSC_GRID = SCALED_WORKGROUPS;
 constexpr int FSC_BUFFERS = 3;         // operand tiles in flight between the unpacking and the multiplying waves
 constexpr int FSC_SPIN_LIMIT = 1 << 20;   // polls of a stage counter before a wave gives up waiting (a few hundred ms)
 
@@ -725,12 +725,11 @@ __global__ __launch_bounds__(FSC_THREADS, 3) void mmq_forward_scaled_kernel(cons
 template <int TYPE>
 static hipError_t launch_forward_scaled_typed(const ForwardArgs & call, hipStream_t stream) {
     ForwardArgs args = call;
-    // (a dense call of fewer row tasks than XCDs is dealt out in plain order, see xcd_tile, and has no empty slots: with those of a
-    // padded list, a wide matrix would need more workgroups than the chip has CUs to hold them in its tables, each with a prologue
-    // and an epilogue that nothing overlaps.  256 rows x 248320 x 2048 Q6_K: 976 workgroups 377 us, 256 workgroups 348.)
-    const int64_t slots = args.task_count != nullptr ? xcd_chunk_slots(args.task_slots)
-                          : args.task_slots < XCDS ? args.task_slots : pad_task_slots(args.task_slots, FWD_XCD_RUN);
-    const int64_t total = static_cast<int64_t>(args.n_tiles) * args.projections * slots;
+    // (No empty slots but one per XCD: a list padded to whole tasks per XCD did not fit the tables of one workgroup per CU where a matrix
+    // is wide and its rows are few, and more workgroups each have a prologue and an epilogue that nothing overlaps.  256 rows x
+    // 248320 x 2048 Q6_K: 976 workgroups 377 us, 256 workgroups 348.)
+    const int64_t total = xcd_slots(static_cast<int64_t>(args.n_tiles) * args.projections *
+                                    (args.task_count != nullptr ? xcd_chunk_slots(args.task_slots) : args.task_slots));
     // grouped calls: tasks of at most FGR_ROWS rows are listed behind the others and go to workgroups of their own (one per CU, whose
     // groups take column tiles until none is left)
     const int64_t late_chunks = args.task_count != nullptr ? static_cast<int64_t>(args.task_slots) * args.n_tiles * args.projections : 0;

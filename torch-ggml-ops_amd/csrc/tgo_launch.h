@@ -97,17 +97,39 @@ constexpr int GEMV_DENSE_ROWS = 32;
 // ranges below it, one range -> ranges: K = 4096, 512 columns, 64 rows Q6_K 102 -> 28 us, Q3_K 50 -> 19, Q4_K 37 -> 17, IQ2_S
 // 42 -> 20; K = 2048, 1024 columns, 64 rows 55 -> 24, 29 -> 18, 22 -> 15, 25 -> 20; K = 1024 mostly a tie, from 2048 columns up
 // also a loss (Q4_K, 517 rows of 2048: 18 -> 23).  (1024 x 4096, on the line, 64 rows: Q6_K 33, Q3_K 20, Q4_K 18.)
+constexpr int SCALED_WORKGROUPS = 256;   // one per CU
 struct ForwardSplit {
     int row_tile;
     int k_splits;
 };
 static inline ForwardSplit forward_split(int64_t rows, int64_t in_features, int64_t out_features, int quant_type, int operand_kind,
-                                         bool scratch) {
+                                         bool scratch, int projections = 1) {
     const int64_t n_tiles = (out_features + 127) / 128;
     const int64_t super_blocks = in_features / 256;
+    if (operand_kind == OPERAND_SCALED) {
+        // One persistent workgroup per CU: a call takes as long as its rounds of items.  An item of T rows costs about 256 + T (256
+        // experts of 2048 x 512 Q4_K with T rows each, one item per expert and column tile: 64 rows 0.64 of the time of 256, 128 rows
+        // 0.75, 192 rows 0.92); the last round costs 0.4 and 1.3 times the share of the CUs that it occupies, at most 1 (4096 x 4096
+        // Q5_K, items of 256 rows: 224 items 88 us, 288 135, 352 173).  Fewer rows are taken where that saves a sixteenth.
+        // 4096 x 4096 Q5_K 2600 rows 178 -> 153 us, 11008 x 2048 2600 rows 235 -> 172, 5000 rows 344 -> 285 (with the tiles dealt out evenly,
+        // see xcd_chunk); a call of one short second round is a little slower for that (2100 rows x 4096 x 4096: 140 -> 148).
+        int best = 256;
+        int64_t least = 0;
+        for (int tile = 256; tile >= 64; tile -= 32) {
+            const int64_t items = n_tiles * projections * ((rows + tile - 1) / tile);
+            const int64_t last = items % SCALED_WORKGROUPS;
+            const int64_t rounds = items / SCALED_WORKGROUPS * 1000 + (last == 0 ? 0 : std::min<int64_t>(1000, 400 + last * 1300 / SCALED_WORKGROUPS));
+            const int64_t cost = rounds * (256 + tile);
+            if (least == 0 || cost * 16 < least * 15) {
+                best = tile;
+                least = cost;
+            }
+        }
+        return {best, 1};
+    }
     const int full_tile = forward_row_tile(quant_type, operand_kind);
     const auto tiles = [&](int tile) { return n_tiles * ((rows + tile - 1) / tile); };
-    if (scratch && operand_kind != OPERAND_SCALED && out_features * in_features >= (INT64_C(1) << 22)) {
+    if (scratch && out_features * in_features >= (INT64_C(1) << 22)) {
         int tile = full_tile;
         int64_t most;   // ranges
         if (full_tile == 128) {
