@@ -55,3 +55,26 @@ def test_grouped(ops, oracle, qname, n, k):
     gate, up = (o.float() for o in outputs)
     expected = (torch.nn.functional.silu(gate) * up)[on_device]
     assert ((activated.float()[on_device] - expected).abs() <= 2.0**-7 * expected.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("qname", tuple(QTYPES))
+@pytest.mark.parametrize("n,sizes", [(512, [1, 15, 16, 17, 33, 5, 0, 2] * 2), (2048, [40, 3, 1, 18])])
+def test_grouped_calls_of_a_few_rows_per_group(oracle, qname, n, sizes):
+    """Beyond the decode regime (more than four rows per group on average): groups of one to three tasks of 16 rows, none, and a list
+    of four groups whose K and columns make up the four million weights; one projection and a pair."""
+    import synth
+    import torch_ggml_ops as tgo
+
+    qtype, k = QTYPES[qname], 512
+    experts = list(range(len(sizes)))[::-1]
+    offsets = np.cumsum(sizes).tolist()
+    assert 4 * len(sizes) < offsets[-1] <= 16 * len(sizes)
+    metadata = (torch.tensor(experts, device="cuda"), torch.tensor(offsets, device="cuda", dtype=torch.int32))
+    hosts = [synth.random_packed_weight(qtype, (len(sizes), n), k, seed=qtype + i) for i in range(2)]
+    weights = [host.cuda() for host in hosts]
+    x = random_bf16((offsets[-1], k), seed=n)
+    expected = [oracle.grouped(oracle.mmq_forward, qtype, bits(x), host.numpy(), experts, offsets, n, k, n) for host in hosts]
+    assert_matches_f32_reference(tgo.grouped_mmq(x, weights[0], *metadata, qtype, n), expected[0])
+    first, second = tgo.grouped_mmq_pair(x, *weights, *metadata, qtype, n)
+    assert_matches_f32_reference(first, expected[0])
+    assert_matches_f32_reference(second, expected[1])

@@ -678,8 +678,8 @@ static int grouped_forward(const void * input_bf16, const int64_t * row_index, i
                                                  static_cast<uint16_t *>(output_second), rows * out_features, hip_stream),
                          "swiglu launch");
     };
-    const bool gemv = tgo::use_gemv(rows, num_groups);
-    const bool tiles = tgo::gemv_takes_tiles(packed_first, packed_second, rows, num_groups, in_features, out_features, quant_type);
+    const bool tiles = tgo::grouped_takes_tiles(packed_first, packed_second, rows, num_groups, in_features, out_features, quant_type);
+    const bool gemv = tiles || tgo::use_gemv(rows, num_groups);
     if (gemv && !tiles && tgo::gemv_fuses(quant_type, rows, num_groups)) {
         // one launch: the decode-regime kernels of these formats quantize their activations and find their tasks
         // themselves

@@ -205,6 +205,17 @@ static inline bool use_gemv(int64_t rows, int64_t groups) {
     return groups <= 0 ? rows <= GEMV_DENSE_ROWS : rows <= 4 * groups;
 }
 
+// Whether the layout of the kernel for tasks of several rows (tgo_gemv_tiles.hip) allows a call: whole tiles of 16 weight rows, aligned weights, offsets within a tile of 32 bits, and four
+// million weights that are read.
+static inline bool tiles_fit(const void * packed, const void * packed_second, int64_t rows, int64_t groups, int64_t in_features,
+                             int64_t out_features) {
+    if (out_features % 16 != 0 || (reinterpret_cast<uintptr_t>(packed) | reinterpret_cast<uintptr_t>(packed_second)) % 16 != 0 ||
+        in_features > (INT64_C(1) << 22) || rows > (1 << 24)) {
+        return false;
+    }
+    const int64_t matrices = groups <= 0 ? 1 : rows < groups ? rows : groups;
+    return matrices * out_features * in_features >= (INT64_C(1) << 22);
+}
 // Decode-regime calls that take the kernel for tasks of several rows (tgo_gemv_tiles.hip), which unpacks every weight once
 // per task, instead of those of tgo_gemv.hip, whose dot products cost the same again for every row.  It needs whole tiles of
 // 16 weight rows and 16-byte aligned weights.  The lines lie where the two measured equal (2048 x 512 and 4096 x 1024 experts
@@ -221,13 +232,7 @@ constexpr int GEMV_TILES_ROWS = 16;              // rows of its tasks
 constexpr int64_t GEMV_TILES_WORKGROUPS = 384;   // workgroups that a launch should have for a wave to take four tiles of 16 weight rows instead of two
 static inline bool gemv_takes_tiles(const void * packed, const void * packed_second, int64_t rows, int64_t groups, int64_t in_features,
                                     int64_t out_features, int quant_type) {
-    if (!use_gemv(rows, groups) || out_features % 16 != 0 ||
-        (reinterpret_cast<uintptr_t>(packed) | reinterpret_cast<uintptr_t>(packed_second)) % 16 != 0 ||
-        in_features > (INT64_C(1) << 22) || rows > (1 << 24)) {   // (the kernel's offsets within a tile have 32 bits)
-        return false;
-    }
-    const int64_t matrices = groups <= 0 ? 1 : rows < groups ? rows : groups;
-    if (matrices * out_features * in_features < (INT64_C(1) << 22)) {
+    if (!use_gemv(rows, groups) || !tiles_fit(packed, packed_second, rows, groups, in_features, out_features)) {
         return false;
     }
     const int64_t super_blocks = in_features / 256;
@@ -248,6 +253,27 @@ static inline bool gemv_takes_tiles(const void * packed, const void * packed_sec
         case 14: return super_blocks <= 2 ? 2 * rows >= groups : super_blocks <= 4 ? rows >= 16 : 2 * rows >= 3 * groups;
         default: return rows >= 24;
     }
+}
+// Grouped calls beyond the decode regime (use_gemv) that take it all the same: its tasks of 16 rows unpack a group's weights once or
+// twice, the matrix-core kernels once per 128 or 256 rows and with a fraction of the chip.  The line is a number of rows per group on
+// average, by the operand kind that the call has otherwise.
+// Exact kinds, gate and up of 256 experts of 2048 x 512, us matrix-core kernel -> this one: 8 rows Q3_K 141 -> 80, Q4_K 123 -> 99,
+// Q5_K 135 -> 112, Q6_K 435 -> 149, IQ2_S 174 -> 94; 12 rows Q6_K 437 -> 156, IQ2_S 175 -> 98; 16 rows of 64 experts of 2048 x 768 Q3_K 69 ->
+// 38, Q4_K 50 -> 43, Q6_K 162 -> 58.  Layers with power-law 1.1 routing, whose large groups are cut into many tasks: 12 rows on average
+// 0.35 to 0.95 of the time, 14 rows IQ2_S 1.18, Q4_K 1.05, Q6_K 0.83.
+// Scaled operands: 512 columns of K to 2048, 12 rows Q3_K 72 -> 52, Q4_K 62 -> 48, Q5_K 69 -> 54, Q6_K 90 -> 82, IQ2_S 70 -> 68.
+// Not where the operand kind was forced: the caller asked for that kind's kernels.
+static inline bool grouped_takes_tiles(const void * packed, const void * packed_second, int64_t rows, int64_t groups, int64_t in_features,
+                                       int64_t out_features, int quant_type) {
+    if (use_gemv(rows, groups)) {
+        return gemv_takes_tiles(packed, packed_second, rows, groups, in_features, out_features, quant_type);
+    }
+    if (forward_operand_setting() != OPERAND_AUTO || !tiles_fit(packed, packed_second, rows, groups, in_features, out_features)) {
+        return false;
+    }
+    const bool scaled = forward_operand_kind(quant_type, rows, out_features, packed_second != nullptr ? 2 : 1) == OPERAND_SCALED;
+    const int64_t most = quant_type == 14 ? (scaled ? 8 : 32) : quant_type == 22 ? (scaled ? 8 : 12) : scaled ? 12 : 16;
+    return rows <= most * groups;
 }
 
 // q8_1 workspace: quantized values, then fp32 scales, then fp32 sums, in one of four layouts over the same bytes.
