@@ -78,3 +78,16 @@ def test_grouped_calls_of_a_few_rows_per_group(oracle, qname, n, sizes):
     first, second = tgo.grouped_mmq_pair(x, *weights, *metadata, qtype, n)
     assert_matches_f32_reference(first, expected[0])
     assert_matches_f32_reference(second, expected[1])
+
+
+@pytest.mark.parametrize("qname", tuple(QTYPES))
+@pytest.mark.parametrize("rows,n,k", [(33, 4096, 1024), (64, 16400, 768), (81, 2064, 4096), (128, 5120, 1024), (129, 5120, 1024)])
+def test_dense_beyond_the_decode_regime(oracle, qname, rows, n, k):
+    """Three to eight tasks of 16 rows, the last one not full, and one row beyond the line."""
+    import synth
+    import torch_ggml_ops as tgo
+
+    qtype = QTYPES[qname]
+    host = synth.random_packed_weight(qtype, (n,), k, seed=qtype + rows)
+    x = random_bf16((rows, k), seed=rows)
+    assert_matches_f32_reference(tgo.mmq(x, host.cuda(), qtype, n), oracle.mmq_forward(qtype, bits(x), host.numpy(), n, k))

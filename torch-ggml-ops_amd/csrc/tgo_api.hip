@@ -366,7 +366,8 @@ int tgo_mmq_forward_scratch(const void * input_bf16, const void * packed, void *
     TGO_TRY(check_pointer(workspace, "workspace"));
     TGO_TRY(check_scratch(scratch, rows, in_features, out_features, quant_type));
     hipStream_t hip_stream = static_cast<hipStream_t>(stream);
-    if (tgo::gemv_fuses(quant_type, rows, 0) && !tgo::gemv_takes_tiles(packed, nullptr, rows, 0, in_features, out_features, quant_type)) {
+    const bool tiles = tgo::dense_takes_tiles(packed, rows, in_features, out_features, quant_type);
+    if (!tiles && tgo::gemv_fuses(quant_type, rows, 0)) {
         // one launch: the decode-regime kernels of these formats quantize their activations themselves
         return check_hip(tgo::launch_mmq_gemv_fused(static_cast<const uint8_t *>(packed), nullptr, 0,
                                                     static_cast<const uint16_t *>(input_bf16), nullptr, rows, nullptr,
@@ -375,11 +376,17 @@ int tgo_mmq_forward_scratch(const void * input_bf16, const void * packed, void *
                                                     static_cast<int>(out_features), quant_type, hip_stream),
                          "mmq_forward launch");
     }
-    const tgo::Q8Workspace view = tgo::q8_workspace_view(workspace, rows, in_features, tgo::use_gemv(rows, 0),
+    const tgo::Q8Workspace view = tgo::q8_workspace_view(workspace, rows, in_features, tiles || tgo::use_gemv(rows, 0),
                                                          tgo::forward_operand_kind(quant_type, rows, out_features, 1));
     TGO_TRY(check_hip(tgo::launch_quantize_q8_1(static_cast<const uint16_t *>(input_bf16), view, rows, in_features,
                                                 hip_stream),
                       "quantize_q8_1 launch"));
+    if (tiles) {
+        return check_hip(tgo::launch_mmq_gemv_tiles(static_cast<const uint8_t *>(packed), nullptr, 0, view, static_cast<uint16_t *>(output_bf16),
+                                                    nullptr, nullptr, static_cast<int>(rows), static_cast<int>(in_features),
+                                                    static_cast<int>(out_features), quant_type, false, hip_stream),
+                         "mmq_forward launch");
+    }
     return check_hip(launch_dense(packed, view, output_bf16, scratch, rows, in_features, out_features, quant_type, hip_stream),
                      "mmq_forward launch");
 }

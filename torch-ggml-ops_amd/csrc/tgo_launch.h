@@ -254,6 +254,24 @@ static inline bool gemv_takes_tiles(const void * packed, const void * packed_sec
         default: return rows >= 24;
     }
 }
+// Dense calls beyond the decode regime that take it all the same: three to eight tasks of 16 rows, each of which unpacks all weights,
+// keep the chip busier than the matrix-core kernels' tiles of 128 columns, up to a number of rows that falls with the matrix (us,
+// matrix-core kernel -> this one): 2048 x 2048 Q4_K 64 rows 23 -> 10, 128 rows 16 -> 11; Q6_K 128 rows 27 -> 15; 5120 x 1024 IQ2_S 128
+// rows 18 -> 18; 4096 x 4096 Q3_K 64 rows 23 -> 17, 96 rows 28 -> 24, Q5_K 96 rows 24 -> 24, Q6_K 64 rows 28 -> 22, 80 rows 30 -> 31; 11008 x 4096
+// 64 rows Q3_K 42 -> 32, Q4_K 34 -> 30, 80 rows 38 -> 37; 28672 x 8192 34 rows Q4_K 103 -> 102, Q6_K 140 -> 160.
+static inline bool dense_takes_tiles(const void * packed, int64_t rows, int64_t in_features, int64_t out_features, int quant_type) {
+    if (use_gemv(rows, 0)) {
+        return gemv_takes_tiles(packed, nullptr, rows, 0, in_features, out_features, quant_type);
+    }
+    if (forward_operand_setting() != OPERAND_AUTO || !tiles_fit(packed, nullptr, rows, 0, in_features, out_features)) {
+        return false;
+    }
+    const int64_t weights = out_features * in_features;
+    return rows <= (weights <= (INT64_C(1) << 23)   ? 128
+                    : weights <= (INT64_C(1) << 24) ? (quant_type == 14 ? 64 : 96)
+                    : weights <= (INT64_C(1) << 26) ? 64
+                                                    : GEMV_DENSE_ROWS);
+}
 // Grouped calls beyond the decode regime (use_gemv) that take it all the same: its tasks of 16 rows unpack a group's weights once or
 // twice, the matrix-core kernels once per 128 or 256 rows and with a fraction of the chip.  The line is a number of rows per group on
 // average, by the operand kind that the call has otherwise.
