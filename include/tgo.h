@@ -344,7 +344,9 @@ int tgo_grouped_mmq_grad_input_weighted(const void * grad_tokens_bf16, const int
                                         int64_t num_groups, int quant_type, void * stream);
 
 /* Name of the kernel family the forward entry points pick for a shape ("mfma" or "gemv");
- * host pointer to a static string.  Lets callers and benchmarks label what they measure. */
+ * host pointer to a static string.  Lets callers and benchmarks label what they measure.  Beyond the
+ * decode regime the answer is "mfma" by rows alone; the 16-row decode kernel still takes calls of few rows
+ * per group, or of up to 128 dense rows, by format, size and alignment. */
 const char * tgo_forward_kernel_family(int64_t rows, int64_t num_groups);
 
 /* ---- optional per-kernel timing (benchmarks only) ---------------------------------------
@@ -389,7 +391,8 @@ int tgo_profile_read(int kernel, double * total_ms, int64_t * launches);
  * KiB: tgo_q8_workspace_unpack follows that tag, and tgo_mmq_forward_prepared turns its outputs into NaN when the
  * setting was changed between quantizing a workspace and using it.  A call reads the setting once.
  * tgo_forward_operand() returns the current setting; tgo_forward_operand_for() the kind (never AUTO) that a forward
- * call of this format and shape would use under it (`projections`: 2 for a pair).  No counterpart in the reference. */
+ * call of this format and shape would use under it on those kernels (`projections`: 2 for a pair); under AUTO
+ * some calls take the 16-row decode kernel instead (see tgo_forward_kernel_family), whose operands are exact.  No counterpart in the reference. */
 #define TGO_OPERAND_INT8 0
 #define TGO_OPERAND_HALF 1
 #define TGO_OPERAND_AUTO 2

@@ -12,7 +12,7 @@
 // weight underflows: S of a weight row follows its super-blocks here instead of a scan over the row (which would fetch a line of every
 // block for four bytes of it, ahead of the first), see FGR_BASE.
 // 256 experts of 2048 x 512 IQ2_S with 128 rows each, gate and up: 0.64 PFLOP/s (0.53 by role-split tasks); under that load the chip's
-// clock is down to 1.7 GHz, and neither the order of a stage's instructions nor 64 weight rows per wave (half the fragment reads, two
+// clock is below 2 GHz (counted cycles over traced time), and neither the order of a stage's instructions nor 64 weight rows per wave (half the fragment reads, two
 // waves per SIMD) changed the time.
 #pragma once
 

@@ -25,7 +25,8 @@
 // cores 11 %, 3.5 TB/s of packed bytes); what is left is each wave's own chain of fetch, park, read back, unpack and multiply at two workgroups per CU,
 // and a fetch ring of four steps or a third workgroup changed nothing.  The kernels of tgo_gemv.hip
 // pay four v_dot4 plus scaling per 16 weights and activation row instead and need no whole tiles: better for one to three
-// rows.  Measured against them in a layer of 97 tokens of eight choices among 256 experts (kernel time, the fused SwiGLU on top of it
+// rows.  Calls of more tasks than the decode regime has, up to 128 dense rows, come here too (dense_takes_tiles, grouped_takes_tiles).
+// Measured against them in a layer of 97 tokens of eight choices among 256 experts (kernel time, the fused SwiGLU on top of it
 // not counted): gate and up (2048 x 512) Q3_K 179 -> 75 us, Q5_K 135 -> 92, IQ2_S 140 -> 91; down (512 x 2048) Q4_K 100 -> 42, Q6_K
 // 91 -> 84.  Dense 28672 x 8192, 16 rows: Q3_K 230 -> 44, Q4_K 65 -> 46, Q6_K 160 -> 69.
 #include <algorithm>

@@ -278,7 +278,8 @@ static inline bool dense_takes_tiles(const void * packed, int64_t rows, int64_t 
 // Exact kinds, gate and up of 256 experts of 2048 x 512, us matrix-core kernel -> this one: 8 rows Q3_K 141 -> 80, Q4_K 123 -> 99,
 // Q5_K 135 -> 112, Q6_K 435 -> 149, IQ2_S 174 -> 94; 12 rows Q6_K 437 -> 156, IQ2_S 175 -> 98; 16 rows of 64 experts of 2048 x 768 Q3_K 69 ->
 // 38, Q4_K 50 -> 43, Q6_K 162 -> 58.  Layers with power-law 1.1 routing, whose large groups are cut into many tasks: 12 rows on average
-// 0.35 to 0.95 of the time, 14 rows IQ2_S 1.18, Q4_K 1.05, Q6_K 0.83.
+// 0.35 to 0.95 of the time, 14 rows IQ2_S 1.18, Q4_K 1.05, Q6_K 0.83.  At the line it can lose a little: 16 rows of 64 experts of 2048 x 512 gate and up
+// Q4_K 34.7 -> 35.8, where the down projection (512 x 2048) wins, 25.4 -> 20.7.
 // Scaled operands: 512 columns of K to 2048, 12 rows Q3_K 72 -> 52, Q4_K 62 -> 48, Q5_K 69 -> 54, Q6_K 90 -> 82, IQ2_S 70 -> 68.
 // Not where the operand kind was forced: the caller asked for that kind's kernels.
 static inline bool grouped_takes_tiles(const void * packed, const void * packed_second, int64_t rows, int64_t groups, int64_t in_features,
