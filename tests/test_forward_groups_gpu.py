@@ -105,3 +105,50 @@ def test_more_groups_than_one_round_of_the_list_builder(ops, oracle):
     sizes = rng.choice([0, 1, 3, 30, 33, 50, 130], size=600, p=[0.1, 0.4, 0.2, 0.1, 0.1, 0.07, 0.03]).tolist()
     host = ops[2].random_packed_weight(qtype, (len(sizes), n), k, seed=9)
     _check(ops, oracle, qtype, host, sizes, k, n)
+
+
+def _spread_weights(ops, qtype, experts, n, k, power):
+    """Random packed weights whose super-block s has scales 2^power[s] times those of a usual one."""
+    host = ops[2].random_packed_weight(qtype, (experts, n), k, seed=qtype)
+    blocks = host.view(experts, n, k // 256, -1)
+    factor = torch.exp2(torch.tensor(power, dtype=torch.float32)).expand(experts, n, k // 256)
+    for offset in SCALE_OFFSETS[qtype]:
+        scale = blocks[..., offset : offset + 2].contiguous().view(torch.float16)[..., 0].float()
+        blocks[..., offset : offset + 2] = (scale * factor).to(torch.float16).contiguous().view(torch.uint8).view(*factor.shape, 2)
+    return host
+
+
+@pytest.mark.parametrize("qname", tuple(QTYPES))
+@pytest.mark.parametrize("largest_first", (True, False))
+def test_up_to_32_rows_every_super_block_keeps_its_own_bits(ops, oracle, qname, largest_first):
+    """Weights 2^18 below another super-block of their row, which meets activations of zero: the result is theirs alone, and as
+    exact as if the other were not there."""
+    tgo, _, _ = ops
+    qtype, k, n, sizes = QTYPES[qname], 768, 96, [1, 20, 32]
+    power = [9, -9, -9] if largest_first else [-9, -9, 9]
+    host = _spread_weights(ops, qtype, len(sizes), n, k, power)
+    offsets = np.cumsum(sizes).tolist()
+    x = random_bf16((offsets[-1], k), seed=3)
+    x[:, :256] = 0 if largest_first else x[:, :256]
+    x[:, 512:] = 0 if not largest_first else x[:, 512:]
+    metadata = (torch.arange(len(sizes), device="cuda"), torch.tensor(offsets, device="cuda", dtype=torch.int32))
+    output = tgo.grouped_mmq(x, host.cuda(), *metadata, qtype, n)
+    expected = oracle.grouped(oracle.mmq_forward, qtype, bits(x), host.numpy(), list(range(len(sizes))), offsets, n, k, n)
+    assert_matches_f32_reference(output, expected, OPERAND_NOISE["scaled"])
+
+
+@pytest.mark.parametrize("qname", tuple(QTYPES))
+def test_33_to_128_rows_are_as_exact_as_a_dense_call(ops, qname):
+    """With the row's largest super-block first, the weights are normalised as in the role-split kernel of a dense call, also those
+    that lose bits: the same results bit for bit.  2^14 and 2^20 below the largest, at which the activations are small."""
+    tgo, _, _ = ops
+    qtype, k, n, sizes = QTYPES[qname], 768, 96, [33, 64, 70, 96, 100, 128]
+    host = _spread_weights(ops, qtype, len(sizes), n, k, [9, -5, -11]).cuda()
+    offsets = np.cumsum(sizes).tolist()
+    x = random_bf16((offsets[-1], k), seed=4)
+    x[:, :256] *= 2.0**-20
+    metadata = (torch.arange(len(sizes), device="cuda"), torch.tensor(offsets, device="cuda", dtype=torch.int32))
+    output = tgo.grouped_mmq(x, host, *metadata, qtype, n)
+    for expert, (begin, end) in enumerate(zip([0] + offsets, offsets)):
+        dense = tgo.mmq(x[begin:end].clone(), host[expert].clone(), qtype, n)
+        torch.testing.assert_close(output[begin:end], dense, rtol=0, atol=0)

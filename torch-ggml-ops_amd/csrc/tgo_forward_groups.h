@@ -8,9 +8,10 @@
 // (v_permlane32_swap) per register puts them where the instruction wants them; every fragment then serves all row tiles.  The four
 // waves share the activation fragments, which they bring to LDS in turn, 8 KiB a stage, rescaled to the row's exponent on the way
 // (once per group instead of by each wave that multiplies with them).
-// The algebra, the operands and the order of additions are the role-split routine's, and so are the results, bit for bit, unless a
-// weight underflows: S of a weight row follows its super-blocks here instead of a scan over the row (which would fetch a line of every
-// block for four bytes of it, ahead of the first), see FGR_BASE.
+// The algebra and the operands are the role-split routine's.  S of a weight row is not scanned for ahead of the row (which would fetch a
+// line of every block for four bytes of it) but follows its super-blocks, see FGR_BASE: tasks of more than 32 rows add in the
+// role-split routine's order and have its results bit for bit, unless a weight underflows there; tasks of at most 32 rows normalise
+// every super-block by itself and add its sums to the row's.
 // 256 experts of 2048 x 512 IQ2_S with 128 rows each, gate and up: 0.64 PFLOP/s (0.53 by role-split tasks); under that load the chip's
 // clock is below 2 GHz (counted cycles over traced time), and neither the order of a stage's instructions nor 64 weight rows per wave (half the fragment reads, two
 // waves per SIMD) changed the time.
@@ -76,11 +77,16 @@ struct GroupLds {
     std::conditional_t<TYPE == IQ2_S, Iq2sSelectors, uint2> codebook;
 };
 
-// A weight row's first super-block puts its largest possible weight in [2^FGR_BASE, 2^(FGR_BASE + 1)).  A later one may be up to
-// 2^FGR_SLACK times as large (below 2^9, which Q4_K/Q5_K's -1024 * scale still allows); beyond that S grows to it and the sums so far
-// are divided accordingly (a power of two).  Smaller ones lose bits only below 2^-18 of the largest.
-constexpr int FGR_BASE = 4;
-constexpr int FGR_SLACK = 4;
+// S puts the largest possible weight of a super-block in [2^FGR_BASE, 2^(FGR_BASE + 1)), as the role-split routine does for a row's
+// largest (Q4_K/Q5_K's -1024 * scale allows no more).
+//  - R = 1: every super-block has an S of its own, and no weight loses bits to a larger super-block of its row; 2^S of the super-block
+//    goes into the multiply-add that joins its sums to the row's.
+//  - R > 1: S is that of the largest super-block so far, and where it grows the sums so far are divided accordingly (a power of two):
+//    a weight never has fewer bits than under the row's maximum, which costs 16 R multiplications in the few super-blocks that bring
+//    one of the wave's 32 rows a new one.
+// Against one S from a row's first super-block with room of 2^4 to grow, in which weights 2^14 below the row's largest lost bits: a
+// prefill layer of 2048 tokens, 256 experts 354.7 -> 355.7 us, a training layer of 4096 tokens 1167 -> 1173.
+constexpr int FGR_BASE = 8;
 
 template <int TYPE, bool WIDE, int R>
 TGO_DEVICE void group_task(const ForwardArgs & a, GroupLds<TYPE> & lds, GroupBarrier & barrier, const int tid, int expert, int row_start,
@@ -240,7 +246,9 @@ TGO_DEVICE void group_task(const ForwardArgs & a, GroupLds<TYPE> & lds, GroupBar
     };
 
     const v16f zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    v16f acc[R];
+    constexpr bool APART = R == 1;   // super-blocks normalised by themselves
+    v16f acc[R];                     // (APART: of the super-block)
+    v16f row_sums = zero;            // APART: sum over the super-blocks so far of 2^S * acc
 #pragma unroll
     for (int r = 0; r < R; ++r) acc[r] = zero;
 
@@ -273,10 +281,10 @@ TGO_DEVICE void group_task(const ForwardArgs & a, GroupLds<TYPE> & lds, GroupBar
         }
         int exponent = static_cast<int>(__float_as_uint(reach) >> 23);
         exponent = min(max(exponent, 9), 254);
-        const bool grow = fresh || exponent > w.exponent + FGR_SLACK;
+        const bool grow = fresh || APART || exponent > w.exponent;
         bool changed = false;
         if (__any(grow)) {
-            if (!fresh) {
+            if (!fresh && !APART) {
                 changed = true;
                 if (half == 0) {
                     lds.column_power[wave][l32] = grow ? __uint_as_float(static_cast<uint32_t>(max(127 + w.exponent - exponent, 0)) << 23) : 1.0f;
@@ -467,12 +475,26 @@ TGO_DEVICE void group_task(const ForwardArgs & a, GroupLds<TYPE> & lds, GroupBar
         park(ahead);   // (everything of this super-block has been read from the slot)
         ratio = ratio_next;
         kb = kb_next;
-        if (kb == 0) {
-            // the item is complete: scale by 2^(E[r] + S[n]) and store
+        if (APART || kb == 0) {
             if (half == 0) {
                 lds.column_power[wave][l32] = __uint_as_float(static_cast<uint32_t>(row.exponent - FGR_BASE) << 23);
             }
             asm volatile("" ::: "memory");
+        }
+        if constexpr (APART) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float4 power = *reinterpret_cast<const float4 *>(&lds.column_power[wave][8 * j + 4 * half]);
+                row_sums[4 * j + 0] = __builtin_fmaf(acc[0][4 * j + 0], power.x, row_sums[4 * j + 0]);
+                row_sums[4 * j + 1] = __builtin_fmaf(acc[0][4 * j + 1], power.y, row_sums[4 * j + 1]);
+                row_sums[4 * j + 2] = __builtin_fmaf(acc[0][4 * j + 2], power.z, row_sums[4 * j + 2]);
+                row_sums[4 * j + 3] = __builtin_fmaf(acc[0][4 * j + 3], power.w, row_sums[4 * j + 3]);
+            }
+            acc[0] = zero;
+            asm volatile("" ::: "memory");
+        }
+        if (kb == 0) {
+            // the item is complete: scale by 2^(E[r] + S[n]) (APART: the sums have their 2^S) and store
             const bool second = tile >= a.n_tiles;
             const int n0 = (second ? tile - a.n_tiles : tile) * FWD_TN + 32 * wave;
             uint16_t * const y = second ? a.y_second : a.y;
@@ -482,13 +504,21 @@ TGO_DEVICE void group_task(const ForwardArgs & a, GroupLds<TYPE> & lds, GroupBar
             for (int r = 0; r < R; ++r) {
                 const int first = row_start + 32 * r;
                 if (first < row_end) {
-                    scale_sums(acc[r], lds.row_power[32 * r + l32_here], half_here);
+                    if constexpr (APART) {
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) {
+                            acc[r][v] = row_sums[v] * lds.row_power[l32_here];
+                        }
+                    } else {
+                        scale_sums(acc[r], lds.row_power[32 * r + l32_here], half_here);
+                    }
                     store_rows_32xn<1>(&acc[r], y + static_cast<int64_t>(first) * a.out_stride + n0, a.out_stride, row_end - first,
                                        a.out_features - n0, lane_here);
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 acc[r] = zero;
             }
+            row_sums = zero;
             asm volatile("" ::: "memory");
             ++tile;
         }
