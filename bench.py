@@ -361,7 +361,7 @@ def measure_decode(args, device) -> dict:
         if launches:
             report["skewed_256_rows_57_experts"] = {
                 "weight_MB": skew_bytes / 1e6,
-                "kernel_family": _native.lib.tgo_forward_kernel_family(sum(sizes), experts).decode(),
+                "kernel_family": _native.forward_kernel_for(synth.IQ2_S, sum(sizes), 2048, 512, len(sizes), 2),
                 "gemv_kernel_us": kernel_ms / launches * 1e3,
                 "GBps_gemv_kernel": skew_bytes / (kernel_ms / launches * 1e-3) / 1e9,
             }
@@ -479,7 +479,8 @@ def measure_dense_cell(args, device, qtype, n, m, k=2048, weight=None) -> dict:
         record[label + "_TFLOPs"] = round(2.0 * m * n * k / total / 1e6, 1)
         if m <= 16:
             record[label + "_weight_GBps"] = round(weight.numel() / total / 1e3, 1)
-    record["forward_operands"] = _native.forward_operand_for(qtype, m, n, 1) if m > 32 else "int8 (GEMV family)"
+    kernels_of_call = _native.forward_kernel_for(qtype, m, k, n)
+    record["forward_operands"] = _native.forward_operand_for(qtype, m, n, 1) if kernels_of_call == "mfma" else f"exact ({kernels_of_call} kernels)"
     return record
 
 

@@ -38,7 +38,7 @@ extern "C" {
 
 /* Library version (major*10000 + minor*100 + patch): TGO_VERSION of the header that the library was built with.  It grows with
  * every change of this file that a caller can see. */
-#define TGO_VERSION 113
+#define TGO_VERSION 114
 int tgo_version(void);
 
 /* Message of the last failure on the calling thread ("" if none). Host pointer. */
@@ -343,11 +343,15 @@ int tgo_grouped_mmq_grad_input_weighted(const void * grad_tokens_bf16, const int
                                         int64_t out_features, int64_t in_features, int64_t num_experts,
                                         int64_t num_groups, int quant_type, void * stream);
 
-/* Name of the kernel family the forward entry points pick for a shape ("mfma" or "gemv");
- * host pointer to a static string.  Lets callers and benchmarks label what they measure.  Beyond the
- * decode regime the answer is "mfma" by rows alone; the 16-row decode kernel still takes calls of few rows
- * per group, or of up to 128 dense rows, by format, size and alignment. */
+/* Whether rows and groups alone (num_groups 0: a dense call) put a forward call in the decode regime, "gemv", or not, "mfma".
+ * tgo_forward_kernel_for: the kernels that a call of this format and shape runs under the current setting: "gemv" (dot products,
+ * weights unpacked for every row), "tiles" (decode kernel for tasks of up to 16 rows, which also takes calls beyond the decode regime:
+ * few rows per group, up to 128 dense rows) or "mfma" (matrix-core kernels, with the operands that tgo_forward_operand_for names; the
+ * other two have exact integer operands).  `projections`: 2 for a pair.  NULL for sizes that the forward entry points refuse.
+ * Host pointers to static strings; for callers and benchmarks that label what they measure. */
 const char * tgo_forward_kernel_family(int64_t rows, int64_t num_groups);
+const char * tgo_forward_kernel_for(int quant_type, int64_t rows, int64_t in_features, int64_t out_features, int64_t num_groups,
+                                    int projections);
 
 /* ---- optional per-kernel timing (benchmarks only) ---------------------------------------
  * While enabled, every kernel launch of the library is bracketed by a pair of HIP events
@@ -391,8 +395,8 @@ int tgo_profile_read(int kernel, double * total_ms, int64_t * launches);
  * KiB: tgo_q8_workspace_unpack follows that tag, and tgo_mmq_forward_prepared turns its outputs into NaN when the
  * setting was changed between quantizing a workspace and using it.  A call reads the setting once.
  * tgo_forward_operand() returns the current setting; tgo_forward_operand_for() the kind (never AUTO) that a forward
- * call of this format and shape would use under it on those kernels (`projections`: 2 for a pair); under AUTO
- * some calls take the 16-row decode kernel instead (see tgo_forward_kernel_family), whose operands are exact.  No counterpart in the reference. */
+ * call of this format and shape would use under it on the matrix-core kernels (`projections`: 2 for a pair);
+ * tgo_forward_kernel_for says whether it runs on those.  No counterpart in the reference. */
 #define TGO_OPERAND_INT8 0
 #define TGO_OPERAND_HALF 1
 #define TGO_OPERAND_AUTO 2

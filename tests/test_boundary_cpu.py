@@ -55,6 +55,42 @@ def test_sizes_and_block_bytes(package):
     assert lib.tgo_task_workspace_bytes(100, 7) >= 4 * (1 + 3 * (13 + 7))
 
 
+def test_the_kernels_of_a_call_are_named(package):
+    """tgo_forward_kernel_for follows format, size, groups and setting, where tgo_forward_kernel_family sees rows and groups only."""
+    _, native, _, _ = package
+    assert native.forward_kernel_for(14, 64, 4096, 4096) == "tiles"
+    assert native.forward_kernel_for(14, 64, 4096, 4099) == "mfma"         # no whole tiles of 16 weight rows
+    assert native.forward_kernel_for(14, 64, 1024, 2048) == "mfma"         # fewer than four million weights
+    assert native.forward_kernel_for(14, 129, 4096, 4096) == "mfma"
+    assert native.forward_kernel_for(14, 1, 4096, 4096) == "gemv"
+    assert native.forward_kernel_for(11, 1, 8192, 28672) == "tiles"
+    assert native.forward_kernel_for(22, 8 * 64, 2048, 512, 64, 2) == "tiles"
+    assert native.forward_kernel_for(22, 64 * 64, 2048, 512, 64, 2) == "mfma"
+    assert native.forward_kernel_for(22, 8, 2048, 512, 256, 2) == "gemv"
+    native.set_forward_operand("int8")
+    try:
+        assert native.forward_kernel_for(14, 64, 4096, 4096) == "mfma"     # the kind was asked for
+        assert native.forward_kernel_for(22, 8 * 64, 2048, 512, 64, 2) == "mfma"
+    finally:
+        native.set_forward_operand("auto")
+    for sizes in ((10, 1, 256, 16), (12, 0, 256, 16), (12, 1, 100, 16), (12, 1, 256, 0)):
+        with pytest.raises(RuntimeError):
+            native.forward_kernel_for(*sizes)
+
+
+def test_an_entry_point_reads_the_operand_setting_once():
+    """The rules take the setting as an argument, and no function of the C ABI reads it twice: a change by another thread falls
+    before or after a call, not into it."""
+    csrc = ROOT / "torch-ggml-ops_amd" / "csrc"
+    read = "forward_operand_setting()"
+    for path in sorted(csrc.glob("*.h")):
+        assert path.read_text().replace(f"int {read};", "").count(read) == 0, path.name
+    functions = re.split(r"\n}\n|; }\n", (csrc / "tgo_api.hip").read_text())
+    assert all(body.count(read) <= 1 for body in functions)
+    others = [p for p in csrc.glob("*.hip") if p.name not in ("tgo_api.hip", "tgo_aux.hip")]
+    assert all(read not in p.read_text() for p in others)
+
+
 def test_c_abi_rejects_bad_arguments_before_launch(package):
     _, native, _, _ = package
     lib = native.lib

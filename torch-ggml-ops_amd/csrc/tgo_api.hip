@@ -213,7 +213,7 @@ int tgo_set_forward_operand(int operand) {
 int tgo_forward_operand(void) { return tgo::forward_operand_setting(); }
 
 int tgo_forward_operand_for(int quant_type, int64_t rows, int64_t out_features, int projections) {
-    return tgo::forward_operand_kind(quant_type, rows, out_features, projections);
+    return tgo::forward_operand_kind(tgo::forward_operand_setting(), quant_type, rows, out_features, projections);
 }
 
 int tgo_profile_read(int kernel, double * total_ms, int64_t * launches) {
@@ -273,6 +273,17 @@ const char * tgo_forward_kernel_family(int64_t rows, int64_t num_groups) {
     return tgo::use_gemv(rows, num_groups) ? "gemv" : "mfma";
 }
 
+const char * tgo_forward_kernel_for(int quant_type, int64_t rows, int64_t in_features, int64_t out_features, int64_t num_groups,
+                                    int projections) {
+    if (check_matmul_shape(rows, in_features, out_features, quant_type) != TGO_OK) {
+        return nullptr;
+    }
+    const int setting = tgo::forward_operand_setting();
+    const bool tiles = num_groups <= 0 ? tgo::dense_takes_tiles(setting, rows, in_features, out_features, quant_type)
+                                       : tgo::grouped_takes_tiles(setting, rows, num_groups, in_features, out_features, quant_type, projections);
+    return tiles ? "tiles" : tgo_forward_kernel_family(rows, num_groups);
+}
+
 int tgo_dequant_bf16(const void * packed, void * out_bf16, int64_t rows, int64_t in_features,
                      int quant_type, void * stream) {
     TGO_TRY(check_matmul_shape(rows, in_features, 1, quant_type));
@@ -305,7 +316,7 @@ int tgo_quantize_q8_1_as(const void * input_bf16, void * workspace, int64_t rows
 
 int tgo_quantize_q8_1(const void * input_bf16, void * workspace, int64_t rows, int64_t in_features,
                       void * stream) {
-    return tgo_quantize_q8_1_as(input_bf16, workspace, rows, in_features, tgo::forward_operand_kind(0), stream);
+    return tgo_quantize_q8_1_as(input_bf16, workspace, rows, in_features, tgo::forward_operand_kind(tgo::forward_operand_setting(), 0), stream);
 }
 
 int tgo_q8_workspace_unpack(const void * workspace, void * q_int8, void * d_f32, void * sum_f32,
@@ -316,7 +327,8 @@ int tgo_q8_workspace_unpack(const void * workspace, void * q_int8, void * d_f32,
         return fail(TGO_ERR_INVALID, "output pointers must not be null");
     }
     const tgo::Q8Workspace view =
-        tgo::q8_workspace_view(const_cast<void *>(workspace), rows, in_features, tgo::use_gemv(rows, 0), tgo::forward_operand_kind(0));
+        tgo::q8_workspace_view(const_cast<void *>(workspace), rows, in_features, tgo::use_gemv(rows, 0),
+                               tgo::forward_operand_kind(tgo::forward_operand_setting(), 0));
     return check_hip(tgo::launch_q8_unpack(view, static_cast<int8_t *>(q_int8), static_cast<float *>(d_f32),
                                            static_cast<float *>(sum_f32), rows, in_features,
                                            static_cast<hipStream_t>(stream)),
@@ -366,7 +378,8 @@ int tgo_mmq_forward_scratch(const void * input_bf16, const void * packed, void *
     TGO_TRY(check_pointer(workspace, "workspace"));
     TGO_TRY(check_scratch(scratch, rows, in_features, out_features, quant_type));
     hipStream_t hip_stream = static_cast<hipStream_t>(stream);
-    const bool tiles = tgo::dense_takes_tiles(packed, rows, in_features, out_features, quant_type);
+    const int setting = tgo::forward_operand_setting();
+    const bool tiles = tgo::dense_takes_tiles(setting, rows, in_features, out_features, quant_type);
     if (!tiles && tgo::gemv_fuses(quant_type, rows, 0)) {
         // one launch: the decode-regime kernels of these formats quantize their activations themselves
         return check_hip(tgo::launch_mmq_gemv_fused(static_cast<const uint8_t *>(packed), nullptr, 0,
@@ -377,7 +390,7 @@ int tgo_mmq_forward_scratch(const void * input_bf16, const void * packed, void *
                          "mmq_forward launch");
     }
     const tgo::Q8Workspace view = tgo::q8_workspace_view(workspace, rows, in_features, tiles || tgo::use_gemv(rows, 0),
-                                                         tgo::forward_operand_kind(quant_type, rows, out_features, 1));
+                                                         tgo::forward_operand_kind(setting, quant_type, rows, out_features, 1));
     TGO_TRY(check_hip(tgo::launch_quantize_q8_1(static_cast<const uint16_t *>(input_bf16), view, rows, in_features,
                                                 hip_stream),
                       "quantize_q8_1 launch"));
@@ -438,7 +451,7 @@ int tgo_mmq_forward_prepared_scratch(const void * workspace, const void * packed
 int tgo_mmq_forward_prepared(const void * workspace, const void * packed, void * output_bf16, int64_t rows,
                              int64_t in_features, int64_t out_features, int quant_type, void * stream) {
     return tgo_mmq_forward_prepared_as(workspace, packed, output_bf16, rows, in_features, out_features, quant_type,
-                                       tgo::forward_operand_kind(0), stream);
+                                       tgo::forward_operand_kind(tgo::forward_operand_setting(), 0), stream);
 }
 
 int tgo_mmq_multi_forward(const void * input_bf16, int count, const void * const * packed, void * const * outputs_bf16,
@@ -604,6 +617,7 @@ int tgo_lm_head_loss(const void * hidden_bf16, const void * packed, const int64_
     }
     hipStream_t hip_stream = static_cast<hipStream_t>(stream);
     const int64_t chunk_limit = std::min({chunk_rows, rows, HEAD_CHUNK_LIMIT});
+    const int setting = tgo::forward_operand_setting();
     const HeadWorkspace w = head_workspace(rows, in_features, out_features, chunk_limit, quant_type, gradient);
     uint8_t * const base = static_cast<uint8_t *>(workspace);
     uint16_t * const logits = reinterpret_cast<uint16_t *>(base + w.logits);
@@ -616,7 +630,7 @@ int tgo_lm_head_loss(const void * hidden_bf16, const void * packed, const int64_
         const int r = static_cast<int>(chunk), n = static_cast<int>(out_features), k = static_cast<int>(in_features);
         const bool gemv = tgo::use_gemv(chunk, 0);
         const tgo::Q8Workspace view =
-            tgo::q8_workspace_view(base, chunk, in_features, gemv, tgo::forward_operand_kind(quant_type, chunk, out_features, 1));
+            tgo::q8_workspace_view(base, chunk, in_features, gemv, tgo::forward_operand_kind(setting, quant_type, chunk, out_features, 1));
         TGO_TRY(check_hip(tgo::launch_quantize_q8_1(static_cast<const uint16_t *>(hidden_bf16) + begin * in_features, view, chunk,
                                                     in_features, hip_stream),
                           "quantize_q8_1 launch"));
@@ -685,7 +699,9 @@ static int grouped_forward(const void * input_bf16, const int64_t * row_index, i
                                                  static_cast<uint16_t *>(output_second), rows * out_features, hip_stream),
                          "swiglu launch");
     };
-    const bool tiles = tgo::grouped_takes_tiles(packed_first, packed_second, rows, num_groups, in_features, out_features, quant_type);
+    const int setting = tgo::forward_operand_setting();
+    const int projections = packed_second != nullptr ? 2 : 1;
+    const bool tiles = tgo::grouped_takes_tiles(setting, rows, num_groups, in_features, out_features, quant_type, projections);
     const bool gemv = tiles || tgo::use_gemv(rows, num_groups);
     if (gemv && !tiles && tgo::gemv_fuses(quant_type, rows, num_groups)) {
         // one launch: the decode-regime kernels of these formats quantize their activations and find their tasks
@@ -701,7 +717,7 @@ static int grouped_forward(const void * input_bf16, const int64_t * row_index, i
                          "grouped mmq_forward launch"));
         return swiglu ? finish_swiglu() : TGO_OK;
     }
-    const int operand_kind = tgo::forward_operand_kind(quant_type, rows, out_features, packed_second != nullptr ? 2 : 1);
+    const int operand_kind = tgo::forward_operand_kind(setting, quant_type, rows, out_features, projections);
     // (the scaled-operand kernel without the epilogue plus the elementwise pass costs less than the other kinds'
     // kernels lose to it)
     const bool fused = swiglu && !gemv && operand_kind != tgo::OPERAND_SCALED;

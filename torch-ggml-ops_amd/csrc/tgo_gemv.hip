@@ -1627,7 +1627,7 @@ hipError_t launch_mmq_gemv(const uint8_t * packed, const uint8_t * packed_second
         return hipErrorInvalidValue;   // these kernels read the row-major activation layout
     }
     if (tasks == nullptr && rows <= GEMV_DENSE_ROWS &&
-        gemv_takes_tiles(packed, packed_second, rows, 0, in_features, out_features, quant_type)) {
+        gemv_takes_tiles(rows, 0, in_features, out_features, quant_type)) {
         return launch_mmq_gemv_tiles(packed, packed_second, bytes_per_expert, ws, output, output_second, tasks, rows, in_features,
                                      out_features, quant_type, false, stream, output_stride);
     }

@@ -21,8 +21,8 @@ namespace tgo {
 //                   tiles spread a small call over more CUs).
 // `quant_type` 0 stands for a workspace that is quantized without knowing the format it will be used with
 // (tgo_quantize_q8_1, tgo_mmq_forward_prepared): int8 unless exact fp16 is forced.  The activation workspace is
-// written for one kind of operand and records which (Q8Workspace::tag); it must be consumed as that kind.  A call
-// reads the setting once, so a change by another thread never splits a call between two kinds.
+// written for one kind of operand and records which (Q8Workspace::tag); it must be consumed as that kind.  An entry
+// point reads the setting once and hands it to the rules below, so a change by another thread never splits a call.
 enum ForwardOperand : int { OPERAND_INT8 = 0, OPERAND_HALF = 1, OPERAND_AUTO = 2, OPERAND_SCALED = 3 };
 int forward_operand_setting();
 void set_forward_operand_setting(int operand);
@@ -34,10 +34,9 @@ static constexpr bool scaled_forward_format(int quant_type) {
 // so half a chip's worth is where it starts to beat the kernels with smaller tiles (dense 512 x 4096: 64 tiles, a
 // tie; 4096 x 2048: 256 tiles, 12 % faster).
 constexpr int64_t SCALED_AUTO_MIN_TILES = 128;
-// The operand kind a call of this format and size uses under the current setting (never OPERAND_AUTO).  Grouped
+// The operand kind a call of this format and size uses under `setting` (never OPERAND_AUTO).  Grouped
 // calls pass their total rows: the tiles of a ragged list are at least that many.
-static inline int forward_operand_kind(int quant_type, int64_t rows = 0, int64_t out_features = 0, int projections = 1) {
-    const int setting = forward_operand_setting();
+static inline int forward_operand_kind(int setting, int quant_type, int64_t rows = 0, int64_t out_features = 0, int projections = 1) {
     const int exact = quant_type == 22 ? OPERAND_HALF : OPERAND_INT8;
     if (setting == OPERAND_SCALED) {
         return scaled_forward_format(quant_type) ? OPERAND_SCALED : exact;
@@ -205,12 +204,11 @@ static inline bool use_gemv(int64_t rows, int64_t groups) {
     return groups <= 0 ? rows <= GEMV_DENSE_ROWS : rows <= 4 * groups;
 }
 
-// Whether the layout of the kernel for tasks of several rows (tgo_gemv_tiles.hip) allows a call: whole tiles of 16 weight rows, aligned weights, offsets within a tile of 32 bits, and four
-// million weights that are read.
-static inline bool tiles_fit(const void * packed, const void * packed_second, int64_t rows, int64_t groups, int64_t in_features,
-                             int64_t out_features) {
-    if (out_features % 16 != 0 || (reinterpret_cast<uintptr_t>(packed) | reinterpret_cast<uintptr_t>(packed_second)) % 16 != 0 ||
-        in_features > (INT64_C(1) << 22) || rows > (1 << 24)) {
+// Whether the layout of the kernel for tasks of several rows (tgo_gemv_tiles.hip) allows a call: whole tiles of 16 weight rows (with
+// them every expert is 16-byte aligned, as the entry points demand of the weights), offsets within a tile of 32 bits, and four million
+// weights that are read.
+static inline bool tiles_fit(int64_t rows, int64_t groups, int64_t in_features, int64_t out_features) {
+    if (out_features % 16 != 0 || in_features > (INT64_C(1) << 22) || rows > (1 << 24)) {
         return false;
     }
     const int64_t matrices = groups <= 0 ? 1 : rows < groups ? rows : groups;
@@ -230,9 +228,8 @@ static inline bool tiles_fit(const void * packed, const void * packed_second, in
 //    65 us for Q6_K), Q4_K from four.  Smaller ones: Q3_K and IQ2_S from five rows, Q6_K from nine, Q4_K and Q5_K beyond 16.
 constexpr int GEMV_TILES_ROWS = 16;              // rows of its tasks
 constexpr int64_t GEMV_TILES_WORKGROUPS = 384;   // workgroups that a launch should have for a wave to take four tiles of 16 weight rows instead of two
-static inline bool gemv_takes_tiles(const void * packed, const void * packed_second, int64_t rows, int64_t groups, int64_t in_features,
-                                    int64_t out_features, int quant_type) {
-    if (!use_gemv(rows, groups) || !tiles_fit(packed, packed_second, rows, groups, in_features, out_features)) {
+static inline bool gemv_takes_tiles(int64_t rows, int64_t groups, int64_t in_features, int64_t out_features, int quant_type) {
+    if (!use_gemv(rows, groups) || !tiles_fit(rows, groups, in_features, out_features)) {
         return false;
     }
     const int64_t super_blocks = in_features / 256;
@@ -259,11 +256,11 @@ static inline bool gemv_takes_tiles(const void * packed, const void * packed_sec
 // matrix-core kernel -> this one): 2048 x 2048 Q4_K 64 rows 23 -> 10, 128 rows 16 -> 11; Q6_K 128 rows 27 -> 15; 5120 x 1024 IQ2_S 128
 // rows 18 -> 18; 4096 x 4096 Q3_K 64 rows 23 -> 17, 96 rows 28 -> 24, Q5_K 96 rows 24 -> 24, Q6_K 64 rows 28 -> 22, 80 rows 30 -> 31; 11008 x 4096
 // 64 rows Q3_K 42 -> 32, Q4_K 34 -> 30, 80 rows 38 -> 37; 28672 x 8192 34 rows Q4_K 103 -> 102, Q6_K 140 -> 160.
-static inline bool dense_takes_tiles(const void * packed, int64_t rows, int64_t in_features, int64_t out_features, int quant_type) {
+static inline bool dense_takes_tiles(int setting, int64_t rows, int64_t in_features, int64_t out_features, int quant_type) {
     if (use_gemv(rows, 0)) {
-        return gemv_takes_tiles(packed, nullptr, rows, 0, in_features, out_features, quant_type);
+        return gemv_takes_tiles(rows, 0, in_features, out_features, quant_type);
     }
-    if (forward_operand_setting() != OPERAND_AUTO || !tiles_fit(packed, nullptr, rows, 0, in_features, out_features)) {
+    if (setting != OPERAND_AUTO || !tiles_fit(rows, 0, in_features, out_features)) {
         return false;
     }
     const int64_t weights = out_features * in_features;
@@ -282,15 +279,15 @@ static inline bool dense_takes_tiles(const void * packed, int64_t rows, int64_t 
 // Q4_K 34.7 -> 35.8, where the down projection (512 x 2048) wins, 25.4 -> 20.7.
 // Scaled operands: 512 columns of K to 2048, 12 rows Q3_K 72 -> 52, Q4_K 62 -> 48, Q5_K 69 -> 54, Q6_K 90 -> 82, IQ2_S 70 -> 68.
 // Not where the operand kind was forced: the caller asked for that kind's kernels.
-static inline bool grouped_takes_tiles(const void * packed, const void * packed_second, int64_t rows, int64_t groups, int64_t in_features,
-                                       int64_t out_features, int quant_type) {
+static inline bool grouped_takes_tiles(int setting, int64_t rows, int64_t groups, int64_t in_features, int64_t out_features,
+                                       int quant_type, int projections) {
     if (use_gemv(rows, groups)) {
-        return gemv_takes_tiles(packed, packed_second, rows, groups, in_features, out_features, quant_type);
+        return gemv_takes_tiles(rows, groups, in_features, out_features, quant_type);
     }
-    if (forward_operand_setting() != OPERAND_AUTO || !tiles_fit(packed, packed_second, rows, groups, in_features, out_features)) {
+    if (setting != OPERAND_AUTO || !tiles_fit(rows, groups, in_features, out_features)) {
         return false;
     }
-    const bool scaled = forward_operand_kind(quant_type, rows, out_features, packed_second != nullptr ? 2 : 1) == OPERAND_SCALED;
+    const bool scaled = forward_operand_kind(setting, quant_type, rows, out_features, projections) == OPERAND_SCALED;
     const int64_t most = quant_type == 14 ? (scaled ? 8 : 32) : quant_type == 22 ? (scaled ? 8 : 12) : scaled ? 12 : 16;
     return rows <= most * groups;
 }

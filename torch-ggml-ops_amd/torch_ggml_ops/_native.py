@@ -48,6 +48,8 @@ lib.tgo_task_workspace_bytes.argtypes = [_i64, _i64]
 lib.tgo_task_workspace_bytes.restype = _i64
 lib.tgo_forward_kernel_family.argtypes = [_i64, _i64]
 lib.tgo_forward_kernel_family.restype = ctypes.c_char_p
+lib.tgo_forward_kernel_for.argtypes = [_int, _i64, _i64, _i64, _i64, _int]
+lib.tgo_forward_kernel_for.restype = ctypes.c_char_p
 lib.tgo_dequant_bf16.argtypes = [_p, _p, _i64, _i64, _int, _p]
 lib.tgo_quantize_q8_1.argtypes = [_p, _p, _i64, _i64, _p]
 lib.tgo_q8_workspace_unpack.argtypes = [_p, _p, _p, _p, _i64, _i64, _p]
@@ -111,6 +113,7 @@ EXPORTS = (
     "tgo_q8_workspace_bytes",
     "tgo_task_workspace_bytes",
     "tgo_forward_kernel_family",
+    "tgo_forward_kernel_for",
     "tgo_dequant_bf16",
     "tgo_quantize_q8_1",
     "tgo_q8_workspace_unpack",
@@ -167,8 +170,19 @@ def forward_operand() -> str:
 
 
 def forward_operand_for(quant_type: int, rows: int, out_features: int, projections: int = 1) -> str:
-    """The kind a forward call of this format and shape uses under the current setting (never "auto")."""
+    """The kind a forward call of this format and shape uses under the current setting on the matrix-core kernels (never
+    "auto"); ``forward_kernel_for`` says whether it runs on those."""
     return {value: name for name, value in OPERANDS.items()}[lib.tgo_forward_operand_for(quant_type, rows, out_features, projections)]
+
+
+def forward_kernel_for(
+    quant_type: int, rows: int, in_features: int, out_features: int, num_groups: int = 0, projections: int = 1
+) -> str:
+    """The kernels a forward call of this format and shape runs: "gemv", "tiles" (both decode kernels, exact operands) or "mfma"."""
+    name = lib.tgo_forward_kernel_for(quant_type, rows, in_features, out_features, num_groups, projections)
+    if name is None:
+        raise RuntimeError(lib.tgo_last_error().decode())
+    return name.decode()
 
 
 def profile_read(kernel: str) -> tuple[float, int]:
