@@ -132,7 +132,9 @@ int tgo_mmq_forward_static(const void * input_bf16, const void * packed, void * 
 /* The second half of tgo_mmq_forward alone: `workspace` already holds the q8_1 form of the
  * activations (written by tgo_quantize_q8_1 for the same rows and in_features) and is only read.
  * Several projections of one input (q/k/v, shared gate/up) quantize once and call this once per
- * weight; results are bit-identical to tgo_mmq_forward.  No counterpart in the reference, which
+ * weight; results are bit-identical to tgo_mmq_forward wherever that call has exact operands of the
+ * workspace's kind (int8; tgo_forward_operand_for) or runs on the decode kernels (tgo_forward_kernel_for),
+ * whose sums do not depend on the workspace's layout.  No counterpart in the reference, which
  * quantizes inside every dense call (csrc/mmq_hip.cu:643-665) and names the reuse as its next
  * step (docs/mmq_fwd_optimization.md:299-307). */
 int tgo_mmq_forward_prepared(const void * workspace, const void * packed, void * output_bf16,

@@ -142,3 +142,40 @@ def test_prepared_rejects_mismatched_workspace(ops):
         tgo.mmq_prepared(workspace, weight, 8, 512, 13, 32)
     with pytest.raises(RuntimeError, match="multiple of 256"):
         tgo.quantize_q8_1(random_bf16((4, 100), seed=3))
+
+
+@pytest.mark.parametrize("qname", tuple(QTYPES))
+@pytest.mark.parametrize("rows,n,k", [(33, 4096, 1024), (48, 2048, 2304), (64, 16400, 768), (61, 2064, 4096), (128, 2048, 2048)])
+def test_rows_beyond_the_decode_regime_equal_mmq_bit_for_bit(ops, oracle, qname, rows, n, k):
+    """Matrices of four million weights, which ``mmq`` gives to the 16-row decode kernel for up to 128 rows: a workspace in either
+    exact tile layout, and ``mmq_multi``, give the same bits (the kernel's sums do not depend on how its activations are laid
+    out), also a key and value of one shape and a projection that takes the matrix-core kernels."""
+    from torch_ggml_ops import _native, prepared
+
+    tgo, synth = ops
+    qtype = QTYPES[qname]
+    assert _native.forward_kernel_for(qtype, rows, k, n) == "tiles"
+    host = synth.random_packed_weight(qtype, (n,), k, seed=qtype + rows)
+    weight = host.cuda()
+    x = random_bf16((rows, k), seed=rows)
+    expected = tgo.mmq(x, weight, qtype, n)
+    assert_matches_f32_reference(expected, oracle.mmq_forward(qtype, bits(x), host.numpy(), n, k))
+    for kind in ("int8", "half"):
+        actual = tgo.mmq_prepared(tgo.quantize_q8_1(x, kind), weight, rows, k, qtype, n, kind)
+        torch.testing.assert_close(actual, expected, rtol=0, atol=0)
+    other = synth.random_packed_weight(qtype, (n,), k, seed=1).cuda()
+    small = synth.random_packed_weight(qtype, (n // 16 + 1,), k, seed=2).cuda()
+    widths = (n, n, n // 16 + 1)
+    assert _native.forward_kernel_for(qtype, rows, k, widths[2]) == "mfma"
+    if prepared.multi_operand([qtype] * 3, rows, widths) != "scaled":
+        outputs = tgo.mmq_multi(x, (weight, other, small), [qtype] * 3, widths)
+        for output, w, width in zip(outputs, (weight, other, small), widths):
+            torch.testing.assert_close(output, tgo.mmq(x, w, qtype, width), rtol=0, atol=0)
+
+
+def test_another_layout_than_the_workspaces_is_nan_on_the_decode_kernel_too(ops):
+    tgo, synth = ops
+    rows, n, k = 40, 4096, 1024
+    weight = synth.random_packed_weight(12, (n,), k, seed=3).cuda()
+    workspace = tgo.quantize_q8_1(random_bf16((rows, k), seed=4), operand="half")
+    assert torch.isnan(tgo.mmq_prepared(workspace, weight, rows, k, 12, n, operand="int8").float()).all()

@@ -339,7 +339,8 @@ int64_t tgo_forward_scratch_bytes(int64_t rows, int64_t in_features, int64_t out
     if (rows <= 0 || in_features <= 0 || out_features <= 0 || tgo::use_gemv(rows, 0)) {
         return 0;
     }
-    // (a prepared workspace may hold either kind of exact operands)
+    // (a prepared workspace may hold either kind of exact operands; the setting, by which some calls use no ranges, may change before
+    // the call)
     return std::max(tgo::forward_partial_bytes(rows, in_features, out_features, quant_type, tgo::OPERAND_INT8),
                     tgo::forward_partial_bytes(rows, in_features, out_features, quant_type, tgo::OPERAND_HALF));
 }
@@ -350,12 +351,16 @@ int tgo_mmq_forward(const void * input_bf16, const void * packed, void * output_
                                    stream);
 }
 
-// The matmul half of a dense call of the kernel family that `view` was quantized for.
-static hipError_t launch_dense(const void * packed, const tgo::Q8Workspace & view, void * output_bf16, void * scratch, int64_t rows,
+// The matmul half of a dense call on a workspace: the kernels that tgo_mmq_forward takes for these sizes (`tiles`: dense_takes_tiles),
+// whose results then are the same bits, unless the workspace holds scaled operands.
+static hipError_t launch_dense(const void * packed, const tgo::Q8Workspace & view, bool tiles, void * output_bf16, void * scratch, int64_t rows,
                                int64_t in_features, int64_t out_features, int quant_type, hipStream_t stream) {
     const uint8_t * const weights = static_cast<const uint8_t *>(packed);
     uint16_t * const output = static_cast<uint16_t *>(output_bf16);
     const int r = static_cast<int>(rows), k = static_cast<int>(in_features), n = static_cast<int>(out_features);
+    if (tiles && !view.scaled_tiles()) {
+        return tgo::launch_mmq_gemv_tiles(weights, nullptr, 0, view, output, nullptr, nullptr, r, k, n, quant_type, false, stream);
+    }
     return view.by_rows() ? tgo::launch_mmq_gemv(weights, nullptr, 0, view, output, nullptr, nullptr, r, k, n, quant_type, stream, 0)
                           : tgo::launch_mmq_forward(weights, nullptr, 0, view, output, nullptr, nullptr, r, k, n, quant_type, stream, 0,
                                                     static_cast<float *>(scratch));
@@ -394,13 +399,7 @@ int tgo_mmq_forward_scratch(const void * input_bf16, const void * packed, void *
     TGO_TRY(check_hip(tgo::launch_quantize_q8_1(static_cast<const uint16_t *>(input_bf16), view, rows, in_features,
                                                 hip_stream),
                       "quantize_q8_1 launch"));
-    if (tiles) {
-        return check_hip(tgo::launch_mmq_gemv_tiles(static_cast<const uint8_t *>(packed), nullptr, 0, view, static_cast<uint16_t *>(output_bf16),
-                                                    nullptr, nullptr, static_cast<int>(rows), static_cast<int>(in_features),
-                                                    static_cast<int>(out_features), quant_type, false, hip_stream),
-                         "mmq_forward launch");
-    }
-    return check_hip(launch_dense(packed, view, output_bf16, scratch, rows, in_features, out_features, quant_type, hip_stream),
+    return check_hip(launch_dense(packed, view, tiles, output_bf16, scratch, rows, in_features, out_features, quant_type, hip_stream),
                      "mmq_forward launch");
 }
 
@@ -423,13 +422,8 @@ int tgo_mmq_forward_static(const void * input_bf16, const void * packed, void * 
                            stream);
 }
 
-int tgo_mmq_forward_prepared_as(const void * workspace, const void * packed, void * output_bf16, int64_t rows,
-                                int64_t in_features, int64_t out_features, int quant_type, int operand, void * stream) {
-    return tgo_mmq_forward_prepared_scratch(workspace, packed, output_bf16, nullptr, rows, in_features, out_features, quant_type,
-                                            operand, stream);
-}
-int tgo_mmq_forward_prepared_scratch(const void * workspace, const void * packed, void * output_bf16, void * scratch, int64_t rows,
-                                     int64_t in_features, int64_t out_features, int quant_type, int operand, void * stream) {
+static int prepared_forward(int setting, const void * workspace, const void * packed, void * output_bf16, void * scratch, int64_t rows,
+                            int64_t in_features, int64_t out_features, int quant_type, int operand, void * stream) {
     TGO_TRY(check_matmul_shape(rows, in_features, out_features, quant_type));
     TGO_TRY(check_pointer(workspace, "workspace"));
     TGO_TRY(check_pointer(packed, "packed_weight"));
@@ -438,7 +432,8 @@ int tgo_mmq_forward_prepared_scratch(const void * workspace, const void * packed
     TGO_TRY(check_scratch(scratch, rows, in_features, out_features, quant_type));
     const tgo::Q8Workspace view =
         tgo::q8_workspace_view(const_cast<void *>(workspace), rows, in_features, tgo::use_gemv(rows, 0), operand);
-    TGO_TRY(check_hip(launch_dense(packed, view, output_bf16, scratch, rows, in_features, out_features, quant_type,
+    const bool tiles = tgo::dense_takes_tiles(setting, rows, in_features, out_features, quant_type);
+    TGO_TRY(check_hip(launch_dense(packed, view, tiles, output_bf16, scratch, rows, in_features, out_features, quant_type,
                                    static_cast<hipStream_t>(stream)),
                       "mmq_forward_prepared launch"));
     // (the workspace was quantized by an earlier call: were it of another kind than this call was told, its layout
@@ -450,8 +445,21 @@ int tgo_mmq_forward_prepared_scratch(const void * workspace, const void * packed
 
 int tgo_mmq_forward_prepared(const void * workspace, const void * packed, void * output_bf16, int64_t rows,
                              int64_t in_features, int64_t out_features, int quant_type, void * stream) {
-    return tgo_mmq_forward_prepared_as(workspace, packed, output_bf16, rows, in_features, out_features, quant_type,
-                                       tgo::forward_operand_kind(tgo::forward_operand_setting(), 0), stream);
+    const int setting = tgo::forward_operand_setting();
+    return prepared_forward(setting, workspace, packed, output_bf16, nullptr, rows, in_features, out_features, quant_type,
+                            tgo::forward_operand_kind(setting, 0), stream);
+}
+
+int tgo_mmq_forward_prepared_as(const void * workspace, const void * packed, void * output_bf16, int64_t rows,
+                                int64_t in_features, int64_t out_features, int quant_type, int operand, void * stream) {
+    return prepared_forward(tgo::forward_operand_setting(), workspace, packed, output_bf16, nullptr, rows, in_features, out_features,
+                            quant_type, operand, stream);
+}
+
+int tgo_mmq_forward_prepared_scratch(const void * workspace, const void * packed, void * output_bf16, void * scratch, int64_t rows,
+                                     int64_t in_features, int64_t out_features, int quant_type, int operand, void * stream) {
+    return prepared_forward(tgo::forward_operand_setting(), workspace, packed, output_bf16, scratch, rows, in_features, out_features,
+                            quant_type, operand, stream);
 }
 
 int tgo_mmq_multi_forward(const void * input_bf16, int count, const void * const * packed, void * const * outputs_bf16,
@@ -476,10 +484,12 @@ int tgo_mmq_multi_forward(const void * input_bf16, int count, const void * const
     const tgo::Q8Workspace view = tgo::q8_workspace_view(workspace, rows, in_features, tgo::use_gemv(rows, 0), operand);
     TGO_TRY(check_hip(tgo::launch_quantize_q8_1(static_cast<const uint16_t *>(input_bf16), view, rows, in_features, hip_stream),
                       "quantize_q8_1 launch"));
+    const int setting = tgo::forward_operand_setting();
     for (int i = 0; i < count; ++i) {
+        const bool tiles = !view.scaled_tiles() && tgo::dense_takes_tiles(setting, rows, in_features, out_features[i], quant_types[i]);
         // two projections of one shape and format (key and value) side by side in one launch: alone, either leaves most of the
         // chip idle (2048 rows of 1024 x 4096: 39 us each, 43 us together); calls that take ranges of K fill it by themselves
-        const bool pair = i + 1 < count && !view.by_rows() && quant_types[i] == quant_types[i + 1] && out_features[i] == out_features[i + 1] &&
+        const bool pair = i + 1 < count && !view.by_rows() && !tiles && quant_types[i] == quant_types[i + 1] && out_features[i] == out_features[i + 1] &&
                           tgo::forward_partial_bytes(rows, in_features, out_features[i], quant_types[i], view.operand_kind()) == 0;
         if (pair) {
             TGO_TRY(check_hip(tgo::launch_mmq_forward(static_cast<const uint8_t *>(packed[i]), static_cast<const uint8_t *>(packed[i + 1]), 0,
@@ -490,7 +500,7 @@ int tgo_mmq_multi_forward(const void * input_bf16, int count, const void * const
                               "mmq_multi_forward launch"));
             ++i;
         } else {
-            TGO_TRY(check_hip(launch_dense(packed[i], view, outputs_bf16[i], scratch, rows, in_features, out_features[i], quant_types[i],
+            TGO_TRY(check_hip(launch_dense(packed[i], view, tiles, outputs_bf16[i], scratch, rows, in_features, out_features[i], quant_types[i],
                                            hip_stream),
                               "mmq_multi_forward launch"));
         }

@@ -48,7 +48,7 @@ struct TilesArgs {
     const uint8_t * packed;
     const uint8_t * packed_second;   // second projection of a pair, or nullptr
     int64_t bytes_per_expert;
-    // activations: int8 rows, block scales and block sums (LAYOUT_ROWS)
+    // activations: quants, block scales and block sums, in the kernel's LAYOUT
     const int8_t * qx;
     const float * dx;
     const float * sx;
@@ -60,6 +60,7 @@ struct TilesArgs {
     const int32_t * task_row_end;
     uint32_t row_bytes;
     int rows;
+    int rows_padded;
     int in_features;
     int out_features; // a multiple of 16
     int out_stride;   // values from one row of y to the next (out_features, or more)
@@ -295,7 +296,11 @@ struct TileWaveLds {
 // R: tiles of 16 weight rows per wave and pass over K (more tiles: fewer fetches of the activations, fewer workgroups).
 // SWIGLU (pair): half of a wave's tiles are gate rows, the other half the same rows of up; the workgroup stores
 // silu(gate) * up, both rounded to bf16 first, and the gate.
-template <int TYPE, int R, bool SWIGLU>
+// LAYOUT: of the activations.  The tile layouts are those of a workspace that is quantized before its weights are known
+// (tgo_quantize_q8_1) or for several of them, which the matrix-core kernels may read as well; dense calls only.  The same quants, scales
+// and sums reach LDS from any of them, so the results are the same bits.  2048 x 2048, 33 rows, us: Q6_K 22.4 by the matrix-core kernel's ranges
+// of K, 10.9 here from int8 tiles (10.9 from rows); IQ2_S 21.7 and 9.5; 4096 x 4096, 64 rows: Q4_K 18.6 and 17.2.
+template <int TYPE, int R, bool SWIGLU, int LAYOUT>
 __global__ __launch_bounds__(TILES_THREADS, 2) void mmq_gemv_tiles_kernel(const TilesArgs a) {
     using S = BlockPieces<TYPE>;
     constexpr int REGS = (16 * S::UNITS + 63) / 64;
@@ -303,6 +308,8 @@ __global__ __launch_bounds__(TILES_THREADS, 2) void mmq_gemv_tiles_kernel(const 
     constexpr int SIDES = SWIGLU ? 2 : 1;
     static_assert(R % SIDES == 0, "as many gate as up tiles");
     constexpr int COLUMN_TILES = R / SIDES;   // tiles of output columns per wave
+    constexpr bool BY_ROWS = LAYOUT == LAYOUT_ROWS, HALVES = LAYOUT == LAYOUT_HALF_TILES;
+    static_assert(BY_ROWS || LAYOUT == LAYOUT_INT8_TILES || HALVES, "the scaled tiles hold no quants");
     union WaveLds {
         TileWaveLds<TYPE> walk;
         alignas(16) float reduction[R * 16 * TILES_RED_PITCH];
@@ -405,34 +412,45 @@ __global__ __launch_bounds__(TILES_THREADS, 2) void mmq_gemv_tiles_kernel(const 
         __syncthreads();
     }
 
-    // ---- activations of a super-block: 16 lanes fetch a row, one super-block ahead in registers
-    constexpr int X_REGS = GEMV_TILES_ROWS / 4;
+    // ---- activations of a super-block, one super-block ahead in registers.  Rows: 16 lanes fetch a row.  Tiles: 16 lanes fetch the same
+    // 16 bytes of the task's 16 rows, which lie side by side (the task starts at row 0 or 16 of a tile, and the rows that it does not
+    // have are there as zeros).
+    constexpr int X_REGS = (HALVES ? 2 : 1) * GEMV_TILES_ROWS / 4;
     struct Incoming {
         uint4 bytes[X_REGS];
-        float4 scales;   // lane: row lane / 4, piece lane % 4 of its eight block scales and eight block sums
+        float4 scales;   // rows: row lane / 4, piece lane % 4 of its eight block scales and eight block sums; tiles: rows 4 (lane % 4) .. + 3
+                         // of block lane / 4 % 8, scales (lanes 0-31) or sums
     };
+    constexpr int TILE_STEP = HALVES ? 8 * 2048 : 8 * 1024;   // bytes of a 32-row tile's super-block
     uint32_t x_offset[X_REGS];
 #pragma unroll
     for (int i = 0; i < X_REGS; ++i) {
-        x_offset[i] = static_cast<uint32_t>(min(4 * i + part, nrows - 1)) * static_cast<uint32_t>(a.in_features) + col * 16;
+        x_offset[i] = BY_ROWS ? static_cast<uint32_t>(min(4 * i + part, nrows - 1)) * static_cast<uint32_t>(a.in_features) + col * 16
+                              : static_cast<uint32_t>((4 * i + part) * 512 + ((row_start & 31) + col) * 16);
     }
-    const int8_t * const x_rows = a.qx + static_cast<int64_t>(row_start) * a.in_features;
-    const float * const my_scales = ((lane & 2) == 0 ? a.dx : a.sx) +
-                                    static_cast<int64_t>(row_start + min(lane >> 2, nrows - 1)) * (a.in_features / 32) + 4 * (lane & 1);
+    const int8_t * const x_rows = a.qx + (BY_ROWS ? static_cast<int64_t>(row_start) * a.in_features
+                                                  : static_cast<int64_t>(row_start >> 5) * super_blocks * TILE_STEP);
+    const float * const my_scales =
+        BY_ROWS ? ((lane & 2) == 0 ? a.dx : a.sx) + static_cast<int64_t>(row_start + min(lane >> 2, nrows - 1)) * (a.in_features / 32) + 4 * (lane & 1)
+                : (lane < 32 ? a.dx : a.sx) + static_cast<int64_t>((lane >> 2) & 7) * a.rows_padded + row_start + 4 * (lane & 3);
     auto x_request = [&](Incoming & in, int sb) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < X_REGS; ++i) {
-            if (4 * i < nrows) {   // uniform
-                in.bytes[i] = *reinterpret_cast<const uint4 *>(x_rows + sb * QK_K + x_offset[i]);
+            if (!BY_ROWS || 4 * i < nrows) {   // uniform
+                in.bytes[i] = *reinterpret_cast<const uint4 *>(x_rows + static_cast<int64_t>(sb) * (BY_ROWS ? QK_K : TILE_STEP) + x_offset[i]);
             }
         }
-        in.scales = *reinterpret_cast<const float4 *>(my_scales + sb * 8);
+        in.scales = *reinterpret_cast<const float4 *>(my_scales + static_cast<int64_t>(sb) * 8 * (BY_ROWS ? 1 : a.rows_padded));
     };
     auto x_park = [&](const Incoming & in) __attribute__((always_inline)) {
         asm volatile("" ::: "memory");
 #pragma unroll
         for (int i = 0; i < X_REGS; ++i) {
-            if (4 * i < nrows) {
+            if constexpr (HALVES) {
+                // (word by word: copied whole, the structure that holds them goes through scratch memory)
+                *reinterpret_cast<uint4 *>(mine.x + col * TILES_X_PITCH + (4 * i + part) * 16) =
+                    make_uint4(in.bytes[i].x, in.bytes[i].y, in.bytes[i].z, in.bytes[i].w);
+            } else if (!BY_ROWS || 4 * i < nrows) {
                 const uint32_t words[4] = {in.bytes[i].x, in.bytes[i].y, in.bytes[i].z, in.bytes[i].w};
                 uint32_t halves[8];
 #pragma unroll
@@ -442,12 +460,20 @@ __global__ __launch_bounds__(TILES_THREADS, 2) void mmq_gemv_tiles_kernel(const 
                     halves[2 * w] = half2_add(first, half2_of(-1152));
                     halves[2 * w + 1] = half2_add(second_pair, half2_of(-1152));
                 }
-                uint8_t * const to = mine.x + (4 * i + part) * TILES_X_PITCH + col * 32;
+                uint8_t * const to = mine.x + (BY_ROWS ? (4 * i + part) * TILES_X_PITCH + col * 32 : col * TILES_X_PITCH + (4 * i + part) * 32);
                 *reinterpret_cast<uint4 *>(to) = make_uint4(halves[0], halves[1], halves[2], halves[3]);
                 *reinterpret_cast<uint4 *>(to + 16) = make_uint4(halves[4], halves[5], halves[6], halves[7]);
             }
         }
-        *reinterpret_cast<float4 *>(&mine.scales[(lane >> 2) * TILES_XS_PITCH + 4 * (lane & 3)]) = in.scales;
+        if constexpr (BY_ROWS) {
+            *reinterpret_cast<float4 *>(&mine.scales[(lane >> 2) * TILES_XS_PITCH + 4 * (lane & 3)]) = in.scales;
+        } else {
+            float * const to = &mine.scales[4 * (lane & 3) * TILES_XS_PITCH + (lane >> 2)];   // (scale or sum of block lane / 4 % 8)
+            to[0] = in.scales.x;
+            to[TILES_XS_PITCH] = in.scales.y;
+            to[2 * TILES_XS_PITCH] = in.scales.z;
+            to[3 * TILES_XS_PITCH] = in.scales.w;
+        }
         asm volatile("" ::: "memory");
     };
     half8_t x[8];
@@ -577,7 +603,7 @@ __global__ __launch_bounds__(TILES_THREADS, 2) void mmq_gemv_tiles_kernel(const 
 }
 
 // ---- launch ------------------------------------------------------------------------------------------------------------
-template <int TYPE, bool SWIGLU>
+template <int TYPE, bool SWIGLU, int LAYOUT>
 static hipError_t launch_tiles_typed(TilesArgs args, int64_t task_slots, hipStream_t stream) {
     const int super_blocks = args.in_features / QK_K;
     args.k_split = super_blocks >= 4 ? 4 : super_blocks >= 2 ? 2 : 1;
@@ -597,9 +623,9 @@ static hipError_t launch_tiles_typed(TilesArgs args, int64_t task_slots, hipStre
     const unsigned grid = static_cast<unsigned>(total);
     const ProfileScope scope(5, stream);
     if (tiles == 4) {
-        mmq_gemv_tiles_kernel<TYPE, 4, SWIGLU><<<grid, TILES_THREADS, 0, stream>>>(args);
+        mmq_gemv_tiles_kernel<TYPE, 4, SWIGLU, LAYOUT><<<grid, TILES_THREADS, 0, stream>>>(args);
     } else {
-        mmq_gemv_tiles_kernel<TYPE, 2, SWIGLU><<<grid, TILES_THREADS, 0, stream>>>(args);
+        mmq_gemv_tiles_kernel<TYPE, 2, SWIGLU, LAYOUT><<<grid, TILES_THREADS, 0, stream>>>(args);
     }
     return hipGetLastError();
 }
@@ -609,7 +635,7 @@ hipError_t launch_mmq_gemv_tiles(const uint8_t * packed, const uint8_t * packed_
                                  const TaskList * tasks, int rows, int in_features, int out_features,
                                  int quant_type, bool swiglu, hipStream_t stream, int output_stride) {
     const int64_t row_bytes = static_cast<int64_t>(in_features / QK_K) * block_bytes(quant_type);
-    if (!ws.by_rows() || out_features % 16 != 0 || 16 * row_bytes > 0x7fffffffLL || (swiglu && packed_second == nullptr)) {
+    if (ws.scaled_tiles() || (!ws.by_rows() && (tasks != nullptr || swiglu)) || out_features % 16 != 0 || 16 * row_bytes > 0x7fffffffLL || (swiglu && packed_second == nullptr)) {
         return hipErrorInvalidValue;
     }
     TilesArgs args = {};
@@ -623,6 +649,7 @@ hipError_t launch_mmq_gemv_tiles(const uint8_t * packed, const uint8_t * packed_
     args.y_second = output_second;
     args.row_bytes = static_cast<uint32_t>(row_bytes);
     args.rows = rows;
+    args.rows_padded = static_cast<int>(ws.rows_padded);
     args.in_features = in_features;
     args.out_features = out_features;
     args.out_stride = output_stride > 0 ? output_stride : out_features;
@@ -636,7 +663,10 @@ hipError_t launch_mmq_gemv_tiles(const uint8_t * packed, const uint8_t * packed_
     }
     const auto typed = [&](auto type) {
         constexpr int TYPE = decltype(type)::value;
-        return swiglu ? launch_tiles_typed<TYPE, true>(args, task_slots, stream) : launch_tiles_typed<TYPE, false>(args, task_slots, stream);
+        return swiglu            ? launch_tiles_typed<TYPE, true, LAYOUT_ROWS>(args, task_slots, stream)
+               : ws.by_rows()    ? launch_tiles_typed<TYPE, false, LAYOUT_ROWS>(args, task_slots, stream)
+               : ws.half_tiles() ? launch_tiles_typed<TYPE, false, LAYOUT_HALF_TILES>(args, task_slots, stream)
+                                 : launch_tiles_typed<TYPE, false, LAYOUT_INT8_TILES>(args, task_slots, stream);
     };
     switch (quant_type) {
         case Q3_K: return typed(std::integral_constant<int, Q3_K>{});

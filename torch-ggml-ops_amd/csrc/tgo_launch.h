@@ -485,6 +485,7 @@ hipError_t launch_mmq_gemv(const uint8_t * packed, const uint8_t * packed_second
                            const Q8Workspace & ws, uint16_t * output, uint16_t * output_second,
                            const TaskList * tasks, int rows, int in_features, int out_features,
                            int quant_type, hipStream_t stream, int output_stride = 0);
+// `ws`: plain rows, or for a dense call without SwiGLU the exact tile layouts as well.
 hipError_t launch_mmq_gemv_tiles(const uint8_t * packed, const uint8_t * packed_second, int64_t bytes_per_expert,
                                  const Q8Workspace & ws, uint16_t * output, uint16_t * output_second,
                                  const TaskList * tasks, int rows, int in_features, int out_features,

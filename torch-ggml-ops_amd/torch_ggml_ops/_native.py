@@ -206,9 +206,16 @@ def stream_of(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def forward_scratch_bytes(rows: int, in_features: int, out_features: int, quant_type: int) -> int:
+    """Scratch bytes worth allocating for a dense forward call: none where the decode kernel takes it (a call without
+    scratch is as correct should the setting change in between)."""
+    size = lib.tgo_forward_scratch_bytes(rows, in_features, out_features, int(quant_type))
+    return size if size == 0 or forward_kernel_for(int(quant_type), rows, in_features, out_features) != "tiles" else 0
+
+
 def forward_scratch(tensor: torch.Tensor, rows: int, in_features: int, out_features: int, quant_type: int):
     """(tensor that keeps it, pointer) of the scratch memory of a dense forward call; (None, None) when it needs none."""
-    size = lib.tgo_forward_scratch_bytes(rows, in_features, out_features, int(quant_type))
+    size = forward_scratch_bytes(rows, in_features, out_features, quant_type)
     if size == 0:
         return None, None
     scratch = tensor.new_empty((size,), dtype=torch.uint8)

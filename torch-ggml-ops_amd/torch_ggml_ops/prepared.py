@@ -6,8 +6,9 @@ paid once: ``quantize_q8_1`` returns the library's q8_1 workspace as an opaque u
 ``mmq_prepared`` runs only the matmul half on it.  A workspace that is quantized before its format is
 known holds int8 operands (exact fp16 ones when ``set_forward_operand("half")`` forces them), so the
 results are bit-identical to ``mmq`` wherever ``mmq`` multiplies the same kind: formats other than IQ2_S
-in calls below the size at which ``mmq`` switches to its scaled operands (``forward_operand_for``).
-Otherwise they are the same q8_1 algebra with another summation order or operand rounding (IQ2_S: exact
+in calls below the size at which ``mmq`` switches to its scaled operands (``forward_operand_for``), and every
+format where ``mmq`` runs on the decode kernels (``forward_kernel_for``), which both then do: up to 32 rows, up to
+128 on the matrices that they are the faster for.  Otherwise they are the same q8_1 algebra with another summation order or operand rounding (IQ2_S: exact
 fp16 in ``mmq``, int8 here, whose kernel is about a third slower for that format; large calls: scaled
 operands in ``mmq``, up to 8e-4 of the largest output apart).  A caller that knows what the workspace
 will be multiplied with names the kind itself (``operand=`` of both functions, the same value in both);
@@ -137,7 +138,7 @@ def _multi_device(input, packed_weights, quant_types, out_features, operand):
             _validate.prepared(workspace, weight, rows, in_features, quant_type, features)
         outputs = [input.new_empty((*input.shape[:-1], features)) for features in out_features]
         scratch_bytes = max(
-            _native.lib.tgo_forward_scratch_bytes(rows, in_features, features, quant_type)
+            _native.forward_scratch_bytes(rows, in_features, features, quant_type)
             for quant_type, features in zip(quant_types, out_features)
         )
         scratch = input.new_empty((scratch_bytes,), dtype=torch.uint8) if scratch_bytes > 0 else None
