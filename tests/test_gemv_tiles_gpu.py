@@ -91,3 +91,28 @@ def test_dense_beyond_the_decode_regime(oracle, qname, rows, n, k):
     host = synth.random_packed_weight(qtype, (n,), k, seed=qtype + rows)
     x = random_bf16((rows, k), seed=rows)
     assert_matches_f32_reference(tgo.mmq(x, host.cuda(), qtype, n), oracle.mmq_forward(qtype, bits(x), host.numpy(), n, k))
+
+
+@pytest.mark.parametrize("qname", tuple(QTYPES))
+def test_grouped_and_dense_calls_on_this_kernel_have_the_same_bits(qname):
+    """Groups of 1 to 50 rows of a grouped call that averages eleven, and a dense call on each of them: where both run on this kernel, the
+    same bits."""
+    import synth
+    import torch_ggml_ops as tgo
+    from torch_ggml_ops import _native
+
+    qtype, n, k = QTYPES[qname], 2048, 2048
+    sizes = [50, 1, 40, 3, 16, 17, 1, 2, 1, 33, 1, 1, 1, 1, 2, 5]
+    experts = len(sizes)
+    ends = np.cumsum(sizes).tolist()
+    weight = synth.random_packed_weight(qtype, (experts, n), k, seed=qtype).cuda()
+    x = random_bf16((ends[-1], k), seed=6)
+    assert _native.forward_kernel_for(qtype, ends[-1], k, n, experts) == "tiles" and ends[-1] > 4 * experts
+    output = tgo.grouped_mmq(x, weight, torch.arange(experts, device="cuda"), torch.tensor(ends, device="cuda", dtype=torch.int32), qtype, n)
+    compared = 0
+    for expert, (begin, end) in enumerate(zip([0] + ends, ends)):
+        if _native.forward_kernel_for(qtype, end - begin, k, n) == "tiles":
+            dense = tgo.mmq(x[begin:end].clone(), weight[expert].clone(), qtype, n)
+            torch.testing.assert_close(output[begin:end], dense, rtol=0, atol=0)
+            compared += 1
+    assert compared >= 4

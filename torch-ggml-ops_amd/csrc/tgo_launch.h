@@ -92,7 +92,8 @@ constexpr int GEMV_DENSE_ROWS = 32;
 //  - 256-row fp16 tiles: the narrow variant up to 128 tiles, else the largest tile that yields 128 workgroups; ranges of four
 //    super-blocks (a narrow workgroup's start costs as much as one).  4096 x 8192 IQ2_S, 64 rows: 77 -> 44 us.
 // Matrices of fewer than four million weights keep one range.  That line is not one of speed: it leaves the sums of small
-// dense calls those of the grouped calls on the same rows bit for bit, which the operators' tests hold them to.  With this rule's
+// dense calls those of the grouped calls on the same rows bit for bit, which the operators' tests hold them to (grouped calls on the
+// matrix-core kernels, that is: those of few rows per group that grouped_takes_tiles takes add in another order).  With this rule's
 // ranges below it, one range -> ranges: K = 4096, 512 columns, 64 rows Q6_K 102 -> 28 us, Q3_K 50 -> 19, Q4_K 37 -> 17, IQ2_S
 // 42 -> 20; K = 2048, 1024 columns, 64 rows 55 -> 24, 29 -> 18, 22 -> 15, 25 -> 20; K = 1024 mostly a tie, from 2048 columns up
 // also a loss (Q4_K, 517 rows of 2048: 18 -> 23).  (1024 x 4096, on the line, 64 rows: Q6_K 33, Q3_K 20, Q4_K 18.)
