@@ -78,6 +78,23 @@ def test_the_kernels_of_a_call_are_named(package):
             native.forward_kernel_for(*sizes)
 
 
+def test_rows_per_group_that_the_decode_kernel_takes(package):
+    """By format, operand kind and, where skewed routing makes many tasks of one expert's weights, rows in all."""
+    _, native, _, _ = package
+
+    def most(qtype, groups, k, n, projections=1):
+        rows = [r for r in range(5 * groups, 40 * groups, groups) if native.forward_kernel_for(qtype, r, k, n, groups, projections) == "tiles"]
+        assert rows == list(range(5 * groups, 5 * groups + len(rows) * groups, groups))   # one line, nothing beyond it
+        return rows[-1] // groups if rows else 4
+
+    assert [most(q, 64, 2048, 512, 2) for q in (11, 12, 13, 14, 22)] == [16, 16, 16, 32, 12]
+    assert [most(q, 256, 2048, 512, 2) for q in (11, 12, 13, 14, 22)] == [15, 10, 8, 15, 12]    # (15: scaled operands from 16 on)
+    assert [most(q, 256, 512, 2048) for q in (11, 12, 13, 14, 22)] == [12, 10, 10, 7, 7]        # (scaled from 8 on)
+    assert [most(q, 256, 1024, 4096) for q in (11, 12, 13, 14, 22)] == [6, 6, 6, 4, 4]          # (all scaled)
+    assert [most(q, 128, 1024, 4096) for q in (11, 12, 13)] == [12, 10, 10]
+    assert [most(q, 256, 4096, 1024, 2) for q in (11, 12, 13, 14, 22)] == [7, 7, 7, 7, 7]
+
+
 def test_an_entry_point_reads_the_operand_setting_once():
     """The rules take the setting as an argument, and no function of the C ABI reads it twice: a change by another thread falls
     before or after a call, not into it."""

@@ -272,14 +272,21 @@ static inline bool dense_takes_tiles(int setting, int64_t rows, int64_t in_featu
 }
 // Grouped calls beyond the decode regime (use_gemv) that take it all the same: its tasks of 16 rows unpack a group's weights once or
 // twice, the matrix-core kernels once per 128 or 256 rows and with a fraction of the chip.  The line is a number of rows per group on
-// average, by the operand kind that the call has otherwise.
-// Exact kinds, gate and up of 256 experts of 2048 x 512, us matrix-core kernel -> this one: 8 rows Q3_K 141 -> 80, Q4_K 123 -> 99,
-// Q5_K 135 -> 112, Q6_K 435 -> 149, IQ2_S 174 -> 94; 12 rows Q6_K 437 -> 156, IQ2_S 175 -> 98; 16 rows of 64 experts of 2048 x 768 Q3_K 69 ->
-// 38, Q4_K 50 -> 43, Q6_K 162 -> 58.  Layers with power-law 1.1 routing, whose large groups are cut into many tasks: 12 rows on average
-// 0.35 to 0.95 of the time, 14 rows IQ2_S 1.18, Q4_K 1.05, Q6_K 0.83.  At the line it can lose a little: 16 rows of 64 experts of 2048 x 512 gate and up
-// Q4_K 34.7 -> 35.8, where the down projection (512 x 2048) wins, 25.4 -> 20.7.
-// Scaled operands: 512 columns of K to 2048, 12 rows Q3_K 72 -> 52, Q4_K 62 -> 48, Q5_K 69 -> 54, Q6_K 90 -> 82, IQ2_S 70 -> 68.
+// average, by the operand kind that the call has otherwise; the host does not see the sizes of the groups, and the more of the rows are in few
+// groups, the more tasks unpack the same weights while the other kernels need fewer.  So the lines lie where a routing with a power law of
+// 1.1 over the experts (normal logits on top of it) still gains or ties; of the time of the matrix-core kernels, gate and up of 2048 x 512
+// unless said otherwise, mean of three routings with power 0.3 / 1.1 / 1.5:
+//  - exact kinds, 256 experts: Q3_K 14 rows 0.59 / 0.96 / 1.06; Q4_K 8 rows 0.72 / 0.92 / 1.05, 10 rows 0.75 / 0.97 / 1.20, 12 rows 0.76 / 1.03 / 1.19;
+//    Q5_K 8 rows 0.78 / 0.94 / 1.12, 10 rows 0.78 / 1.07 / 1.09; Q6_K 14 rows 0.41 / 0.70 / 0.99; IQ2_S 10 rows 0.58 / 0.94 / 1.08, 12 rows 0.63 / 1.03 /
+//    1.24.  128 experts of 2048 x 768, 16 rows: Q4_K 0.78 / 0.94 / 1.05, Q5_K 0.82 / 0.96 / 1.12.  64 experts, equal groups of 16 rows: Q4_K
+//    0.97, Q5_K 0.99.  Q4_K and Q5_K, whose other kernels unpack the fastest, lose to skew by rows in all rather than per group.
+//  - scaled operands: 512 columns of K to 2048, 256 experts: Q3_K 12 rows 0.73 / 0.94 / 1.06, Q4_K 10 rows 0.73 / 0.89 / 1.00, Q5_K the same
+//    0.73 / 0.83 / 1.02.  Larger experts lose earlier (1024 columns of K to 4096, 256 experts, power 1.1: 6 rows Q4_K 0.98, Q5_K 1.01, 8 rows 1.09 and 1.14; 128
+//    experts, 12 rows: 0.94 and 0.97).  Q6_K (0.94 to 1.41 at 8 rows) and IQ2_S (0.99 to 1.53) not at all.
+// All rows in one group of 256 is the worst of it: 8 rows on average, Q4_K 1.25 (46 us -> 58), 512 columns of K to 2048 1.73 (24 -> 42), and up to
+// twice the time at the lines.
 // Not where the operand kind was forced: the caller asked for that kind's kernels.
+constexpr int64_t GEMV_TILES_SCALED_WORK = INT64_C(6) << 30;   // rows x columns x K: 1536 rows of 1024 x 4096
 static inline bool grouped_takes_tiles(int setting, int64_t rows, int64_t groups, int64_t in_features, int64_t out_features,
                                        int quant_type, int projections) {
     if (use_gemv(rows, groups)) {
@@ -289,8 +296,15 @@ static inline bool grouped_takes_tiles(int setting, int64_t rows, int64_t groups
         return false;
     }
     const bool scaled = forward_operand_kind(setting, quant_type, rows, out_features, projections) == OPERAND_SCALED;
-    const int64_t most = quant_type == 14 ? (scaled ? 8 : 32) : quant_type == 22 ? (scaled ? 8 : 12) : scaled ? 12 : 16;
-    return rows <= most * groups;
+    switch (quant_type) {
+        case 11: return rows <= (scaled ? 12 : 16) * groups && (!scaled || rows <= GEMV_TILES_SCALED_WORK / (out_features * in_features));
+        case 12:
+        case 13:
+            return scaled ? rows <= 10 * groups && rows <= GEMV_TILES_SCALED_WORK / (out_features * in_features)
+                          : rows <= 16 * groups && rows <= (quant_type == 12 ? 2560 : 2048);
+        case 14: return !scaled && rows <= 32 * groups;
+        default: return !scaled && rows <= 12 * groups;
+    }
 }
 
 // q8_1 workspace: quantized values, then fp32 scales, then fp32 sums, in one of four layouts over the same bytes.
