@@ -95,6 +95,32 @@ def test_rows_per_group_that_the_decode_kernel_takes(package):
     assert [most(q, 256, 4096, 1024, 2) for q in (11, 12, 13, 14, 22)] == [7, 7, 7, 7, 7]
 
 
+def test_dense_rows_that_the_decode_kernel_takes(package):
+    """By format, size and length of K: Q3_K, Q4_K, Q5_K, Q6_K, IQ2_S."""
+    _, native, _, _ = package
+
+    def most(n, k):
+        found = []
+        for qtype in (11, 12, 13, 14, 22):
+            rows = [r for r in range(33, 200) if native.forward_kernel_for(qtype, r, k, n) == "tiles"]
+            assert rows == list(range(33, 33 + len(rows)))   # one line, nothing beyond it
+            found.append(rows[-1] if rows else 32)
+        return found
+
+    assert most(2048, 2048) == most(1024, 8192) == [128] * 5
+    assert most(1024, 4096 - 256) == [32] * 5                      # fewer than four million weights
+    assert most(4096, 4096) == [96, 96, 96, 64, 96]
+    assert most(2048, 8192) == [96, 64, 64, 64, 96]
+    assert most(1024, 16384) == [96, 32, 32, 64, 32]
+    assert most(8192, 4096) == most(11008, 4096) == [64] * 5
+    assert most(8192, 5120) == [64, 64, 48, 64, 64]
+    assert most(14336, 4096) == [64, 48, 48, 64, 48]
+    assert most(8192, 8192) == [64, 32, 32, 64, 48]
+    assert most(4096, 14336) == [64, 32, 32, 64, 32]
+    assert most(16384, 4096) == [64] * 5
+    assert most(28672, 8192) == [32] * 5
+
+
 def test_an_entry_point_reads_the_operand_setting_once():
     """The rules take the setting as an argument, and no function of the C ABI reads it twice: a change by another thread falls
     before or after a call, not into it."""

@@ -253,10 +253,16 @@ static inline bool gemv_takes_tiles(int64_t rows, int64_t groups, int64_t in_fea
     }
 }
 // Dense calls beyond the decode regime that take it all the same: three to eight tasks of 16 rows, each of which unpacks all weights,
-// keep the chip busier than the matrix-core kernels' tiles of 128 columns, up to a number of rows that falls with the matrix (us,
-// matrix-core kernel -> this one): 2048 x 2048 Q4_K 64 rows 23 -> 10, 128 rows 16 -> 11; Q6_K 128 rows 27 -> 15; 5120 x 1024 IQ2_S 128
-// rows 18 -> 18; 4096 x 4096 Q3_K 64 rows 23 -> 17, 96 rows 28 -> 24, Q5_K 96 rows 24 -> 24, Q6_K 64 rows 28 -> 22, 80 rows 30 -> 31; 11008 x 4096
-// 64 rows Q3_K 42 -> 32, Q4_K 34 -> 30, 80 rows 38 -> 37; 28672 x 8192 34 rows Q4_K 103 -> 102, Q6_K 140 -> 160.
+// keep the chip busier than the matrix-core kernels' tiles of 128 columns, up to a number of rows that falls with the matrix; of the time
+// of the matrix-core kernels (with their ranges of K), weights read from memory:
+//  - up to 2^23 weights, 128 rows: 2048 x 2048 Q3_K 0.69, Q4_K 0.73, Q5_K 0.75, Q6_K 0.58, IQ2_S 0.64; 1024 x 8192 Q4_K 0.89, Q5_K 0.92.
+//  - up to 2^24: 4096 x 4096, 96 rows Q3_K 0.88, Q4_K 0.94, Q5_K 0.98, Q6_K 1.03 (64 rows 0.79), IQ2_S 0.90; 8192 x 2048, 128 rows Q4_K 1.04.
+//  - up to 2^26: 8192 x 4096, 64 rows 0.79, 0.89, 0.94, 0.90, 0.90 in this order, 80 rows 0.77, 0.91, 0.95, 1.15, 1.15.  From 48 million weights on
+//    64 rows of a matrix without enough columns for the scaled kernel lose the last round of workgroups (14336 x 4096: 0.89, 1.06, 1.10, 0.98,
+//    1.11; 48 rows 0.72, 0.86, 0.91, 0.78, 0.93); with enough of them they do not (16384 x 4096: 0.67, 0.76, 0.77, 0.85, 0.83).
+//  - a long K is where ranges gain the most: Q4_K and Q5_K, whose other kernel unpacks the fastest, and beyond 12288 IQ2_S.  8192 x 5120,
+//    48 / 64 rows Q4_K 0.96 / 0.95, Q5_K 1.02 / 1.02; 8192 x 8192 Q4_K 1.05 / 1.05, Q5_K 1.09 / 1.09; 4096 x 11008 1.05 / 1.07, 1.09 / 1.11; 1024 x 16384, 64
+//    rows 1.09, 1.12, IQ2_S 1.10 (Q3_K 0.90, Q6_K 0.74).
 static inline bool dense_takes_tiles(int setting, int64_t rows, int64_t in_features, int64_t out_features, int quant_type) {
     if (use_gemv(rows, 0)) {
         return gemv_takes_tiles(rows, 0, in_features, out_features, quant_type);
@@ -265,11 +271,23 @@ static inline bool dense_takes_tiles(int setting, int64_t rows, int64_t in_featu
         return false;
     }
     const int64_t weights = out_features * in_features;
-    return rows <= (weights <= (INT64_C(1) << 23)   ? 128
-                    : weights <= (INT64_C(1) << 24) ? (quant_type == 14 ? 64 : 96)
-                    : weights <= (INT64_C(1) << 26) ? 64
-                                                    : GEMV_DENSE_ROWS);
+    const bool quick = quant_type == 12 || quant_type == 13;   // (to unpack, for the other kernels)
+    if (in_features > (quick ? 8192 : quant_type == 22 ? 12288 : 1 << 22)) {
+        return false;
+    }
+    if (weights <= (INT64_C(1) << 23)) {
+        return rows <= 128;
+    }
+    if (weights <= (INT64_C(1) << 24)) {
+        return rows <= (quant_type == 14 || (quick && in_features > 4096) ? 64 : 96);
+    }
+    if (weights > (INT64_C(1) << 26) || (quick && in_features > 4096 && weights > (INT64_C(44) << 20))) {
+        return false;
+    }
+    const bool last_round = weights > (INT64_C(48) << 20) && out_features < 16384 && (quick || quant_type == 22);
+    return rows <= (last_round || (quant_type == 13 && in_features > 4096) ? 48 : 64);
 }
+
 // Grouped calls beyond the decode regime (use_gemv) that take it all the same: its tasks of 16 rows unpack a group's weights once or
 // twice, the matrix-core kernels once per 128 or 256 rows and with a fraction of the chip.  The line is a number of rows per group on
 // average, by the operand kind that the call has otherwise; the host does not see the sizes of the groups, and the more of the rows are in few
