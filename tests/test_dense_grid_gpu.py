@@ -107,10 +107,10 @@ def test_q4k_32_rows_square_against_the_oracle_everywhere(ops, oracle):
     _check_grad_input(oracle, qtype, dy, packed_host, packed, n, list(range(m)))
 
 
-@pytest.mark.parametrize("rows,n", [(2100, 640), (2305, 2560), (1300, 5000), (704, 11008)])
+@pytest.mark.parametrize("rows,n", [(2100, 640), (2305, 2560), (1300, 5000), (704, 11008), (4200, 640), (300, 16385)])
 def test_row_tiles_chosen_by_rounds_give_every_result(rows, n):
-    """Dense calls with scaled operands whose row tile follows from the rounds of items, nine and ten row tasks over eight XCDs among
-    them: forward and grad-input against the same rows called a few at a time (whose tiles are others)."""
+    """Dense calls with scaled operands, row tasks of 256 rows (nine, ten and seventeen of them over eight XCDs, six, three and
+    two): forward and grad-input against the same rows called a few at a time, most of which have tasks of 128 rows."""
     import synth
     import torch_ggml_ops as tgo
     from torch_ggml_ops import _native

@@ -102,9 +102,10 @@ TGO_DEVICE void xcd_chunk(int linear, int inner, int tasks, int early, int & inn
     task = t < late_end - late_first ? early + late_first + t : tasks;
 }
 
-// Dense launches and the short tasks of the grad-input: XCD x takes the x-th eighth of the items, to within one item.  (Whole tasks
-// per XCD, or runs of four of them, gave one XCD twice the work of the others where a call has nine row tasks: 2600 rows x 5000 x 3072
-// Q5_K 172 -> 127 us.)  At most eight tasks in plain order: every XCD then has its share of the weights for all tasks (1700 rows x
+// Dense launches and the short tasks of the grad-input: as many whole tasks for every XCD as there are, then every XCD takes an
+// eighth of the items of the tasks that are left, to within one item.  (Only whole tasks per XCD gave one XCD twice the work of the others
+// where a call has nine tasks.  An eighth of all items each puts items of two tasks, whose activations then share an XCD's L2, into the
+// first round.)  At most eight tasks in plain order: every XCD then has its share of the weights for all tasks (1700 rows x
 // 4096 x 4096 Q5_K: 98 us with an XCD per task, 88 in plain order).  The grid holds xcd_slots(inner * tasks) workgroups; a slot past its
 // XCD's items returns task = tasks.
 TGO_DEVICE void xcd_tile(int linear, int inner, int tasks, int & inner_id, int & task) {
@@ -113,12 +114,20 @@ TGO_DEVICE void xcd_tile(int linear, int inner, int tasks, int & inner_id, int &
         inner_id = linear - task * inner;
         return;
     }
-    const int xcd = linear % XCDS;
-    const int64_t items = static_cast<int64_t>(tasks) * inner;
-    const int64_t first = xcd * items / XCDS, end = (xcd + 1) * items / XCDS;
-    const int64_t item = first + linear / XCDS < end ? first + linear / XCDS : items;
-    task = static_cast<int>(static_cast<uint32_t>(item) / static_cast<uint32_t>(inner));   // (launches have fewer than 2^31 items)
-    inner_id = static_cast<int>(item) - task * inner;
+    const int xcd = linear % XCDS, slot = linear / XCDS;
+    const int whole = tasks / XCDS;   // tasks of its own that an XCD has
+    if (slot < whole * inner) {
+        const int t = slot / inner;
+        task = xcd * whole + t;
+        inner_id = slot - t * inner;
+        return;
+    }
+    const int rest = (tasks - whole * XCDS) * inner;   // (fewer than eight tasks' items, far below 2^28)
+    const int first = xcd * rest / XCDS, end = (xcd + 1) * rest / XCDS;
+    const int item = min(first + slot - whole * inner, rest);
+    const int t = item < end ? item / inner : tasks - whole * XCDS;
+    task = whole * XCDS + t;
+    inner_id = item < end ? item - t * inner : 0;
 }
 
 static inline int xcd_chunk_slots(int slots) { return ((slots + XCDS - 1) / XCDS + 1) * XCDS; }

@@ -107,25 +107,12 @@ static inline ForwardSplit forward_split(int64_t rows, int64_t in_features, int6
     const int64_t n_tiles = (out_features + 127) / 128;
     const int64_t super_blocks = in_features / 256;
     if (operand_kind == OPERAND_SCALED) {
-        // One persistent workgroup per CU: a call takes as long as its rounds of items.  An item of T rows costs about 256 + T (256
-        // experts of 2048 x 512 Q4_K with T rows each, one item per expert and column tile: 64 rows 0.64 of the time of 256, 128 rows
-        // 0.75, 192 rows 0.92); the last round costs 0.4 and 1.3 times the share of the CUs that it occupies, at most 1 (4096 x 4096
-        // Q5_K, items of 256 rows: 224 items 88 us, 288 135, 352 173).  Fewer rows are taken where that saves a sixteenth.
-        // 4096 x 4096 Q5_K 2600 rows 178 -> 153 us, 11008 x 2048 2600 rows 235 -> 172, 5000 rows 344 -> 285 (with the tiles dealt out evenly,
-        // see xcd_chunk); a call of one short second round is a little slower for that (2100 rows x 4096 x 4096: 140 -> 148).
-        int best = 256;
-        int64_t least = 0;
-        for (int tile = 256; tile >= 64; tile -= 32) {
-            const int64_t items = n_tiles * projections * ((rows + tile - 1) / tile);
-            const int64_t last = items % SCALED_WORKGROUPS;
-            const int64_t rounds = items / SCALED_WORKGROUPS * 1000 + (last == 0 ? 0 : std::min<int64_t>(1000, 400 + last * 1300 / SCALED_WORKGROUPS));
-            const int64_t cost = rounds * (256 + tile);
-            if (least == 0 || cost * 16 < least * 15) {
-                best = tile;
-                least = cost;
-            }
-        }
-        return {best, 1};
+        // One persistent workgroup per CU, items of 256 rows, unless those leave half of the chip without one: then 128 rows (8192 x 4096,
+        // 300 rows: Q3_K 0.97 of the time, Q4_K 0.88, Q5_K 0.90, Q6_K 0.98, IQ2_S 0.97; 4096 x 4096, 900 rows: 1.00, 0.93, 0.96, 0.99, 0.99).
+        // Fewer rows per item where they make the rounds of items come out even gain nothing that holds: the unpacking that the items repeat
+        // costs as much (4096 x 4096, 192 rows per item: 2600 rows 0.97, 0.99, 0.98, 0.97, 0.96; 3000 rows 1.04, 1.06, 1.07, 1.04, 1.03; 11008 x
+        // 2048, 600 rows, 224 per item: Q4_K 1.07).
+        return {n_tiles * projections * ((rows + 255) / 256) <= SCALED_WORKGROUPS / 2 ? 128 : 256, 1};
     }
     const int full_tile = forward_row_tile(quant_type, operand_kind);
     const auto tiles = [&](int tile) { return n_tiles * ((rows + tile - 1) / tile); };
