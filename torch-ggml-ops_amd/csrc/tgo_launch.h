@@ -108,9 +108,9 @@ static inline ForwardSplit forward_split(int64_t rows, int64_t in_features, int6
     const int64_t super_blocks = in_features / 256;
     if (operand_kind == OPERAND_SCALED) {
         // One persistent workgroup per CU, items of 256 rows, unless those leave half of the chip without one: then 128 rows (8192 x 4096,
-        // 300 rows: Q3_K 0.97 of the time, Q4_K 0.88, Q5_K 0.90, Q6_K 0.98, IQ2_S 0.97; 4096 x 4096, 900 rows: 1.00, 0.93, 0.96, 0.99, 0.99).
+        // 300 rows: Q3_K 0.95 of the time, Q4_K 0.88, Q5_K 0.88, Q6_K 0.96, IQ2_S 0.96; 4096 x 4096, 900 rows: 1.01, 0.93, 0.96, 1.00, 1.00).
         // Fewer rows per item where they make the rounds of items come out even gain nothing that holds: the unpacking that the items repeat
-        // costs as much (4096 x 4096, 192 rows per item: 2600 rows 0.97, 0.99, 0.98, 0.97, 0.96; 3000 rows 1.04, 1.06, 1.07, 1.04, 1.03; 11008 x
+        // costs as much (4096 x 4096, 192 rows per item: 2600 rows 0.97, 0.99, 1.00, 0.97, 0.97; 3000 rows 1.04, 1.06, 1.07, 1.05, 1.04; 11008 x
         // 2048, 600 rows, 224 per item: Q4_K 1.07).
         return {n_tiles * projections * ((rows + 255) / 256) <= SCALED_WORKGROUPS / 2 ? 128 : 256, 1};
     }

@@ -142,12 +142,6 @@ TGO_DEVICE void decode16_scaled(const uint8_t * blk, int u, const Codebook * cod
     }
 }
 
-// Stores the wave's 32 rows x (32 * TILES) columns of results, which the matrix instructions left transposed (weights as the
-// A operand: the lane holds row l32 and, as element v of tile t, column 32 t + 8 (v / 4) + 4 (lane / 32) + v % 4), as
-// bf16.  The two half-waves exchange runs of four columns, after which a lane holds eight neighbouring columns and
-// stores 16 bytes; a row gets 32 contiguous bytes per instruction.  `dst` points at row 0, column 0; rows >=
-// valid_rows and columns >= valid_cols are skipped.  The 16-byte path needs row_stride % 8 == 0 (dst is then 16-byte
-// aligned: the tensor is, and column tiles start at multiples of 128).
 // The lane's number computed from nothing, and opaque: what is derived from it is derived where it is used instead of
 // being kept in a register through a loop (where such a register is spilled, its reload waits for every load in flight).
 TGO_DEVICE int lane_afresh() {
@@ -156,6 +150,12 @@ TGO_DEVICE int lane_afresh() {
     return lane;
 }
 
+// Stores the wave's 32 rows x (32 * TILES) columns of results, which the matrix instructions left transposed (weights as the
+// A operand: the lane holds row l32 and, as element v of tile t, column 32 t + 8 (v / 4) + 4 (lane / 32) + v % 4), as
+// bf16.  The two half-waves exchange runs of four columns, after which a lane holds eight neighbouring columns and
+// stores 16 bytes; a row gets 32 contiguous bytes per instruction.  `dst` points at row 0, column 0; rows >=
+// valid_rows and columns >= valid_cols are skipped.  The 16-byte path needs row_stride % 8 == 0 (dst is then 16-byte
+// aligned: the tensor is, and column tiles start at multiples of 128).
 template <int TILES>
 TGO_DEVICE void store_rows_32xn(const v16f * tiles, uint16_t * dst, int64_t row_stride, int valid_rows, int valid_cols, int lane) {
     const int l32 = lane & 31;
