@@ -122,7 +122,7 @@ TGO_DEVICE void xcd_tile(int linear, int inner, int tasks, int & inner_id, int &
         inner_id = slot - t * inner;
         return;
     }
-    const int rest = (tasks - whole * XCDS) * inner;   // (fewer than eight tasks' items, far below 2^28)
+    const int rest = (tasks - whole * XCDS) * inner;   // (at most seven tasks' items, below 2^28 for any width)
     const int first = xcd * rest / XCDS, end = (xcd + 1) * rest / XCDS;
     const int item = min(first + slot - whole * inner, rest);
     const int t = item < end ? item / inner : tasks - whole * XCDS;
