@@ -38,7 +38,7 @@ extern "C" {
 
 /* Library version (major*10000 + minor*100 + patch): TGO_VERSION of the header that the library was built with.  It grows with
  * every change of this file that a caller can see. */
-#define TGO_VERSION 114
+#define TGO_VERSION 115
 int tgo_version(void);
 
 /* Message of the last failure on the calling thread ("" if none). Host pointer. */
@@ -112,6 +112,13 @@ int64_t tgo_pair_grad_workspace_bytes(int64_t rows, int64_t out_features, int64_
 int tgo_mmq_pair_grad_input(const void * grad_output_first, const void * grad_output_second, const void * packed_first,
                             const void * packed_second, void * grad_input_bf16, void * workspace, int64_t rows, int64_t out_features,
                             int64_t in_features, int quant_type, void * stream);
+/* The gradient of the input of up to four projections of any shapes and formats, summed in fp32 and rounded once, as one product over
+ * all their weight rows: the weights are unpacked into `workspace`, which holds tgo_multi_grad_workspace_bytes() bytes.  0 bytes:
+ * projections of these sizes are better taken one by one, and the call is refused.  The arrays lie in host memory. */
+int64_t tgo_multi_grad_workspace_bytes(int count, const int64_t * out_features, int64_t rows, int64_t in_features);
+int tgo_mmq_multi_grad_input(int count, const void * const * grad_outputs_bf16, const void * const * packed, const int64_t * out_features,
+                             const int * quant_types, void * grad_input_bf16, void * workspace, int64_t rows, int64_t in_features,
+                             void * stream);
 
 /* tgo_mmq_forward without a workspace argument and without any allocation: the q8_1 activation
  * workspace is a fixed array inside the library's code object (one copy per GPU, held until the
@@ -163,14 +170,14 @@ int64_t tgo_grad_workspace_bytes(int64_t rows, int64_t out_features, int64_t num
 
 /* Bytes of `workspace` for tgo_mmq_grad_input: the packed cotangent as above, plus, for calls of so
  * few rows that whole reductions per workgroup would leave most of the chip idle, room for the
- * fp32 partial results of a reduction split over several workgroups (added up in a fixed order);
- * which calls split depends on the format, hence `quant_type`.
+ * fp32 partial results of a reduction split over several workgroups (added up in a fixed order), plus, for
+ * calls that unpack their weights first, two bytes per weight.
  * No counterpart in the reference.  -1 on invalid sizes. */
 int64_t tgo_dense_grad_workspace_bytes(int64_t rows, int64_t out_features, int64_t in_features,
                                        int quant_type);
 
 /* grad_input[rows, in_features] = bf16( grad_output[rows, out_features] x bf16(W) ), weights
- * dequantized to bf16 in LDS, bf16 MFMA, fp32 accumulation, one rounding.
+ * dequantized to bf16 (in LDS, or once into the workspace), bf16 MFMA, fp32 accumulation, one rounding.
  * `workspace` holds tgo_dense_grad_workspace_bytes(rows, out_features, in_features, quant_type) bytes.
  * Replaces launch_dense_mmq_grad_input<type>, csrc/ck/mmq_backward.cuh:1066-1241. */
 int tgo_mmq_grad_input(const void * grad_output_bf16, const void * packed, void * grad_input_bf16,

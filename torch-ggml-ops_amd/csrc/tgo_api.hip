@@ -252,13 +252,69 @@ int64_t tgo_task_workspace_bytes(int64_t rows, int64_t num_groups) {
     return (tgo::task_workspace_bytes(rows, num_groups) + 15) / 16 * 16;
 }
 
+// Packed cotangent and split sums of the kernels that unpack as they multiply.
+static int64_t single_grad_bytes(int64_t rows, int64_t out_features, int64_t in_features) {
+    return (tgo::cotangent_workspace_bytes(rows, out_features) + 15) / 16 * 16 + tgo::dense_grad_partial_bytes(rows, out_features, in_features);
+}
+
 int64_t tgo_dense_grad_workspace_bytes(int64_t rows, int64_t out_features, int64_t in_features, int quant_type) {
     if (rows <= 0 || out_features <= 0 || in_features <= 0 || in_features % tgo::QK_K != 0 ||
         tgo::block_bytes(quant_type) == 0) {
         return -1;
     }
-    return (tgo::cotangent_workspace_bytes(rows, out_features) + 15) / 16 * 16 +
-           tgo::dense_grad_partial_bytes(rows, out_features, in_features);
+    if (tgo::grad_unpacks(rows, out_features, in_features)) {
+        return tgo::unpacked_grad_workspace(nullptr, rows, tgo::cotangent_chunks(out_features), in_features).bytes;
+    }
+    return single_grad_bytes(rows, out_features, in_features);
+}
+
+// Reduction steps of 16 weight rows of several projections side by side, each in whole steps of 64, and their weight rows.
+static int64_t multi_chunks(int count, const int64_t * out_features, int64_t & total) {
+    int64_t chunks = 0;
+    total = 0;
+    for (int i = 0; i < count; ++i) {
+        if (out_features[i] <= 0 || out_features[i] > INT_LIMIT) {
+            return -1;
+        }
+        total += out_features[i];
+        chunks += tgo::cotangent_chunks(out_features[i]);
+    }
+    return chunks > INT_LIMIT ? -1 : chunks;
+}
+
+int64_t tgo_multi_grad_workspace_bytes(int count, const int64_t * out_features, int64_t rows, int64_t in_features) {
+    if (count < 1 || count > tgo::UNPACKED_SOURCES || out_features == nullptr || rows <= 0 || in_features <= 0 || in_features % tgo::QK_K != 0) {
+        return 0;
+    }
+    int64_t total;
+    const int64_t chunks = multi_chunks(count, out_features, total);
+    return chunks > 0 && tgo::multi_grad_unpacks(rows, total, in_features, count) ? tgo::unpacked_grad_workspace(nullptr, rows, chunks, in_features).bytes : 0;
+}
+
+int tgo_mmq_multi_grad_input(int count, const void * const * grad_outputs_bf16, const void * const * packed, const int64_t * out_features,
+                             const int * quant_types, void * grad_input_bf16, void * workspace, int64_t rows, int64_t in_features,
+                             void * stream) {
+    if (grad_outputs_bf16 == nullptr || packed == nullptr || out_features == nullptr || quant_types == nullptr) {
+        return fail(TGO_ERR_INVALID, "grad_outputs_bf16, packed, out_features and quant_types must not be null");
+    }
+    if (count < 1 || count > tgo::UNPACKED_SOURCES) {
+        return fail(TGO_ERR_INVALID, "between 1 and %d projections are required; got %d", tgo::UNPACKED_SOURCES, count);
+    }
+    tgo::DenseSource sources[tgo::UNPACKED_SOURCES];
+    for (int i = 0; i < count; ++i) {
+        TGO_TRY(check_matmul_shape(rows, in_features, out_features[i], quant_types[i]));
+        TGO_TRY(check_pointer(grad_outputs_bf16[i], "grad_output"));
+        TGO_TRY(check_pointer(packed[i], "packed_weight"));
+        sources[i] = {static_cast<const uint8_t *>(packed[i]), static_cast<const uint16_t *>(grad_outputs_bf16[i]), out_features[i], quant_types[i]};
+    }
+    TGO_TRY(check_pointer(grad_input_bf16, "grad_input"));
+    TGO_TRY(check_pointer(workspace, "workspace"));
+    if (tgo_multi_grad_workspace_bytes(count, out_features, rows, in_features) == 0) {
+        return fail(TGO_ERR_INVALID, "projections of these sizes have their gradients taken one by one");
+    }
+    return check_hip(tgo::launch_grad_input_unpacked(sources, count, workspace, static_cast<uint16_t *>(grad_input_bf16), rows, in_features,
+                                                     static_cast<hipStream_t>(stream)),
+                     "mmq_multi_grad_input launch");
 }
 
 int64_t tgo_grad_workspace_bytes(int64_t rows, int64_t out_features, int64_t num_groups, int sources) {
@@ -517,6 +573,13 @@ int tgo_mmq_grad_input(const void * grad_output_bf16, const void * packed, void 
     TGO_TRY(check_pointer(grad_input_bf16, "grad_input"));
     TGO_TRY(check_pointer(workspace, "workspace"));
     hipStream_t hip_stream = static_cast<hipStream_t>(stream);
+    if (tgo::grad_unpacks(rows, out_features, in_features)) {
+        const tgo::DenseSource source = {static_cast<const uint8_t *>(packed), static_cast<const uint16_t *>(grad_output_bf16), out_features,
+                                         quant_type};
+        return check_hip(tgo::launch_grad_input_unpacked(&source, 1, workspace, static_cast<uint16_t *>(grad_input_bf16), rows, in_features,
+                                                         hip_stream),
+                         "mmq_grad_input launch");
+    }
     uint8_t * cotangent = static_cast<uint8_t *>(workspace);
     TGO_TRY(check_hip(tgo::launch_pack_cotangent(static_cast<const uint16_t *>(grad_output_bf16), nullptr, cotangent,
                                                  nullptr, static_cast<int>(rows), static_cast<int>(out_features),
@@ -534,8 +597,12 @@ int tgo_mmq_grad_input(const void * grad_output_bf16, const void * packed, void 
 }
 
 int64_t tgo_pair_grad_workspace_bytes(int64_t rows, int64_t out_features, int64_t in_features, int quant_type) {
-    const int64_t single = tgo_dense_grad_workspace_bytes(rows, out_features, in_features, quant_type);
-    return single < 0 ? single : single + (tgo::cotangent_workspace_bytes(rows, out_features) + 15) / 16 * 16;
+    if (rows <= 0 || out_features <= 0 || in_features <= 0 || in_features % tgo::QK_K != 0 || tgo::block_bytes(quant_type) == 0) {
+        return -1;
+    }
+    const int64_t both[2] = {out_features, out_features};
+    const int64_t unpacked = tgo_multi_grad_workspace_bytes(2, both, rows, in_features);
+    return unpacked > 0 ? unpacked : single_grad_bytes(rows, out_features, in_features) + (tgo::cotangent_workspace_bytes(rows, out_features) + 15) / 16 * 16;
 }
 
 int tgo_mmq_pair_grad_input(const void * grad_output_first, const void * grad_output_second, const void * packed_first,
@@ -549,6 +616,14 @@ int tgo_mmq_pair_grad_input(const void * grad_output_first, const void * grad_ou
     TGO_TRY(check_pointer(grad_input_bf16, "grad_input"));
     TGO_TRY(check_pointer(workspace, "workspace"));
     hipStream_t hip_stream = static_cast<hipStream_t>(stream);
+    if (tgo::multi_grad_unpacks(rows, 2 * out_features, in_features, 2)) {
+        const tgo::DenseSource sources[2] = {
+            {static_cast<const uint8_t *>(packed_first), static_cast<const uint16_t *>(grad_output_first), out_features, quant_type},
+            {static_cast<const uint8_t *>(packed_second), static_cast<const uint16_t *>(grad_output_second), out_features, quant_type}};
+        return check_hip(tgo::launch_grad_input_unpacked(sources, 2, workspace, static_cast<uint16_t *>(grad_input_bf16), rows, in_features,
+                                                         hip_stream),
+                         "mmq_pair_grad_input launch");
+    }
     const int64_t cotangent_bytes = (tgo::cotangent_workspace_bytes(rows, out_features) + 15) / 16 * 16;
     uint8_t * const cotangent = static_cast<uint8_t *>(workspace);
     TGO_TRY(check_hip(tgo::launch_pack_cotangent(static_cast<const uint16_t *>(grad_output_first),

@@ -567,4 +567,104 @@ hipError_t launch_mmq_grad_input(const uint8_t * cotangent_first, const uint8_t 
                                  int rows, int out_features, int in_features, int quant_type,
                                  hipStream_t stream, float * partial = nullptr);
 
+// ---- dense products whose weights are unpacked once per call (tgo_unpacked.hip) ----
+// One projection: its packed weight, and its input (forward) or the cotangent of its output (grad-input).
+struct DenseSource {
+    const uint8_t * packed;
+    const uint16_t * activations;
+    int64_t out_features;
+    int quant_type;
+};
+// How a product of slabs is cut into workgroups: `full_rows` rows in tiles of 256 x 256 that fill the chip a whole number of times
+// (one workgroup per CU), the rest in tiles of `rest_tile_rows` x `rest_tile_columns`, and what that takes, in microseconds.
+struct ProductPlan {
+    int64_t full_rows;
+    int rest_tile_rows, rest_tile_columns;
+    float microseconds;
+};
+// One reduction step of 16 of `tiles` workgroups, 256 to a round: a round is the faster the emptier it is, down to `half` for half a
+// round, below which the CUs at work no longer gain from those that are idle.
+static inline float rounds_microseconds(int64_t tiles, float half, float whole) {
+    const int64_t rounds = (tiles - 1) / 256;
+    const float last = static_cast<float>(tiles - 256 * rounds);
+    return static_cast<float>(rounds) * whole + (last <= 128.0f ? half : half + (whole - half) * (last - 128.0f) / 128.0f);
+}
+// Measured per reduction step of 16 (100 to 8192 rows, 2048 to 11008 columns, reduction 512 to 11008, bf16), half a round and a whole one:
+// 256 x 256 tiles 0.29 and 0.45 us, 128 x 256 0.18 and 0.27, 128 x 128 0.115 and 0.155, 0.145 for each of several rounds (two workgroups
+// share a CU).
+static inline ProductPlan product_plan(int64_t rows, int64_t columns, int64_t steps) {
+    const auto up = [](int64_t count, int64_t tile) { return (count + tile - 1) / tile; };
+    const int64_t across = up(columns, 256);
+    const auto with_rounds = [&](int64_t rounds, int64_t row_tiles) {
+        ProductPlan plan = {rounds * row_tiles * 256, 256, 256, static_cast<float>(rounds * steps) * rounds_microseconds(row_tiles * across, 0.29f, 0.45f)};
+        const int64_t rest = rows - plan.full_rows;
+        if (rest > 0) {
+            const float a = rounds_microseconds(up(rest, 256) * across, 0.29f, 0.45f);
+            const float b = rounds_microseconds(up(rest, 128) * across, 0.18f, 0.27f);
+            const int64_t small = up(rest, 128) * up(columns, 128);
+            const float c = small <= 256 ? rounds_microseconds(small, 0.115f, 0.155f) : static_cast<float>(up(small, 256)) * 0.145f;
+            const float least = std::min(a, std::min(b, c));
+            plan.rest_tile_rows = least == a ? 256 : 128;
+            plan.rest_tile_columns = least == a || least == b ? 256 : 128;
+            plan.microseconds += static_cast<float>(steps) * least + 4.0f;
+        }
+        return plan;
+    };
+    const ProductPlan plain = with_rounds(0, 1);
+    const int64_t row_tiles = across <= 256 ? 256 / across : 0;
+    if (row_tiles * across < 160 || rows < row_tiles * 256) {
+        return plain;
+    }
+    const ProductPlan whole = with_rounds(rows / (row_tiles * 256), row_tiles);
+    return whole.microseconds < plain.microseconds ? whole : plain;
+}
+// Writing both operands: two bytes per weight leave.
+static inline float unpack_microseconds(int64_t out_features, int64_t in_features) {
+    return 5.0f + static_cast<float>(out_features) * static_cast<float>(in_features) * 0.6e-6f;
+}
+constexpr int UNPACKED_SOURCES = 4;
+struct UnpackedGradWorkspace {
+    uint8_t * cotangent;
+    uint8_t * weights;
+    int64_t bytes;
+};
+static inline UnpackedGradWorkspace unpacked_grad_workspace(void * base, int64_t rows, int64_t chunks, int64_t in_features) {
+    UnpackedGradWorkspace view;
+    view.cotangent = static_cast<uint8_t *>(base);
+    const int64_t weights = pad_rows(rows) / 32 * chunks * 1024;
+    view.weights = view.cotangent + weights;
+    view.bytes = weights + in_features / 32 * chunks * 1024;
+    return view;
+}
+// Whether a dense grad-input unpacks its weights once (tgo_unpacked.hip) or leaves it to every workgroup (tgo_backward.hip): by what
+// either takes.  The latter packs the cotangent, then runs items of 256 x 128, a round of 256 taking 0.27 us per 16 weight rows and half a
+// round 0.18, and cuts the reduction where that leaves half of the chip idle, for fp32 sums to be written and read again.  `count`
+// projections of one input (their weight rows together) would take a call each and an addition.
+// Of the time of the kernels that unpack as they multiply, where this rule leaves them (250 calls of 96 to 16384 rows, 512 to 28672 weight rows, K
+// 512 to 8192, all formats): 0.78 on the mean, 0.5 to 1.07.  4096 x 2048: 2000 rows Q4_K 58.9 -> 51.0 us, Q6_K 63.7 -> 47.8; 4096 rows 87.2 -> 74.8,
+// 96.3 -> 73.0; 8192 rows 165.6 -> 122.6, 184.0 -> 121.9.  On the other side of it, always unpacked: 28672 x 8192, 300 rows 206 -> 413 us (Q4_K); 4096 x
+// 2048, 300 rows 28.5 -> 30.2.
+static inline bool grad_unpacks(int64_t rows, int64_t out_features, int64_t in_features, int count = 1) {
+    // (32-bit lane offsets; a workspace of at most 1 GiB for the weights)
+    if (rows < 96 || out_features > (1 << 24) || out_features * in_features > (INT64_C(1) << 29) || rows > (1 << 24)) {
+        return false;
+    }
+    const int64_t steps = (out_features + 15) / 16;
+    const int splits = dense_grad_splits(rows, out_features, in_features);
+    const int64_t items = (rows + BACKWARD_ROW_TILE - 1) / BACKWARD_ROW_TILE * (in_features / 128) * splits;
+    const float together = 9.0f + static_cast<float>(rows) * static_cast<float>(out_features) * 0.8e-6f +
+                           static_cast<float>(steps / splits) * rounds_microseconds(items, 0.18f, 0.27f) +
+                           (splits > 1 ? 4.0f + static_cast<float>(rows) * static_cast<float>(in_features) * static_cast<float>(splits) * 1.2e-6f : 0.0f) +
+                           static_cast<float>(count - 1) * (9.0f + static_cast<float>(rows) * static_cast<float>(in_features) * 1.5e-6f);
+    return 1.05f * (unpack_microseconds(out_features, in_features) + product_plan(rows, in_features, steps).microseconds) < together;
+}
+// Of several projections as one reduction: their sums in fp32.  (Below a million weights the terms keep being rounded one by one.)
+static inline bool multi_grad_unpacks(int64_t rows, int64_t out_features, int64_t in_features, int count) {
+    return (count == 1 || out_features * in_features >= (1 << 20)) && grad_unpacks(rows, out_features, in_features, count);
+}
+// Grad-input of up to four projections of one input: the sum of their Jacobian products, rounded once.  `workspace`:
+// unpacked_grad_workspace().bytes.
+hipError_t launch_grad_input_unpacked(const DenseSource * sources, int count, void * workspace, uint16_t * grad_input, int64_t rows,
+                                      int64_t in_features, hipStream_t stream);
+
 }  // namespace tgo

@@ -64,6 +64,11 @@ lib.tgo_mmq_multi_forward.argtypes = [
 lib.tgo_pair_grad_workspace_bytes.argtypes = [_i64, _i64, _i64, _int]
 lib.tgo_pair_grad_workspace_bytes.restype = _i64
 lib.tgo_mmq_pair_grad_input.argtypes = [_p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _int, _p]
+lib.tgo_multi_grad_workspace_bytes.argtypes = [_int, ctypes.POINTER(_i64), _i64, _i64]
+lib.tgo_multi_grad_workspace_bytes.restype = _i64
+lib.tgo_mmq_multi_grad_input.argtypes = [
+    _int, ctypes.POINTER(_p), ctypes.POINTER(_p), ctypes.POINTER(_i64), ctypes.POINTER(_int), _p, _p, _i64, _i64, _p,
+]
 lib.tgo_mmq_forward_static.argtypes = [_p, _p, _p, _i64, _i64, _i64, _int, _p]
 lib.tgo_mmq_forward_prepared.argtypes = [_p, _p, _p, _i64, _i64, _i64, _int, _p]
 lib.tgo_quantize_q8_1_as.argtypes = [_p, _p, _i64, _i64, _int, _p]
@@ -124,6 +129,8 @@ EXPORTS = (
     "tgo_mmq_multi_forward",
     "tgo_pair_grad_workspace_bytes",
     "tgo_mmq_pair_grad_input",
+    "tgo_multi_grad_workspace_bytes",
+    "tgo_mmq_multi_grad_input",
     "tgo_mmq_forward_static",
     "tgo_mmq_forward_prepared",
     "tgo_quantize_q8_1_as",

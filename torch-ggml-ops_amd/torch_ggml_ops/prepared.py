@@ -193,6 +193,60 @@ def _pair_grad_input_backward(ctx, grad_grad_input):
 torch.library.register_autograd("torch_ggml_ops::mmq_pair_grad_input", _pair_grad_input_backward)
 
 
+torch.library.define(
+    "torch_ggml_ops::mmq_multi_grad_input",
+    "(Tensor[] grad_outputs, Tensor[] packed_weights, int[] quant_types, int in_features) -> Tensor",
+)
+
+
+def _multi_grad_workspace_bytes(rows: int, out_features: Sequence[int], in_features: int) -> int:
+    """Workspace of ``mmq_multi_grad_input``; 0 where the projections' gradients are better taken one by one."""
+    count = len(out_features)
+    return _native.lib.tgo_multi_grad_workspace_bytes(count, (ctypes.c_int64 * count)(*out_features), rows, in_features)
+
+
+@torch.library.impl("torch_ggml_ops::mmq_multi_grad_input", "CUDA")
+def _multi_grad_input_device(grad_outputs, packed_weights, quant_types, in_features):
+    if not (len(grad_outputs) == len(packed_weights) == len(quant_types)) or not grad_outputs:
+        raise ValueError("grad_outputs, packed_weights and quant_types must be non-empty and of equal length")
+    first = grad_outputs[0]
+    shapes = [
+        _validate.dense(grad, weight, quant_type, in_features, backward=True)
+        for grad, weight, quant_type in zip(grad_outputs, packed_weights, quant_types)
+    ]
+    rows, in_features, _ = shapes[0]
+    if any(shape[0] != rows for shape in shapes):
+        raise RuntimeError("all gradients must have the same rows")
+    if any(grad.device != first.device for grad in grad_outputs):
+        raise RuntimeError("all gradients must be on the same device")
+    out_features = [shape[2] for shape in shapes]
+    count = len(grad_outputs)
+    pointers = ctypes.c_void_p * count
+    with _native.on_device(first.device):
+        grad_input = first.new_empty((*first.shape[:-1], in_features))
+        workspace = first.new_empty((_multi_grad_workspace_bytes(rows, out_features, in_features),), dtype=torch.uint8)
+        _native.check(
+            _native.lib.tgo_mmq_multi_grad_input(
+                count, pointers(*(g.data_ptr() for g in grad_outputs)), pointers(*(w.data_ptr() for w in packed_weights)),
+                (ctypes.c_int64 * count)(*out_features), (ctypes.c_int * count)(*quant_types), grad_input.data_ptr(),
+                workspace.data_ptr(), rows, in_features, _stream(first),
+            )
+        )
+    return grad_input
+
+
+@torch.library.register_fake("torch_ggml_ops::mmq_multi_grad_input")
+def _multi_grad_input_fake(grad_outputs, packed_weights, quant_types, in_features):
+    return grad_outputs[0].new_empty((*grad_outputs[0].shape[:-1], in_features))
+
+
+def _multi_grad_input_backward(ctx, grad_grad_input):
+    raise RuntimeError("torch_ggml_ops::mmq_multi_grad_input does not support higher-order gradients")
+
+
+torch.library.register_autograd("torch_ggml_ops::mmq_multi_grad_input", _multi_grad_input_backward)
+
+
 class _MultiProjection(torch.autograd.Function):
     @staticmethod
     def forward(ctx, input, quant_types, out_features, *packed_weights):
@@ -210,6 +264,16 @@ class _MultiProjection(torch.autograd.Function):
         grad_input = None
         if ctx.needs_input_grad[0]:
             weights = ctx.saved_tensors
+            present = [i for i, grad in enumerate(grad_outputs) if grad is not None]
+            if len(present) > 1:
+                rows = grad_outputs[present[0]].numel() // ctx.out_features[present[0]]
+                if _multi_grad_workspace_bytes(rows, [ctx.out_features[i] for i in present], ctx.in_features) > 0:
+                    # one product over the weight rows of all projections
+                    grad_input = torch.ops.torch_ggml_ops.mmq_multi_grad_input.default(
+                        [grad_outputs[i].contiguous() for i in present], [weights[i] for i in present],
+                        [ctx.quant_types[i] for i in present], ctx.in_features,
+                    )
+                    return (grad_input, None, None) + (None,) * len(weights)
             i = 0
             while i < len(weights):
                 grad, weight, quant_type = grad_outputs[i], weights[i], ctx.quant_types[i]
