@@ -92,8 +92,8 @@ int tgo_mmq_forward(const void * input_bf16, const void * packed, void * output_
 
 /* tgo_mmq_forward and tgo_mmq_forward_prepared_as with tgo_forward_scratch_bytes() bytes of `scratch` (0: NULL is as good): dense
  * calls of more rows than the decode kernels take, whose tiles would not fill the chip, then cut K into ranges that run side by
- * side and leave fp32 sums there, which a second kernel adds up in a fixed order.  No counterpart in
- * the reference. */
+ * side and leave fp32 sums there, which a second kernel adds up in a fixed order; tgo_mmq_forward_scratch with scaled operands unpacks the
+ * weights there once where that pays (the same bits).  No counterpart in the reference. */
 int64_t tgo_forward_scratch_bytes(int64_t rows, int64_t in_features, int64_t out_features, int quant_type);
 int tgo_mmq_forward_scratch(const void * input_bf16, const void * packed, void * output_bf16, void * workspace, void * scratch,
                             int64_t rows, int64_t in_features, int64_t out_features, int quant_type, void * stream);
@@ -112,6 +112,13 @@ int64_t tgo_pair_grad_workspace_bytes(int64_t rows, int64_t out_features, int64_
 int tgo_mmq_pair_grad_input(const void * grad_output_first, const void * grad_output_second, const void * packed_first,
                             const void * packed_second, void * grad_input_bf16, void * workspace, int64_t rows, int64_t out_features,
                             int64_t in_features, int quant_type, void * stream);
+/* tgo_mmq_multi_forward with scaled operands of up to four projections of one format as one product over all their columns: the weights are
+ * unpacked into `scratch`, which holds tgo_multi_forward_scratch_bytes() bytes; `workspace`: tgo_q8_workspace_bytes().  0 bytes: such projections
+ * are better taken by tgo_mmq_multi_forward, whose results are the same bits, and the call is refused. */
+int64_t tgo_multi_forward_scratch_bytes(int count, const int64_t * out_features, const int * quant_types, int64_t rows, int64_t in_features);
+int tgo_mmq_multi_forward_unpacked(const void * input_bf16, int count, const void * const * packed, void * const * outputs_bf16,
+                                   const int64_t * out_features, const int * quant_types, void * workspace, void * scratch, int64_t rows,
+                                   int64_t in_features, void * stream);
 /* The gradient of the input of up to four projections of any shapes and formats, summed in fp32 and rounded once, as one product over
  * all their weight rows: the weights are unpacked into `workspace`, which holds tgo_multi_grad_workspace_bytes() bytes.  0 bytes:
  * projections of these sizes are better taken one by one, and the call is refused.  The arrays lie in host memory. */

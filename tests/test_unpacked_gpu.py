@@ -30,7 +30,7 @@ def _unpacks_gradient(rows, widths, k):
 
 # (rows, weight rows, K): 128 x 128 tiles, one row behind a tile and one short of it; odd reductions, which pack; 128 x 256 tiles; whole rounds of
 # 256 x 256 tiles and rows behind them, packed and not; more than eight row tiles, which are dealt out in bands
-GRADIENTS = [(257, 640, 768), (255, 623, 2304), (1731, 1859, 512), (4000, 1056, 2048), (4200, 544, 4096), (4133, 521, 4096), (9000, 96, 512)]
+GRADIENTS = [(257, 640, 768), (255, 623, 2304), (1731, 1859, 512), (4000, 1056, 2048), (4200, 1568, 4096), (4133, 1569, 4096), (9000, 96, 512)]
 
 
 @pytest.mark.parametrize("qname", tuple(QTYPES))
@@ -62,3 +62,65 @@ def test_gradient_of_several_projections(oracle, widths):
     (grad,) = torch.autograd.grad(outputs, x, grads)
     expected = sum(g.double() @ p for g, p in zip(grads, plain))
     assert_matches_f32_reference(grad, expected.cpu().numpy(), accumulate_noise=1e-5)
+
+
+# (rows, columns, K): as above, an odd number of steps with the minima's (K = 768, 1280), columns that end inside a tile, rows of 16-byte units
+# and not (Q3_K, Q6_K and IQ2_S of K = 768 and an odd number of columns)
+FORWARDS = [(2000, 2048, 2048), (1000, 5003, 1280), (545, 6017, 768), (8200, 769, 768), (9000, 520, 512), (4097, 4096, 1024), (500, 8192, 2816)]
+
+
+@pytest.mark.parametrize("qname", tuple(QTYPES))
+@pytest.mark.parametrize("rows,n,k", FORWARDS)
+def test_forward_has_the_bits_of_the_scaled_kernel(qname, rows, n, k):
+    """The same operands in the same order: a call without scratch, which the scaled kernel takes, gives the same bits.  Super-blocks far below
+    their row's largest one, a row of zeros, an infinity, and a weight row of zeros and of the format's largest scales among them."""
+    import synth
+    import torch_ggml_ops as tgo  # noqa: F401
+    from torch_ggml_ops import _native
+
+    qtype, lib = QTYPES[qname], _native.lib
+    if _native.forward_operand_for(qtype, rows, n) != "scaled":
+        pytest.skip("not a call with scaled operands")
+    packed = synth.random_packed_weight(qtype, (n,), k, seed=qtype + n)
+    packed[1] = 0
+    packed = packed.cuda()
+    x = random_bf16((rows, k), seed=rows)
+    x[3] = 0
+    x[5, 256:] *= 2.0**-20
+    x[6, :32] *= 2.0**-30
+    x[rows - 1, 7] = float("inf")
+    workspace = torch.empty(lib.tgo_q8_workspace_bytes(rows, k), dtype=torch.uint8, device="cuda")
+    outputs = []
+    for scratch_bytes in (0, lib.tgo_forward_scratch_bytes(rows, k, n, qtype)):
+        scratch = torch.empty(max(scratch_bytes, 16), dtype=torch.uint8, device="cuda")
+        # (whatever an earlier call left there must not be read)
+        scratch.fill_(0xFF)
+        workspace.fill_(0xFF)
+        output = torch.empty((rows, n), dtype=torch.bfloat16, device="cuda")
+        _native.check(
+            lib.tgo_mmq_forward_scratch(
+                x.data_ptr(), packed.data_ptr(), output.data_ptr(), workspace.data_ptr(), scratch.data_ptr() if scratch_bytes else None,
+                rows, k, n, qtype, _native.stream_of(x.device),
+            )
+        )
+        outputs.append(output.view(torch.int16))
+    assert torch.equal(*outputs)
+
+
+@pytest.mark.parametrize("qname", ("Q5_K", "IQ2_S"))
+@pytest.mark.parametrize("widths", [(2048, 512, 512), (2010, 500, 490, 70)])
+def test_forward_of_several_projections(qname, widths):
+    """One product over all columns: the bits of ``mmq_prepared``."""
+    import synth
+    import torch_ggml_ops as tgo
+    from torch_ggml_ops import _native, prepared
+
+    rows, k, qtype = 2000, 2048, QTYPES[qname]
+    count = len(widths)
+    assert prepared.multi_operand([qtype] * count, rows, widths) == "scaled"
+    assert _native.lib.tgo_multi_forward_scratch_bytes(count, (ctypes.c_int64 * count)(*widths), (ctypes.c_int * count)(*[qtype] * count), rows, k) > 0
+    packed = [synth.random_packed_weight(qtype, (n,), k, seed=3 + i).cuda() for i, n in enumerate(widths)]
+    x = random_bf16((rows, k), seed=2)
+    workspace = tgo.quantize_q8_1(x, "scaled")
+    for output, weight, n in zip(tgo.mmq_multi(x, packed, [qtype] * count, widths), packed, widths):
+        assert torch.equal(output, tgo.mmq_prepared(workspace, weight, rows, k, qtype, n, "scaled"))

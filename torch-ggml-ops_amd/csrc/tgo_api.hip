@@ -397,8 +397,10 @@ int64_t tgo_forward_scratch_bytes(int64_t rows, int64_t in_features, int64_t out
     }
     // (a prepared workspace may hold either kind of exact operands; the setting, by which some calls use no ranges, may change before
     // the call)
-    return std::max(tgo::forward_partial_bytes(rows, in_features, out_features, quant_type, tgo::OPERAND_INT8),
-                    tgo::forward_partial_bytes(rows, in_features, out_features, quant_type, tgo::OPERAND_HALF));
+    const int64_t unpacked = tgo::forward_unpacks(quant_type, rows, in_features, out_features)
+        ? tgo::unpacked_forward_bytes(quant_type, (out_features + 31) / 32, in_features) : 0;
+    return std::max({unpacked, tgo::forward_partial_bytes(rows, in_features, out_features, quant_type, tgo::OPERAND_INT8),
+                     tgo::forward_partial_bytes(rows, in_features, out_features, quant_type, tgo::OPERAND_HALF)});
 }
 
 int tgo_mmq_forward(const void * input_bf16, const void * packed, void * output_bf16, void * workspace,
@@ -450,8 +452,16 @@ int tgo_mmq_forward_scratch(const void * input_bf16, const void * packed, void *
                                                     static_cast<int>(out_features), quant_type, hip_stream),
                          "mmq_forward launch");
     }
-    const tgo::Q8Workspace view = tgo::q8_workspace_view(workspace, rows, in_features, tiles || tgo::use_gemv(rows, 0),
-                                                         tgo::forward_operand_kind(setting, quant_type, rows, out_features, 1));
+    const int kind = tgo::forward_operand_kind(setting, quant_type, rows, out_features, 1);
+    if (!tiles && scratch != nullptr && kind == tgo::OPERAND_SCALED && !tgo::use_gemv(rows, 0) &&
+        tgo::forward_unpacks(quant_type, rows, in_features, out_features)) {
+        const tgo::DenseSource source = {static_cast<const uint8_t *>(packed), nullptr, out_features, quant_type};
+        uint16_t * const output = static_cast<uint16_t *>(output_bf16);
+        return check_hip(tgo::launch_forward_unpacked(static_cast<const uint16_t *>(input_bf16), workspace, &source, &output, 1, scratch, rows,
+                                                      in_features, hip_stream),
+                         "mmq_forward launch");
+    }
+    const tgo::Q8Workspace view = tgo::q8_workspace_view(workspace, rows, in_features, tiles || tgo::use_gemv(rows, 0), kind);
     TGO_TRY(check_hip(tgo::launch_quantize_q8_1(static_cast<const uint16_t *>(input_bf16), view, rows, in_features,
                                                 hip_stream),
                       "quantize_q8_1 launch"));
@@ -562,6 +572,51 @@ int tgo_mmq_multi_forward(const void * input_bf16, int count, const void * const
         }
     }
     return TGO_OK;
+}
+
+int64_t tgo_multi_forward_scratch_bytes(int count, const int64_t * out_features, const int * quant_types, int64_t rows, int64_t in_features) {
+    if (count < 1 || count > tgo::UNPACKED_SOURCES || out_features == nullptr || quant_types == nullptr || rows <= 0 || in_features <= 0 ||
+        in_features % tgo::QK_K != 0 || tgo::use_gemv(rows, 0)) {
+        return 0;
+    }
+    int64_t total = 0, tiles = 0;
+    for (int i = 0; i < count; ++i) {
+        if (out_features[i] <= 0 || out_features[i] > INT_LIMIT || quant_types[i] != quant_types[0]) {
+            return 0;
+        }
+        total += out_features[i];
+        tiles += (out_features[i] + 31) / 32;
+    }
+    return tgo::forward_unpacks(quant_types[0], rows, in_features, total) ? tgo::unpacked_forward_bytes(quant_types[0], tiles, in_features) : 0;
+}
+
+int tgo_mmq_multi_forward_unpacked(const void * input_bf16, int count, const void * const * packed, void * const * outputs_bf16,
+                                   const int64_t * out_features, const int * quant_types, void * workspace, void * scratch, int64_t rows,
+                                   int64_t in_features, void * stream) {
+    TGO_TRY(check_pointer(input_bf16, "input"));
+    TGO_TRY(check_pointer(workspace, "workspace"));
+    TGO_TRY(check_pointer(scratch, "scratch"));
+    if (packed == nullptr || outputs_bf16 == nullptr || out_features == nullptr || quant_types == nullptr) {
+        return fail(TGO_ERR_INVALID, "packed, outputs_bf16, out_features and quant_types must not be null");
+    }
+    if (count < 1 || count > tgo::UNPACKED_SOURCES) {
+        return fail(TGO_ERR_INVALID, "between 1 and %d projections are required; got %d", tgo::UNPACKED_SOURCES, count);
+    }
+    tgo::DenseSource sources[tgo::UNPACKED_SOURCES];
+    uint16_t * outputs[tgo::UNPACKED_SOURCES];
+    for (int i = 0; i < count; ++i) {
+        TGO_TRY(check_matmul_shape(rows, in_features, out_features[i], quant_types[i]));
+        TGO_TRY(check_pointer(packed[i], "packed_weight"));
+        TGO_TRY(check_pointer(outputs_bf16[i], "output"));
+        sources[i] = {static_cast<const uint8_t *>(packed[i]), nullptr, out_features[i], quant_types[i]};
+        outputs[i] = static_cast<uint16_t *>(outputs_bf16[i]);
+    }
+    if (tgo_multi_forward_scratch_bytes(count, out_features, quant_types, rows, in_features) == 0) {
+        return fail(TGO_ERR_INVALID, "projections of these sizes and formats are taken one by one");
+    }
+    return check_hip(tgo::launch_forward_unpacked(static_cast<const uint16_t *>(input_bf16), workspace, sources, outputs, count, scratch, rows,
+                                                  in_features, static_cast<hipStream_t>(stream)),
+                     "mmq_multi_forward launch");
 }
 
 int tgo_mmq_grad_input(const void * grad_output_bf16, const void * packed, void * grad_input_bf16,

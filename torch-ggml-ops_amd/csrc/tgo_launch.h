@@ -582,31 +582,34 @@ struct ProductPlan {
     int rest_tile_rows, rest_tile_columns;
     float microseconds;
 };
-// One reduction step of 16 of `tiles` workgroups, 256 to a round: a round is the faster the emptier it is, down to `half` for half a
-// round, below which the CUs at work no longer gain from those that are idle.
+// `tiles` workgroups, 256 to a round: a round is the faster the emptier it is, down to `half` for half a round, below which the CUs at
+// work no longer gain from those that are idle.
 static inline float rounds_microseconds(int64_t tiles, float half, float whole) {
     const int64_t rounds = (tiles - 1) / 256;
     const float last = static_cast<float>(tiles - 256 * rounds);
     return static_cast<float>(rounds) * whole + (last <= 128.0f ? half : half + (whole - half) * (last - 128.0f) / 128.0f);
 }
-// Measured per reduction step of 16 (100 to 8192 rows, 2048 to 11008 columns, reduction 512 to 11008, bf16), half a round and a whole one:
-// 256 x 256 tiles 0.29 and 0.45 us, 128 x 256 0.18 and 0.27, 128 x 128 0.115 and 0.155, 0.145 for each of several rounds (two workgroups
-// share a CU).
+// Measured (100 to 8192 rows, 2048 to 28672 columns, reduction 512 to 11008), half a round and a whole one, per reduction step of 16 and for
+// the stores: 256 x 256 tiles 0.29 us + 5 and 0.42 + 9, 128 x 256 0.18 + 3 and 0.255 + 5, 128 x 128 0.115 + 3 and 0.15 + 4, each of several
+// rounds 0.125 + 2.5 (two workgroups share a CU).
 static inline ProductPlan product_plan(int64_t rows, int64_t columns, int64_t steps) {
     const auto up = [](int64_t count, int64_t tile) { return (count + tile - 1) / tile; };
     const int64_t across = up(columns, 256);
+    const float n = static_cast<float>(steps);
+    const auto large = [&](int64_t tiles) { return rounds_microseconds(tiles, 0.29f * n + 5.0f, 0.42f * n + 9.0f); };
     const auto with_rounds = [&](int64_t rounds, int64_t row_tiles) {
-        ProductPlan plan = {rounds * row_tiles * 256, 256, 256, static_cast<float>(rounds * steps) * rounds_microseconds(row_tiles * across, 0.29f, 0.45f)};
+        ProductPlan plan = {rounds * row_tiles * 256, 256, 256, static_cast<float>(rounds) * large(row_tiles * across)};
         const int64_t rest = rows - plan.full_rows;
         if (rest > 0) {
-            const float a = rounds_microseconds(up(rest, 256) * across, 0.29f, 0.45f);
-            const float b = rounds_microseconds(up(rest, 128) * across, 0.18f, 0.27f);
+            const float a = large(up(rest, 256) * across);
+            const float b = rounds_microseconds(up(rest, 128) * across, 0.18f * n + 3.0f, 0.255f * n + 5.0f);
             const int64_t small = up(rest, 128) * up(columns, 128);
-            const float c = small <= 256 ? rounds_microseconds(small, 0.115f, 0.155f) : static_cast<float>(up(small, 256)) * 0.145f;
+            const float c = small <= 256 ? rounds_microseconds(small, 0.115f * n + 3.0f, 0.15f * n + 4.0f)
+                                         : static_cast<float>(up(small, 256)) * (0.125f * n + 2.5f) + 3.0f;
             const float least = std::min(a, std::min(b, c));
             plan.rest_tile_rows = least == a ? 256 : 128;
             plan.rest_tile_columns = least == a || least == b ? 256 : 128;
-            plan.microseconds += static_cast<float>(steps) * least + 4.0f;
+            plan.microseconds += least + (rounds > 0 ? 4.0f : 0.0f);
         }
         return plan;
     };
@@ -666,5 +669,49 @@ static inline bool multi_grad_unpacks(int64_t rows, int64_t out_features, int64_
 // unpacked_grad_workspace().bytes.
 hipError_t launch_grad_input_unpacked(const DenseSource * sources, int count, void * workspace, uint16_t * grad_input, int64_t rows,
                                       int64_t in_features, hipStream_t stream);
+
+// Reduction steps of 16 of the forward: with Q4_K (12) and Q5_K (13) one more per super-block, for the minima, and an even number.
+static inline int64_t unpacked_forward_steps(int quant_type, int64_t in_features) {
+    const int64_t super_blocks = in_features / 256;
+    return quant_type == 12 || quant_type == 13 ? (17 * super_blocks + 1) / 2 * 2 : 16 * super_blocks;
+}
+// Scratch: the slabs of `tiles` times 32 weight rows and their powers.  (The activations fit the q8_1 workspace: 2.125 bytes per value and
+// 36 per row of the 2.3 and 4 that it holds.)
+static inline int64_t unpacked_forward_bytes(int quant_type, int64_t tiles, int64_t in_features) {
+    return tiles * (unpacked_forward_steps(quant_type, in_features) * 1024 + 128);
+}
+// Whether a dense forward call with scaled operands unpacks its weights once (tgo_unpacked.hip) or leaves it to the unpacking waves of
+// every workgroup (tgo_forward_scaled.hip): by what either takes.  The latter quantizes in two launches, then runs items of 256 x 128 on
+// persistent workgroups, half a round and a whole round of 256 in 0.19 and 0.27 us per step of 16 (Q6_K 0.31) and 1.3 for the stores, or of 128
+// x 128 (forward_split) in 0.145 and 0.185, the slower formats to unpack 0.22.
+// Results of more than 100 million values no longer stay in the last cache, which only the kernel without an overlapped epilogue notices.
+// Of the time of the scaled kernel, where this rule leaves it (100 calls of 300 to 16000 rows, 512 to 28672 columns, K 512 to 8192): 0.83 on the
+// mean, 0.38 (Q6_K, rows of which no tile is a whole number of 16-byte units) to 1.05.  4096 x 4096, 4096 rows: Q4_K 173 -> 152 us, Q3_K 178 ->
+// 144, Q6_K 196 -> 147; 2048 x 2048, 2000 rows Q4_K 43.7 -> 34.8.  On the other side of it, always unpacked: 28672 x 8192, 300 rows Q4_K 235 -> 389 us;
+// 16384 x 1024, 8192 rows Q4_K 315 -> 367.
+static inline bool forward_unpacks(int quant_type, int64_t rows, int64_t in_features, int64_t out_features) {
+    const int64_t tiles = ((rows + 255) / 256) * ((out_features + 127) / 128);
+    if (!scaled_forward_format(quant_type) || tiles < SCALED_AUTO_MIN_TILES || out_features > (1 << 24) ||
+        out_features * in_features > (INT64_C(1) << 29) || rows > (1 << 24)) {
+        return false;
+    }
+    const float input = static_cast<float>(rows) * static_cast<float>(in_features), results = static_cast<float>(rows) * static_cast<float>(out_features);
+    const float steps = static_cast<float>(in_features / 16);
+    const bool quick = quant_type == 12 || quant_type == 13;
+    const int row_tile = forward_split(rows, in_features, out_features, quant_type, OPERAND_SCALED, false).row_tile;
+    const float half = row_tile == 128 ? (quick ? 0.145f : 0.19f) : quant_type == 14 ? 0.22f : 0.19f;
+    const float whole = row_tile == 128 ? (quick ? 0.185f : 0.22f) : quant_type == 14 ? 0.311f : 0.273f;
+    const int64_t items = ((rows + row_tile - 1) / row_tile) * ((out_features + 127) / 128);
+    const float together = (row_tile == 128 ? 12.0f : 16.0f) + input * 1.0e-6f + rounds_microseconds(items, half * steps + 1.3f, whole * steps + 1.3f);
+    const float apart = unpack_microseconds(out_features, in_features) + input * 0.9e-6f + (results > 1.0e8f ? results * 0.3e-6f : 0.0f) +
+                        product_plan(rows, out_features, unpacked_forward_steps(quant_type, in_features)).microseconds;
+    // (short reductions, but for those of Q6_K, are what the model is least sure of)
+    const float margin = quant_type == 14 ? 1.03f : 1.02f + 128.0f / static_cast<float>(in_features);
+    return margin * apart < together;
+}
+// y[i] = x W[i]^T for up to four projections of one format: the bits of the scaled kernel.  `workspace`: q8_workspace_bytes(),
+// `scratch`: unpacked_forward_bytes() of all tiles of 32 weight rows.
+hipError_t launch_forward_unpacked(const uint16_t * input, void * workspace, const DenseSource * sources, uint16_t * const * outputs, int count,
+                                   void * scratch, int64_t rows, int64_t in_features, hipStream_t stream);
 
 }  // namespace tgo

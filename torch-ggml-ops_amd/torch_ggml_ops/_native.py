@@ -69,6 +69,11 @@ lib.tgo_multi_grad_workspace_bytes.restype = _i64
 lib.tgo_mmq_multi_grad_input.argtypes = [
     _int, ctypes.POINTER(_p), ctypes.POINTER(_p), ctypes.POINTER(_i64), ctypes.POINTER(_int), _p, _p, _i64, _i64, _p,
 ]
+lib.tgo_multi_forward_scratch_bytes.argtypes = [_int, ctypes.POINTER(_i64), ctypes.POINTER(_int), _i64, _i64]
+lib.tgo_multi_forward_scratch_bytes.restype = _i64
+lib.tgo_mmq_multi_forward_unpacked.argtypes = [
+    _p, _int, ctypes.POINTER(_p), ctypes.POINTER(_p), ctypes.POINTER(_i64), ctypes.POINTER(_int), _p, _p, _i64, _i64, _p,
+]
 lib.tgo_mmq_forward_static.argtypes = [_p, _p, _p, _i64, _i64, _i64, _int, _p]
 lib.tgo_mmq_forward_prepared.argtypes = [_p, _p, _p, _i64, _i64, _i64, _int, _p]
 lib.tgo_quantize_q8_1_as.argtypes = [_p, _p, _i64, _i64, _int, _p]
@@ -131,6 +136,8 @@ EXPORTS = (
     "tgo_mmq_pair_grad_input",
     "tgo_multi_grad_workspace_bytes",
     "tgo_mmq_multi_grad_input",
+    "tgo_multi_forward_scratch_bytes",
+    "tgo_mmq_multi_forward_unpacked",
     "tgo_mmq_forward_static",
     "tgo_mmq_forward_prepared",
     "tgo_quantize_q8_1_as",

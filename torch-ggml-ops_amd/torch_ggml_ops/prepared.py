@@ -137,19 +137,33 @@ def _multi_device(input, packed_weights, quant_types, out_features, operand):
         for weight, quant_type, features in zip(packed_weights, quant_types, out_features):
             _validate.prepared(workspace, weight, rows, in_features, quant_type, features)
         outputs = [input.new_empty((*input.shape[:-1], features)) for features in out_features]
+        count = len(outputs)
+        pointers = ctypes.c_void_p * count
+        widths, types = (ctypes.c_int64 * count)(*out_features), (ctypes.c_int * count)(*quant_types)
+        projections = (
+            input.data_ptr(), count, pointers(*(w.data_ptr() for w in packed_weights)),
+            pointers(*(o.data_ptr() for o in outputs)), widths, types, workspace.data_ptr(),
+        )
+        # one product over the columns of all projections, where that pays: the same bits
+        unpacked_bytes = (
+            _native.lib.tgo_multi_forward_scratch_bytes(count, widths, types, rows, in_features) if operand == "scaled" else 0
+        )
+        if unpacked_bytes > 0:
+            scratch = input.new_empty((unpacked_bytes,), dtype=torch.uint8)
+            _native.check(
+                _native.lib.tgo_mmq_multi_forward_unpacked(
+                    *projections, scratch.data_ptr(), rows, in_features, _stream(input)
+                )
+            )
+            return outputs
         scratch_bytes = max(
             _native.forward_scratch_bytes(rows, in_features, features, quant_type)
             for quant_type, features in zip(quant_types, out_features)
         )
         scratch = input.new_empty((scratch_bytes,), dtype=torch.uint8) if scratch_bytes > 0 else None
-        count = len(outputs)
-        pointers = ctypes.c_void_p * count
         _native.check(
             _native.lib.tgo_mmq_multi_forward(
-                input.data_ptr(), count, pointers(*(w.data_ptr() for w in packed_weights)),
-                pointers(*(o.data_ptr() for o in outputs)), (ctypes.c_int64 * count)(*out_features),
-                (ctypes.c_int * count)(*quant_types), workspace.data_ptr(), None if scratch is None else scratch.data_ptr(),
-                rows, in_features, kind, _stream(input),
+                *projections, None if scratch is None else scratch.data_ptr(), rows, in_features, kind, _stream(input)
             )
         )
     return outputs
