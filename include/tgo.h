@@ -330,6 +330,19 @@ int tgo_moe_combine(const void * rows_bf16, const int64_t * slot_rows, const flo
                     void * output_bf16, int64_t tokens, int64_t top_k, int64_t num_rows, int64_t features,
                     void * stream);
 
+/* A whole mixture-of-experts layer without a gradient for a few tokens, in two launches:
+ * output[t] = sum over j of slot_weights[t, j] * down[e](silu(gate[e](hidden[t])) * up[e](hidden[t])), e = slot_experts[t, j]; choices outside
+ * [0, num_experts) contribute nothing.  q8_1 activations as everywhere, gate, up and their product rounded to bf16, the sum over the experts
+ * in fp32 and rounded once.  `workspace` holds tgo_moe_decode_workspace_bytes() bytes; 0 bytes: a layer of these sizes is better taken by
+ * tgo_route, tgo_grouped_mmq_swiglu, tgo_grouped_mmq_forward and tgo_moe_combine, and the call is refused.  No counterpart in the
+ * reference. */
+int64_t tgo_moe_decode_workspace_bytes(int64_t tokens, int64_t top_k, int64_t num_experts, int64_t features, int64_t intermediate,
+                                       int gate_up_type, int down_type);
+int tgo_moe_decode(const void * hidden_bf16, const int64_t * slot_experts, const float * slot_weights, const void * gate, const void * up,
+                   const void * down, void * output_bf16, void * workspace, int64_t tokens, int64_t top_k, int64_t num_experts,
+                   int64_t features, int64_t intermediate, int gate_up_type, int down_type, void * stream);
+
+
 /* Grouped grad-input.  With `grad_output_second`/`packed_second` set, both Jacobian products
  * are summed in one fp32 accumulator and rounded once.  `workspace` holds
  * tgo_grad_workspace_bytes(rows, out_features, num_groups, 1 or 2) bytes.

@@ -969,6 +969,39 @@ int tgo_swiglu_backward(const void * gate_bf16, const void * up_bf16, const void
                      "swiglu_backward launch");
 }
 
+int64_t tgo_moe_decode_workspace_bytes(int64_t tokens, int64_t top_k, int64_t num_experts, int64_t features, int64_t intermediate,
+                                       int gate_up_type, int down_type) {
+    if (tokens <= 0 || top_k <= 0 || num_experts <= 0 || features <= 0 || intermediate <= 0 || tgo::block_bytes(gate_up_type) == 0 ||
+        tgo::block_bytes(down_type) == 0 || tokens > INT_LIMIT || top_k > INT_LIMIT || num_experts > INT_LIMIT ||
+        !tgo::moe_decodes(tokens, top_k, num_experts, features, intermediate)) {
+        return 0;
+    }
+    return tokens * top_k * intermediate * 2;
+}
+
+int tgo_moe_decode(const void * hidden_bf16, const int64_t * slot_experts, const float * slot_weights, const void * gate, const void * up,
+                   const void * down, void * output_bf16, void * workspace, int64_t tokens, int64_t top_k, int64_t num_experts,
+                   int64_t features, int64_t intermediate, int gate_up_type, int down_type, void * stream) {
+    TGO_TRY(check_pointer(hidden_bf16, "hidden"));
+    TGO_TRY(check_pointer(gate, "gate_weight"));
+    TGO_TRY(check_pointer(up, "up_weight"));
+    TGO_TRY(check_pointer(down, "down_weight"));
+    TGO_TRY(check_pointer(output_bf16, "output"));
+    TGO_TRY(check_pointer(workspace, "workspace"));
+    if (slot_experts == nullptr || slot_weights == nullptr) {
+        return fail(TGO_ERR_INVALID, "slot_experts and slot_weights must not be null");
+    }
+    if (tgo_moe_decode_workspace_bytes(tokens, top_k, num_experts, features, intermediate, gate_up_type, down_type) == 0) {
+        return fail(TGO_ERR_INVALID, "a layer of these sizes and formats is not taken by tgo_moe_decode");
+    }
+    const tgo::MoeDecodeArgs args = {static_cast<const uint16_t *>(hidden_bf16), slot_experts, slot_weights,
+                                     static_cast<const uint8_t *>(gate), static_cast<const uint8_t *>(up), static_cast<const uint8_t *>(down),
+                                     static_cast<uint16_t *>(workspace), static_cast<uint16_t *>(output_bf16), static_cast<int>(tokens),
+                                     static_cast<int>(top_k), static_cast<int>(tokens * top_k), static_cast<int>(num_experts),
+                                     static_cast<int>(features), static_cast<int>(intermediate)};
+    return check_hip(tgo::launch_moe_decode(args, gate_up_type, down_type, static_cast<hipStream_t>(stream)), "moe_decode launch");
+}
+
 int tgo_moe_combine(const void * rows_bf16, const int64_t * slot_rows, const float * slot_weights,
                     void * output_bf16, int64_t tokens, int64_t top_k, int64_t num_rows, int64_t features,
                     void * stream) {

@@ -3,7 +3,7 @@
 //
 // What bounds a decode-sized call is the host: 15 us for one projection whose kernel takes 6, 67 us for a
 // mixture-of-experts layer whose five kernels take 23.  Here the projection costs two allocations and a launch, the layer two
-// allocations and its launches.
+// allocations and its launches, of which a layer of a few tokens has two (tgo_moe_decode).
 //
 // A function returns None for every call that is not plainly its own -- a gradient may be wanted, a tensor is not an ordinary
 // device tensor, a transform, a mode or a tracer is active, an argument would not pass the operator's checks -- and its
@@ -185,35 +185,45 @@ PyObject * direct_moe_layer(PyObject *, PyObject * const * args, Py_ssize_t coun
         pybind11::gil_scoped_release release;
         RECORD_FUNCTION("torch_ggml_ops::moe_layer", c10::ArrayRef<const c10::IValue>());
         output = at::detail::empty_cuda({tokens, features}, at::kBFloat16, hidden.device(), std::nullopt);
-        Pieces pieces;
-        const int64_t row_index = pieces.take(slots * 8), slot_rows = pieces.take(slots * 8), indices = pieces.take(experts * 8),
-                      offsets = pieces.take(experts * 4), activated = pieces.take(slots * intermediate * 2),
-                      rows = pieces.take(slots * std::max(features, intermediate) * 2),   // the gate, then the expert-sorted results
-                      route_workspace = pieces.take(tgo_route_workspace_bytes(slots, experts)),
-                      workspace = pieces.take(tgo_q8_workspace_bytes(slots, std::max(features, intermediate)) +
-                                              tgo_task_workspace_bytes(slots, experts));
-        const c10::DataPtr memory = c10::GetAllocator(c10::kCUDA)->allocate(pieces.bytes);
-        uint8_t * const base = static_cast<uint8_t *>(memory.get());
-        int64_t * const index = reinterpret_cast<int64_t *>(base + row_index);
-        int64_t * const of_slot = reinterpret_cast<int64_t *>(base + slot_rows);
-        int64_t * const group_expert = reinterpret_cast<int64_t *>(base + indices);
-        int32_t * const group_end = reinterpret_cast<int32_t *>(base + offsets);
-        void * const stream = c10::hip::getCurrentHIPStream(device).stream();
-        status = tgo_route(slot_experts.const_data_ptr<int64_t>(), tokens, top_k, experts, index, of_slot, group_expert, group_end,
-                           base + route_workspace, stream);
-        if (status == TGO_OK) {
-            status = tgo_grouped_mmq_swiglu(hidden.data_ptr(), index, tokens, gate.data_ptr(), up.data_ptr(), base + rows,
-                                            base + activated, group_expert, group_end, base + workspace, slots, features,
-                                            intermediate, experts, experts, static_cast<int>(gate_up_type), stream);
-        }
-        if (status == TGO_OK) {
-            status = tgo_grouped_mmq_forward(base + activated, down.data_ptr(), nullptr, base + rows, nullptr, group_expert,
-                                             group_end, base + workspace, slots, intermediate, features, down.size(0), experts,
-                                             static_cast<int>(down_type), stream);
-        }
-        if (status == TGO_OK) {
-            status = tgo_moe_combine(base + rows, of_slot, slot_weights.const_data_ptr<float>(), output.data_ptr(), tokens, top_k,
-                                     slots, features, stream);
+        const int64_t decode_bytes = tgo_moe_decode_workspace_bytes(tokens, top_k, experts, features, intermediate, static_cast<int>(gate_up_type),
+                                                                    static_cast<int>(down_type));
+        if (decode_bytes > 0) {
+            const c10::DataPtr memory = c10::GetAllocator(c10::kCUDA)->allocate(decode_bytes);
+            status = tgo_moe_decode(hidden.data_ptr(), slot_experts.const_data_ptr<int64_t>(), slot_weights.const_data_ptr<float>(),
+                                    gate.data_ptr(), up.data_ptr(), down.data_ptr(), output.data_ptr(), memory.get(), tokens, top_k, experts,
+                                    features, intermediate, static_cast<int>(gate_up_type), static_cast<int>(down_type),
+                                    c10::hip::getCurrentHIPStream(device).stream());
+        } else {
+            Pieces pieces;
+            const int64_t row_index = pieces.take(slots * 8), slot_rows = pieces.take(slots * 8), indices = pieces.take(experts * 8),
+                          offsets = pieces.take(experts * 4), activated = pieces.take(slots * intermediate * 2),
+                          rows = pieces.take(slots * std::max(features, intermediate) * 2),   // the gate, then the expert-sorted results
+                          route_workspace = pieces.take(tgo_route_workspace_bytes(slots, experts)),
+                          workspace = pieces.take(tgo_q8_workspace_bytes(slots, std::max(features, intermediate)) +
+                                                  tgo_task_workspace_bytes(slots, experts));
+            const c10::DataPtr memory = c10::GetAllocator(c10::kCUDA)->allocate(pieces.bytes);
+            uint8_t * const base = static_cast<uint8_t *>(memory.get());
+            int64_t * const index = reinterpret_cast<int64_t *>(base + row_index);
+            int64_t * const of_slot = reinterpret_cast<int64_t *>(base + slot_rows);
+            int64_t * const group_expert = reinterpret_cast<int64_t *>(base + indices);
+            int32_t * const group_end = reinterpret_cast<int32_t *>(base + offsets);
+            void * const stream = c10::hip::getCurrentHIPStream(device).stream();
+            status = tgo_route(slot_experts.const_data_ptr<int64_t>(), tokens, top_k, experts, index, of_slot, group_expert, group_end,
+                               base + route_workspace, stream);
+            if (status == TGO_OK) {
+                status = tgo_grouped_mmq_swiglu(hidden.data_ptr(), index, tokens, gate.data_ptr(), up.data_ptr(), base + rows,
+                                                base + activated, group_expert, group_end, base + workspace, slots, features,
+                                                intermediate, experts, experts, static_cast<int>(gate_up_type), stream);
+            }
+            if (status == TGO_OK) {
+                status = tgo_grouped_mmq_forward(base + activated, down.data_ptr(), nullptr, base + rows, nullptr, group_expert,
+                                                 group_end, base + workspace, slots, intermediate, features, down.size(0), experts,
+                                                 static_cast<int>(down_type), stream);
+            }
+            if (status == TGO_OK) {
+                status = tgo_moe_combine(base + rows, of_slot, slot_weights.const_data_ptr<float>(), output.data_ptr(), tokens, top_k,
+                                         slots, features, stream);
+            }
         }
     }
     return finished(status, output);

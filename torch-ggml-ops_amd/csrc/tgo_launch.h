@@ -714,4 +714,30 @@ static inline bool forward_unpacks(int quant_type, int64_t rows, int64_t in_feat
 hipError_t launch_forward_unpacked(const uint16_t * input, void * workspace, const DenseSource * sources, uint16_t * const * outputs, int count,
                                    void * scratch, int64_t rows, int64_t in_features, hipStream_t stream);
 
+// ---- a mixture-of-experts layer of a few tokens (tgo_moe_decode.hip) ----
+constexpr int MOE_DECODE_SLOTS = 64;
+constexpr int MOE_DECODE_TOP_K = 8;
+struct MoeDecodeArgs {
+    const uint16_t * hidden;        // [tokens][features]
+    const int64_t * slot_experts;   // [tokens][top_k]
+    const float * slot_weights;
+    const uint8_t * gate, * up, * down;
+    uint16_t * activated;           // [slots][intermediate]
+    uint16_t * output;              // [tokens][features]
+    int tokens, top_k, slots, experts, features, intermediate;
+};
+// Layers that take it: 64 slots at most (its waves look them over a slot per lane), and as long as the tokens' experts are mostly
+// different ones: every token unpacks its experts' down projections again.  Of the time of routing, grouped kernels and combine, eight layers with
+// weights of their own in a graph, all formats: a token 0.42 to 0.66 (256 experts of 2048 x 512, IQ2_S and Q6_K: 22.9 -> 12.0 us), six tokens of
+// 256 experts with power-law 0.3 routing 0.56 to 0.67 (50.5 -> 32.1), of 128 experts of 2048 x 768 with power-law 1.1 routing 0.66 to 0.90, five
+// of 64 of 4096 x 1024 0.83 to 0.94.  Beyond the lines: 8 tokens of 128 of 2048 x 768, 1.1: 0.71 to 1.05; 8 of 64 of 4096 x 1024: 0.98 to 1.29; 16 of
+// 256 of 2048 x 512: 0.77 to 0.92 at 0.3, 1.08 to 1.35 at 1.1.  Experts of less than half a million weights keep the operators, and with them
+// the operators' bits: those round every expert's row before they add it, and their sums have another order.
+static inline bool moe_decodes(int64_t tokens, int64_t top_k, int64_t experts, int64_t features, int64_t intermediate) {
+    const int64_t slots = tokens * top_k;
+    return top_k <= MOE_DECODE_TOP_K && slots <= MOE_DECODE_SLOTS && features % 256 == 0 && features <= 4096 && intermediate % 256 == 0 &&
+           intermediate <= 1024 && experts > 0 && features * intermediate >= (1 << 19) && slots * features * intermediate <= (slots <= 32 ? INT64_C(1) << 27 : INT64_C(96000000));
+}
+hipError_t launch_moe_decode(const MoeDecodeArgs & args, int gate_up_type, int down_type, hipStream_t stream);
+
 }  // namespace tgo

@@ -74,6 +74,9 @@ lib.tgo_multi_forward_scratch_bytes.restype = _i64
 lib.tgo_mmq_multi_forward_unpacked.argtypes = [
     _p, _int, ctypes.POINTER(_p), ctypes.POINTER(_p), ctypes.POINTER(_i64), ctypes.POINTER(_int), _p, _p, _i64, _i64, _p,
 ]
+lib.tgo_moe_decode_workspace_bytes.argtypes = [_i64, _i64, _i64, _i64, _i64, _int, _int]
+lib.tgo_moe_decode_workspace_bytes.restype = _i64
+lib.tgo_moe_decode.argtypes = [_p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _int, _int, _p]
 lib.tgo_mmq_forward_static.argtypes = [_p, _p, _p, _i64, _i64, _i64, _int, _p]
 lib.tgo_mmq_forward_prepared.argtypes = [_p, _p, _p, _i64, _i64, _i64, _int, _p]
 lib.tgo_quantize_q8_1_as.argtypes = [_p, _p, _i64, _i64, _int, _p]
@@ -159,6 +162,8 @@ EXPORTS = (
     "tgo_scale_bf16",
     "tgo_rows_to_tokens",
     "tgo_moe_combine",
+    "tgo_moe_decode_workspace_bytes",
+    "tgo_moe_decode",
     "tgo_grouped_mmq_grad_input",
     "tgo_grouped_mmq_grad_input_weighted",
     "tgo_profile_enable",
