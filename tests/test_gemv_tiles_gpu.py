@@ -94,6 +94,23 @@ def test_dense_beyond_the_decode_regime(oracle, qname, rows, n, k):
 
 
 @pytest.mark.parametrize("qname", tuple(QTYPES))
+@pytest.mark.parametrize("rows,n,k,taken", [(17, 256, 512, True), (31, 16, 8192, True), (32, 1040, 2304, True), (24, 2064, 1024, True), (33, 256, 512, False),
+                                            (20, 480, 256, False), (32, 520, 1024, False)])
+def test_dense_decode_on_few_weights(oracle, qname, rows, n, k, taken):
+    """From 2^17 to below 2^22 weights: one tile of weight rows, a last workgroup that lacks tiles, a task of one row less than two, the most rows
+    and one more, too few weights, a matrix that is not made of whole tiles."""
+    import synth
+    import torch_ggml_ops as tgo
+    from torch_ggml_ops import _native
+
+    qtype = QTYPES[qname]
+    assert (_native.forward_kernel_for(qtype, rows, k, n) == "tiles") == taken
+    host = synth.random_packed_weight(qtype, (n,), k, seed=qtype + rows)
+    x = random_bf16((rows, k), seed=rows)
+    assert_matches_f32_reference(tgo.mmq(x, host.cuda(), qtype, n), oracle.mmq_forward(qtype, bits(x), host.numpy(), n, k))
+
+
+@pytest.mark.parametrize("qname", tuple(QTYPES))
 def test_grouped_and_dense_calls_on_this_kernel_have_the_same_bits(qname):
     """Groups of 1 to 50 rows of a grouped call that averages eleven, and a dense call on each of them: where both run on this kernel, the
     same bits."""

@@ -193,14 +193,15 @@ static inline bool use_gemv(int64_t rows, int64_t groups) {
 }
 
 // Whether the layout of the kernel for tasks of several rows (tgo_gemv_tiles.hip) allows a call: whole tiles of 16 weight rows (with
-// them every expert is 16-byte aligned, as the entry points demand of the weights), offsets within a tile of 32 bits, and four million
-// weights that are read.
+// them every expert is 16-byte aligned, as the entry points demand of the weights), offsets within a tile of 32 bits, and enough weights that
+// are read: four million in grouped calls (fewer: their time is their launches and latencies, and most of them are one launch of the other
+// kernel), a hundred thousand in dense ones (of the decode regime; dense_takes_tiles asks for four million).
 static inline bool tiles_fit(int64_t rows, int64_t groups, int64_t in_features, int64_t out_features) {
     if (out_features % 16 != 0 || in_features > (INT64_C(1) << 22) || rows > (1 << 24)) {
         return false;
     }
     const int64_t matrices = groups <= 0 ? 1 : rows < groups ? rows : groups;
-    return matrices * out_features * in_features >= (INT64_C(1) << 22);
+    return matrices * out_features * in_features >= (groups <= 0 ? INT64_C(1) << 17 : INT64_C(1) << 22);
 }
 // Decode-regime calls that take the kernel for tasks of several rows (tgo_gemv_tiles.hip), which unpacks every weight once
 // per task, instead of those of tgo_gemv.hip, whose dot products cost the same again for every row.  It needs whole tiles of
@@ -210,10 +211,9 @@ static inline bool tiles_fit(int64_t rows, int64_t groups, int64_t in_features, 
 //    instructions to pay; Q3_K and IQ2_S from 16 and 24 rows.  Q6_K, whose unpacking is the longest: from 16 rows if K is three or
 //    four super-blocks, from half as many rows as groups below that (the other kernel folds rows there), from one and a half
 //    times as many above.
-//  - calls of fewer than four million weights never: their time is their launches and latencies, and most of them are one
-//    launch of the other kernel.
 //  - dense matrices that fill the chip: Q3_K always (28672 x 8192, one row: 54 -> 41 us), Q5_K, Q6_K and IQ2_S from three rows (80 ->
-//    65 us for Q6_K), Q4_K from four.  Smaller ones: Q3_K and IQ2_S from five rows, Q6_K from nine, Q4_K and Q5_K beyond 16.
+//    65 us for Q6_K), Q4_K from four.  Smaller ones: Q3_K and IQ2_S from five rows, Q6_K from nine, Q4_K and Q5_K beyond 16 (1024 x 2048: 5 rows
+//    Q3_K 8.8 -> 7.9 us, 12 rows Q6_K 12.6 -> 11.0, 32 rows Q4_K 10.6 -> 8.8, IQ2_S 20.2 -> 9.8; 512 x 512, 32 rows: Q3_K 24.3 -> 7.3).
 constexpr int GEMV_TILES_ROWS = 16;              // rows of its tasks
 constexpr int64_t GEMV_TILES_WORKGROUPS = 384;   // workgroups that a launch should have for a wave to take four tiles of 16 weight rows instead of two
 static inline bool gemv_takes_tiles(int64_t rows, int64_t groups, int64_t in_features, int64_t out_features, int quant_type) {
@@ -260,6 +260,9 @@ static inline bool dense_takes_tiles(int setting, int64_t rows, int64_t in_featu
     const int64_t weights = out_features * in_features;
     const bool quick = quant_type == 12 || quant_type == 13;   // (to unpack, for the other kernels)
     if (in_features > (quick ? 8192 : quant_type == 22 ? 12288 : 1 << 22)) {
+        return false;
+    }
+    if (weights < (INT64_C(1) << 22)) {
         return false;
     }
     if (weights <= (INT64_C(1) << 23)) {
