@@ -1380,13 +1380,28 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
 // workgroup barrier), one barrier per step publishes the tile, and then every wave multiplies the task's rows with
 // one 32-column slice of it (4 or 8 matrix instructions).  Small footprint: three workgroups share a CU, so one's
 // barrier and memory waits are covered by the others' decoding.  One workgroup per (task, column tile).
-// Q4_K / Q5_K fetch their blocks as the 16-byte units they consist of and have the block-scale stage; the other
-// formats fetch the aligned units that cover their blocks (wide_fetch, callers check wide_stage_ok) and decode
-// 16-value units straight from the parked blocks.
+// Q4_K / Q5_K fetch their blocks as the 16-byte units they consist of; the other formats fetch the aligned units that cover their blocks
+// (wide_fetch, callers check wide_stage_ok).  A lane decodes 32 values of one weight row and stores them along K; the transposition to the fragments'
+// order happens in the reads (ds_read_b64_tr_b16).  Against a lane that decodes four values of eight rows and stores a transposed tile
+// (24 four- and eight-byte reads of LDS per lane and step instead of three of 16 bytes): groups of 8192 tokens with power-law 1.1 routing over 256
+// experts of 2 x 512 x 2048 Q5_K 133 -> 115 us, 4096 tokens with 0.3, 512 x 2048 Q5_K 57 -> 48, 2 x 512 x 2048 IQ2_S 93 -> 86.  Bound by the
+// vector unit (0.53 of the time at 2.7 waves per SIMD; LDS 0.42, of which a third bank conflicts, matrix cores 0.11).
 constexpr int BSH_THREADS = 256;
 constexpr int BSH_ROWS_PER_WAVE = BWD_NS / 4;
-constexpr int BSH_SM_PITCH = BSH_ROWS_PER_WAVE + 1;
 constexpr int BSH_DEPTH = 2;
+
+// The tile lies as the weights do, [weight row][K column], and is transposed on its way out (the fragments want eight weight rows of a column
+// per lane).  The 16-byte granules of a row are exchanged by the row's number, so that the lanes which the LDS serves together, eight that store
+// along two rows or 16 that read from four, find theirs on different banks.
+constexpr int BSH_TILE_PITCH = BWD_TK * 2;
+TGO_DEVICE int tile_granule(int row, int granule) { return granule ^ ((row & 3) * 5); }
+TGO_DEVICE v8bf transposed_fragment(const uint8_t * first, const uint8_t * second) {
+    typedef short four_t __attribute__((ext_vector_type(4)));
+    typedef short eight_t __attribute__((ext_vector_type(8)));
+    const four_t low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) four_t *)(first));
+    const four_t high = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) four_t *)(second));
+    return __builtin_bit_cast(v8bf, eight_t{low.x, low.y, low.z, low.w, high.x, high.y, high.z, high.w});
+}
 
 template <int TYPE>
 __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(const BackwardArgs a) {
@@ -1399,9 +1414,8 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
     constexpr int SLOT_PITCH = K45 ? BSH_RAW_PITCH : W::PITCH;
     constexpr int SLOT_FRONT = K45 ? 0 : W::FRONT;
     constexpr int QS = TYPE == Q4_K ? 16 : 48;
-    __shared__ __attribute__((aligned(16))) uint16_t wb[2][BWD_TK * BWD_PITCH];
+    __shared__ __attribute__((aligned(16))) uint8_t wb[2][BWD_NS * BSH_TILE_PITCH];   // [weight row][K column], bf16 (tile_granule)
     __shared__ __attribute__((aligned(16))) uint8_t raw_all[4][BSH_ROWS_PER_WAVE * SLOT_PITCH];
-    __shared__ float2 scale_min_all[K45 ? 4 : 1][4 * BSH_SM_PITCH];
     // (the magnitude grid, not the 16 KiB selector table of decode16_bf16: with that table only two of these
     // workgroups fit a CU instead of three, which costs more than the cheaper decode brings -- measured)
     __shared__ uint2 grid[TYPE == IQ2_S ? TGO_IQ2S_GRID_ENTRIES : 1];
@@ -1431,7 +1445,6 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
     const int last = steps - 1;
 
     uint8_t * const raw = raw_all[wave];
-    float2 * const scale_min = scale_min_all[K45 ? wave : 0];
     if constexpr (TYPE == IQ2_S) {
         expand_iq2s_grid(grid, tid, BSH_THREADS);   // (visible after the barrier that follows the first decode's inputs)
         __syncthreads();
@@ -1508,95 +1521,68 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
     };
-    // (d * sc, dmin * m) of this lane's (row, 32-value group); rows past the end of the weight matrix get (0, 0)
-    // and therefore decode to exact zeros
-    auto scales = [&](int step) __attribute__((always_inline)) {
-        const int n = lane & 15;
-        const int group_local = lane >> 4;
-        const uint8_t * blk = raw + n * BSH_RAW_PITCH;
-        const uint32_t d_dmin = lds_u32(blk), low = lds_u32(blk + 4), mid = lds_u32(blk + 8), high = lds_u32(blk + 12);
-        const int shift = 8 * group_local;
-        const uint32_t b0 = (low >> shift) & 0xffu, b1 = (mid >> shift) & 0xffu, b2 = (high >> shift) & 0xffu;
-        uint32_t sc, mn;
-        if (half_block == 0) {   // groups 0..3 of the super-block: plain 6-bit fields
-            sc = b0 & 63u;
-            mn = b1 & 63u;
-        } else {                 // groups 4..7: low nibbles in the third word, top two bits above the first eight
-            sc = (b2 & 15u) | ((b0 >> 6) << 4);
-            mn = (b2 >> 4) | ((b1 >> 6) << 4);
-        }
-        const int source = step >= steps_per_source ? 1 : 0;
-        const int n0 = (step - source * steps_per_source) * BWD_NS;
-        const bool valid = n0 + wave * BSH_ROWS_PER_WAVE + n < n_total;
-        scale_min[group_local * BSH_SM_PITCH + n] =
-            valid ? make_float2(half_bits_to_float(d_dmin & 0xffffu) * static_cast<float>(sc),
-                                half_bits_to_float(d_dmin >> 16) * static_cast<float>(mn))
-                  : make_float2(0.0f, 0.0f);
+    // A lane decodes 32 values of one weight row (its own, lane / 4): whole 16-byte pieces of the block, the scales from its header, and
+    // four 16-byte stores along K.  Rows past the end of the weight matrix decode to exact zeros.
+    const int n = lane >> 2;
+    uint8_t * const tile_row = &wb[0][(wave * BSH_ROWS_PER_WAVE + n) * BSH_TILE_PITCH];
+    auto store_sixteen = [&](int buffer, int column, const uint32_t (&pairs)[8]) __attribute__((always_inline)) {
+        uint8_t * const row = tile_row + buffer * sizeof(wb[0]);
+        *reinterpret_cast<uint4 *>(row + tile_granule(n, column / 8) * 16) = make_uint4(pairs[0], pairs[1], pairs[2], pairs[3]);
+        *reinterpret_cast<uint4 *>(row + tile_granule(n, column / 8 + 1) * 16) = make_uint4(pairs[4], pairs[5], pairs[6], pairs[7]);
     };
-    // a lane decodes 8 weight rows x 4 consecutive K positions and stores each K position's eight bf16 values with
-    // one 16-byte write
-    const int octet = lane & 1;
-    const int word = (lane >> 1) & 15;
-    const int nibble = lane >> 5;
-    const int position = (word & 7) * 4;
-    const int group_local = 2 * (word >> 3) + nibble;
-    const int group = 4 * half_block + group_local;
-    auto decode = [&](int step, uint16_t * tile) __attribute__((always_inline)) {
-        if constexpr (!K45) {
-            // 16 rows x 8 units of 16 values: a lane takes one row and two units; neighbouring lanes hold neighbouring
-            // rows of the same values and swap halves so that each writes both rows of one k, four bytes at a time
-            const uint8_t * rows;
-            int rows_valid, n0;
-            wave_rows(step, rows, rows_valid, n0);
-            const int n = lane & 15;
-            uint32_t keep = n0 + wave * BSH_ROWS_PER_WAVE + n < n_total ? 0xffffffffu : 0u;
-            asm volatile("" : "+v"(keep));   // (a mask, not a branch around part of the arithmetic)
-            const uint32_t selector = (lane & 1) != 0 ? 0x03020706u : 0x05040100u;
+    auto decode = [&](int step, int buffer) __attribute__((always_inline)) {
+        const uint8_t * rows;
+        int rows_valid, n0;
+        wave_rows(step, rows, rows_valid, n0);
+        uint32_t keep = n0 + wave * BSH_ROWS_PER_WAVE + n < n_total ? 0xffffffffu : 0u;
+        asm volatile("" : "+v"(keep));   // (a mask, not a branch around part of the arithmetic)
+        if constexpr (K45) {
+            // 16 bytes of nibbles: 16 values of group 2 chunk of the half block and 16 of the next one
+            const int chunk = (lane >> 1) & 1, part = lane & 1;
+            const uint8_t * const blk = raw + n * BSH_RAW_PITCH;
+            const uint4 header = *reinterpret_cast<const uint4 *>(blk);
+            const uint4 nibbles = *reinterpret_cast<const uint4 *>(blk + QS + 64 * half_block + 32 * chunk + 16 * part);
+            const uint4 planes = TYPE == Q5_K ? *reinterpret_cast<const uint4 *>(blk + 16 + 16 * part) : uint4{0, 0, 0, 0};
+            const uint32_t word[4] = {nibbles.x, nibbles.y, nibbles.z, nibbles.w}, plane[4] = {planes.x, planes.y, planes.z, planes.w};
+            const uint32_t first = header.y >> (16 * chunk), second = header.z >> (16 * chunk), third = header.w >> (16 * chunk);
+            // groups 0 .. 3 of the super-block: plain 6-bit fields; 4 .. 7: nibbles of the third word, their top bits above the first four's
+            const uint32_t scales = half_block == 0 ? first & 0x3f3fu : (third & 0x0f0fu) | ((first >> 2) & 0x3030u);
+            const uint32_t minima = half_block == 0 ? second & 0x3f3fu : ((third >> 4) & 0x0f0fu) | ((second >> 2) & 0x3030u);
+            const uint32_t d_dmin = header.x & keep;
+            const float d = half_bits_to_float(d_dmin & 0xffffu), dmin = half_bits_to_float(d_dmin >> 16);
+#pragma unroll
+            for (int high = 0; high < 2; ++high) {
+                const float scale = d * static_cast<float>((scales >> (8 * high)) & 0xffu);
+                const float minimum = dmin * static_cast<float>((minima >> (8 * high)) & 0xffu);
+                uint32_t pairs[8];
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    uint32_t q = (word[w] >> (4 * high)) & 0x0f0f0f0fu;
+                    if constexpr (TYPE == Q5_K) {
+                        q |= ((plane[w] >> (4 * half_block + 2 * chunk + high)) & 0x01010101u) << 4;
+                    }
+                    float value[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        value[e] = scale * static_cast<float>((q >> (8 * e)) & 0xffu) - minimum;
+                    }
+                    pairs[2 * w] = pack_bf16x2(value[0], value[1]);
+                    pairs[2 * w + 1] = pack_bf16x2(value[2], value[3]);
+                }
+                store_sixteen(buffer, 64 * chunk + 32 * high + 16 * part, pairs);
+            }
+        } else {
 #pragma unroll
             for (int pass = 0; pass < 2; ++pass) {
-                const int unit = (lane >> 4) + 4 * pass;
+                const int unit = 2 * (lane & 3) + pass;
                 uint32_t pairs[8];
                 decode16_bf16<TYPE>(raw + n * SLOT_PITCH + SLOT_FRONT, 8 * half_block + unit, grid, pairs);
-                uint32_t * const pair_row = reinterpret_cast<uint32_t *>(
-                    &tile[(unit * 16 + (lane & 1)) * BWD_PITCH + wave * BSH_ROWS_PER_WAVE + (n & ~1)]);
 #pragma unroll
-                for (int j = 0; j < 16; j += 2) {
-                    const uint32_t own = pairs[j / 2] & keep;
-                    const uint32_t other = static_cast<uint32_t>(
-                        __builtin_amdgcn_mov_dpp(static_cast<int>(own), 0xB1, 0xf, 0xf, true));   // lane ^ 1
-                    pair_row[j * (BWD_PITCH / 2)] = __builtin_amdgcn_perm(other, own, selector);
+                for (int i = 0; i < 8; ++i) {
+                    pairs[i] &= keep;
                 }
+                store_sixteen(buffer, 16 * unit, pairs);
             }
-            return;
-        }
-        uint32_t qs[8], qh[8];
-        float2 sm[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int n = 8 * octet + i;
-            const uint8_t * blk = raw + n * BSH_RAW_PITCH;
-            qs[i] = lds_u32(blk + QS + 64 * half_block + 4 * word);
-            qh[i] = TYPE == Q5_K ? lds_u32(blk + 16 + position) : 0u;
-            sm[i] = scale_min[group_local * BSH_SM_PITCH + n];
-        }
-        float w[4][8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            uint32_t q = (qs[i] >> (4 * nibble)) & 0x0f0f0f0fu;
-            if constexpr (TYPE == Q5_K) {
-                q |= ((qh[i] >> group) & 0x01010101u) << 4;
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                w[e][i] = sm[i].x * static_cast<float>((q >> (8 * e)) & 0xffu) - sm[i].y;
-            }
-        }
-        const int k_local = 32 * group_local + position;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const uint4 packed = make_uint4(pack_bf16x2(w[e][0], w[e][1]), pack_bf16x2(w[e][2], w[e][3]),
-                                            pack_bf16x2(w[e][4], w[e][5]), pack_bf16x2(w[e][6], w[e][7]));
-            *reinterpret_cast<uint4 *>(&tile[(k_local + e) * BWD_PITCH + wave * BSH_ROWS_PER_WAVE + 8 * octet]) = packed;
         }
     };
 
@@ -1631,11 +1617,16 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
     for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[rt][v] = 0.0f;
-    auto multiply = [&](const uint16_t * tile) __attribute__((always_inline)) {
+    // Fragments of the wave's 32 columns: lane (column, half) wants eight weight rows of its column.  ds_read_b64_tr_b16 gives lane i of 16 the
+    // i-th column of the four rows x 16 columns that the 16 lanes address, four lanes side by side in a row.
+    const int tr_row = (lane >> 2) & 3;
+    const uint8_t * const tr_from = &wb[0][(8 * half + tr_row) * BSH_TILE_PITCH + tile_granule(tr_row, 4 * wave + 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1)) * 16 +
+                                           8 * (lane & 1)];
+    auto multiply = [&](int buffer) __attribute__((always_inline)) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            const uint4 bits = *reinterpret_cast<const uint4 *>(&tile[(wave * 32 + l32) * BWD_PITCH + 16 * c + 8 * half]);
-            const v8bf bfrag = __builtin_bit_cast(v8bf, bits);
+            const uint8_t * const from = tr_from + buffer * sizeof(wb[0]) + 16 * c * BSH_TILE_PITCH;
+            const v8bf bfrag = transposed_fragment(from, from + 4 * BSH_TILE_PITCH);
 #pragma unroll
             for (int rt = 0; rt < 2; ++rt) {
                 if (rt < row_tiles) {
@@ -1654,11 +1645,7 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
     park(0, ring[0]);
     request(BSH_DEPTH, ring[0]);
     wave_sync();
-    if constexpr (K45) {
-        scales(0);
-        wave_sync();
-    }
-    decode(0, wb[0]);
+    decode(0, 0);
     __syncthreads();
     // A step that has a successor: multiply its tile and prepare the next one.  The loop below holds no branch, so
     // the compiler's wait-count bookkeeping sees every request on every path; with the last step's exceptions inside
@@ -1671,17 +1658,13 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
         // the chain of dependent waits goes first, the arithmetic of the decode fills in (measured: 1 %)
         __builtin_amdgcn_s_setprio(3);
         park(step + 1, ring[u ^ 1]);
-        multiply(wb[u]);
+        multiply(u);
         // both requests go out behind the matrix instructions, which wait for the previous step's cotangent only
         request_cotangent(step + 1);
         request(step + 1 + BSH_DEPTH, ring[u ^ 1]);
         wave_sync();
-        if constexpr (K45) {
-            scales(step + 1);
-            wave_sync();
-        }
         __builtin_amdgcn_s_setprio(0);
-        decode(step + 1, wb[u ^ 1]);
+        decode(step + 1, u ^ 1);
         __syncthreads();
     };
     int step = 0;
@@ -1692,17 +1675,17 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
     }
     if (step < last) {   // uniform
         advance(step, std::integral_constant<int, 0>{});
-        multiply(wb[1]);
+        multiply(1);
     } else {
-        multiply(wb[0]);
+        multiply(0);
     }
     __syncthreads();
     // the tiles are free (every wave is past its last multiplication): the four 32-column slices of a 32-row tile
     // meet in LDS and leave as whole 256-byte rows
     constexpr int STAGE_PITCH = BWD_TK + 8;
-    static_assert(2 * 32 * STAGE_PITCH <= 2 * BWD_TK * BWD_PITCH, "both row tiles fit the weight tiles");
+    static_assert(2 * 32 * STAGE_PITCH * 2 <= sizeof(wb), "both row tiles fit the weight tiles");
     static_assert(BSH_DEPTH % 2 == 0, "tile parity follows the position in the unrolled round");
-    uint16_t * stage = &wb[0][0];
+    uint16_t * stage = reinterpret_cast<uint16_t *>(&wb[0][0]);
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt) {
         if (rt < row_tiles) {
