@@ -9,8 +9,8 @@
 //
 // mmq_grad_input_split_kernel: a workgroup owns 256 rows x 128 values of K (half a super-block column) and walks the
 // reduction dimension N in steps of 64 weight rows.  Per step the 64 packed blocks are copied to LDS, dequantized once to bf16
-// (bit-exact with the scalar reference decoder) into a transposed tile [k][n] whose rows are what a lane needs as its B
-// operand; half of the waves dequantize, half multiply.  Dense calls whose tiles do not fill the chip cut N into ranges.
+// (bit-exact with the scalar reference decoder) into a tile that the multiplying waves read transposed; half of the waves dequantize, half
+// multiply.  Dense calls whose tiles do not fill the chip cut N into ranges.
 //
 // mmq_grad_input_short_kernel: tasks of a few rows of a grouped call; described where it is defined.
 //
@@ -734,6 +734,26 @@ __global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_ker
     }
 }
 
+// A tile of the two kernels below lies as the weights do, [weight row][K column], and is transposed on its way out (the fragments want eight weight rows of a column
+// per lane).  The 16-byte granules of a row are exchanged by the row's number, so that the lanes which the LDS serves together, eight that store
+// along two rows or 16 that read from four, find theirs on different banks.
+constexpr int BWD_ROW_PITCH = BWD_TK * 2;
+TGO_DEVICE int tile_granule(int row, int granule) { return granule ^ ((row & 3) * 5); }
+// A fragment of 16 weight rows x 32 K columns (column tile kt): lane (column, half) wants eight weight rows of its column.  ds_read_b64_tr_b16 gives
+// lane i of 16 the i-th column of the four rows x 16 columns that the 16 lanes address, four lanes side by side in a row; two of them make the
+// fragment, the second four rows further on.
+TGO_DEVICE uint32_t transposed_offset(int lane, int kt) {
+    const int row = (lane >> 2) & 3, half = lane >> 5;
+    return (8 * half + row) * BWD_ROW_PITCH + tile_granule(row, 4 * kt + 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1)) * 16 + 8 * (lane & 1);
+}
+TGO_DEVICE v8bf transposed_fragment(const uint8_t * first, const uint8_t * second) {
+    typedef short four_t __attribute__((ext_vector_type(4)));
+    typedef short eight_t __attribute__((ext_vector_type(8)));
+    const four_t low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) four_t *)(first));
+    const four_t high = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) four_t *)(second));
+    return __builtin_bit_cast(v8bf, eight_t{low.x, low.y, low.z, low.w, high.x, high.y, high.z, high.w});
+}
+
 // ---- role-split variant --------------------------------------------------------------------------------------
 // 256 rows x 128 values of K, reduction steps of 64 weight rows, double-buffered bf16
 // tile; the eight waves of a workgroup are specialised: waves 0-3 only multiply (64 rows each), waves
@@ -745,21 +765,23 @@ __global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_ker
 // steps as one stream, so the memory latency of an item's first loads and the drain of its last step are
 // paid once per workgroup instead of once per item.  Nothing is loaded where it is used.  A decoder wave owns
 // 16 of a step's 64 weight rows from global load to tile write (no barrier of its own; LDS traffic inside a
-// wave is ordered) and works on four consecutive steps at once: while the multipliers consume step g it
-// dequantizes step g+1, derives the block scales of step g+2, parks the packed blocks of step g+3 in LDS and
-// has the blocks of steps g+4..g+7 in flight in registers, so no stage waits for the one before it.  A
+// wave is ordered) and works on several consecutive steps at once: while the multipliers consume step g it
+// dequantizes step g+1 from what it read of LDS during the previous round, parks the packed blocks of step g+3 in LDS, reads the inputs of
+// step g+2 (IQ2_S: looks up its codebook words, and reads the indices of g+3) and has the blocks of steps g+4..g+7 in flight in registers, so no
+// stage waits for the one before it.  A
 // multiplier wave keeps the cotangent fragments of the next step in flight (two steps were measured: no faster, and
 // the registers serve the weight-fragment look-ahead better).
 //
 // Measured, 256 rows of a 248320 x 2048 head (16 ranges): Q4_K 955 -> 316 us, Q6_K 655 -> 356, IQ2_S 527 -> 333 (820 TFLOP/s)
-// against the general kernel, whose waves dequantize and multiply in turn; the matrix pipe is busy for
-// a third of the time at the clock the card then holds, the decoder waves' LDS traffic and arithmetic for the rest.
+// against the general kernel, whose waves dequantize and multiply in turn.  Then a lane decoded four values of eight weight rows, for a tile that
+// was stored transposed, after a stage for the block scales; with 32 values of a row per lane and the transposition in the reads (tile_granule) the
+// LDS is busy for 0.29 to 0.36 of the time instead of 0.43 to 0.6: 4096 tokens of eight choices among 256 experts with power-law 0.3 routing, 2 x
+// 512 x 2048 IQ2_S 276 -> 254 us, 512 x 2048 Q5_K 150 -> 138; dense calls of 33 to 900 rows 0.97 on the mean.  What is left: the matrix pipe is busy
+// for 0.32 (tasks that half fill 256 rows) to 0.44 of the time at the clock that the card's power leaves (1.9 GHz with 256 rows of the head).
 constexpr int BSP_THREADS = 512;
 constexpr int BSP_ROWS_PER_DECODER = BWD_NS / 4;   // weight rows a decoder wave owns per step
 constexpr int BSP_RAW_DEPTH = 4;                   // steps of packed blocks in flight per decoder wave
 constexpr int BSP_COT_DEPTH = 2;                   // cotangent fragment sets per multiplier wave (1 in use)
-constexpr int BSP_SM_PITCH = BSP_ROWS_PER_DECODER + 1;
-constexpr int BSP_OCTET_PITCH = BSP_ROWS_PER_DECODER + 4;
 constexpr int BSP_MAX_ITEMS = 64;                  // items per workgroup (one wave builds the table)
 constexpr int BSP_GRID = 256;                      // one workgroup per CU
 
@@ -812,7 +834,6 @@ struct SplitBlock : BlockPieces<TYPE> {
     using P = BlockPieces<TYPE>;
     static constexpr int SLOT_BYTES = BSP_ROWS_PER_DECODER * P::PITCH;
     static constexpr int REGS = (BSP_ROWS_PER_DECODER * P::UNITS + 63) / 64;
-    static constexpr int SCALE_GROUPS = P::ALIGNED ? 4 : 8;   // scales in half a super-block
     static constexpr int BIAS = TYPE == Q3_K ? 4 : TYPE == Q6_K ? 32 : TYPE == IQ2_S ? 128 : 0;   // of the quants as unsigned bytes
 };
 
@@ -839,12 +860,9 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
     constexpr int BSP_RAW_PITCH = B::PITCH;
     constexpr int RAW_REGS = B::REGS;
     constexpr int QS = TYPE == Q4_K ? 16 : 48;
-    __shared__ __attribute__((aligned(16))) uint16_t wb[2][BWD_TK * BWD_PITCH];
+    __shared__ __attribute__((aligned(16))) uint8_t wb[2][BWD_NS * BWD_ROW_PITCH];   // [weight row][K column], bf16 (tile_granule)
     __shared__ __attribute__((aligned(16))) uint8_t raw_all[4][3][B::SLOT_BYTES];
-    __shared__ float2 scale_min_all[4][2][B::SCALE_GROUPS * BSP_SM_PITCH];
-    // IQ2_S: codebook, and per decoder wave and step the (codebook index, signs) of each eight values and weight row
-    __shared__ uint2 grid[TYPE == IQ2_S ? TGO_IQ2S_GRID_ENTRIES : 1];
-    __shared__ __attribute__((aligned(16))) uint32_t octets_all[TYPE == IQ2_S ? 4 : 1][2][TYPE == IQ2_S ? 16 * BSP_OCTET_PITCH : 4];
+    __shared__ uint2 grid[TYPE == IQ2_S ? TGO_IQ2S_GRID_ENTRIES : 1];   // codebook
     __shared__ __attribute__((aligned(16))) uint16_t stage_all[4][32 * (BWD_TK + 8)];
     __shared__ SplitItem items[BSP_MAX_ITEMS];
     __shared__ int item_count, step_count;
@@ -1012,165 +1030,138 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
                 *reinterpret_cast<u32x4 *>(raw + lane_row(i) * BSP_RAW_PITCH + 16 * lane_unit(i)) = regs[i];
             }
         };
-        // Stages 2 and 3 are each split into the LDS reads and the arithmetic on what was read, so that the
-        // reads can be issued well before their results are needed (a lone wave has nothing else to cover an
-        // LDS round trip with).
-        //
-        // stage 2: (d * sc, dmin * m) of this lane's (row, 32-value group); rows past the end of the weight
-        // matrix get (0, 0) and therefore decode to exact zeros
-        // The other formats have a scale per 16 values and a constant bias of the quants instead: (s, bias * s), and the
-        // lane's two groups.  IQ2_S: also the codebook indices and signs of the lane's four octets of values.
-        struct ScaleInputs {
-            uint32_t d_dmin, low, mid, high;   // Q4_K / Q5_K: the 16-byte block header: two halves, then 12 bytes of 6-bit fields
+        // stage 2: a lane decodes 32 values of one weight row (lane / 4) in two runs of 16 along K.  The LDS reads and the arithmetic on
+        // what was read are apart, so that the reads can be issued well before their results are needed (a lone wave has nothing else to
+        // cover an LDS round trip with).
+        struct DecodeInputs {
+            uint32_t low[4], high[4];   // K45: nibbles and fifth bits; Q3_K, Q6_K: low and high bits; IQ2_S: codebook words of the runs
+            uint32_t header[4];         // scales
         };
-        auto scales_fetch = [&](int info, const uint8_t * raw) {
-            const uint8_t * blk = raw + (lane & 15) * BSP_RAW_PITCH;
-            const int pair = lane >> 4;
+        const int n = lane >> 2, quarter = lane & 3;
+        const auto unpack4 = [](const uint4 v, uint32_t (&to)[4]) {
+            to[0] = v.x; to[1] = v.y; to[2] = v.z; to[3] = v.w;
+        };
+        auto decode_fetch = [&](int info, const uint8_t * raw) {
             const int half_block = info & 1;
-            ScaleInputs in = {0, 0, 0, 0};
+            const uint8_t * const blk = raw + n * BSP_RAW_PITCH;
+            DecodeInputs in = {};
+            const auto bytes16 = [&](int at) { return *reinterpret_cast<const uint4 *>(blk + at); };
             if constexpr (K45) {
-                in.d_dmin = lds_u32(blk);
-                in.low = lds_u32(blk + 4);
-                in.mid = lds_u32(blk + 8);
-                in.high = lds_u32(blk + 12);
+                unpack4(bytes16(0), in.header);
+                unpack4(bytes16(QS + 64 * half_block + 16 * quarter), in.low);
+                if constexpr (TYPE == Q5_K) {
+                    unpack4(bytes16(16 + 16 * (quarter & 1)), in.high);
+                }
             } else if constexpr (TYPE == Q3_K) {
-                in.d_dmin = lds_u16(blk + 110);
-                in.low = lds_u16(blk + 98 + 2 * pair);
-                in.mid = lds_u16(blk + 106 + 2 * (pair & 1));
+                unpack4(bytes16(32 + 32 * half_block + 16 * (quarter & 1)), in.low);
+                unpack4(bytes16(16 * (quarter & 1)), in.high);
+                const int unit = 4 * (quarter >> 1) + (quarter & 1);   // of the half block, and the one two behind it
+                in.header[0] = lds_u16(blk + 110);
+                in.header[1] = (static_cast<uint32_t>(blk[98 + unit]) >> (4 * half_block)) | (static_cast<uint32_t>(blk[100 + unit]) >> (4 * half_block) << 16);
+                in.header[2] = blk[106 + (quarter & 1)] | (static_cast<uint32_t>(blk[108 + (quarter & 1)]) << 16);
             } else if constexpr (TYPE == Q6_K) {
-                in.d_dmin = lds_u16(blk + 222);
-                in.low = lds_u16(blk + 192 + 8 * half_block + 2 * pair);
+                unpack4(bytes16(64 * half_block + 16 * quarter), in.low);
+                unpack4(bytes16(128 + 32 * half_block + 16 * (quarter & 1)), in.high);
+                in.header[0] = lds_u16(blk + 222);
+                in.header[1] = blk[192 + 8 * half_block + quarter];
+                in.header[2] = blk[196 + 8 * half_block + quarter];
             } else {
-                in.d_dmin = lds_u16(blk + 80) | (static_cast<uint32_t>(blk[72 + 4 * half_block + pair]) << 16);
-                in.low = lds_u32(blk + 16 * half_block + 4 * pair);        // codebook indices of four octets, eight bits each
-                in.mid = lds_u32(blk + 32 + 16 * half_block + 4 * pair);   // their signs
-                in.high = blk[64 + 4 * half_block + pair];                 // the indices' upper two bits
+                in.low[0] = lds_u32(blk + 16 * half_block + 4 * quarter);        // codebook indices of four octets, eight bits each
+                in.low[1] = lds_u32(blk + 32 + 16 * half_block + 4 * quarter);   // their signs
+                in.low[2] = blk[64 + 4 * half_block + quarter];                  // the indices' upper two bits
+                in.header[0] = lds_u16(blk + 80);
+                in.header[1] = blk[72 + 4 * half_block + quarter];
             }
             return in;
         };
-        auto scales_finish = [&](int info, const ScaleInputs & in, float2 * scale_min, uint32_t * octets) {
-            const int n = lane & 15;
-            const bool valid = (info >> 1) * BWD_NS + dw * BSP_ROWS_PER_DECODER + n < n_total;
-            if constexpr (K45) {
-                const int group_local = lane >> 4;
-                const int shift = 8 * group_local;
-                const uint32_t b0 = (in.low >> shift) & 0xffu, b1 = (in.mid >> shift) & 0xffu, b2 = (in.high >> shift) & 0xffu;
-                uint32_t sc, mn;
-                if ((info & 1) == 0) {   // groups 0..3 of the super-block: plain 6-bit fields
-                    sc = b0 & 63u;
-                    mn = b1 & 63u;
-                } else {                 // groups 4..7: low nibbles in the third word, top two bits above the first eight
-                    sc = (b2 & 15u) | ((b0 >> 6) << 4);
-                    mn = (b2 >> 4) | ((b1 >> 6) << 4);
-                }
-                scale_min[group_local * BSP_SM_PITCH + n] =
-                    valid ? make_float2(half_bits_to_float(in.d_dmin & 0xffffu) * static_cast<float>(sc),
-                                        half_bits_to_float(in.d_dmin >> 16) * static_cast<float>(mn))
-                          : make_float2(0.0f, 0.0f);
-            } else {
-                const int pair = lane >> 4;
-                const float d = half_bits_to_float(in.d_dmin & 0xffffu);
+        // IQ2_S: the codebook words that a step's indices name, a round before they are needed
+        auto codebook_fetch = [&](const DecodeInputs & in) {
+            DecodeInputs out = in;
+            if constexpr (TYPE == IQ2_S) {
+                uint32_t words[8];
 #pragma unroll
-                for (int g = 0; g < 2; ++g) {
-                    float scale;
+                for (int o = 0; o < 4; ++o) {
+                    const uint2 entry = grid[((in.low[0] >> (8 * o)) & 0xffu) | (((in.low[2] >> (2 * o)) & 3u) << 8)];
+                    words[2 * o] = entry.x;
+                    words[2 * o + 1] = entry.y;
+                }
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    out.low[w] = words[w];
+                    out.high[w] = words[4 + w];
+                }
+                out.header[2] = in.low[1];
+            }
+            return out;
+        };
+        auto decode_finish = [&](int info, const DecodeInputs & in, uint8_t * tile) {
+            const int half_block = info & 1;
+            uint32_t keep = (info >> 1) * BWD_NS + dw * BSP_ROWS_PER_DECODER + n < n_total ? 0xffffffffu : 0u;
+            asm volatile("" : "+v"(keep));   // (a mask, not a branch around part of the arithmetic; rows past the end become exact zeros)
+            const uint32_t header = in.header[0] & keep;
+            const float d = half_bits_to_float(header & 0xffffu);
+            uint8_t * const row = tile + (dw * BSP_ROWS_PER_DECODER + n) * BWD_ROW_PITCH;
+            uint32_t k45_scales = 0, k45_minima = 0;
+            if constexpr (K45) {
+                const int shift = 16 * (quarter >> 1);
+                const uint32_t first = in.header[1] >> shift, second = in.header[2] >> shift, third = in.header[3] >> shift;
+                // groups 0 .. 3 of the super-block: plain 6-bit fields; 4 .. 7: nibbles of the third word, their top bits above the first four's
+                k45_scales = half_block == 0 ? first & 0x3f3fu : (third & 0x0f0fu) | ((first >> 2) & 0x3030u);
+                k45_minima = half_block == 0 ? second & 0x3f3fu : ((third >> 4) & 0x0f0fu) | ((second >> 2) & 0x3030u);
+            }
+#pragma unroll
+            for (int run = 0; run < 2; ++run) {
+                float scale, offset;
+                int column;
+                if constexpr (K45) {
+                    scale = d * static_cast<float>((k45_scales >> (8 * run)) & 0xffu);
+                    offset = half_bits_to_float(header >> 16) * static_cast<float>((k45_minima >> (8 * run)) & 0xffu);
+                    column = 64 * (quarter >> 1) + 32 * run + 16 * (quarter & 1);
+                } else {
                     if constexpr (TYPE == Q3_K) {
-                        const uint32_t low = (in.low >> (8 * g + 4 * (info & 1))) & 15u;
-                        const uint32_t high = (in.mid >> (8 * g + 4 * (info & 1) + 2 * (pair >> 1))) & 3u;
+                        const uint32_t low = (in.header[1] >> (16 * run)) & 15u;
+                        const uint32_t high = (in.header[2] >> (16 * run + 4 * half_block + 2 * (quarter >> 1))) & 3u;
                         scale = d * static_cast<float>(static_cast<int>(low | (high << 4)) - 32);
+                        column = 64 * (quarter >> 1) + 32 * run + 16 * (quarter & 1);
                     } else if constexpr (TYPE == Q6_K) {
-                        scale = d * static_cast<float>(static_cast<int>(in.low << (24 - 8 * g)) >> 24);
+                        scale = d * static_cast<float>(static_cast<int>(in.header[1 + run] << 24) >> 24);
+                        column = 64 * run + 16 * quarter;
                     } else {
-                        scale = d * 0.125f * static_cast<float>(((in.d_dmin >> (16 + 4 * g)) & 15u) * 2 + 1);
+                        scale = d * 0.125f * static_cast<float>(((in.header[1] >> (4 * run)) & 15u) * 2 + 1);
+                        column = 32 * quarter + 16 * run;
                     }
                     // (products of an 11-bit and an at most 8-bit number: exact, and so is the bias, a power of two)
-                    scale = valid ? scale : 0.0f;
-                    scale_min[(2 * pair + g) * BSP_SM_PITCH + n] = make_float2(scale, scale * B::BIAS);
+                    offset = scale * B::BIAS;
                 }
-                if constexpr (TYPE == IQ2_S) {
+                uint32_t pairs[8];
 #pragma unroll
-                    for (int o = 0; o < 4; ++o) {
-                        const uint32_t index = ((in.low >> (8 * o)) & 0xffu) | (((in.high >> (2 * o)) & 3u) << 8);
-                        octets[(4 * pair + o) * BSP_OCTET_PITCH + n] = index | (((in.mid >> (8 * o)) & 0xffu) << 16);
+                for (int w = 0; w < 4; ++w) {
+                    uint32_t q;   // four quants as unsigned bytes, above their true values by the bias
+                    if constexpr (K45) {
+                        q = (in.low[w] >> (4 * run)) & 0x0f0f0f0fu;
+                        if constexpr (TYPE == Q5_K) {
+                            q |= ((in.high[w] >> (4 * half_block + 2 * (quarter >> 1) + run)) & 0x01010101u) << 4;
+                        }
+                    } else if constexpr (TYPE == Q3_K) {
+                        const int group = 2 * (quarter >> 1) + run;   // 32-value group of the half block
+                        q = ((in.low[w] >> (2 * group)) & 0x03030303u) | (((in.high[w] >> (4 * half_block + group)) & 0x01010101u) << 2);
+                    } else if constexpr (TYPE == Q6_K) {
+                        q = ((in.low[w] >> (4 * run)) & 0x0f0f0f0fu) | (((in.high[w] >> (2 * (quarter >> 1) + 4 * run)) & 0x03030303u) << 4);
+                    } else {
+                        // the four signs spread to a bit per byte; a negative magnitude is its complement plus one
+                        const uint32_t negative = (((in.header[2] >> (16 * run + 4 * w)) & 15u) * 0x00204081u) & 0x01010101u;
+                        q = (((run == 0 ? in.low[w] : in.high[w]) ^ (negative * 0xffu)) + negative) ^ 0x80808080u;
                     }
-                }
-            }
-        };
-        // stage 3: a lane decodes 8 weight rows x 4 consecutive K positions and stores each K position's
-        // eight bf16 values with one 16-byte write
-        struct DecodeInputs {
-            uint32_t qs[8], qh[8];
-            float2 sm[8];
-        };
-        const int octet = lane & 1;
-        const int word = (lane >> 1) & 15;
-        const int nibble = lane >> 5;
-        const int position = (word & 7) * 4;
-        // Q4_K / Q5_K: two lanes share a word, a nibble each.  The others: 4 * (lane >> 1) is the lane's position in the half.
-        const int group_local = K45 ? 2 * (word >> 3) + nibble : lane >> 4;                  // 32-value group inside the half block
-        const int scale_group = K45 ? group_local : lane >> 3;
-        auto decode_fetch = [&](int info, const uint8_t * raw, const float2 * scale_min, const uint32_t * octets) {
-            const int half_block = info & 1;
-            DecodeInputs in;
-            if constexpr (TYPE == IQ2_S) {
-                const uint32_t * mine = octets + (lane >> 2) * BSP_OCTET_PITCH + 8 * octet;
-                const uint4 low = *reinterpret_cast<const uint4 *>(mine), high = *reinterpret_cast<const uint4 *>(mine + 4);
-                const uint32_t records[8] = {low.x, low.y, low.z, low.w, high.x, high.y, high.z, high.w};
+                    float value[4];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    in.qs[i] = reinterpret_cast<const uint32_t *>(grid)[2 * (records[i] & 0x3ffu) + ((lane >> 1) & 1)];
-                    in.qh[i] = records[i] >> 16;
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int n = 8 * octet + i;
-                const uint8_t * blk = raw + n * BSP_RAW_PITCH;
-                if constexpr (K45) {
-                    in.qs[i] = lds_u32(blk + QS + 64 * half_block + 4 * word);
-                    in.qh[i] = TYPE == Q5_K ? lds_u32(blk + 16 + position) : 0u;
-                } else if constexpr (TYPE == Q3_K) {
-                    in.qs[i] = lds_u32(blk + 32 + 32 * half_block + 4 * ((lane >> 1) & 7));
-                    in.qh[i] = lds_u32(blk + 4 * ((lane >> 1) & 7));
-                } else if constexpr (TYPE == Q6_K) {
-                    in.qs[i] = lds_u32(blk + 64 * half_block + 4 * ((lane >> 1) & 15));
-                    in.qh[i] = lds_u32(blk + 128 + 32 * half_block + 4 * ((lane >> 1) & 7));
-                }
-                in.sm[i] = scale_min[scale_group * BSP_SM_PITCH + n];
-            }
-            return in;
-        };
-        auto decode_finish = [&](int info, const DecodeInputs & in, uint16_t * tile) {
-            const int group = 4 * (info & 1) + group_local;
-            float w[4][8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                uint32_t q;   // four quants as unsigned bytes, above their true values by the bias
-                if constexpr (K45) {
-                    q = (in.qs[i] >> (4 * nibble)) & 0x0f0f0f0fu;
-                    if constexpr (TYPE == Q5_K) {
-                        q |= ((in.qh[i] >> group) & 0x01010101u) << 4;
+                    for (int e = 0; e < 4; ++e) {
+                        value[e] = scale * static_cast<float>((q >> (8 * e)) & 0xffu) - offset;
                     }
-                } else if constexpr (TYPE == Q3_K) {
-                    q = ((in.qs[i] >> (2 * group_local)) & 0x03030303u) | (((in.qh[i] >> group) & 0x01010101u) << 2);
-                } else if constexpr (TYPE == Q6_K) {
-                    q = ((in.qs[i] >> (4 * nibble)) & 0x0f0f0f0fu) | (((in.qh[i] >> (2 * group_local)) & 0x03030303u) << 4);
-                } else {
-                    // the four signs spread to a bit per byte; a negative magnitude is its complement plus one
-                    const uint32_t negative = (((in.qh[i] >> (4 * ((lane >> 1) & 1))) & 15u) * 0x00204081u) & 0x01010101u;
-                    q = ((in.qs[i] ^ (negative * 0xffu)) + negative) ^ 0x80808080u;
+                    pairs[2 * w] = pack_bf16x2(value[0], value[1]);
+                    pairs[2 * w + 1] = pack_bf16x2(value[2], value[3]);
                 }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    w[e][i] = in.sm[i].x * static_cast<float>((q >> (8 * e)) & 0xffu) - in.sm[i].y;
-                }
-            }
-            const int k_local = K45 ? 32 * group_local + position : 4 * (lane >> 1);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint4 packed = make_uint4(pack_bf16x2(w[e][0], w[e][1]), pack_bf16x2(w[e][2], w[e][3]),
-                                                pack_bf16x2(w[e][4], w[e][5]), pack_bf16x2(w[e][6], w[e][7]));
-                *reinterpret_cast<uint4 *>(
-                    &tile[(k_local + e) * BWD_PITCH + dw * BSP_ROWS_PER_DECODER + 8 * octet]) = packed;
+                *reinterpret_cast<uint4 *>(row + tile_granule(n, column / 8) * 16) = make_uint4(pairs[0], pairs[1], pairs[2], pairs[3]);
+                *reinterpret_cast<uint4 *>(row + tile_granule(n, column / 8 + 1) * 16) = make_uint4(pairs[4], pairs[5], pairs[6], pairs[7]);
             }
         };
         auto wave_sync = [&]() {
@@ -1178,10 +1169,8 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
             __builtin_amdgcn_wave_barrier();
         };
         auto raw_slot = [&](int slot) { return raw_all[dw][slot]; };
-        auto sm_slot = [&](int slot) { return scale_min_all[dw][slot]; };
-        auto octet_slot = [&](int slot) { return octets_all[TYPE == IQ2_S ? dw : 0][slot]; };
 
-        // Step t uses raw slot t % 3, scale slot t & 1, tile t & 1 and register set t % 4.  Only the load
+        // Step t uses raw slot t % 3, tile t & 1 and register set t % 4.  Only the load
         // stage walks the item list; what the later stages need to know about a step (which half of the
         // super-block, which 64 weight rows) follows it through a seven-deep queue of scalars.
         SplitCursor c_load = first_step(rebase);
@@ -1205,15 +1194,18 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
             request(ring[t]);
         }
         wave_sync();
-        scales_finish(info[6], scales_fetch(info[6], raw_slot(0)), sm_slot(0), octet_slot(0));
-        scales_finish(info[5], scales_fetch(info[5], raw_slot(1)), sm_slot(1), octet_slot(1));
-        wave_sync();
-        decode_finish(info[6], decode_fetch(info[6], raw_slot(0), sm_slot(0), octet_slot(0)), wb[0]);
-        DecodeInputs pending = decode_fetch(info[5], raw_slot(1), sm_slot(1), octet_slot(1));   // step 1
+        decode_finish(info[6], codebook_fetch(decode_fetch(info[6], raw_slot(0))), wb[0]);
+        // IQ2_S has its codebook words looked up in the round before they are decoded, and the indices read in the round before that
+        constexpr bool LOOKS_UP = TYPE == IQ2_S;
+        DecodeInputs pending = codebook_fetch(decode_fetch(info[5], raw_slot(1)));   // step 1
+        DecodeInputs indices = {};
+        if constexpr (LOOKS_UP) {
+            indices = decode_fetch(info[4], raw_slot(2));   // step 2
+        }
         __syncthreads();
         // While the multipliers consume step g: finish decoding g + 1 (its inputs were read from LDS during
-        // the previous round), scales of g + 2 (inputs read first thing, used after the decode), park g + 3,
-        // request g + 7, and read the decode inputs of g + 2 so that they arrive during the barrier.  LDS
+        // the previous round), park g + 3, request g + 7, and read the decode inputs of g + 2 so that they arrive during the barrier (IQ2_S: look
+        // up what g + 2 needs first thing, and read the indices of g + 3).  LDS
         // executes a wave's accesses in order, so a stage may read what an earlier stage of the same round
         // wrote without waiting; the fences only keep the compiler from reordering them.
         int g3 = 0;   // g % 3
@@ -1224,13 +1216,20 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
                 const int g = base + u;
                 const int g3_plus1 = g3 == 2 ? 0 : g3 + 1;
                 const int g3_plus2 = g3_plus1 == 2 ? 0 : g3_plus1 + 1;
-                const ScaleInputs scale_inputs = scales_fetch(info[4], raw_slot(g3_plus2));
-                __builtin_amdgcn_sched_barrier(0);
+                DecodeInputs next;
+                if constexpr (LOOKS_UP) {
+                    next = codebook_fetch(indices);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
                 decode_finish(info[5], pending, wb[(g + 1) & 1]);
-                scales_finish(info[4], scale_inputs, sm_slot(g & 1), octet_slot(g & 1));
                 park(ring[(u + 3) % BSP_RAW_DEPTH], raw_slot(g3));
                 wave_sync();
-                pending = decode_fetch(info[4], raw_slot(g3_plus2), sm_slot(g & 1), octet_slot(g & 1));
+                if constexpr (LOOKS_UP) {
+                    indices = decode_fetch(info[3], raw_slot(g3));
+                    pending = next;
+                } else {
+                    pending = decode_fetch(info[4], raw_slot(g3_plus2));
+                }
                 request(ring[(u + 3) % BSP_RAW_DEPTH]);
                 __builtin_amdgcn_sched_barrier(0);
                 g3 = g3_plus1;
@@ -1272,6 +1271,12 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
     };
     auto rebase_none = [&](SplitCursor &) {};
 
+    // where the lane's share of a fragment of column tile kt lies (ds_read_b64_tr_b16, see transposed_fragment)
+    uint32_t fragment_offset[4];
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) {
+        fragment_offset[kt] = transposed_offset(lane, kt);
+    }
     v16f acc[2][4];
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt)
@@ -1307,12 +1312,13 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
                 // 16 weight fragments (4 chunks x 4 column tiles), two MFMAs each.  An LDS read takes
                 // longer than the two MFMAs it feeds, so fragment j + AHEAD is requested before fragment j
                 // is used; the scheduling groups below pin that interleaving.
-                const uint16_t * tile = wb[g & 1] + l32 * BWD_PITCH + 8 * half;
+                const uint8_t * const tile = wb[g & 1];
                 auto read_fragment = [&](int j) {
-                    return *reinterpret_cast<const uint4 *>(&tile[(j & 3) * 32 * BWD_PITCH + 16 * (j >> 2)]);
+                    const uint8_t * const from = tile + fragment_offset[j & 3] + 16 * (j >> 2) * BWD_ROW_PITCH;
+                    return transposed_fragment(from, from + 4 * BWD_ROW_PITCH);
                 };
                 constexpr int AHEAD = 6;
-                uint4 fragment[16];
+                v8bf fragment[16];
 #pragma unroll
                 for (int j = 0; j < AHEAD; ++j) {
                     fragment[j] = read_fragment(j);
@@ -1327,15 +1333,15 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
                         // (operands swapped: the lane ends up with one task row and runs of four neighbouring
                         // columns, which the epilogue stages with 8-byte LDS writes instead of 2-byte ones)
                         acc[rt][j & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                            __builtin_bit_cast(v8bf, fragment[j]), __builtin_bit_cast(v8bf, cot[u][rt][j >> 2]),
+                            fragment[j], __builtin_bit_cast(v8bf, cot[u][rt][j >> 2]),
                             acc[rt][j & 3], 0, 0, 0);
                     }
                 }
-                __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);   // LDS reads
+                __builtin_amdgcn_sched_group_barrier(0x100, 2 * AHEAD, 0);   // LDS reads
 #pragma unroll
                 for (int j = 0; j < 16; ++j) {
                     if (j + AHEAD < 16) {
-                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
                     }
                     __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);   // MFMAs
                 }
@@ -1390,19 +1396,6 @@ constexpr int BSH_THREADS = 256;
 constexpr int BSH_ROWS_PER_WAVE = BWD_NS / 4;
 constexpr int BSH_DEPTH = 2;
 
-// The tile lies as the weights do, [weight row][K column], and is transposed on its way out (the fragments want eight weight rows of a column
-// per lane).  The 16-byte granules of a row are exchanged by the row's number, so that the lanes which the LDS serves together, eight that store
-// along two rows or 16 that read from four, find theirs on different banks.
-constexpr int BSH_TILE_PITCH = BWD_TK * 2;
-TGO_DEVICE int tile_granule(int row, int granule) { return granule ^ ((row & 3) * 5); }
-TGO_DEVICE v8bf transposed_fragment(const uint8_t * first, const uint8_t * second) {
-    typedef short four_t __attribute__((ext_vector_type(4)));
-    typedef short eight_t __attribute__((ext_vector_type(8)));
-    const four_t low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) four_t *)(first));
-    const four_t high = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) four_t *)(second));
-    return __builtin_bit_cast(v8bf, eight_t{low.x, low.y, low.z, low.w, high.x, high.y, high.z, high.w});
-}
-
 template <int TYPE>
 __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(const BackwardArgs a) {
     using F = Format<TYPE>;
@@ -1414,7 +1407,7 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
     constexpr int SLOT_PITCH = K45 ? BSH_RAW_PITCH : W::PITCH;
     constexpr int SLOT_FRONT = K45 ? 0 : W::FRONT;
     constexpr int QS = TYPE == Q4_K ? 16 : 48;
-    __shared__ __attribute__((aligned(16))) uint8_t wb[2][BWD_NS * BSH_TILE_PITCH];   // [weight row][K column], bf16 (tile_granule)
+    __shared__ __attribute__((aligned(16))) uint8_t wb[2][BWD_NS * BWD_ROW_PITCH];   // [weight row][K column], bf16 (tile_granule)
     __shared__ __attribute__((aligned(16))) uint8_t raw_all[4][BSH_ROWS_PER_WAVE * SLOT_PITCH];
     // (the magnitude grid, not the 16 KiB selector table of decode16_bf16: with that table only two of these
     // workgroups fit a CU instead of three, which costs more than the cheaper decode brings -- measured)
@@ -1524,7 +1517,7 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
     // A lane decodes 32 values of one weight row (its own, lane / 4): whole 16-byte pieces of the block, the scales from its header, and
     // four 16-byte stores along K.  Rows past the end of the weight matrix decode to exact zeros.
     const int n = lane >> 2;
-    uint8_t * const tile_row = &wb[0][(wave * BSH_ROWS_PER_WAVE + n) * BSH_TILE_PITCH];
+    uint8_t * const tile_row = &wb[0][(wave * BSH_ROWS_PER_WAVE + n) * BWD_ROW_PITCH];
     auto store_sixteen = [&](int buffer, int column, const uint32_t (&pairs)[8]) __attribute__((always_inline)) {
         uint8_t * const row = tile_row + buffer * sizeof(wb[0]);
         *reinterpret_cast<uint4 *>(row + tile_granule(n, column / 8) * 16) = make_uint4(pairs[0], pairs[1], pairs[2], pairs[3]);
@@ -1617,16 +1610,12 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
     for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[rt][v] = 0.0f;
-    // Fragments of the wave's 32 columns: lane (column, half) wants eight weight rows of its column.  ds_read_b64_tr_b16 gives lane i of 16 the
-    // i-th column of the four rows x 16 columns that the 16 lanes address, four lanes side by side in a row.
-    const int tr_row = (lane >> 2) & 3;
-    const uint8_t * const tr_from = &wb[0][(8 * half + tr_row) * BSH_TILE_PITCH + tile_granule(tr_row, 4 * wave + 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1)) * 16 +
-                                           8 * (lane & 1)];
+    const uint8_t * const tr_from = &wb[0][transposed_offset(lane, wave)];   // the wave's 32 columns
     auto multiply = [&](int buffer) __attribute__((always_inline)) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            const uint8_t * const from = tr_from + buffer * sizeof(wb[0]) + 16 * c * BSH_TILE_PITCH;
-            const v8bf bfrag = transposed_fragment(from, from + 4 * BSH_TILE_PITCH);
+            const uint8_t * const from = tr_from + buffer * sizeof(wb[0]) + 16 * c * BWD_ROW_PITCH;
+            const v8bf bfrag = transposed_fragment(from, from + 4 * BWD_ROW_PITCH);
 #pragma unroll
             for (int rt = 0; rt < 2; ++rt) {
                 if (rt < row_tiles) {
