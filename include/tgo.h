@@ -84,7 +84,7 @@ int tgo_q8_workspace_unpack(const void * workspace, void * q_int8, void * d_f32,
  * Decode-sized calls of Q3_K / Q6_K / IQ2_S (dense: at most 8 rows; grouped: at most 64 rows that
  * average at most 4 per listed group, over at most 1024 listed groups) are a single launch whose workgroups quantize their own rows
  * (same q8_1 arithmetic) and, in the grouped entry points, find their task in the group list; such a
- * call leaves `workspace` untouched.
+ * call leaves `workspace` untouched.  (Not where tgo_forward_kernel_for names the kernel for several rows.)
  * Replaces launch_dense_mmq<type>, csrc/mmq_hip.cu:117-147 (called by mmq_cuda, :587-678). */
 int tgo_mmq_forward(const void * input_bf16, const void * packed, void * output_bf16,
                     void * workspace, int64_t rows, int64_t in_features, int64_t out_features,
@@ -93,7 +93,8 @@ int tgo_mmq_forward(const void * input_bf16, const void * packed, void * output_
 /* tgo_mmq_forward and tgo_mmq_forward_prepared_as with tgo_forward_scratch_bytes() bytes of `scratch` (0: NULL is as good): dense
  * calls of more rows than the decode kernels take, whose tiles would not fill the chip, then cut K into ranges that run side by
  * side and leave fp32 sums there, which a second kernel adds up in a fixed order; tgo_mmq_forward_scratch with scaled operands unpacks the
- * weights there once where that pays (the same bits).  No counterpart in the reference. */
+ * weights there once where that pays (the same bits; `workspace` then holds the activations as that product reads them and is no workspace for
+ * the prepared entry points, which give NaN on it, nor for tgo_q8_workspace_unpack, which gives zeros).  No counterpart in the reference. */
 int64_t tgo_forward_scratch_bytes(int64_t rows, int64_t in_features, int64_t out_features, int quant_type);
 int tgo_mmq_forward_scratch(const void * input_bf16, const void * packed, void * output_bf16, void * workspace, void * scratch,
                             int64_t rows, int64_t in_features, int64_t out_features, int quant_type, void * stream);

@@ -124,3 +124,29 @@ def test_forward_of_several_projections(qname, widths):
     workspace = tgo.quantize_q8_1(x, "scaled")
     for output, weight, n in zip(tgo.mmq_multi(x, packed, [qtype] * count, widths), packed, widths):
         assert torch.equal(output, tgo.mmq_prepared(workspace, weight, rows, k, qtype, n, "scaled"))
+
+
+def test_a_workspace_that_such_a_call_used_is_refused():
+    """It holds the activations as the product reads them, whatever it held before: NaN where it is multiplied as a workspace, zeros where it is unpacked."""
+    import synth
+    import torch_ggml_ops as tgo
+    from torch_ggml_ops import _native
+
+    rows, n, k, qtype, lib = 2000, 2048, 2048, QTYPES["Q4_K"], _native.lib
+    packed = synth.random_packed_weight(qtype, (n,), k, seed=1).cuda()
+    x = random_bf16((rows, k), seed=1)
+    workspace = tgo.quantize_q8_1(x, "scaled")
+    assert torch.isfinite(tgo.mmq_prepared(workspace, packed, rows, k, qtype, n, "scaled").float()).all()
+    scratch = torch.empty(lib.tgo_forward_scratch_bytes(rows, k, n, qtype), dtype=torch.uint8, device="cuda")
+    output = torch.empty((rows, n), dtype=torch.bfloat16, device="cuda")
+    stream = _native.stream_of(x.device)
+    _native.check(lib.tgo_mmq_forward_scratch(x.data_ptr(), packed.data_ptr(), output.data_ptr(), workspace.data_ptr(), scratch.data_ptr(), rows, k, n, qtype,
+                                              stream))
+    assert torch.isfinite(output.float()).all()
+    for kind in ("scaled", "int8"):
+        assert torch.isnan(tgo.mmq_prepared(workspace, packed, rows, k, qtype, n, kind).float()).all()
+    q = torch.ones(rows, k, dtype=torch.int8, device="cuda")
+    d = torch.ones(rows, k // 32, device="cuda")
+    s = torch.ones(rows, k // 32, device="cuda")
+    _native.check(lib.tgo_q8_workspace_unpack(workspace.data_ptr(), q.data_ptr(), d.data_ptr(), s.data_ptr(), rows, k, stream))
+    assert not q.any() and not d.any() and not s.any()

@@ -159,6 +159,7 @@ struct ForwardOperandArgs {
     const uint16_t * input;
     uint8_t * x;            // slabs [rows / 32][steps]
     float * row_power;      // 2^E of every activation row
+    uint32_t * tag;         // of the workspace, which holds no q8_1 layout afterwards
 };
 constexpr int UNF_ROWS = 16;   // weight rows of a workgroup
 constexpr int UNF_X_ROWS = 8;  // activation rows of a workgroup
@@ -427,6 +428,9 @@ __global__ __launch_bounds__(256) void forward_operands_kernel(const ForwardOper
     __shared__ float reach[64];
     __shared__ std::conditional_t<TYPE == IQ2_S, Iq2sSelectors, uint2> codebook;
     const int tid = threadIdx.x;
+    if (blockIdx.x == 0 && tid == 0) {
+        *args.tag = 0;
+    }
     if (static_cast<int>(blockIdx.x) >= args.quantize_first) {
         quantize_forward_rows<TYPE == Q4_K || TYPE == Q5_K>(args, static_cast<int>(blockIdx.x) - args.quantize_first, reach, tid);
         return;
@@ -878,6 +882,7 @@ hipError_t launch_forward_unpacked(const uint16_t * input, void * workspace, con
     operands.input = input;
     operands.x = static_cast<uint8_t *>(workspace);
     operands.row_power = reinterpret_cast<float *>(operands.x + pad_rows(rows) * operands.steps * 32);
+    operands.tag = q8_workspace_view(workspace, rows, in_features, false, OPERAND_SCALED).tag;
     int tiles = 0;
     int64_t columns = 0;
     for (int i = 0; i < count; ++i) {
