@@ -1401,8 +1401,10 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
 // (wide_fetch, callers check wide_stage_ok).  A lane decodes 32 values of one weight row and stores them along K; the transposition to the fragments'
 // order happens in the reads (ds_read_b64_tr_b16).  Against a lane that decodes four values of eight rows and stores a transposed tile
 // (24 four- and eight-byte reads of LDS per lane and step instead of three of 16 bytes): groups of 8192 tokens with power-law 1.1 routing over 256
-// experts of 2 x 512 x 2048 Q5_K 133 -> 115 us, 4096 tokens with 0.3, 512 x 2048 Q5_K 57 -> 48, 2 x 512 x 2048 IQ2_S 93 -> 86.  Bound by the
-// vector unit (0.53 of the time at 2.7 waves per SIMD; LDS 0.42, of which a third bank conflicts, matrix cores 0.11).
+// experts of 2 x 512 x 2048 Q5_K 133 -> 115 us, 4096 tokens with 0.3, 512 x 2048 Q5_K 57 -> 48, 2 x 512 x 2048 IQ2_S 93 -> 86.  The formats with a
+// scale per 16 values unpack four quants per operation as the role-split kernel does, instead of one by one: the whole gradient of 1024 tokens of
+// eight choices, 256 experts of 2 x 512 x 2048, IQ2_S 215 -> 175 us, Q3_K 205 -> 188, Q6_K 240 -> 227.  Bound by the
+// vector unit (Q5_K 0.53 of the time at 2.7 waves per SIMD; LDS 0.42, of which a third bank conflicts, matrix cores 0.11).
 constexpr int BSH_THREADS = 256;
 constexpr int BSH_ROWS_PER_WAVE = BWD_NS / 4;
 constexpr int BSH_DEPTH = 2;
@@ -1575,17 +1577,86 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
                 }
                 store_sixteen(buffer, 64 * chunk + 32 * high + 16 * part, pairs);
             }
-        } else {
+        } else if constexpr (TYPE == IQ2_S) {
+            // a block of 32 values: codebook magnitudes with their signs applied, four bytes at a time, above their true values by 128 (as in the
+            // role-split kernel; exact before its rounding)
+            const int quarter = lane & 3, block = 4 * half_block + quarter;
+            const uint8_t * const blk = raw + n * SLOT_PITCH + SLOT_FRONT;
+            const uint32_t indices = lds_u16(blk + 2 + 4 * block) | (lds_u16(blk + 4 + 4 * block) << 16);
+            const uint32_t signs = lds_u16(blk + 34 + 4 * block) | (lds_u16(blk + 36 + 4 * block) << 16);
+            const uint32_t upper = blk[66 + block], scales = blk[74 + block];
+            const float d = half_bits_to_float(lds_u16(blk) & keep);
 #pragma unroll
-            for (int pass = 0; pass < 2; ++pass) {
-                const int unit = 2 * (lane & 3) + pass;
+            for (int run = 0; run < 2; ++run) {
+                const float scale = d * 0.125f * static_cast<float>(((scales >> (4 * run)) & 15u) * 2 + 1);
+                const float offset = scale * 128.0f;
                 uint32_t pairs[8];
-                decode16_bf16<TYPE>(raw + n * SLOT_PITCH + SLOT_FRONT, 8 * half_block + unit, grid, pairs);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    pairs[i] &= keep;
+                for (int o = 0; o < 2; ++o) {
+                    const int octet = 2 * run + o;
+                    const uint2 entry = grid[((indices >> (8 * octet)) & 0xffu) | (((upper >> (2 * octet)) & 3u) << 8)];
+#pragma unroll
+                    for (int w = 0; w < 2; ++w) {
+                        // the four signs spread to a bit per byte; a negative magnitude is its complement plus one
+                        const uint32_t negative = (((signs >> (8 * octet + 4 * w)) & 15u) * 0x00204081u) & 0x01010101u;
+                        const uint32_t q = (((w == 0 ? entry.x : entry.y) ^ (negative * 0xffu)) + negative) ^ 0x80808080u;
+                        float value[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            value[e] = scale * static_cast<float>((q >> (8 * e)) & 0xffu) - offset;
+                        }
+                        pairs[4 * o + 2 * w] = pack_bf16x2(value[0], value[1]);
+                        pairs[4 * o + 2 * w + 1] = pack_bf16x2(value[2], value[3]);
+                    }
                 }
-                store_sixteen(buffer, 16 * unit, pairs);
+                store_sixteen(buffer, 32 * quarter + 16 * run, pairs);
+            }
+        } else {
+            // two runs of 16 values that share their bytes, four quants at a time, above their true values by the bias
+            const int quarter = lane & 3, part = quarter & 1, upper = quarter >> 1;
+            const uint8_t * const blk = raw + n * SLOT_PITCH + SLOT_FRONT;
+            const uint8_t * const low_bits = TYPE == Q6_K ? blk + 64 * half_block + 16 * quarter : blk + 32 + 32 * half_block + 16 * part;
+            const uint8_t * const high_bits = TYPE == Q6_K ? blk + 128 + 32 * half_block + 16 * part : blk + 16 * part;
+            uint32_t low[4], high[4];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                low[w] = lds_u32(low_bits + 4 * w);
+                high[w] = lds_u32(high_bits + 4 * w);
+            }
+            const float d = half_bits_to_float(lds_u16(blk + (TYPE == Q6_K ? 208 : 108)) & keep);
+#pragma unroll
+            for (int run = 0; run < 2; ++run) {
+                int sub, column;
+                if constexpr (TYPE == Q6_K) {
+                    sub = static_cast<int8_t>(blk[192 + 8 * half_block + quarter + 4 * run]);
+                    column = 64 * run + 16 * quarter;
+                } else {
+                    const uint32_t nibble = blk[96 + 4 * upper + 2 * run + part] >> (4 * half_block);
+                    const uint32_t top = blk[104 + 2 * run + part] >> (4 * half_block + 2 * upper);
+                    sub = static_cast<int>((nibble & 15u) | ((top & 3u) << 4)) - 32;
+                    column = 64 * upper + 32 * run + 16 * part;
+                }
+                const float scale = d * static_cast<float>(sub);
+                const float offset = scale * (TYPE == Q6_K ? 32.0f : 4.0f);
+                uint32_t pairs[8];
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    uint32_t q;
+                    if constexpr (TYPE == Q6_K) {
+                        q = ((low[w] >> (4 * run)) & 0x0f0f0f0fu) | (((high[w] >> (2 * upper + 4 * run)) & 0x03030303u) << 4);
+                    } else {
+                        const int group = 2 * upper + run;   // 32-value group of the half block
+                        q = ((low[w] >> (2 * group)) & 0x03030303u) | (((high[w] >> (4 * half_block + group)) & 0x01010101u) << 2);
+                    }
+                    float value[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        value[e] = scale * static_cast<float>((q >> (8 * e)) & 0xffu) - offset;
+                    }
+                    pairs[2 * w] = pack_bf16x2(value[0], value[1]);
+                    pairs[2 * w + 1] = pack_bf16x2(value[2], value[3]);
+                }
+                store_sixteen(buffer, column, pairs);
             }
         }
     };
