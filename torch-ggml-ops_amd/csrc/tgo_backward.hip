@@ -1397,13 +1397,13 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
 // workgroup barrier), one barrier per step publishes the tile, and then every wave multiplies the task's rows with
 // one 32-column slice of it (4 or 8 matrix instructions).  Small footprint: three workgroups share a CU, so one's
 // barrier and memory waits are covered by the others' decoding.  One workgroup per (task, column tile).
-// Q4_K / Q5_K fetch their blocks as the 16-byte units they consist of; the other formats fetch the aligned units that cover their blocks
-// (wide_fetch, callers check wide_stage_ok).  A lane decodes 32 values of one weight row and stores them along K; the transposition to the fragments'
+// Blocks are fetched as 16-byte pieces at their own addresses (BlockPieces).  A lane decodes 32 values of one weight row and stores them along K; the transposition to the fragments'
 // order happens in the reads (ds_read_b64_tr_b16).  Against a lane that decodes four values of eight rows and stores a transposed tile
 // (24 four- and eight-byte reads of LDS per lane and step instead of three of 16 bytes): groups of 8192 tokens with power-law 1.1 routing over 256
 // experts of 2 x 512 x 2048 Q5_K 133 -> 115 us, 4096 tokens with 0.3, 512 x 2048 Q5_K 57 -> 48, 2 x 512 x 2048 IQ2_S 93 -> 86.  The formats with a
 // scale per 16 values unpack four quants per operation as the role-split kernel does, instead of one by one: the whole gradient of 1024 tokens of
-// eight choices, 256 experts of 2 x 512 x 2048, IQ2_S 215 -> 175 us, Q3_K 205 -> 188, Q6_K 240 -> 227.  Bound by the
+// eight choices, 256 experts of 2 x 512 x 2048, IQ2_S 215 -> 175 us, Q3_K 205 -> 188, Q6_K 240 -> 227, and with pieces instead of the aligned units
+// that cover a block 166, 178 and 233 (600 tokens of 128 experts of 2048 x 768: 94, 91 and 105 of 118, 104 and 115).  Bound by the
 // vector unit (Q5_K 0.53 of the time at 2.7 waves per SIMD; LDS 0.42, of which a third bank conflicts, matrix cores 0.11).
 constexpr int BSH_THREADS = 256;
 constexpr int BSH_ROWS_PER_WAVE = BWD_NS / 4;
@@ -1411,17 +1411,15 @@ constexpr int BSH_DEPTH = 2;
 
 template <int TYPE>
 __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(const BackwardArgs a) {
-    using F = Format<TYPE>;
+    using B = SplitBlock<TYPE>;
     constexpr bool K45 = TYPE == Q4_K || TYPE == Q5_K;
-    using W = WideStage<TYPE>;
-    constexpr int RAW_UNITS = K45 ? F::BLOCK_BYTES / 16 : W::UNITS;
-    constexpr int BSH_RAW_PITCH = F::BLOCK_BYTES;   // Q4_K / Q5_K: as in the role-split kernel (16-byte park writes)
-    constexpr int RAW_REGS = (BSH_ROWS_PER_WAVE * RAW_UNITS + 63) / 64;
-    constexpr int SLOT_PITCH = K45 ? BSH_RAW_PITCH : W::PITCH;
-    constexpr int SLOT_FRONT = K45 ? 0 : W::FRONT;
+    constexpr int RAW_UNITS = B::UNITS;
+    constexpr int RAW_PITCH = B::PITCH;
+    constexpr int RAW_REGS = B::REGS;
+    static_assert(BSH_ROWS_PER_WAVE == BSP_ROWS_PER_DECODER, "a wave holds as many weight rows as a decoder wave of the role-split kernel");
     constexpr int QS = TYPE == Q4_K ? 16 : 48;
     __shared__ __attribute__((aligned(16))) uint8_t wb[2][BWD_NS * BWD_ROW_PITCH];   // [weight row][K column], bf16 (tile_granule)
-    __shared__ __attribute__((aligned(16))) uint8_t raw_all[4][BSH_ROWS_PER_WAVE * SLOT_PITCH];
+    __shared__ __attribute__((aligned(16))) uint8_t raw_all[4][B::SLOT_BYTES];
     // (the magnitude grid, not the 16 KiB selector table of decode16_bf16: with that table only two of these
     // workgroups fit a CU instead of three, which costs more than the cheaper decode brings -- measured)
     __shared__ uint2 grid[TYPE == IQ2_S ? TGO_IQ2S_GRID_ENTRIES : 1];
@@ -1460,67 +1458,44 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
     // (the last step of a source clamps rows past the end of the matrix to its last row)
     const int tail_rows = n_total - (steps_per_source - 1) * BWD_NS;
     uint32_t unit_offset[RAW_REGS], unit_offset_tail[RAW_REGS];
-    if constexpr (K45) {
+#pragma unroll
+    for (int i = 0; i < RAW_REGS; ++i) {
+        const int id = min(lane + 64 * i, BSH_ROWS_PER_WAVE * RAW_UNITS - 1);
+        const int row = wave * BSH_ROWS_PER_WAVE + id / RAW_UNITS;
+        const int piece = B::offset(id % RAW_UNITS);
+        unit_offset[i] = static_cast<uint32_t>(row * a.row_bytes + piece);
+        unit_offset_tail[i] = static_cast<uint32_t>(min(row, tail_rows - 1) * a.row_bytes + piece);
+    }
+    const int64_t expert_offset = static_cast<int64_t>(expert) * a.bytes_per_expert + static_cast<int64_t>(kb) * B::BLOCK;
+    // A step's packed blocks in flight.  (Pieces of the 2-byte aligned formats start on any even address.)
+    typedef uint32_t even_t __attribute__((ext_vector_type(4), aligned(2)));
+    struct InFlight {
+        u32x4 unit[RAW_REGS];
+    };
+    auto request = [&](int step, InFlight & regs) __attribute__((always_inline)) {
+        step = min(step, last);
+        const int source = step >= steps_per_source ? 1 : 0;
+        const int n_step = step - source * steps_per_source;
+        const uint8_t * base = (source == 0 ? a.packed[0] : a.packed[1]) + expert_offset +
+                               static_cast<int64_t>(n_step) * BWD_NS * a.row_bytes;
+        const bool tail = n_step == steps_per_source - 1;
+#pragma unroll
+        for (int i = 0; i < RAW_REGS; ++i) {
+            const uint8_t * const from = base + (tail ? unit_offset_tail[i] : unit_offset[i]);
+            if constexpr (B::ALIGNED) {
+                regs.unit[i] = *reinterpret_cast<const u32x4 *>(from);
+            } else {
+                regs.unit[i] = *reinterpret_cast<const even_t *>(from);
+            }
+        }
+    };
+    auto park = [&](const InFlight & regs) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < RAW_REGS; ++i) {
             const int id = min(lane + 64 * i, BSH_ROWS_PER_WAVE * RAW_UNITS - 1);
-            const int row = wave * BSH_ROWS_PER_WAVE + id / RAW_UNITS;
-            const int unit = id % RAW_UNITS;
-            unit_offset[i] = static_cast<uint32_t>(row * a.row_bytes + unit * 16);
-            unit_offset_tail[i] = static_cast<uint32_t>(min(row, tail_rows - 1) * a.row_bytes + unit * 16);
-        }
-    }
-    const int64_t expert_offset = static_cast<int64_t>(expert) * a.bytes_per_expert + static_cast<int64_t>(kb) * F::BLOCK_BYTES;
-    // A step's packed blocks in flight: the units themselves (Q4_K / Q5_K) or the covering aligned units.
-    struct InFlight {
-        u32x4 unit[RAW_REGS];
-        WideRegs<K45 ? 1 : RAW_REGS> wide;
-    };
-    // first of this wave's weight rows in a step and how many of them exist (at least one is read: a wave whose rows
-    // all lie past the end of the matrix repeats the last row and decodes zeros)
-    auto wave_rows = [&](int step, const uint8_t *& rows, int & rows_valid, int & n0) __attribute__((always_inline)) {
-        step = min(step, last);
-        const int source = step >= steps_per_source ? 1 : 0;
-        n0 = (step - source * steps_per_source) * BWD_NS;
-        const int first = min(n0 + wave * BSH_ROWS_PER_WAVE, n_total - 1);
-        rows_valid = min(BSH_ROWS_PER_WAVE, n_total - first);
-        rows = (source == 0 ? a.packed[0] : a.packed[1]) + static_cast<int64_t>(expert) * a.bytes_per_expert +
-               static_cast<int64_t>(first) * a.row_bytes;
-    };
-    auto request = [&](int step, InFlight & regs) __attribute__((always_inline)) {
-        if constexpr (K45) {
-            step = min(step, last);
-            const int source = step >= steps_per_source ? 1 : 0;
-            const int n_step = step - source * steps_per_source;
-            const uint8_t * base = (source == 0 ? a.packed[0] : a.packed[1]) + expert_offset +
-                                   static_cast<int64_t>(n_step) * BWD_NS * a.row_bytes;
-            const bool tail = n_step == steps_per_source - 1;
-#pragma unroll
-            for (int i = 0; i < RAW_REGS; ++i) {
-                regs.unit[i] = *reinterpret_cast<const u32x4 *>(base + (tail ? unit_offset_tail[i] : unit_offset[i]));
-            }
-        } else {
-            const uint8_t * rows;
-            int rows_valid, n0;
-            wave_rows(step, rows, rows_valid, n0);
-            wide_fetch<TYPE, BSH_ROWS_PER_WAVE, 64, RAW_REGS>(regs.wide, rows, static_cast<int>(a.row_bytes), rows_valid, kb, lane);
-        }
-    };
-    // (`step`: the one the registers were requested for)
-    auto park = [&](int step, const InFlight & regs) __attribute__((always_inline)) {
-        if constexpr (K45) {
-#pragma unroll
-            for (int i = 0; i < RAW_REGS; ++i) {
-                const int id = min(lane + 64 * i, BSH_ROWS_PER_WAVE * RAW_UNITS - 1);
-                const int row = id / RAW_UNITS;
-                const int unit = id - row * RAW_UNITS;
-                *reinterpret_cast<u32x4 *>(raw + row * BSH_RAW_PITCH + unit * 16) = regs.unit[i];
-            }
-        } else {
-            const uint8_t * rows;
-            int rows_valid, n0;
-            wave_rows(step, rows, rows_valid, n0);
-            wide_park<TYPE, BSH_ROWS_PER_WAVE, 64, RAW_REGS>(raw, regs.wide, rows, static_cast<int>(a.row_bytes), rows_valid, kb, lane);
+            const int row = id / RAW_UNITS;
+            const int unit = id - row * RAW_UNITS;
+            *reinterpret_cast<u32x4 *>(raw + row * RAW_PITCH + unit * 16) = regs.unit[i];
         }
     };
     auto wave_sync = [&]() __attribute__((always_inline)) {
@@ -1537,15 +1512,13 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
         *reinterpret_cast<uint4 *>(row + tile_granule(n, column / 8 + 1) * 16) = make_uint4(pairs[4], pairs[5], pairs[6], pairs[7]);
     };
     auto decode = [&](int step, int buffer) __attribute__((always_inline)) {
-        const uint8_t * rows;
-        int rows_valid, n0;
-        wave_rows(step, rows, rows_valid, n0);
+        const int n0 = (step >= steps_per_source ? step - steps_per_source : step) * BWD_NS;
         uint32_t keep = n0 + wave * BSH_ROWS_PER_WAVE + n < n_total ? 0xffffffffu : 0u;
         asm volatile("" : "+v"(keep));   // (a mask, not a branch around part of the arithmetic)
+        const uint8_t * const blk = raw + n * RAW_PITCH;
         if constexpr (K45) {
             // 16 bytes of nibbles: 16 values of group 2 chunk of the half block and 16 of the next one
             const int chunk = (lane >> 1) & 1, part = lane & 1;
-            const uint8_t * const blk = raw + n * BSH_RAW_PITCH;
             const uint4 header = *reinterpret_cast<const uint4 *>(blk);
             const uint4 nibbles = *reinterpret_cast<const uint4 *>(blk + QS + 64 * half_block + 32 * chunk + 16 * part);
             const uint4 planes = TYPE == Q5_K ? *reinterpret_cast<const uint4 *>(blk + 16 + 16 * part) : uint4{0, 0, 0, 0};
@@ -1581,11 +1554,9 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
             // a block of 32 values: codebook magnitudes with their signs applied, four bytes at a time, above their true values by 128 (as in the
             // role-split kernel; exact before its rounding)
             const int quarter = lane & 3, block = 4 * half_block + quarter;
-            const uint8_t * const blk = raw + n * SLOT_PITCH + SLOT_FRONT;
-            const uint32_t indices = lds_u16(blk + 2 + 4 * block) | (lds_u16(blk + 4 + 4 * block) << 16);
-            const uint32_t signs = lds_u16(blk + 34 + 4 * block) | (lds_u16(blk + 36 + 4 * block) << 16);
-            const uint32_t upper = blk[66 + block], scales = blk[74 + block];
-            const float d = half_bits_to_float(lds_u16(blk) & keep);
+            const uint32_t indices = lds_u32(blk + 4 * block), signs = lds_u32(blk + 32 + 4 * block);
+            const uint32_t upper = blk[64 + block], scales = blk[72 + block];
+            const float d = half_bits_to_float(lds_u16(blk + 80) & keep);
 #pragma unroll
             for (int run = 0; run < 2; ++run) {
                 const float scale = d * 0.125f * static_cast<float>(((scales >> (4 * run)) & 15u) * 2 + 1);
@@ -1614,16 +1585,10 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
         } else {
             // two runs of 16 values that share their bytes, four quants at a time, above their true values by the bias
             const int quarter = lane & 3, part = quarter & 1, upper = quarter >> 1;
-            const uint8_t * const blk = raw + n * SLOT_PITCH + SLOT_FRONT;
-            const uint8_t * const low_bits = TYPE == Q6_K ? blk + 64 * half_block + 16 * quarter : blk + 32 + 32 * half_block + 16 * part;
-            const uint8_t * const high_bits = TYPE == Q6_K ? blk + 128 + 32 * half_block + 16 * part : blk + 16 * part;
-            uint32_t low[4], high[4];
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                low[w] = lds_u32(low_bits + 4 * w);
-                high[w] = lds_u32(high_bits + 4 * w);
-            }
-            const float d = half_bits_to_float(lds_u16(blk + (TYPE == Q6_K ? 208 : 108)) & keep);
+            const uint4 low_bits = *reinterpret_cast<const uint4 *>(TYPE == Q6_K ? blk + 64 * half_block + 16 * quarter : blk + 32 + 32 * half_block + 16 * part);
+            const uint4 high_bits = *reinterpret_cast<const uint4 *>(TYPE == Q6_K ? blk + 128 + 32 * half_block + 16 * part : blk + 16 * part);
+            const uint32_t low[4] = {low_bits.x, low_bits.y, low_bits.z, low_bits.w}, high[4] = {high_bits.x, high_bits.y, high_bits.z, high_bits.w};
+            const float d = half_bits_to_float(lds_u16(blk + (TYPE == Q6_K ? 222 : 110)) & keep);
 #pragma unroll
             for (int run = 0; run < 2; ++run) {
                 int sub, column;
@@ -1631,8 +1596,8 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
                     sub = static_cast<int8_t>(blk[192 + 8 * half_block + quarter + 4 * run]);
                     column = 64 * run + 16 * quarter;
                 } else {
-                    const uint32_t nibble = blk[96 + 4 * upper + 2 * run + part] >> (4 * half_block);
-                    const uint32_t top = blk[104 + 2 * run + part] >> (4 * half_block + 2 * upper);
+                    const uint32_t nibble = blk[98 + 4 * upper + 2 * run + part] >> (4 * half_block);
+                    const uint32_t top = blk[106 + 2 * run + part] >> (4 * half_block + 2 * upper);
                     sub = static_cast<int>((nibble & 15u) | ((top & 3u) << 4)) - 32;
                     column = 64 * upper + 32 * run + 16 * part;
                 }
@@ -1713,7 +1678,7 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
         request(d, ring[d]);
     }
     request_cotangent(0);
-    park(0, ring[0]);
+    park(ring[0]);
     request(BSH_DEPTH, ring[0]);
     wave_sync();
     decode(0, 0);
@@ -1728,7 +1693,7 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
         // (this wave's decode of the current step, the last reader of its slot, is behind it in program order)
         // the chain of dependent waits goes first, the arithmetic of the decode fills in (measured: 1 %)
         __builtin_amdgcn_s_setprio(3);
-        park(step + 1, ring[u ^ 1]);
+        park(ring[u ^ 1]);
         multiply(u);
         // both requests go out behind the matrix instructions, which wait for the previous step's cotangent only
         request_cotangent(step + 1);
@@ -1826,16 +1791,8 @@ static hipError_t launch_backward_typed(const BackwardArgs & args, hipStream_t s
         // (32-bit lane offsets into the packed cotangent and a step's weight rows, as in the role-split kernel)
         if (cotangent_workspace_bytes(args.rows, args.out_features) < (int64_t{1} << 32) &&
             args.row_bytes * 2 * BWD_NS < (int64_t{1} << 32)) {
-            bool fits = true;
-            if constexpr (Format<TYPE>::BLOCK_BYTES % 16 != 0) {
-                const int64_t weight_bytes = static_cast<int64_t>(args.out_features) * args.row_bytes;
-                fits = args.row_bytes < (1 << 24) && wide_stage_ok(args.packed[0], weight_bytes) &&
-                       (args.packed[1] == nullptr || wide_stage_ok(args.packed[1], weight_bytes));
-            }
-            if (fits) {
-                mmq_grad_input_short_kernel<TYPE><<<static_cast<unsigned>(total_short), BSH_THREADS, 0, stream>>>(short_args);
-                launched = true;
-            }
+            mmq_grad_input_short_kernel<TYPE><<<static_cast<unsigned>(total_short), BSH_THREADS, 0, stream>>>(short_args);
+            launched = true;
         }
         if (!launched) {
             general(std::true_type{}, dim3(static_cast<unsigned>(total_short)), short_args);
