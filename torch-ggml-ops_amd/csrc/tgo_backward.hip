@@ -1420,8 +1420,7 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
     constexpr int QS = TYPE == Q4_K ? 16 : 48;
     __shared__ __attribute__((aligned(16))) uint8_t wb[2][BWD_NS * BWD_ROW_PITCH];   // [weight row][K column], bf16 (tile_granule)
     __shared__ __attribute__((aligned(16))) uint8_t raw_all[4][B::SLOT_BYTES];
-    // (the magnitude grid, not the 16 KiB selector table of decode16_bf16: with that table only two of these
-    // workgroups fit a CU instead of three, which costs more than the cheaper decode brings -- measured)
+    // (the magnitude grid: with the 16 KiB selector table of decode16_bf16 only two of these workgroups fit a CU instead of three)
     __shared__ uint2 grid[TYPE == IQ2_S ? TGO_IQ2S_GRID_ENTRIES : 1];
 
     const int tid = threadIdx.x;
