@@ -646,8 +646,8 @@ static inline UnpackedGradWorkspace unpacked_grad_workspace(void * base, int64_t
 // either takes.  The latter packs the cotangent, then runs items of 256 x 128, a round of 256 taking 0.27 us per 16 weight rows and half a
 // round 0.18, and cuts the reduction where that leaves half of the chip idle, for fp32 sums to be written and read again.  `count`
 // projections of one input (their weight rows together) would take a call each and an addition.
-// Of the time of the kernels that unpack as they multiply (3 % more on the mean than they take since their tile lies along K), where this rule leaves them (250 calls of 96 to 16384 rows, 512 to 28672 weight rows, K
-// 512 to 8192, all formats): 0.78 on the mean, 0.5 to 1.07.  4096 x 2048: 2000 rows Q4_K 58.9 -> 51.0 us, Q6_K 63.7 -> 47.8; 4096 rows 87.2 -> 74.8,
+// Of the time of the kernels that unpack as they multiply, where this rule leaves them (70 calls of 96 to 16384 rows, 512 to 28672 weight rows, K
+// 512 to 8192, all formats): 0.82 on the mean, 1.09 at most (257 rows of 1260 x 4608 IQ2_S 25.3 -> 27.5 us); before those kernels' tile lay along K:  4096 x 2048: 2000 rows Q4_K 58.9 -> 51.0 us, Q6_K 63.7 -> 47.8; 4096 rows 87.2 -> 74.8,
 // 96.3 -> 73.0; 8192 rows 165.6 -> 122.6, 184.0 -> 121.9.  On the other side of it, always unpacked: 28672 x 8192, 300 rows 206 -> 413 us (Q4_K); 4096 x
 // 2048, 300 rows 28.5 -> 30.2.
 static inline bool grad_unpacks(int64_t rows, int64_t out_features, int64_t in_features, int count = 1) {
