@@ -1397,29 +1397,53 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
 // workgroup barrier), one barrier per step publishes the tile, and then every wave multiplies the task's rows with
 // one 32-column slice of it (4 or 8 matrix instructions).  Small footprint: three workgroups share a CU, so one's
 // barrier and memory waits are covered by the others' decoding.  One workgroup per (task, column tile).
-// Blocks are fetched as 16-byte pieces at their own addresses (BlockPieces).  A lane decodes 32 values of one weight row and stores them along K; the transposition to the fragments'
+// Blocks are fetched as 16-byte pieces at their own addresses, those that the column tile needs (HalfBlockPieces).  A lane decodes 32 values of one weight row and stores them along K; the transposition to the fragments'
 // order happens in the reads (ds_read_b64_tr_b16).  Against a lane that decodes four values of eight rows and stores a transposed tile
 // (24 four- and eight-byte reads of LDS per lane and step instead of three of 16 bytes): groups of 8192 tokens with power-law 1.1 routing over 256
 // experts of 2 x 512 x 2048 Q5_K 133 -> 115 us, 4096 tokens with 0.3, 512 x 2048 Q5_K 57 -> 48, 2 x 512 x 2048 IQ2_S 93 -> 86.  The formats with a
 // scale per 16 values unpack four quants per operation as the role-split kernel does, instead of one by one: the whole gradient of 1024 tokens of
 // eight choices, 256 experts of 2 x 512 x 2048, IQ2_S 215 -> 175 us, Q3_K 205 -> 188, Q6_K 240 -> 227, and with pieces instead of the aligned units
-// that cover a block 166, 178 and 233 (600 tokens of 128 experts of 2048 x 768: 94, 91 and 105 of 118, 104 and 115).  Bound by the
+// that cover a block, and of those only what the tile needs, 155, 177 and 193 (Q5_K 187 -> 179, Q4_K 176 -> 162; 600 tokens of 128 experts of 2048 x
+// 768: IQ2_S 118 -> 90, Q3_K 104 -> 89, Q6_K 115 -> 91).  Four workgroups per CU, which Q3_K to Q5_K then have room for, are no faster.  Bound by the
 // vector unit (Q5_K 0.53 of the time at 2.7 waves per SIMD; LDS 0.42, of which a third bank conflicts, matrix cores 0.11).
 constexpr int BSH_THREADS = 256;
 constexpr int BSH_ROWS_PER_WAVE = BWD_NS / 4;
 constexpr int BSH_DEPTH = 2;
 
+// What a column tile, half a super-block, needs of a block, in 16-byte pieces at their own addresses.  Slot of a row in LDS, PITCH bytes:
+//   Q4_K   header 0, nibbles 16            Q5_K   header 0, fifth bits 16, nibbles 48
+//   Q3_K   high bits 0, low bits 32, the block's last 16 bytes 64: scales from 66, d at 78
+//   Q6_K   low bits 0, high bits 64, scales 96, the block's last 16 bytes 112: d at 126
+//   IQ2_S  indices 0, signs 16, upper index bits 32, scales 40, the block's first 16 bytes 48: d there
+template <int TYPE>
+struct HalfBlockPieces {
+    static constexpr int UNITS = TYPE == Q5_K ? 7 : TYPE == Q6_K ? 8 : TYPE == IQ2_S ? 4 : 5;
+    static constexpr int PITCH = UNITS % 2 == 1 ? 16 * UNITS : 16 * UNITS + 16;   // (4 * odd words: rows spread over the banks)
+    static constexpr int REGS = (BSH_ROWS_PER_WAVE * UNITS + 63) / 64;
+    __device__ __forceinline__ static int offset(int unit, int half_block) {   // of a piece in the block
+        if constexpr (TYPE == Q4_K) {
+            return unit == 0 ? 0 : 64 * half_block + 16 * unit;
+        } else if constexpr (TYPE == Q5_K) {
+            return unit < 3 ? 16 * unit : 64 * half_block + 16 * unit;
+        } else if constexpr (TYPE == Q3_K) {
+            return unit < 2 ? 16 * unit : unit < 4 ? 32 * half_block + 16 * unit : Format<TYPE>::BLOCK_BYTES - 16;
+        } else if constexpr (TYPE == Q6_K) {
+            return unit < 4 ? 64 * half_block + 16 * unit : unit < 6 ? 64 + 32 * half_block + 16 * unit : unit == 6 ? 192 : Format<TYPE>::BLOCK_BYTES - 16;
+        } else {
+            return unit < 2 ? 2 + 32 * unit + 16 * half_block : unit == 2 ? 66 : 0;
+        }
+    }
+};
+
 template <int TYPE>
 __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(const BackwardArgs a) {
-    using B = SplitBlock<TYPE>;
+    using B = HalfBlockPieces<TYPE>;
     constexpr bool K45 = TYPE == Q4_K || TYPE == Q5_K;
     constexpr int RAW_UNITS = B::UNITS;
     constexpr int RAW_PITCH = B::PITCH;
     constexpr int RAW_REGS = B::REGS;
-    static_assert(BSH_ROWS_PER_WAVE == BSP_ROWS_PER_DECODER, "a wave holds as many weight rows as a decoder wave of the role-split kernel");
-    constexpr int QS = TYPE == Q4_K ? 16 : 48;
     __shared__ __attribute__((aligned(16))) uint8_t wb[2][BWD_NS * BWD_ROW_PITCH];   // [weight row][K column], bf16 (tile_granule)
-    __shared__ __attribute__((aligned(16))) uint8_t raw_all[4][B::SLOT_BYTES];
+    __shared__ __attribute__((aligned(16))) uint8_t raw_all[4][BSH_ROWS_PER_WAVE * RAW_PITCH];
     // (the magnitude grid: with the 16 KiB selector table of decode16_bf16 only two of these workgroups fit a CU instead of three)
     __shared__ uint2 grid[TYPE == IQ2_S ? TGO_IQ2S_GRID_ENTRIES : 1];
 
@@ -1461,11 +1485,11 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
     for (int i = 0; i < RAW_REGS; ++i) {
         const int id = min(lane + 64 * i, BSH_ROWS_PER_WAVE * RAW_UNITS - 1);
         const int row = wave * BSH_ROWS_PER_WAVE + id / RAW_UNITS;
-        const int piece = B::offset(id % RAW_UNITS);
+        const int piece = B::offset(id % RAW_UNITS, half_block);
         unit_offset[i] = static_cast<uint32_t>(row * a.row_bytes + piece);
         unit_offset_tail[i] = static_cast<uint32_t>(min(row, tail_rows - 1) * a.row_bytes + piece);
     }
-    const int64_t expert_offset = static_cast<int64_t>(expert) * a.bytes_per_expert + static_cast<int64_t>(kb) * B::BLOCK;
+    const int64_t expert_offset = static_cast<int64_t>(expert) * a.bytes_per_expert + static_cast<int64_t>(kb) * Format<TYPE>::BLOCK_BYTES;
     // A step's packed blocks in flight.  (Pieces of the 2-byte aligned formats start on any even address.)
     typedef uint32_t even_t __attribute__((ext_vector_type(4), aligned(2)));
     struct InFlight {
@@ -1481,7 +1505,7 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
 #pragma unroll
         for (int i = 0; i < RAW_REGS; ++i) {
             const uint8_t * const from = base + (tail ? unit_offset_tail[i] : unit_offset[i]);
-            if constexpr (B::ALIGNED) {
+            if constexpr (K45) {
                 regs.unit[i] = *reinterpret_cast<const u32x4 *>(from);
             } else {
                 regs.unit[i] = *reinterpret_cast<const even_t *>(from);
@@ -1519,7 +1543,7 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
             // 16 bytes of nibbles: 16 values of group 2 chunk of the half block and 16 of the next one
             const int chunk = (lane >> 1) & 1, part = lane & 1;
             const uint4 header = *reinterpret_cast<const uint4 *>(blk);
-            const uint4 nibbles = *reinterpret_cast<const uint4 *>(blk + QS + 64 * half_block + 32 * chunk + 16 * part);
+            const uint4 nibbles = *reinterpret_cast<const uint4 *>(blk + (TYPE == Q4_K ? 16 : 48) + 32 * chunk + 16 * part);
             const uint4 planes = TYPE == Q5_K ? *reinterpret_cast<const uint4 *>(blk + 16 + 16 * part) : uint4{0, 0, 0, 0};
             const uint32_t word[4] = {nibbles.x, nibbles.y, nibbles.z, nibbles.w}, plane[4] = {planes.x, planes.y, planes.z, planes.w};
             const uint32_t first = header.y >> (16 * chunk), second = header.z >> (16 * chunk), third = header.w >> (16 * chunk);
@@ -1553,9 +1577,9 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
             // a block of 32 values: codebook magnitudes with their signs applied, four bytes at a time, above their true values by 128 (as in the
             // role-split kernel; exact before its rounding)
             const int quarter = lane & 3, block = 4 * half_block + quarter;
-            const uint32_t indices = lds_u32(blk + 4 * block), signs = lds_u32(blk + 32 + 4 * block);
-            const uint32_t upper = blk[64 + block], scales = blk[72 + block];
-            const float d = half_bits_to_float(lds_u16(blk + 80) & keep);
+            const uint32_t indices = lds_u32(blk + 4 * quarter), signs = lds_u32(blk + 16 + 4 * quarter);
+            const uint32_t upper = blk[32 + block], scales = blk[40 + block];
+            const float d = half_bits_to_float(lds_u16(blk + 48) & keep);
 #pragma unroll
             for (int run = 0; run < 2; ++run) {
                 const float scale = d * 0.125f * static_cast<float>(((scales >> (4 * run)) & 15u) * 2 + 1);
@@ -1584,19 +1608,19 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
         } else {
             // two runs of 16 values that share their bytes, four quants at a time, above their true values by the bias
             const int quarter = lane & 3, part = quarter & 1, upper = quarter >> 1;
-            const uint4 low_bits = *reinterpret_cast<const uint4 *>(TYPE == Q6_K ? blk + 64 * half_block + 16 * quarter : blk + 32 + 32 * half_block + 16 * part);
-            const uint4 high_bits = *reinterpret_cast<const uint4 *>(TYPE == Q6_K ? blk + 128 + 32 * half_block + 16 * part : blk + 16 * part);
+            const uint4 low_bits = *reinterpret_cast<const uint4 *>(TYPE == Q6_K ? blk + 16 * quarter : blk + 32 + 16 * part);
+            const uint4 high_bits = *reinterpret_cast<const uint4 *>(TYPE == Q6_K ? blk + 64 + 16 * part : blk + 16 * part);
             const uint32_t low[4] = {low_bits.x, low_bits.y, low_bits.z, low_bits.w}, high[4] = {high_bits.x, high_bits.y, high_bits.z, high_bits.w};
-            const float d = half_bits_to_float(lds_u16(blk + (TYPE == Q6_K ? 222 : 110)) & keep);
+            const float d = half_bits_to_float(lds_u16(blk + (TYPE == Q6_K ? 126 : 78)) & keep);
 #pragma unroll
             for (int run = 0; run < 2; ++run) {
                 int sub, column;
                 if constexpr (TYPE == Q6_K) {
-                    sub = static_cast<int8_t>(blk[192 + 8 * half_block + quarter + 4 * run]);
+                    sub = static_cast<int8_t>(blk[96 + 8 * half_block + quarter + 4 * run]);
                     column = 64 * run + 16 * quarter;
                 } else {
-                    const uint32_t nibble = blk[98 + 4 * upper + 2 * run + part] >> (4 * half_block);
-                    const uint32_t top = blk[106 + 2 * run + part] >> (4 * half_block + 2 * upper);
+                    const uint32_t nibble = blk[66 + 4 * upper + 2 * run + part] >> (4 * half_block);
+                    const uint32_t top = blk[74 + 2 * run + part] >> (4 * half_block + 2 * upper);
                     sub = static_cast<int>((nibble & 15u) | ((top & 3u) << 4)) - 32;
                     column = 64 * upper + 32 * run + 16 * part;
                 }

@@ -647,8 +647,8 @@ static inline UnpackedGradWorkspace unpacked_grad_workspace(void * base, int64_t
 // round 0.18, and cuts the reduction where that leaves half of the chip idle, for fp32 sums to be written and read again.  `count`
 // projections of one input (their weight rows together) would take a call each and an addition.
 // Of the time of the kernels that unpack as they multiply, where this rule leaves them (70 calls of 96 to 16384 rows, 512 to 28672 weight rows, K
-// 512 to 8192, all formats): 0.82 on the mean, 1.09 at most (257 rows of 1260 x 4608 IQ2_S 25.3 -> 27.5 us); before those kernels' tile lay along K:  4096 x 2048: 2000 rows Q4_K 58.9 -> 51.0 us, Q6_K 63.7 -> 47.8; 4096 rows 87.2 -> 74.8,
-// 96.3 -> 73.0; 8192 rows 165.6 -> 122.6, 184.0 -> 121.9.  On the other side of it, always unpacked: 28672 x 8192, 300 rows 206 -> 413 us (Q4_K); 4096 x
+// 512 to 8192, all formats): 0.82 on the mean, 1.09 at most (257 rows of 1260 x 4608 IQ2_S 25.3 -> 27.5 us); before those kernels'
+// tile lay along K: 4096 x 2048, 2000 rows Q4_K 58.9 -> 51.0 us, Q6_K 63.7 -> 47.8; 4096 rows 87.2 -> 74.8, 96.3 -> 73.0; 8192 rows 165.6 -> 122.6, 184.0 -> 121.9.  On the other side of it, always unpacked: 28672 x 8192, 300 rows 206 -> 413 us (Q4_K); 4096 x
 // 2048, 300 rows 28.5 -> 30.2.
 static inline bool grad_unpacks(int64_t rows, int64_t out_features, int64_t in_features, int count = 1) {
     // (32-bit lane offsets; a workspace of at most 1 GiB for the weights)
