@@ -754,6 +754,31 @@ TGO_DEVICE v8bf transposed_fragment(const uint8_t * first, const uint8_t * secon
     return __builtin_bit_cast(v8bf, eight_t{low.x, low.y, low.z, low.w, high.x, high.y, high.z, high.w});
 }
 
+// What a column tile, half a super-block, needs of a block, in 16-byte pieces at their own addresses.  Slot of a row in LDS, PITCH bytes:
+//   Q4_K   header 0, nibbles 16            Q5_K   header 0, fifth bits 16, nibbles 48
+//   Q3_K   high bits 0, low bits 32, the block's last 16 bytes 64: scales from 66, d at 78
+//   Q6_K   low bits 0, high bits 64, scales 96, the block's last 16 bytes 112: d at 126
+//   IQ2_S  indices 0, signs 16, upper index bits 32, scales 40, the block's first 16 bytes 48: d there
+template <int TYPE>
+struct HalfBlockPieces {
+    static constexpr int UNITS = TYPE == Q5_K ? 7 : TYPE == Q6_K ? 8 : TYPE == IQ2_S ? 4 : 5;
+    static constexpr int PITCH = UNITS % 2 == 1 ? 16 * UNITS : 16 * UNITS + 16;   // (4 * odd words: rows spread over the banks)
+    static constexpr int REGS = (BWD_NS / 4 * UNITS + 63) / 64;   // of a wave's 16 weight rows, per lane
+    __device__ __forceinline__ static int offset(int unit, int half_block) {   // of a piece in the block
+        if constexpr (TYPE == Q4_K) {
+            return unit == 0 ? 0 : 64 * half_block + 16 * unit;
+        } else if constexpr (TYPE == Q5_K) {
+            return unit < 3 ? 16 * unit : 64 * half_block + 16 * unit;
+        } else if constexpr (TYPE == Q3_K) {
+            return unit < 2 ? 16 * unit : unit < 4 ? 32 * half_block + 16 * unit : Format<TYPE>::BLOCK_BYTES - 16;
+        } else if constexpr (TYPE == Q6_K) {
+            return unit < 4 ? 64 * half_block + 16 * unit : unit < 6 ? 64 + 32 * half_block + 16 * unit : unit == 6 ? 192 : Format<TYPE>::BLOCK_BYTES - 16;
+        } else {
+            return unit < 2 ? 2 + 32 * unit + 16 * half_block : unit == 2 ? 66 : 0;
+        }
+    }
+};
+
 // ---- role-split variant --------------------------------------------------------------------------------------
 // 256 rows x 128 values of K, reduction steps of 64 weight rows, double-buffered bf16
 // tile; the eight waves of a workgroup are specialised: waves 0-3 only multiply (64 rows each), waves
@@ -776,7 +801,9 @@ TGO_DEVICE v8bf transposed_fragment(const uint8_t * first, const uint8_t * secon
 // against the general kernel, whose waves dequantize and multiply in turn.  Then a lane decoded four values of eight weight rows, for a tile that
 // was stored transposed, after a stage for the block scales; with 32 values of a row per lane and the transposition in the reads (tile_granule) the
 // LDS is busy for 0.29 to 0.36 of the time instead of 0.43 to 0.6: 4096 tokens of eight choices among 256 experts with power-law 0.3 routing, 2 x
-// 512 x 2048 IQ2_S 276 -> 254 us, 512 x 2048 Q5_K 150 -> 138; dense calls of 33 to 900 rows 0.97 on the mean.  What is left: the matrix pipe is busy
+// 512 x 2048 IQ2_S 276 -> 254 us, 512 x 2048 Q5_K 150 -> 138; dense calls of 33 to 900 rows 0.97 on the mean.  With the pieces of the column tile's
+// half block in place of the whole block (5 to 8 of 9 to 14) the head Q6_K 344 -> 317, IQ2_S 313 -> 305, Q5_K 319 -> 315; a pair of 8192 tokens
+// Q6_K 497 -> 478, IQ2_S 448 -> 439, Q5_K 458 -> 454.  What is left: the matrix pipe is busy
 // for 0.32 (tasks that half fill 256 rows) to 0.44 of the time at the clock that the card's power leaves (1.9 GHz with 256 rows of the head).
 constexpr int BSP_THREADS = 512;
 constexpr int BSP_ROWS_PER_DECODER = BWD_NS / 4;   // weight rows a decoder wave owns per step
@@ -797,6 +824,10 @@ constexpr int BSP_GRID = 256;                      // one workgroup per CU
 template <int IMMEDIATE = 0>
 TGO_DEVICE void async_load16(u32x4 & destination, const void * base, uint32_t offset) {
     asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(destination) : "v"(offset), "s"(base), "n"(IMMEDIATE));
+}
+template <int YOUNGER>
+TGO_DEVICE void await_loads(u32x4 (&r)[1]) {
+    asm volatile("s_waitcnt vmcnt(%1)" : "+v"(r[0]) : "n"(YOUNGER));
 }
 template <int YOUNGER>
 TGO_DEVICE void await_loads(u32x4 (&r)[2]) {
@@ -830,10 +861,8 @@ struct SplitItem {
 
 // How the decoder waves hold a format's packed blocks.
 template <int TYPE>
-struct SplitBlock : BlockPieces<TYPE> {
-    using P = BlockPieces<TYPE>;
-    static constexpr int SLOT_BYTES = BSP_ROWS_PER_DECODER * P::PITCH;
-    static constexpr int REGS = (BSP_ROWS_PER_DECODER * P::UNITS + 63) / 64;
+struct SplitBlock : HalfBlockPieces<TYPE> {
+    static constexpr int SLOT_BYTES = BSP_ROWS_PER_DECODER * HalfBlockPieces<TYPE>::PITCH;
     static constexpr int BIAS = TYPE == Q3_K ? 4 : TYPE == Q6_K ? 32 : TYPE == IQ2_S ? 128 : 0;   // of the quants as unsigned bytes
 };
 
@@ -859,7 +888,6 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
     constexpr int RAW_UNITS = B::UNITS;
     constexpr int BSP_RAW_PITCH = B::PITCH;
     constexpr int RAW_REGS = B::REGS;
-    constexpr int QS = TYPE == Q4_K ? 16 : 48;
     __shared__ __attribute__((aligned(16))) uint8_t wb[2][BWD_NS * BWD_ROW_PITCH];   // [weight row][K column], bf16 (tile_granule)
     __shared__ __attribute__((aligned(16))) uint8_t raw_all[4][3][B::SLOT_BYTES];
     __shared__ uint2 grid[TYPE == IQ2_S ? TGO_IQ2S_GRID_ENTRIES : 1];   // codebook
@@ -1011,26 +1039,27 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
         // Lane offsets of the 16-byte units this lane fetches per step, relative to the step's first weight
         // row; the last step of a source clamps rows past the end of the matrix to its last row.
         const int tail_rows = n_total - (steps_per_source - 1) * BWD_NS;
-        uint32_t unit_offset[RAW_REGS], unit_offset_tail[RAW_REGS];
+        uint32_t unit_offset[RAW_REGS], unit_offset_tail[RAW_REGS], second_half[RAW_REGS];   // (second_half: from a piece of the first half block to the other's)
         const auto lane_row = [&](int i) { return min(lane + 64 * i, BSP_ROWS_PER_DECODER * RAW_UNITS - 1) / RAW_UNITS; };
         const auto lane_unit = [&](int i) { return min(lane + 64 * i, BSP_ROWS_PER_DECODER * RAW_UNITS - 1) % RAW_UNITS; };
 #pragma unroll
         for (int i = 0; i < RAW_REGS; ++i) {
             const int row = dw * BSP_ROWS_PER_DECODER + lane_row(i);
-            const int piece = B::offset(lane_unit(i));
+            const int piece = B::offset(lane_unit(i), 0);
             unit_offset[i] = static_cast<uint32_t>(row * a.row_bytes + piece);
             unit_offset_tail[i] = static_cast<uint32_t>(min(row, tail_rows - 1) * a.row_bytes + piece);
+            second_half[i] = static_cast<uint32_t>(B::offset(lane_unit(i), 1) - piece);
         }
         const int64_t step_bytes = BWD_NS * a.row_bytes;
         auto rebase = [&](SplitCursor & c) {
             c.base = (c.source == 0 ? packed_of[0] : packed_of[1]) + static_cast<int64_t>(c.expert) * a.bytes_per_expert +
-                     static_cast<int64_t>(c.k_tile >> 1) * B::BLOCK + c.step_begin * step_bytes;
+                     static_cast<int64_t>(c.k_tile >> 1) * Format<TYPE>::BLOCK_BYTES + c.step_begin * step_bytes;
         };
         auto load_raw = [&](const SplitCursor & c, u32x4 (&regs)[RAW_REGS]) {
             const bool tail = c.n_step == steps_per_source - 1;
 #pragma unroll
             for (int i = 0; i < RAW_REGS; ++i) {
-                async_load16(regs[i], c.base, tail ? unit_offset_tail[i] : unit_offset[i]);
+                async_load16(regs[i], c.base, (tail ? unit_offset_tail[i] : unit_offset[i]) + ((c.k_tile & 1) != 0 ? second_half[i] : 0u));
             }
         };
         // stage 1: packed blocks from registers to an LDS slot
@@ -1059,29 +1088,29 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
             const auto bytes16 = [&](int at) { return *reinterpret_cast<const uint4 *>(blk + at); };
             if constexpr (K45) {
                 unpack4(bytes16(0), in.header);
-                unpack4(bytes16(QS + 64 * half_block + 16 * quarter), in.low);
+                unpack4(bytes16((TYPE == Q4_K ? 16 : 48) + 16 * quarter), in.low);
                 if constexpr (TYPE == Q5_K) {
                     unpack4(bytes16(16 + 16 * (quarter & 1)), in.high);
                 }
             } else if constexpr (TYPE == Q3_K) {
-                unpack4(bytes16(32 + 32 * half_block + 16 * (quarter & 1)), in.low);
+                unpack4(bytes16(32 + 16 * (quarter & 1)), in.low);
                 unpack4(bytes16(16 * (quarter & 1)), in.high);
                 const int unit = 4 * (quarter >> 1) + (quarter & 1);   // of the half block, and the one two behind it
-                in.header[0] = lds_u16(blk + 110);
-                in.header[1] = (static_cast<uint32_t>(blk[98 + unit]) >> (4 * half_block)) | (static_cast<uint32_t>(blk[100 + unit]) >> (4 * half_block) << 16);
-                in.header[2] = blk[106 + (quarter & 1)] | (static_cast<uint32_t>(blk[108 + (quarter & 1)]) << 16);
+                in.header[0] = lds_u16(blk + 78);
+                in.header[1] = (static_cast<uint32_t>(blk[66 + unit]) >> (4 * half_block)) | (static_cast<uint32_t>(blk[68 + unit]) >> (4 * half_block) << 16);
+                in.header[2] = blk[74 + (quarter & 1)] | (static_cast<uint32_t>(blk[76 + (quarter & 1)]) << 16);
             } else if constexpr (TYPE == Q6_K) {
-                unpack4(bytes16(64 * half_block + 16 * quarter), in.low);
-                unpack4(bytes16(128 + 32 * half_block + 16 * (quarter & 1)), in.high);
-                in.header[0] = lds_u16(blk + 222);
-                in.header[1] = blk[192 + 8 * half_block + quarter];
-                in.header[2] = blk[196 + 8 * half_block + quarter];
+                unpack4(bytes16(16 * quarter), in.low);
+                unpack4(bytes16(64 + 16 * (quarter & 1)), in.high);
+                in.header[0] = lds_u16(blk + 126);
+                in.header[1] = blk[96 + 8 * half_block + quarter];
+                in.header[2] = blk[100 + 8 * half_block + quarter];
             } else {
-                in.low[0] = lds_u32(blk + 16 * half_block + 4 * quarter);        // codebook indices of four octets, eight bits each
-                in.low[1] = lds_u32(blk + 32 + 16 * half_block + 4 * quarter);   // their signs
-                in.low[2] = blk[64 + 4 * half_block + quarter];                  // the indices' upper two bits
-                in.header[0] = lds_u16(blk + 80);
-                in.header[1] = blk[72 + 4 * half_block + quarter];
+                in.low[0] = lds_u32(blk + 4 * quarter);        // codebook indices of four octets, eight bits each
+                in.low[1] = lds_u32(blk + 16 + 4 * quarter);   // their signs
+                in.low[2] = blk[32 + 4 * half_block + quarter];   // the indices' upper two bits
+                in.header[0] = lds_u16(blk + 48);
+                in.header[1] = blk[40 + 4 * half_block + quarter];
             }
             return in;
         };
@@ -1409,31 +1438,6 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
 constexpr int BSH_THREADS = 256;
 constexpr int BSH_ROWS_PER_WAVE = BWD_NS / 4;
 constexpr int BSH_DEPTH = 2;
-
-// What a column tile, half a super-block, needs of a block, in 16-byte pieces at their own addresses.  Slot of a row in LDS, PITCH bytes:
-//   Q4_K   header 0, nibbles 16            Q5_K   header 0, fifth bits 16, nibbles 48
-//   Q3_K   high bits 0, low bits 32, the block's last 16 bytes 64: scales from 66, d at 78
-//   Q6_K   low bits 0, high bits 64, scales 96, the block's last 16 bytes 112: d at 126
-//   IQ2_S  indices 0, signs 16, upper index bits 32, scales 40, the block's first 16 bytes 48: d there
-template <int TYPE>
-struct HalfBlockPieces {
-    static constexpr int UNITS = TYPE == Q5_K ? 7 : TYPE == Q6_K ? 8 : TYPE == IQ2_S ? 4 : 5;
-    static constexpr int PITCH = UNITS % 2 == 1 ? 16 * UNITS : 16 * UNITS + 16;   // (4 * odd words: rows spread over the banks)
-    static constexpr int REGS = (BSH_ROWS_PER_WAVE * UNITS + 63) / 64;
-    __device__ __forceinline__ static int offset(int unit, int half_block) {   // of a piece in the block
-        if constexpr (TYPE == Q4_K) {
-            return unit == 0 ? 0 : 64 * half_block + 16 * unit;
-        } else if constexpr (TYPE == Q5_K) {
-            return unit < 3 ? 16 * unit : 64 * half_block + 16 * unit;
-        } else if constexpr (TYPE == Q3_K) {
-            return unit < 2 ? 16 * unit : unit < 4 ? 32 * half_block + 16 * unit : Format<TYPE>::BLOCK_BYTES - 16;
-        } else if constexpr (TYPE == Q6_K) {
-            return unit < 4 ? 64 * half_block + 16 * unit : unit < 6 ? 64 + 32 * half_block + 16 * unit : unit == 6 ? 192 : Format<TYPE>::BLOCK_BYTES - 16;
-        } else {
-            return unit < 2 ? 2 + 32 * unit + 16 * half_block : unit == 2 ? 66 : 0;
-        }
-    }
-};
 
 template <int TYPE>
 __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(const BackwardArgs a) {
