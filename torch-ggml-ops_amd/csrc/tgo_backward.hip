@@ -804,7 +804,7 @@ struct HalfBlockPieces {
 // 512 x 2048 IQ2_S 276 -> 254 us, 512 x 2048 Q5_K 150 -> 138; dense calls of 33 to 900 rows 0.97 on the mean.  With the pieces of the column tile's
 // half block in place of the whole block (5 to 8 of 9 to 14) the head Q6_K 344 -> 317, IQ2_S 313 -> 305, Q5_K 319 -> 315; a pair of 8192 tokens
 // Q6_K 497 -> 478, IQ2_S 448 -> 439, Q5_K 458 -> 454.  What is left: the matrix pipe is busy
-// for 0.32 (tasks that half fill 256 rows) to 0.44 of the time at the clock that the card's power leaves (1.9 GHz with 256 rows of the head).
+// for 0.24 (tasks that half fill 256 rows, Q5_K) to 0.47 of the time (256 rows of the Q6_K head) at the clock that the card's power leaves (1.9 GHz with 256 rows of the head).
 constexpr int BSP_THREADS = 512;
 constexpr int BSP_ROWS_PER_DECODER = BWD_NS / 4;   // weight rows a decoder wave owns per step
 constexpr int BSP_RAW_DEPTH = 4;                   // steps of packed blocks in flight per decoder wave
