@@ -481,6 +481,14 @@ TGO_DEVICE uint32_t lds_address(const void * p) {
     return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) uint8_t *)p));
 }
 
+// Requests 16 bytes per lane, from `base` + the lane's `offset` to the LDS address `to` + 16 x lane.  The load takes its LDS address from m0 as it
+// issues, and one that follows a scalar write of m0 at once may still see the old value: a wait state lies between them, which the compiler
+// does not add inside a piece of assembly.  m0 is one of its reserved registers, which a clobber list does not protect: nothing else in these
+// kernels may use it.  (check_lds_loads.py looks for both in every build.)
+TGO_DEVICE void slab_to_lds(uint32_t to, uint32_t offset, const uint8_t * base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(offset), "s"(base) : "memory");
+}
+
 // A wave's tile is MT x 32 rows by NT x 32 columns, the workgroup's WM x WN of those.
 // ROW_MAJOR: x are rows as they stand (bf16, whole stages of 32 values, 16-byte aligned).  The lanes of a request then take 64 bytes
 // from each of 16 rows, which land row by row; the 16-byte pieces of a row are exchanged by (row / 2) % 4 on the way, so that the eight
@@ -576,14 +584,11 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void fragment_product_kernel(const
         const uint32_t to = ring_address + buffer * STAGE;
 #pragma unroll
         for (int i = 0; i < W_PER; ++i) {
-            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to + (wave * W_PER + i) * 1024), "v"(lane16), "s"(w_source[i])
-                         : "memory");
+            slab_to_lds(to + (wave * W_PER + i) * 1024, lane16, w_source[i]);
         }
 #pragma unroll
         for (int i = 0; i < X_PER; ++i) {
-            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to + (W_TILES * SS + wave * X_PER + i) * 1024), "v"(x_lane[i]),
-                         "s"(x_source[i])
-                         : "memory");
+            slab_to_lds(to + (W_TILES * SS + wave * X_PER + i) * 1024, x_lane[i], x_source[i]);
         }
         if (++requested < stages) {
 #pragma unroll
