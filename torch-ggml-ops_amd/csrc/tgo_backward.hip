@@ -14,8 +14,9 @@
 //
 // mmq_grad_input_short_kernel: tasks of a few rows of a grouped call; described where it is defined.
 //
-// mmq_grad_input_kernel: the same tile as the split kernel's by four waves that all dequantize and multiply, for calls
-// beyond the 32-bit offsets of the two others (a cotangent of 4 GiB).
+// mmq_grad_input_kernel: the same tile as the split kernel's by four waves that all dequantize and multiply, for what lies
+// beyond the 32-bit offsets of the two others: tasks of more than 64 rows of calls whose packed cotangent has 4 GiB, and every
+// task of calls of 22 million weight rows.
 //
 // The pair variant of both walks a second (dY, W) in the same loop with one fp32 accumulator, so the sum of
 // both Jacobian products is rounded to bf16 once.
@@ -173,18 +174,13 @@ TGO_DEVICE void task_segment(const BackwardArgs & a, int & first, int & tasks) {
     task_segment(a, first, tasks, ordinary);
 }
 
-// SHORT: the variant for tasks of at most BACKWARD_SHORT_ROWS rows.  Dequantizing a step's weights costs the same
-// however few rows multiply them, so for these tasks it is nearly all of the work: every wave takes the task's 64
-// rows and one 32-column slice of the tile (8 instead of 32 matrix instructions per step, spread over all four
-// SIMDs, 32 accumulator registers instead of 128), and with the smaller register footprint three workgroups share
-// a CU, so that one's barriers and memory waits are covered by another's decoding.
 // WIDE (formats whose blocks are not multiples of 16 bytes, when wide_stage_ok holds): a step's packed blocks are
 // requested as aligned 16-byte units while the previous step multiplies, like those of Q4_K / Q5_K, instead of
 // being copied two bytes at a time between the multiplications and the decoding.
-template <int TYPE, bool SHORT, bool WIDE>
-__global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_kernel(const BackwardArgs a) {
+template <int TYPE, bool WIDE>
+__global__ __launch_bounds__(BWD_THREADS, 2) void mmq_grad_input_kernel(const BackwardArgs a) {
     using F = Format<TYPE>;
-    constexpr int KT = SHORT ? 1 : 4;   // 32-column tiles per wave
+    constexpr int KT = 4;   // 32-column tiles per wave
     constexpr bool FAST_K45 = TYPE == Q4_K || TYPE == Q5_K;
     constexpr int RAW_UNITS = F::BLOCK_BYTES / 16;                              // 16-byte units per block (fast types)
     constexpr int RAW_REGS = (BWD_NS * RAW_UNITS + BWD_THREADS - 1) / BWD_THREADS;  // units in flight per thread
@@ -214,7 +210,7 @@ __global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_ker
     if (a.task_count != nullptr) {
         task_segment(a, first_task, tasks, ordinary);
     }
-    if (!SHORT && a.task_count != nullptr) {
+    if (a.task_count != nullptr) {
         xcd_chunk(blockIdx.x, a.k_tiles, tasks, ordinary, k_tile, task);
     } else {
         xcd_tile(blockIdx.x, a.k_tiles, tasks, k_tile, task);
@@ -242,9 +238,8 @@ __global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_ker
         expand_iq2s_selectors(codebook_storage, tid, BWD_THREADS);
     }
 
-    const int wave_row = SHORT ? row_start : row_start + wave * 64;
-    const bool wave_active = SHORT || wave_row < row_end;
-    const int row_tiles = SHORT ? (row_end - row_start + 31) / 32 : 2;   // 32-row tiles this wave multiplies
+    const int wave_row = row_start + wave * 64;
+    const bool wave_active = wave_row < row_end;
     const int n_total = a.out_features;
     const int steps_per_source = (n_total + BWD_NS - 1) / BWD_NS;
     const int steps = steps_per_source * a.sources;
@@ -280,9 +275,6 @@ __global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_ker
         const uint8_t * base = a.cotangent[source];
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt) {
-            if (SHORT && rt >= row_tiles) {
-                break;
-            }
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 const int chunk = (n0 >> 4) + s;
@@ -380,97 +372,7 @@ __global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_ker
         __syncthreads();   // tile visible
     };
 
-    if constexpr (SHORT && FAST_K45) {
-        // The multiplications of a step are too short here to cover a memory round trip, so the packed blocks travel
-        // DEPTH steps ahead through a ring of register sets and the cotangent fragments two steps ahead; steps past
-        // the end repeat the last one (harmless re-reads instead of branches around loads).
-        constexpr int DEPTH = 1;
-        const int last = step_end - 1;
-        u32x4 ring[DEPTH][RAW_REGS];
-        u32x4 cot[2][2][4] = {};
-        auto request_raw = [&](int step, u32x4 (&regs)[RAW_REGS]) {
-            step = min(step, last);
-            const int source = step / steps_per_source;
-            const int n0 = (step - source * steps_per_source) * BWD_NS;
-            const uint8_t * weights = a.packed[source] + static_cast<int64_t>(expert) * a.bytes_per_expert +
-                                      static_cast<int64_t>(kb) * F::BLOCK_BYTES;
-#pragma unroll
-            for (int i = 0; i < RAW_REGS; ++i) {
-                const int id = min(tid + BWD_THREADS * i, BWD_NS * RAW_UNITS - 1);
-                const int row = id / RAW_UNITS;
-                const int unit = id - row * RAW_UNITS;
-                const int src_row = min(n0 + row, n_total - 1);
-                regs[i] = *reinterpret_cast<const u32x4 *>(weights + src_row * a.row_bytes + unit * 16);
-            }
-        };
-        auto park_raw = [&](const u32x4 (&regs)[RAW_REGS]) {
-#pragma unroll
-            for (int i = 0; i < RAW_REGS; ++i) {
-                const int id = tid + BWD_THREADS * i;
-                const int row = id / RAW_UNITS;
-                const int unit = id - row * RAW_UNITS;
-                if (row < BWD_NS) {
-                    *reinterpret_cast<u32x4 *>(raw + row * F::RAW_PITCH + unit * 16) = regs[i];
-                }
-            }
-        };
-        auto request_cotangent = [&](int step, u32x4 (&regs)[2][4]) {
-            step = min(step, last);
-            const int source = step / steps_per_source;
-            const int n0 = (step - source * steps_per_source) * BWD_NS;
-            const uint8_t * base = a.cotangent[source];
-#pragma unroll
-            for (int rt = 0; rt < 2; ++rt) {
-                if (rt < row_tiles) {
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        // (the packed cotangent is zero padded to whole steps of 64 columns)
-                        regs[rt][c] = *reinterpret_cast<const u32x4 *>(
-                            base + lane_offset[rt] + static_cast<int64_t>((n0 >> 4) + c) * 1024);
-                    }
-                }
-            }
-        };
-        auto multiply = [&](const uint16_t * tile, const u32x4 (&regs)[2][4]) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const uint4 bits = *reinterpret_cast<const uint4 *>(&tile[(wave * 32 + l32) * BWD_PITCH + 16 * c + 8 * half]);
-                const v8bf bfrag = __builtin_bit_cast(v8bf, bits);
-#pragma unroll
-                for (int rt = 0; rt < 2; ++rt) {
-                    if (rt < row_tiles) {
-                        acc[rt][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, regs[rt][c]), bfrag,
-                                                                             acc[rt][0], 0, 0, 0);
-                    }
-                }
-            }
-        };
-#pragma unroll
-        for (int d = 0; d < DEPTH; ++d) {
-            request_raw(step_begin + d, ring[d]);
-        }
-        request_cotangent(step_begin, cot[0]);
-        request_cotangent(step_begin + 1, cot[1]);
-        park_raw(ring[0]);
-        request_raw(step_begin + DEPTH, ring[0]);
-        decode(step_begin, wb[0]);
-#pragma unroll 1
-        for (int first = step_begin; first < step_end; first += DEPTH) {
-#pragma unroll
-            for (int u = 0; u < DEPTH; ++u) {
-                const int step = first + u;
-                if (step < step_end) {
-                    multiply(wb[u & 1], cot[u & 1]);
-                    request_cotangent(step + 2, cot[u & 1]);
-                    if (step + 1 < step_end) {
-                        park_raw(ring[(u + 1) % DEPTH]);
-                        request_raw(step + 1 + DEPTH, ring[(u + 1) % DEPTH]);
-                        decode(step + 1, wb[(u + 1) & 1]);
-                    }
-                }
-            }
-        }
-    } else if constexpr (WIDE) {
+    if constexpr (WIDE) {
         // One barrier per step, and every wave both multiplies and dequantizes between two barriers: while the matrix
         // instructions of step i run on tile i % 2, the same wave's vector instructions decode step i + 1 from its
         // parked blocks into the other tile (the two kinds of instruction issue independently, so inside one block
@@ -528,11 +430,9 @@ __global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_ker
             const uint8_t * base = a.cotangent[source];
 #pragma unroll
             for (int rt = 0; rt < 2; ++rt) {
-                if (!SHORT || rt < row_tiles) {
-                    // (the packed cotangent is zero padded to whole steps of 64 columns)
-                    afrag[rt][s] = *reinterpret_cast<const uint4 *>(
-                        base + lane_offset[rt] + static_cast<int64_t>((n0 >> 4) + s) * 1024);
-                }
+                // (the packed cotangent is zero padded to whole steps of 64 columns)
+                afrag[rt][s] = *reinterpret_cast<const uint4 *>(
+                    base + lane_offset[rt] + static_cast<int64_t>((n0 >> 4) + s) * 1024);
             }
         };
         // the weight fragments of chunk s of a tile (one per 32-column tile of the wave), and the chunk's multiplications
@@ -540,7 +440,7 @@ __global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_ker
         auto read_fragments = [&](const uint16_t * tile, int s) __attribute__((always_inline)) {
 #pragma unroll
             for (int kt = 0; kt < KT; ++kt) {
-                const int k = (SHORT ? wave : kt) * 32 + l32;
+                const int k = kt * 32 + l32;
                 fragment[s & 1][kt] = *reinterpret_cast<const uint4 *>(&tile[k * BWD_PITCH + 16 * s + 8 * half]);
             }
         };
@@ -550,14 +450,9 @@ __global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_ker
                 const v8bf bfrag = __builtin_bit_cast(v8bf, fragment[s & 1][kt]);
 #pragma unroll
                 for (int rt = 0; rt < 2; ++rt) {
-                    if (!SHORT || rt < row_tiles) {
-                        // (full-size tasks swap the operands: the lane then holds one task row and runs of four
-                        // neighbouring columns, which the epilogue stages with 8-byte LDS writes)
-                        acc[rt][kt] = SHORT ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                                                  __builtin_bit_cast(v8bf, afrag[rt][s]), bfrag, acc[rt][kt], 0, 0, 0)
-                                            : __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                                                  bfrag, __builtin_bit_cast(v8bf, afrag[rt][s]), acc[rt][kt], 0, 0, 0);
-                    }
+                    // (operands swapped: the lane then holds one task row and runs of four neighbouring columns, which
+                    // the epilogue stages with 8-byte LDS writes)
+                    acc[rt][kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfrag, __builtin_bit_cast(v8bf, afrag[rt][s]), acc[rt][kt], 0, 0, 0);
                 }
             }
         };
@@ -607,7 +502,7 @@ __global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_ker
                     if (s == 3) {
                         request(step + 3);
                     }
-                    if constexpr (ACTIVE && !SHORT) {
+                    if constexpr (ACTIVE) {
                         // one matrix instruction, then a run of the vector instructions that share its chunk
 #pragma unroll
                         for (int i = 0; i < 2 * KT; ++i) {
@@ -657,18 +552,13 @@ __global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_ker
                 for (int s = 0; s < 4; ++s) {
 #pragma unroll
                     for (int kt = 0; kt < KT; ++kt) {
-                        const int k = (SHORT ? wave : kt) * 32 + l32;
+                        const int k = kt * 32 + l32;
                         const uint4 bits = *reinterpret_cast<const uint4 *>(&tile[k * BWD_PITCH + 16 * s + 8 * half]);
                         const v8bf bfrag = __builtin_bit_cast(v8bf, bits);
 #pragma unroll
                         for (int rt = 0; rt < 2; ++rt) {
-                            if (SHORT && rt >= row_tiles) {
-                                break;
-                            }
-                            acc[rt][kt] = SHORT ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                                                      __builtin_bit_cast(v8bf, afrag[rt][s]), bfrag, acc[rt][kt], 0, 0, 0)
-                                                : __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                                                      bfrag, __builtin_bit_cast(v8bf, afrag[rt][s]), acc[rt][kt], 0, 0, 0);
+                            acc[rt][kt] =
+                                __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfrag, __builtin_bit_cast(v8bf, afrag[rt][s]), acc[rt][kt], 0, 0, 0);
                         }
                     }
                 }
@@ -689,29 +579,6 @@ __global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_ker
     }
 
     __syncthreads();   // the tiles are free: each wave reuses 8.5 KiB of them to transpose its results
-    if constexpr (SHORT) {
-        // the four 32-column slices of a 32-row tile meet in LDS and leave as whole 256-byte rows
-        constexpr int STAGE_PITCH = BWD_TK + 8;
-        static_assert(2 * 32 * STAGE_PITCH <= 2 * BWD_TK * BWD_PITCH, "both row tiles fit the weight tiles");
-        uint16_t * stage = &wb[0][0];
-#pragma unroll
-        for (int rt = 0; rt < 2; ++rt) {
-            if (rt < row_tiles) {
-                stage_tile_32x32<STAGE_PITCH>(stage + rt * 32 * STAGE_PITCH, acc[rt][0], wave * 32, lane);
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int rt = 0; rt < 2; ++rt) {
-            const int r0 = row_start + rt * 32;
-            if (rt < row_tiles) {
-                store_staged_rows<STAGE_PITCH>(stage + rt * 32 * STAGE_PITCH,
-                                               a.dx + static_cast<int64_t>(r0) * a.in_features + k_tile * BWD_TK,
-                                               a.in_features, row_end - r0, BWD_TK, tid, BWD_THREADS);
-            }
-        }
-        return;
-    } else {
     if (!wave_active) {
         return;
     }
@@ -730,7 +597,6 @@ __global__ __launch_bounds__(BWD_THREADS, SHORT ? 3 : 2) void mmq_grad_input_ker
             store_rows_32x128<BWD_TK + 8, true, true>(stage, acc[rt], a.dx + static_cast<int64_t>(r0) * a.in_features + k_tile * BWD_TK,
                                                 a.in_features, row_end - r0, BWD_TK, lane);
         }
-    }
     }
 }
 
@@ -1655,12 +1521,15 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
 
     // cotangent fragments of the task's (up to) two 32-row tiles; one set, requested right after the
     // multiplications that used the previous one and awaited a whole decode later
+    // (offsets from the 32-row tile that the task starts in: it reaches into two more at most)
+    const int first_tile = row_start >> 5;
+    const int64_t task_offset = static_cast<int64_t>(first_tile) * a.n_chunks * 1024;
     uint32_t lane_offset[2];
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt) {
         int r = row_start + rt * 32 + l32;
         r = r < a.rows_padded ? r : a.rows_padded - 1;
-        lane_offset[rt] = static_cast<uint32_t>(r >> 5) * a.n_chunks * 1024 + ((r & 31) + 32 * half) * 16;
+        lane_offset[rt] = static_cast<uint32_t>((r >> 5) - first_tile) * a.n_chunks * 1024 + ((r & 31) + 32 * half) * 16;
     }
     u32x4 cot[2][4] = {};
     auto request_cotangent = [&](int step) __attribute__((always_inline)) {
@@ -1668,7 +1537,7 @@ __global__ __launch_bounds__(BSH_THREADS, 3) void mmq_grad_input_short_kernel(co
         const int source = step >= steps_per_source ? 1 : 0;
         const int n0 = (step - source * steps_per_source) * BWD_NS;
         // (the packed cotangent is zero padded to whole steps of 64 columns)
-        const uint8_t * base = (source == 0 ? a.cotangent[0] : a.cotangent[1]) + static_cast<int64_t>(n0 >> 4) * 1024;
+        const uint8_t * base = (source == 0 ? a.cotangent[0] : a.cotangent[1]) + task_offset + static_cast<int64_t>(n0 >> 4) * 1024;
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt) {
             if (rt < row_tiles) {
@@ -1795,43 +1664,43 @@ static hipError_t launch_backward_typed(const BackwardArgs & args, hipStream_t s
         return hipErrorInvalidValue;
     }
     const ProfileScope scope(3, stream);
-    // the general kernel, in its variant for short tasks or not, with the packed blocks fetched as wide units
-    // where the format needs that and the weights allow it
-    const auto general = [&](auto short_tag, dim3 grid, const BackwardArgs & launch_args) {
-        constexpr bool SHORT = decltype(short_tag)::value;
+    // the general kernel, with the packed blocks fetched as wide units where the format needs that and the weights allow it
+    const auto general = [&](dim3 grid, const BackwardArgs & launch_args) {
         if constexpr (Format<TYPE>::BLOCK_BYTES % 16 != 0) {
             const int64_t weight_bytes = static_cast<int64_t>(args.out_features) * args.row_bytes;
             // (and the rows short enough for the 24-bit multiplies of the unit offsets)
             if (args.row_bytes < (1 << 24) && wide_stage_ok(args.packed[0], weight_bytes) &&
                 (args.packed[1] == nullptr || wide_stage_ok(args.packed[1], weight_bytes))) {
-                mmq_grad_input_kernel<TYPE, SHORT, true><<<grid, BWD_THREADS, 0, stream>>>(launch_args);
+                mmq_grad_input_kernel<TYPE, true><<<grid, BWD_THREADS, 0, stream>>>(launch_args);
                 return;
             }
         }
-        mmq_grad_input_kernel<TYPE, SHORT, false><<<grid, BWD_THREADS, 0, stream>>>(launch_args);
+        mmq_grad_input_kernel<TYPE, false><<<grid, BWD_THREADS, 0, stream>>>(launch_args);
     };
+    // (32-bit lane offsets into a step's weight rows, in both kernels below; in_features ends far below)
+    if (args.row_bytes * 2 * BWD_NS >= (int64_t{1} << 32)) {
+        return hipErrorInvalidValue;
+    }
     if (args.segment == 1) {
+        // (32-bit lane offsets into the three row tiles that a task may touch)
+        if (int64_t{3} * args.n_chunks * 1024 >= (int64_t{1} << 32)) {
+            // twenty million weight rows and more: all tasks in one launch of the general kernel
+            BackwardArgs all_args = args;
+            all_args.segment = 0;
+            general(dim3(static_cast<unsigned>(total)), all_args);
+            return hipGetLastError();
+        }
         // grouped call: the short tasks (a separate segment of the task list) run in a launch of their own
         BackwardArgs short_args = args;
         short_args.segment = 2;
-        bool launched = false;
-        // (32-bit lane offsets into the packed cotangent and a step's weight rows, as in the role-split kernel)
-        if (cotangent_workspace_bytes(args.rows, args.out_features) < (int64_t{1} << 32) &&
-            args.row_bytes * 2 * BWD_NS < (int64_t{1} << 32)) {
-            mmq_grad_input_short_kernel<TYPE><<<static_cast<unsigned>(total_short), BSH_THREADS, 0, stream>>>(short_args);
-            launched = true;
-        }
-        if (!launched) {
-            general(std::true_type{}, dim3(static_cast<unsigned>(total_short)), short_args);
-        }
+        mmq_grad_input_short_kernel<TYPE><<<static_cast<unsigned>(total_short), BSH_THREADS, 0, stream>>>(short_args);
         const hipError_t status = hipGetLastError();
         if (status != hipSuccess) {
             return status;
         }
     }
-    // the role-split kernel addresses the packed cotangent and a step's weight rows with 32-bit lane offsets
-    const bool role_split = cotangent_workspace_bytes(args.rows, args.out_features) < (int64_t{1} << 32) &&
-                      args.row_bytes * 2 * BWD_NS < (int64_t{1} << 32);
+    // the role-split kernel addresses the packed cotangent with 32-bit lane offsets
+    const bool role_split = cotangent_workspace_bytes(args.rows, args.out_features) < (int64_t{1} << 32);
     const bool splits = args.n_splits > 1;
     if (role_split) {
         // one persistent workgroup per CU, more only when a workgroup's item table would overflow
@@ -1841,7 +1710,7 @@ static hipError_t launch_backward_typed(const BackwardArgs & args, hipStream_t s
         const int64_t grid = (std::max<int64_t>(std::min<int64_t>(items, BSP_GRID), needed) + XCDS - 1) / XCDS * XCDS;
         mmq_grad_input_split_kernel<TYPE><<<static_cast<unsigned>(grid), BSP_THREADS, 0, stream>>>(args, static_cast<int>(items));
     } else {
-        general(std::false_type{}, dim3(static_cast<unsigned>(total), static_cast<unsigned>(args.n_splits)), args);
+        general(dim3(static_cast<unsigned>(total), static_cast<unsigned>(args.n_splits)), args);
     }
     if (splits) {
         const int64_t count = static_cast<int64_t>(args.rows) * args.in_features;
