@@ -467,14 +467,23 @@ __global__ __launch_bounds__(MDE_THREADS) void moe_down_kernel(const MoeDecodeAr
     }
     __syncthreads();
     float acc[2][1] = {};
+    // (lanes read what other lanes of their wave have parked: LDS executes a wave's accesses in order, the compiler has to keep them so)
+    const auto wave_sync = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
 #pragma unroll
     for (int first = 0; first < EXPERTS; first += AT_ONCE) {
+        if (first != 0) {
+            wave_sync();   // the experts before have been read
+        }
 #pragma unroll
         for (int j = 0; j < AT_ONCE; ++j) {
             if ((valid >> (first + j) & 1) != 0) {
                 weights[first + j].park(raw[wave][j], 2 * BLOCKS, lane);
             }
         }
+        wave_sync();   // parked
 #pragma unroll
         for (int i = 0; i < (AT_ONCE * UNITS + 63) / 64; ++i) {
             const int id = lane + 64 * i;
