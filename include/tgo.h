@@ -38,7 +38,7 @@ extern "C" {
 
 /* Library version (major*10000 + minor*100 + patch): TGO_VERSION of the header that the library was built with.  It grows with
  * every change of this file that a caller can see. */
-#define TGO_VERSION 115
+#define TGO_VERSION 116
 int tgo_version(void);
 
 /* Message of the last failure on the calling thread ("" if none). Host pointer. */
@@ -90,12 +90,21 @@ int tgo_mmq_forward(const void * input_bf16, const void * packed, void * output_
                     void * workspace, int64_t rows, int64_t in_features, int64_t out_features,
                     int quant_type, void * stream);
 
-/* tgo_mmq_forward and tgo_mmq_forward_prepared_as with tgo_forward_scratch_bytes() bytes of `scratch` (0: NULL is as good): dense
+/* tgo_mmq_forward and tgo_mmq_forward_prepared_as with `scratch` (0 bytes: NULL is as good): dense
  * calls of more rows than the decode kernels take, whose tiles would not fill the chip, then cut K into ranges that run side by
  * side and leave fp32 sums there, which a second kernel adds up in a fixed order; tgo_mmq_forward_scratch with scaled operands unpacks the
  * weights there once where that pays (the same bits; `workspace` then holds the activations as that product reads them and is no workspace for
- * the prepared entry points, which give NaN on it, nor for tgo_q8_workspace_unpack, which gives zeros).  No counterpart in the reference. */
+ * the prepared entry points, which give NaN on it, nor for tgo_q8_workspace_unpack, which gives zeros).  No counterpart in the reference.
+ *   tgo_forward_scratch_bytes     what tgo_mmq_forward_scratch may use, under any setting of the operands
+ *   tgo_forward_scratch_bytes_as  what a call on operands of that kind uses: TGO_OPERAND_SCALED the unpacked weights (which may be hundreds of
+ *                                 MiB), TGO_OPERAND_INT8 and _HALF the ranges' sums, which are also all that the prepared entry points and
+ *                                 tgo_mmq_multi_forward use, with operands of any kind
+ *   tgo_mmq_forward_sized         tgo_mmq_forward_scratch with any number of bytes there: a call does without what does not fit, and so a
+ *                                 caller may ask for what tgo_forward_operand_for's present kind uses */
 int64_t tgo_forward_scratch_bytes(int64_t rows, int64_t in_features, int64_t out_features, int quant_type);
+int64_t tgo_forward_scratch_bytes_as(int64_t rows, int64_t in_features, int64_t out_features, int quant_type, int operand);
+int tgo_mmq_forward_sized(const void * input_bf16, const void * packed, void * output_bf16, void * workspace, void * scratch,
+                          int64_t scratch_bytes, int64_t rows, int64_t in_features, int64_t out_features, int quant_type, void * stream);
 int tgo_mmq_forward_scratch(const void * input_bf16, const void * packed, void * output_bf16, void * workspace, void * scratch,
                             int64_t rows, int64_t in_features, int64_t out_features, int quant_type, void * stream);
 int tgo_mmq_forward_prepared_scratch(const void * workspace, const void * packed, void * output_bf16, void * scratch, int64_t rows,
@@ -103,7 +112,7 @@ int tgo_mmq_forward_prepared_scratch(const void * workspace, const void * packed
 
 /* Several dense projections of one input: the activations are quantized once, as `operand` (TGO_OPERAND_INT8, _HALF or _SCALED), into
  * `workspace` (tgo_q8_workspace_bytes), and multiplied with each packed weight; `scratch`: the largest
- * tgo_forward_scratch_bytes() of the projections, or NULL.  The arrays have `count` entries and lie in host memory.
+ * tgo_forward_scratch_bytes_as(TGO_OPERAND_INT8) of the projections, or NULL.  The arrays have `count` entries and lie in host memory.
  * tgo_mmq_pair_grad_input: the gradient of the input of two projections of one shape and format, summed in fp32 and rounded
  * once; `workspace` holds tgo_pair_grad_workspace_bytes() bytes.  No counterparts in the reference. */
 int tgo_mmq_multi_forward(const void * input_bf16, int count, const void * const * packed, void * const * outputs_bf16,

@@ -179,3 +179,59 @@ def test_another_layout_than_the_workspaces_is_nan_on_the_decode_kernel_too(ops)
     weight = synth.random_packed_weight(12, (n,), k, seed=3).cuda()
     workspace = tgo.quantize_q8_1(random_bf16((rows, k), seed=4), operand="half")
     assert torch.isnan(tgo.mmq_prepared(workspace, weight, rows, k, 12, n, operand="int8").float()).all()
+
+
+@pytest.mark.parametrize("call", ("prepared", "multi", "int8", "half"))
+def test_calls_that_do_not_unpack_their_weights_have_no_scratch_for_them(ops, call):
+    """Two bytes per weight, where ``mmq`` with scaled operands has them."""
+    tgo, synth = ops
+    from torch_ggml_ops import _native
+
+    qtype, rows, k, n = 12, 4096, 4096, 4096
+    unpacked = _native.lib.tgo_forward_scratch_bytes_as(rows, k, n, qtype, _native.OPERANDS["scaled"])
+    assert unpacked >= 2 * n * k
+    packed = synth.random_packed_weight(qtype, (n,), k, seed=1).cuda()
+    other = synth.random_packed_weight(14, (n,), k, seed=2).cuda()   # (of another format: not one product)
+    x = random_bf16((rows, k), seed=3)
+    workspace = tgo.quantize_q8_1(x, "scaled")
+    try:
+        if call in ("int8", "half"):
+            _native.set_forward_operand(call)
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        if call == "prepared":
+            outputs = [tgo.mmq_prepared(workspace, packed, rows, k, qtype, n, "scaled")]
+        elif call == "multi":
+            outputs = tgo.mmq_multi(x, [packed, other], [qtype, 14], [n, n])
+        else:
+            outputs = [tgo.mmq(x, packed, qtype, n)]
+        taken = torch.cuda.max_memory_allocated() - before
+    finally:
+        _native.set_forward_operand("auto")
+    kept = sum(o.numel() * 2 for o in outputs) + (0 if call == "prepared" else workspace.numel())
+    assert taken < kept + unpacked // 4
+
+
+def test_scratch_that_is_too_small_is_done_without(ops):
+    """A call whose scratch was sized under another setting: the same bits as without scratch, and nothing written beyond it."""
+    _, synth = ops
+    from torch_ggml_ops import _native
+
+    qtype, rows, k, n, lib = 12, 2048, 2048, 2048, _native.lib
+    needed = lib.tgo_forward_scratch_bytes_as(rows, k, n, qtype, _native.OPERANDS["scaled"])
+    assert needed > 0
+    packed = synth.random_packed_weight(qtype, (n,), k, seed=1).cuda()
+    x = random_bf16((rows, k), seed=3)
+    workspace = torch.empty(lib.tgo_q8_workspace_bytes(rows, k), dtype=torch.uint8, device="cuda")
+    scratch = torch.full((needed,), 0x5A, dtype=torch.uint8, device="cuda")
+    outputs = []
+    for size in (0, needed - 1, needed):
+        assert bool((scratch == 0x5A).all())
+        output = torch.empty((rows, n), dtype=torch.bfloat16, device="cuda")
+        _native.check(lib.tgo_mmq_forward_sized(x.data_ptr(), packed.data_ptr(), output.data_ptr(), workspace.data_ptr(), scratch.data_ptr(), size,
+                                                rows, k, n, qtype, _native.stream_of(x.device)))
+        outputs.append(output)
+    assert torch.equal(outputs[0], outputs[1]) and torch.equal(outputs[0], outputs[2])
+    assert not bool((scratch == 0x5A).all())

@@ -391,16 +391,22 @@ int tgo_q8_workspace_unpack(const void * workspace, void * q_int8, void * d_f32,
                      "q8_unpack launch");
 }
 
-int64_t tgo_forward_scratch_bytes(int64_t rows, int64_t in_features, int64_t out_features, int quant_type) {
+int64_t tgo_forward_scratch_bytes_as(int64_t rows, int64_t in_features, int64_t out_features, int quant_type, int operand) {
     if (rows <= 0 || in_features <= 0 || out_features <= 0 || tgo::use_gemv(rows, 0)) {
         return 0;
     }
-    // (a prepared workspace may hold either kind of exact operands; the setting, by which some calls use no ranges, may change before
-    // the call)
-    const int64_t unpacked = tgo::forward_unpacks(quant_type, rows, in_features, out_features)
-        ? tgo::unpacked_forward_bytes(quant_type, (out_features + 31) / 32, in_features) : 0;
-    return std::max({unpacked, tgo::forward_partial_bytes(rows, in_features, out_features, quant_type, tgo::OPERAND_INT8),
-                     tgo::forward_partial_bytes(rows, in_features, out_features, quant_type, tgo::OPERAND_HALF)});
+    if (operand == TGO_OPERAND_SCALED) {
+        return tgo::forward_unpacks(quant_type, rows, in_features, out_features)
+            ? tgo::unpacked_forward_bytes(quant_type, (out_features + 31) / 32, in_features) : 0;
+    }
+    // (either kind of exact operands: a call's row tile depends on whether it has scratch)
+    return std::max(tgo::forward_partial_bytes(rows, in_features, out_features, quant_type, tgo::OPERAND_INT8),
+                    tgo::forward_partial_bytes(rows, in_features, out_features, quant_type, tgo::OPERAND_HALF));
+}
+
+int64_t tgo_forward_scratch_bytes(int64_t rows, int64_t in_features, int64_t out_features, int quant_type) {
+    return std::max(tgo_forward_scratch_bytes_as(rows, in_features, out_features, quant_type, TGO_OPERAND_SCALED),
+                    tgo_forward_scratch_bytes_as(rows, in_features, out_features, quant_type, TGO_OPERAND_INT8));
 }
 
 int tgo_mmq_forward(const void * input_bf16, const void * packed, void * output_bf16, void * workspace,
@@ -424,22 +430,26 @@ static hipError_t launch_dense(const void * packed, const tgo::Q8Workspace & vie
                                                     static_cast<float *>(scratch));
 }
 
-// `scratch` of a dense call that cuts K into ranges (tgo_forward_scratch_bytes); any pointer will do where nothing is cut.
-static int check_scratch(const void * scratch, int64_t rows, int64_t in_features, int64_t out_features, int quant_type) {
-    if (scratch != nullptr && tgo_forward_scratch_bytes(rows, in_features, out_features, quant_type) > 0) {
-        return check_pointer(scratch, "scratch");
-    }
-    return TGO_OK;
+// `scratch` of a dense call; any pointer will do where none is `needed`.
+static int check_scratch(const void * scratch, int64_t needed) {
+    return scratch != nullptr && needed > 0 ? check_pointer(scratch, "scratch") : TGO_OK;
 }
 
 int tgo_mmq_forward_scratch(const void * input_bf16, const void * packed, void * output_bf16, void * workspace, void * scratch,
                             int64_t rows, int64_t in_features, int64_t out_features, int quant_type, void * stream) {
+    // (that many bytes by contract)
+    return tgo_mmq_forward_sized(input_bf16, packed, output_bf16, workspace, scratch, INT64_MAX, rows, in_features, out_features, quant_type,
+                                 stream);
+}
+
+int tgo_mmq_forward_sized(const void * input_bf16, const void * packed, void * output_bf16, void * workspace, void * scratch,
+                          int64_t scratch_bytes, int64_t rows, int64_t in_features, int64_t out_features, int quant_type, void * stream) {
     TGO_TRY(check_matmul_shape(rows, in_features, out_features, quant_type));
     TGO_TRY(check_pointer(input_bf16, "input"));
     TGO_TRY(check_pointer(packed, "packed_weight"));
     TGO_TRY(check_pointer(output_bf16, "output"));
     TGO_TRY(check_pointer(workspace, "workspace"));
-    TGO_TRY(check_scratch(scratch, rows, in_features, out_features, quant_type));
+    TGO_TRY(check_scratch(scratch, tgo_forward_scratch_bytes(rows, in_features, out_features, quant_type)));
     hipStream_t hip_stream = static_cast<hipStream_t>(stream);
     const int setting = tgo::forward_operand_setting();
     const bool tiles = tgo::dense_takes_tiles(setting, rows, in_features, out_features, quant_type);
@@ -453,8 +463,11 @@ int tgo_mmq_forward_scratch(const void * input_bf16, const void * packed, void *
                          "mmq_forward launch");
     }
     const int kind = tgo::forward_operand_kind(setting, quant_type, rows, out_features, 1);
-    if (!tiles && scratch != nullptr && kind == tgo::OPERAND_SCALED && !tgo::use_gemv(rows, 0) &&
-        tgo::forward_unpacks(quant_type, rows, in_features, out_features)) {
+    const int64_t needed = tgo_forward_scratch_bytes_as(rows, in_features, out_features, quant_type, kind);
+    if (scratch_bytes < needed) {
+        scratch = nullptr;   // (it may have been sized under another setting)
+    }
+    if (!tiles && scratch != nullptr && kind == tgo::OPERAND_SCALED && needed > 0) {
         const tgo::DenseSource source = {static_cast<const uint8_t *>(packed), nullptr, out_features, quant_type};
         uint16_t * const output = static_cast<uint16_t *>(output_bf16);
         return check_hip(tgo::launch_forward_unpacked(static_cast<const uint16_t *>(input_bf16), workspace, &source, &output, 1, scratch, rows,
@@ -495,7 +508,7 @@ static int prepared_forward(int setting, const void * workspace, const void * pa
     TGO_TRY(check_pointer(packed, "packed_weight"));
     TGO_TRY(check_pointer(output_bf16, "output"));
     TGO_TRY(check_workspace_operand(operand));
-    TGO_TRY(check_scratch(scratch, rows, in_features, out_features, quant_type));
+    TGO_TRY(check_scratch(scratch, tgo_forward_scratch_bytes_as(rows, in_features, out_features, quant_type, TGO_OPERAND_INT8)));
     const tgo::Q8Workspace view =
         tgo::q8_workspace_view(const_cast<void *>(workspace), rows, in_features, tgo::use_gemv(rows, 0), operand);
     const bool tiles = tgo::dense_takes_tiles(setting, rows, in_features, out_features, quant_type);
@@ -544,7 +557,7 @@ int tgo_mmq_multi_forward(const void * input_bf16, int count, const void * const
         TGO_TRY(check_matmul_shape(rows, in_features, out_features[i], quant_types[i]));
         TGO_TRY(check_pointer(packed[i], "packed_weight"));
         TGO_TRY(check_pointer(outputs_bf16[i], "output"));
-        TGO_TRY(check_scratch(scratch, rows, in_features, out_features[i], quant_types[i]));
+        TGO_TRY(check_scratch(scratch, tgo_forward_scratch_bytes_as(rows, in_features, out_features[i], quant_types[i], TGO_OPERAND_INT8)));
     }
     hipStream_t hip_stream = static_cast<hipStream_t>(stream);
     const tgo::Q8Workspace view = tgo::q8_workspace_view(workspace, rows, in_features, tgo::use_gemv(rows, 0), operand);

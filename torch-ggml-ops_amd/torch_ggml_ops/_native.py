@@ -56,6 +56,9 @@ lib.tgo_q8_workspace_unpack.argtypes = [_p, _p, _p, _p, _i64, _i64, _p]
 lib.tgo_mmq_forward.argtypes = [_p, _p, _p, _p, _i64, _i64, _i64, _int, _p]
 lib.tgo_forward_scratch_bytes.argtypes = [_i64, _i64, _i64, _int]
 lib.tgo_forward_scratch_bytes.restype = _i64
+lib.tgo_forward_scratch_bytes_as.argtypes = [_i64, _i64, _i64, _int, _int]
+lib.tgo_forward_scratch_bytes_as.restype = _i64
+lib.tgo_mmq_forward_sized.argtypes = [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _int, _p]
 lib.tgo_mmq_forward_scratch.argtypes = [_p, _p, _p, _p, _p, _i64, _i64, _i64, _int, _p]
 lib.tgo_mmq_forward_prepared_scratch.argtypes = [_p, _p, _p, _p, _i64, _i64, _i64, _int, _int, _p]
 lib.tgo_mmq_multi_forward.argtypes = [
@@ -132,7 +135,9 @@ EXPORTS = (
     "tgo_q8_workspace_unpack",
     "tgo_mmq_forward",
     "tgo_forward_scratch_bytes",
+    "tgo_forward_scratch_bytes_as",
     "tgo_mmq_forward_scratch",
+    "tgo_mmq_forward_sized",
     "tgo_mmq_forward_prepared_scratch",
     "tgo_mmq_multi_forward",
     "tgo_pair_grad_workspace_bytes",
@@ -225,20 +230,20 @@ def stream_of(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
-def forward_scratch_bytes(rows: int, in_features: int, out_features: int, quant_type: int) -> int:
-    """Scratch bytes worth allocating for a dense forward call: none where the decode kernel takes it (a call without
-    scratch is as correct should the setting change in between)."""
-    size = lib.tgo_forward_scratch_bytes(rows, in_features, out_features, int(quant_type))
+def forward_scratch_bytes(rows: int, in_features: int, out_features: int, quant_type: int, kind: int) -> int:
+    """Scratch bytes worth allocating for a dense forward call on operands of this kind: none where the decode kernel takes it (a
+    call without scratch is as correct should the setting change in between)."""
+    size = lib.tgo_forward_scratch_bytes_as(rows, in_features, out_features, int(quant_type), kind)
     return size if size == 0 or forward_kernel_for(int(quant_type), rows, in_features, out_features) != "tiles" else 0
 
 
-def forward_scratch(tensor: torch.Tensor, rows: int, in_features: int, out_features: int, quant_type: int):
-    """(tensor that keeps it, pointer) of the scratch memory of a dense forward call; (None, None) when it needs none."""
-    size = forward_scratch_bytes(rows, in_features, out_features, quant_type)
+def forward_scratch(tensor: torch.Tensor, rows: int, in_features: int, out_features: int, quant_type: int, kind: int):
+    """(tensor that keeps it, pointer, bytes) of the scratch memory of a dense forward call; (None, None, 0) when it needs none."""
+    size = forward_scratch_bytes(rows, in_features, out_features, quant_type, kind)
     if size == 0:
-        return None, None
+        return None, None, 0
     scratch = tensor.new_empty((size,), dtype=torch.uint8)
-    return scratch, scratch.data_ptr()
+    return scratch, scratch.data_ptr(), size
 
 
 def on_device(device: torch.device):

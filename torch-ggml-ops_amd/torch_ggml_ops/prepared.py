@@ -96,7 +96,10 @@ def _mmq_prepared_device(
         )
     with _native.on_device(workspace.device):
         output = workspace.new_empty((rows, out_features), dtype=torch.bfloat16)
-        _scratch, scratch = _native.forward_scratch(workspace, rows, in_features, out_features, quant_type)
+        # (the ranges' sums of exact operands: weights are unpacked once per call only together with their activations)
+        _scratch, scratch, _ = _native.forward_scratch(
+            workspace, rows, in_features, out_features, quant_type, _native.OPERANDS["int8"]
+        )
         _native.check(
             _native.lib.tgo_mmq_forward_prepared_scratch(
                 workspace.data_ptr(), packed_weight.data_ptr(), output.data_ptr(), scratch,
@@ -157,7 +160,7 @@ def _multi_device(input, packed_weights, quant_types, out_features, operand):
             )
             return outputs
         scratch_bytes = max(
-            _native.forward_scratch_bytes(rows, in_features, features, quant_type)
+            _native.forward_scratch_bytes(rows, in_features, features, quant_type, _native.OPERANDS["int8"])
             for quant_type, features in zip(quant_types, out_features)
         )
         scratch = input.new_empty((scratch_bytes,), dtype=torch.uint8) if scratch_bytes > 0 else None
