@@ -187,8 +187,8 @@ int64_t tgo_grad_workspace_bytes(int64_t rows, int64_t out_features, int64_t num
 
 /* Bytes of `workspace` for tgo_mmq_grad_input: the packed cotangent as above, plus, for calls of so
  * few rows that whole reductions per workgroup would leave most of the chip idle, room for the
- * fp32 partial results of a reduction split over several workgroups (added up in a fixed order), plus, for
- * calls that unpack their weights first, two bytes per weight.
+ * fp32 partial results of a reduction split over several workgroups (added up in a fixed order).  Calls that unpack their weights
+ * first: two bytes per weight, and the packed cotangent unless out_features is a multiple of 32.
  * No counterpart in the reference.  -1 on invalid sizes. */
 int64_t tgo_dense_grad_workspace_bytes(int64_t rows, int64_t out_features, int64_t in_features,
                                        int quant_type);

@@ -458,3 +458,14 @@ def test_version_is_the_headers(package):
     assert native.lib.tgo_version() == version >= 113
     for name in ("tgo_forward_scratch_bytes", "tgo_mmq_multi_forward", "tgo_mmq_pair_grad_input", "tgo_route", "tgo_lm_head_loss"):
         assert f"{name}(" in header
+
+
+def test_gradient_workspace_without_a_cotangent_that_is_not_packed(package):
+    """Calls that unpack their weights read cotangents of whole stages as they stand: room for the weights is all that they ask for."""
+    _, native, _, _ = package
+    lib = native.lib
+    both = (ctypes.c_int64 * 2)(2048, 512)
+    assert lib.tgo_dense_grad_workspace_bytes(16384, 28672, 1024, 12) == 2 * 28672 * 1024
+    assert lib.tgo_multi_grad_workspace_bytes(2, both, 4096, 2048) == 2 * 2560 * 2048
+    assert lib.tgo_pair_grad_workspace_bytes(4096, 2048, 2048, 14) == 2 * 2 * 2048 * 2048
+    assert lib.tgo_dense_grad_workspace_bytes(4096, 2047, 2048, 12) == 2 * 2048 * 2048 + 2 * 4096 * 2048   # (both packed)

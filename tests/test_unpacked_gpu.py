@@ -64,6 +64,33 @@ def test_gradient_of_several_projections(oracle, widths):
     assert_matches_f32_reference(grad, expected.cpu().numpy(), accumulate_noise=1e-5)
 
 
+@pytest.mark.parametrize("qname", ("Q4_K", "IQ2_S"))
+def test_gradient_workspaces(qname):
+    """One buffer for calls on either side of the rule: nothing that an earlier call left there is read, and nothing is written beyond the bytes that a
+    call asks for, with cotangents that are read as they stand and cotangents that are packed."""
+    import synth
+    import torch_ggml_ops  # noqa: F401
+    from torch_ggml_ops import _native
+
+    qtype, lib, k = QTYPES[qname], _native.lib, 2048
+    buffer = torch.full((1 << 26,), 0xFF, dtype=torch.uint8, device="cuda")
+    stream = _native.stream_of(buffer.device)
+    unpack = []
+    for rows, n in ((4000, 1056), (40, 1056), (4133, 1569), (300, 640), (4000, 1056), (64, 1569), (4133, 1569)):
+        size = lib.tgo_dense_grad_workspace_bytes(rows, n, k, qtype)
+        unpack.append(_unpacks_gradient(rows, [n], k))
+        if unpack[-1]:
+            assert size == 2 * n * k if n % 32 == 0 else size >= 2 * n * (k + rows)
+        packed = synth.random_packed_weight(qtype, (n,), k, seed=qtype + n).cuda()
+        grad = random_bf16((rows, n), seed=rows)
+        expected = torch.ops.torch_ggml_ops.mmq_grad_input.default(grad, packed, qtype, k)
+        actual = torch.empty((rows, k), dtype=torch.bfloat16, device="cuda")
+        buffer[size:] = 0xA5
+        _native.check(lib.tgo_mmq_grad_input(grad.data_ptr(), packed.data_ptr(), actual.data_ptr(), buffer.data_ptr(), rows, n, k, qtype, stream))
+        assert torch.equal(actual, expected) and bool((buffer[size:] == 0xA5).all())
+    assert unpack.count(True) >= 4 and not unpack[1] and not unpack[5]
+
+
 # (rows, columns, K): as above, an odd number of steps with the minima's (K = 768, 1280), columns that end inside a tile, rows of 16-byte units
 # and not (Q3_K, Q6_K and IQ2_S of K = 768 and an odd number of columns)
 FORWARDS = [(2000, 2048, 2048), (1000, 5003, 1280), (545, 6017, 768), (8200, 769, 768), (9000, 520, 512), (4097, 4096, 1024), (500, 8192, 2816)]

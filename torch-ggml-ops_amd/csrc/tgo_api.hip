@@ -263,32 +263,24 @@ int64_t tgo_dense_grad_workspace_bytes(int64_t rows, int64_t out_features, int64
         return -1;
     }
     if (tgo::grad_unpacks(rows, out_features, in_features)) {
-        return tgo::unpacked_grad_workspace(nullptr, rows, tgo::cotangent_chunks(out_features), in_features).bytes;
+        return tgo::unpacked_grad_workspace(nullptr, rows, 1, &out_features, in_features).bytes;
     }
     return single_grad_bytes(rows, out_features, in_features);
-}
-
-// Reduction steps of 16 weight rows of several projections side by side, each in whole steps of 64, and their weight rows.
-static int64_t multi_chunks(int count, const int64_t * out_features, int64_t & total) {
-    int64_t chunks = 0;
-    total = 0;
-    for (int i = 0; i < count; ++i) {
-        if (out_features[i] <= 0 || out_features[i] > INT_LIMIT) {
-            return -1;
-        }
-        total += out_features[i];
-        chunks += tgo::cotangent_chunks(out_features[i]);
-    }
-    return chunks > INT_LIMIT ? -1 : chunks;
 }
 
 int64_t tgo_multi_grad_workspace_bytes(int count, const int64_t * out_features, int64_t rows, int64_t in_features) {
     if (count < 1 || count > tgo::UNPACKED_SOURCES || out_features == nullptr || rows <= 0 || in_features <= 0 || in_features % tgo::QK_K != 0) {
         return 0;
     }
-    int64_t total;
-    const int64_t chunks = multi_chunks(count, out_features, total);
-    return chunks > 0 && tgo::multi_grad_unpacks(rows, total, in_features, count) ? tgo::unpacked_grad_workspace(nullptr, rows, chunks, in_features).bytes : 0;
+    int64_t total = 0;
+    for (int i = 0; i < count; ++i) {
+        if (out_features[i] <= 0 || out_features[i] > INT_LIMIT) {
+            return 0;
+        }
+        total += out_features[i];
+    }
+    return tgo::multi_grad_unpacks(rows, total, in_features, count)
+        ? tgo::unpacked_grad_workspace(nullptr, rows, count, out_features, in_features).bytes : 0;
 }
 
 int tgo_mmq_multi_grad_input(int count, const void * const * grad_outputs_bf16, const void * const * packed, const int64_t * out_features,

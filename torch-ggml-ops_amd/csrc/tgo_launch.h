@@ -629,17 +629,28 @@ static inline float unpack_microseconds(int64_t out_features, int64_t in_feature
     return 5.0f + static_cast<float>(out_features) * static_cast<float>(in_features) * 0.6e-6f;
 }
 constexpr int UNPACKED_SOURCES = 4;
+// Workspace of a grad-input of `count` projections: slabs of 16 weight rows (`chunks` of all projections together), and those of the cotangents,
+// unless all of them have rows of whole stages (32 values), which the product reads as they stand.
 struct UnpackedGradWorkspace {
+    bool row_major;
+    int64_t chunks;
     uint8_t * cotangent;
     uint8_t * weights;
     int64_t bytes;
+    // of one projection: row-major it ends with its weight rows, packed with a whole step of 64
+    int64_t chunks_of(int64_t out_features) const { return row_major ? out_features / 16 : (out_features + 63) / 64 * 4; }
 };
-static inline UnpackedGradWorkspace unpacked_grad_workspace(void * base, int64_t rows, int64_t chunks, int64_t in_features) {
+static inline UnpackedGradWorkspace unpacked_grad_workspace(void * base, int64_t rows, int count, const int64_t * out_features, int64_t in_features) {
     UnpackedGradWorkspace view;
+    view.row_major = std::all_of(out_features, out_features + count, [](int64_t features) { return features % 32 == 0; });
+    view.chunks = 0;
+    for (int i = 0; i < count; ++i) {
+        view.chunks += view.chunks_of(out_features[i]);
+    }
+    const int64_t cotangent_bytes = view.row_major ? 0 : pad_rows(rows) / 32 * view.chunks * 1024;
     view.cotangent = static_cast<uint8_t *>(base);
-    const int64_t weights = pad_rows(rows) / 32 * chunks * 1024;
-    view.weights = view.cotangent + weights;
-    view.bytes = weights + in_features / 32 * chunks * 1024;
+    view.weights = view.cotangent + cotangent_bytes;
+    view.bytes = cotangent_bytes + in_features / 32 * view.chunks * 1024;
     return view;
 }
 // Whether a dense grad-input unpacks its weights once (tgo_unpacked.hip) or leaves it to every workgroup (tgo_backward.hip): by what

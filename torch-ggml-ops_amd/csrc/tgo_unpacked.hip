@@ -784,16 +784,14 @@ hipError_t launch_grad_input_unpacked(const DenseSource * sources, int count, vo
     if (count < 1 || count > UNP_SOURCES) {
         return hipErrorInvalidValue;
     }
-    int64_t chunks = 0;
-    // cotangents whose rows are whole stages are multiplied as they stand
-    bool row_major = true;
+    int64_t widths[UNP_SOURCES];
     for (int i = 0; i < count; ++i) {
-        chunks += cotangent_chunks(sources[i].out_features);
-        row_major = row_major && sources[i].out_features % 32 == 0;
+        widths[i] = sources[i].out_features;
     }
-    const UnpackedGradWorkspace view = unpacked_grad_workspace(workspace, rows, chunks, in_features);
-    // (row-major: a source ends with its weight rows, a multiple of 32, and not with a whole step of 64)
-    const auto chunks_of = [&](int i) { return row_major ? static_cast<int>(sources[i].out_features / 16) : cotangent_chunks(sources[i].out_features); };
+    // cotangents whose rows are whole stages are multiplied as they stand
+    const UnpackedGradWorkspace view = unpacked_grad_workspace(workspace, rows, count, widths, in_features);
+    const bool row_major = view.row_major;
+    const auto chunks_of = [&](int i) { return static_cast<int>(view.chunks_of(widths[i])); };
     ProductArgs args = {};
     for (int i = 0; i < count; ++i) {
         args.x_source[i] = reinterpret_cast<const uint8_t *>(sources[i].activations);
