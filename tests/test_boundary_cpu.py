@@ -469,3 +469,17 @@ def test_gradient_workspace_without_a_cotangent_that_is_not_packed(package):
     assert lib.tgo_multi_grad_workspace_bytes(2, both, 4096, 2048) == 2 * 2560 * 2048
     assert lib.tgo_pair_grad_workspace_bytes(4096, 2048, 2048, 14) == 2 * 2 * 2048 * 2048
     assert lib.tgo_dense_grad_workspace_bytes(4096, 2047, 2048, 12) == 2 * 2048 * 2048 + 2 * 4096 * 2048   # (both packed)
+
+
+def test_gradients_that_unpack_their_weights_once(package):
+    """Not where that measured slower: long reductions over a few columns, which wait for their cotangent, and pairs of one shape, which are one call
+    otherwise too."""
+    _, native, _, _ = package
+
+    def unpacks(rows, widths, k):
+        return native.lib.tgo_multi_grad_workspace_bytes(len(widths), (ctypes.c_int64 * len(widths))(*widths), rows, k) > 0
+
+    for rows, widths, k in ((4096, [28672], 512), (3193, [15872], 768), (2048, [8192], 1536), (195, [832, 832], 2560), (2857, [5632, 5632], 1024)):
+        assert not unpacks(rows, widths, k)
+    for rows, widths, k in ((4096, [4096], 2048), (2048, [4096, 1024, 1024], 4096), (8192, [15872], 512), (4096, [2048, 2048], 2048)):
+        assert unpacks(rows, widths, k)

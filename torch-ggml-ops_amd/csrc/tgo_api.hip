@@ -272,14 +272,12 @@ int64_t tgo_multi_grad_workspace_bytes(int count, const int64_t * out_features, 
     if (count < 1 || count > tgo::UNPACKED_SOURCES || out_features == nullptr || rows <= 0 || in_features <= 0 || in_features % tgo::QK_K != 0) {
         return 0;
     }
-    int64_t total = 0;
     for (int i = 0; i < count; ++i) {
         if (out_features[i] <= 0 || out_features[i] > INT_LIMIT) {
             return 0;
         }
-        total += out_features[i];
     }
-    return tgo::multi_grad_unpacks(rows, total, in_features, count)
+    return tgo::multi_grad_unpacks(rows, count, out_features, in_features)
         ? tgo::unpacked_grad_workspace(nullptr, rows, count, out_features, in_features).bytes : 0;
 }
 
@@ -676,7 +674,8 @@ int tgo_mmq_pair_grad_input(const void * grad_output_first, const void * grad_ou
     TGO_TRY(check_pointer(grad_input_bf16, "grad_input"));
     TGO_TRY(check_pointer(workspace, "workspace"));
     hipStream_t hip_stream = static_cast<hipStream_t>(stream);
-    if (tgo::multi_grad_unpacks(rows, 2 * out_features, in_features, 2)) {
+    const int64_t both[2] = {out_features, out_features};
+    if (tgo::multi_grad_unpacks(rows, 2, both, in_features)) {
         const tgo::DenseSource sources[2] = {
             {static_cast<const uint8_t *>(packed_first), static_cast<const uint16_t *>(grad_output_first), out_features, quant_type},
             {static_cast<const uint8_t *>(packed_second), static_cast<const uint16_t *>(grad_output_second), out_features, quant_type}};

@@ -655,13 +655,16 @@ static inline UnpackedGradWorkspace unpacked_grad_workspace(void * base, int64_t
 }
 // Whether a dense grad-input unpacks its weights once (tgo_unpacked.hip) or leaves it to every workgroup (tgo_backward.hip): by what
 // either takes.  The latter packs the cotangent, then runs items of 256 x 128, a round of 256 taking 0.27 us per 16 weight rows and half a
-// round 0.18, and cuts the reduction where that leaves half of the chip idle, for fp32 sums to be written and read again.  `count`
-// projections of one input (their weight rows together) would take a call each and an addition.
-// Of the time of the kernels that unpack as they multiply, where this rule leaves them (70 calls of 96 to 16384 rows, 512 to 28672 weight rows, K
-// 512 to 8192, all formats): 0.82 on the mean, 1.09 at most (257 rows of 1260 x 4608 IQ2_S 25.3 -> 27.5 us); before those kernels'
-// tile lay along K: 4096 x 2048, 2000 rows Q4_K 58.9 -> 51.0 us, Q6_K 63.7 -> 47.8; 4096 rows 87.2 -> 74.8, 96.3 -> 73.0; 8192 rows 165.6 -> 122.6, 184.0 -> 121.9.  On the other side of it, always unpacked: 28672 x 8192, 300 rows 206 -> 413 us (Q4_K); 4096 x
-// 2048, 300 rows 28.5 -> 30.2.
-static inline bool grad_unpacks(int64_t rows, int64_t out_features, int64_t in_features, int count = 1) {
+// round 0.18, and cuts the reduction where that leaves half of the chip idle, for fp32 sums to be written and read again.  Projections of one
+// input (`out_features`: their weight rows together) would take `calls` calls and an addition for each but the first.
+// A product that reads 32 MB of cotangent waits for them at 0.165 us per step, however few tiles it has (rows x weight rows x K: 2048 x 8192 x
+// 1536 93 us, 3193 x 15872 x 768 172, 4096 x 28672 x 512 302; the other kernels 85, 129 and 214).
+// Of the time of the kernels that unpack as they multiply, where this rule leaves them, inputs from memory, all formats: 246 of 460 calls of 96 to
+// 16384 rows, 256 to 28672 weight rows, K 512 to 8192: 0.83 on the mean, 1.17 at most (2 us of an IQ2_S call of 11); 31 of 68 pairs of one shape
+// 0.87, 1.11; 45 of 62 calls of three projections 0.67, 1.00.
+// 4096 x 2048, 4096 rows Q4_K 85.2 -> 76.2 us, Q6_K 87.4 -> 77.0; 8192 rows 164 -> 125, 168 -> 127.  On the other side of it, always unpacked:
+// 28672 x 8192, 300 rows Q4_K 211 -> 439 us; 4096 x 2048, 300 rows 27.6 -> 44.8; and the wrong one: 257 rows of 1260 x 4608 IQ2_S 24.7 -> 27.3.
+static inline bool grad_unpacks(int64_t rows, int64_t out_features, int64_t in_features, int calls = 1) {
     // (32-bit lane offsets; a workspace of at most 1 GiB for the weights)
     if (rows < 96 || out_features > (1 << 24) || out_features * in_features > (INT64_C(1) << 29) || rows > (1 << 24)) {
         return false;
@@ -672,12 +675,22 @@ static inline bool grad_unpacks(int64_t rows, int64_t out_features, int64_t in_f
     const float together = 9.0f + static_cast<float>(rows) * static_cast<float>(out_features) * 0.8e-6f +
                            static_cast<float>(steps / splits) * rounds_microseconds(items, 0.18f, 0.27f) +
                            (splits > 1 ? 4.0f + static_cast<float>(rows) * static_cast<float>(in_features) * static_cast<float>(splits) * 1.2e-6f : 0.0f) +
-                           static_cast<float>(count - 1) * (9.0f + static_cast<float>(rows) * static_cast<float>(in_features) * 1.5e-6f);
-    return 1.05f * (unpack_microseconds(out_features, in_features) + product_plan(rows, in_features, steps).microseconds) < together;
+                           static_cast<float>(calls - 1) * (9.0f + static_cast<float>(rows) * static_cast<float>(in_features) * 1.5e-6f);
+    const float waiting = rows * out_features >= (1 << 24) ? 0.165f * static_cast<float>(steps) : 0.0f;
+    return 1.05f * (unpack_microseconds(out_features, in_features) + std::max(product_plan(rows, in_features, steps).microseconds, waiting)) < together;
 }
-// Of several projections as one reduction: their sums in fp32.  (Below a million weights the terms keep being rounded one by one.)
-static inline bool multi_grad_unpacks(int64_t rows, int64_t out_features, int64_t in_features, int count) {
-    return (count == 1 || out_features * in_features >= (1 << 20)) && grad_unpacks(rows, out_features, in_features, count);
+// Of several projections as one reduction: their sums in fp32.  (Below a million weights the terms keep being rounded one by one.)  Neighbours of
+// one width are a call otherwise (mmq_pair_grad_input, if their formats agree).
+static inline bool multi_grad_unpacks(int64_t rows, int count, const int64_t * out_features, int64_t in_features) {
+    int64_t total = 0;
+    int calls = 0;
+    for (int i = 0; i < count; ++i, ++calls) {
+        total += out_features[i];
+        if (i + 1 < count && out_features[i + 1] == out_features[i]) {
+            total += out_features[++i];
+        }
+    }
+    return (count == 1 || total * in_features >= (1 << 20)) && grad_unpacks(rows, total, in_features, calls);
 }
 // Grad-input of up to four projections of one input: the sum of their Jacobian products, rounded once.  `workspace`:
 // unpacked_grad_workspace().bytes.
