@@ -483,3 +483,16 @@ def test_gradients_that_unpack_their_weights_once(package):
         assert not unpacks(rows, widths, k)
     for rows, widths, k in ((4096, [4096], 2048), (2048, [4096, 1024, 1024], 4096), (8192, [15872], 512), (4096, [2048, 2048], 2048)):
         assert unpacks(rows, widths, k)
+
+
+def test_forward_calls_that_unpack_their_weights_once(package):
+    """Not short reductions of a few hundred rows, whose activations the other kernels quantize in less time than the rule once held against them."""
+    _, native, _, _ = package
+
+    def unpacks(qtype, rows, n, k):
+        return native.lib.tgo_forward_scratch_bytes_as(rows, k, n, qtype, native.OPERANDS["scaled"]) > 0
+
+    for call in ((11, 123, 18688, 512), (12, 320, 18752, 512), (11, 463, 9216, 768), (13, 374, 11281, 512)):
+        assert not unpacks(*call)
+    for call in ((12, 4096, 4096, 4096), (12, 2000, 2048, 2048), (13, 4096, 4096, 2048), (11, 2424, 13878, 3584)):
+        assert unpacks(*call)

@@ -708,14 +708,14 @@ static inline int64_t unpacked_forward_bytes(int quant_type, int64_t tiles, int6
     return tiles * (unpacked_forward_steps(quant_type, in_features) * 1024 + 128);
 }
 // Whether a dense forward call with scaled operands unpacks its weights once (tgo_unpacked.hip) or leaves it to the unpacking waves of
-// every workgroup (tgo_forward_scaled.hip): by what either takes.  The latter quantizes in two launches, then runs items of 256 x 128 on
-// persistent workgroups, half a round and a whole round of 256 in 0.19 and 0.27 us per step of 16 (Q6_K 0.31) and 1.3 for the stores, or of 128
+// every workgroup (tgo_forward_scaled.hip): by what either takes.  The latter quantizes in two launches (with their gaps 9 us for 256 rows, 16
+// from 1024 on, 12 where tiles of 128 rows follow), then runs items of 256 x 128 on persistent workgroups, half a round and a whole round of 256 in 0.19 and 0.27 us per step of 16 (Q6_K 0.31) and 1.3 for the stores, or of 128
 // x 128 (forward_split) in 0.145 and 0.185, the slower formats to unpack 0.22.
 // Results of more than 100 million values no longer stay in the last cache, which only the kernel without an overlapped epilogue notices.
-// Of the time of the scaled kernel, where this rule leaves it (100 calls of 300 to 16000 rows, 512 to 28672 columns, K 512 to 8192): 0.83 on the
-// mean, 0.38 (Q6_K, rows of which no tile is a whole number of 16-byte units) to 1.05.  4096 x 4096, 4096 rows: Q4_K 173 -> 152 us, Q3_K 178 ->
-// 144, Q6_K 196 -> 147; 2048 x 2048, 2000 rows Q4_K 43.7 -> 34.8.  On the other side of it, always unpacked: 28672 x 8192, 300 rows Q4_K 235 -> 389 us;
-// 16384 x 1024, 8192 rows Q4_K 315 -> 367.
+// Of the time of the scaled kernel, where this rule leaves it: 277 of 453 calls of 96 to 16384 rows, 512 to 28672 columns, K 512 to 8192 0.84 on the
+// mean, 1.12 at most (4 us of 34); with 16 us for any number of rows 296, 0.85 and 1.46 (123 rows of 18688 x 512 Q3_K 18.2 -> 26.6).  Calls of three
+// projections (57) 0.73, 1.01.  4096 x 4096, 4096 rows: Q4_K 173 -> 152 us, Q3_K 178 -> 144, Q6_K 196 -> 147; 2048 x 2048, 2000 rows Q4_K 43.7 -> 34.8.
+// On the other side of it, always unpacked: 28672 x 8192, 300 rows Q4_K 235 -> 389 us; 16384 x 1024, 8192 rows Q4_K 315 -> 367.
 static inline bool forward_unpacks(int quant_type, int64_t rows, int64_t in_features, int64_t out_features) {
     const int64_t tiles = ((rows + 255) / 256) * ((out_features + 127) / 128);
     if (!scaled_forward_format(quant_type) || tiles < SCALED_AUTO_MIN_TILES || out_features > (1 << 24) ||
@@ -729,7 +729,8 @@ static inline bool forward_unpacks(int quant_type, int64_t rows, int64_t in_feat
     const float half = row_tile == 128 ? (quick ? 0.145f : 0.19f) : quant_type == 14 ? 0.22f : 0.19f;
     const float whole = row_tile == 128 ? (quick ? 0.185f : 0.22f) : quant_type == 14 ? 0.311f : 0.273f;
     const int64_t items = ((rows + row_tile - 1) / row_tile) * ((out_features + 127) / 128);
-    const float together = (row_tile == 128 ? 12.0f : 16.0f) + input * 1.0e-6f + rounds_microseconds(items, half * steps + 1.3f, whole * steps + 1.3f);
+    const float many_rows = std::min(1.0f, std::max(0.0f, (static_cast<float>(rows) - 256.0f) / 768.0f));
+    const float together = 9.0f + (row_tile == 128 ? 3.0f : 7.0f) * many_rows + input * 1.0e-6f + rounds_microseconds(items, half * steps + 1.3f, whole * steps + 1.3f);
     const float apart = unpack_microseconds(out_features, in_features) + input * 0.9e-6f + (results > 1.0e8f ? results * 0.3e-6f : 0.0f) +
                         product_plan(rows, out_features, unpacked_forward_steps(quant_type, in_features)).microseconds;
     // (short reductions, but for those of Q6_K, are what the model is least sure of)
