@@ -77,13 +77,26 @@ def test_layer(ops, oracle, gate_up, down, tokens, top_k, experts, k, n):
 
 
 def test_choices_that_are_no_expert_contribute_nothing(ops, oracle):
-    """Also where a whole token has none, and where what an earlier call left in the workspace would be read for them."""
+    """Also where a whole token has none, where a token names one expert twice, and with a workspace of NaN, of which the slots without an expert are
+    never written."""
+    from torch_ggml_ops import _native
+
     tgo, lib, synth = ops
-    hidden, chosen, weights, *experts = _layer(synth, 4, 3, 5, 1024, 512, "Q6_K", "Q4_K", seed=11)
+    hidden, chosen, weights, *experts = _layer(synth, 5, 3, 5, 1024, 512, "Q6_K", "Q4_K", seed=11)
     chosen[1] = torch.tensor([-1, 5, 1 << 40])
     chosen[2, 1] = -7
-    torch.full((1 << 22,), float("nan"), device="cuda")   # (given back to the allocator, from which the workspace comes)
-    _check(tgo, lib, oracle, hidden, chosen, weights, *experts, "Q6_K", "Q4_K", 512)
+    chosen[3] = torch.tensor([4, 2, 4])
+    device = _check(tgo, lib, oracle, hidden, chosen, weights, *experts, "Q6_K", "Q4_K", 512)
+    with torch.no_grad():
+        expected = tgo.moe_layer(hidden, *device, QTYPES["Q6_K"], QTYPES["Q4_K"], 512)
+    sizes = (5, 3, 5, 1024, 512, QTYPES["Q6_K"], QTYPES["Q4_K"])
+    workspace = torch.full((lib.tgo_moe_decode_workspace_bytes(*sizes),), 0xFF, dtype=torch.uint8, device="cuda")
+    assert workspace.view(torch.bfloat16).isnan().all()
+    actual = torch.empty_like(expected)
+    pointers = [t.data_ptr() for t in (hidden, *device, actual, workspace)]
+    _native.check(lib.tgo_moe_decode(*pointers, *sizes, _native.stream_of(hidden.device)))
+    assert torch.equal(actual, expected) and not actual[1].any()
+    assert workspace.view(torch.bfloat16).view(15, 512)[[3, 4, 5, 7]].isnan().all()
 
 
 def test_graph(ops):

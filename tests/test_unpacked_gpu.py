@@ -91,30 +91,46 @@ def test_gradient_workspaces(qname):
     assert unpack.count(True) >= 4 and not unpack[1] and not unpack[5]
 
 
-# (rows, columns, K): as above, an odd number of steps with the minima's (K = 768, 1280), columns that end inside a tile, rows of 16-byte units
-# and not (Q3_K, Q6_K and IQ2_S of K = 768 and an odd number of columns)
-FORWARDS = [(2000, 2048, 2048), (1000, 5003, 1280), (545, 6017, 768), (8200, 769, 768), (9000, 520, 512), (4097, 4096, 1024), (500, 8192, 2816)]
+# (rows, columns, K): 128 x 128 and 128 x 256 tiles; an odd number of super-blocks and with it of the minima's steps (K = 768, 1280); columns that end
+# inside a tile; rows of 16-byte units and not (Q3_K, Q6_K and IQ2_S of K = 768 and an odd number of columns); 256 x 256 tiles, whole rounds of them
+# and rows behind those.  Every call here has to unpack its weights: of short reductions Q4_K and Q5_K do not.
+FORWARDS = [(2000, 2048, 2048), (1000, 5003, 1280), (9000, 520, 512), (4097, 4096, 1280), (8300, 2041, 1280), (2600, 5000, 1280)]
+SHORT_FORWARDS = [(545, 6017, 768), (8200, 769, 768), (4097, 4096, 1024)]
 
 
-@pytest.mark.parametrize("qname", tuple(QTYPES))
-@pytest.mark.parametrize("rows,n,k", FORWARDS)
+@pytest.mark.parametrize(
+    "qname,rows,n,k", [(q, *f) for q in QTYPES for f in FORWARDS + (SHORT_FORWARDS if q in ("Q3_K", "Q6_K", "IQ2_S") else [])]
+)
 def test_forward_has_the_bits_of_the_scaled_kernel(qname, rows, n, k):
     """The same operands in the same order: a call without scratch, which the scaled kernel takes, gives the same bits.  Super-blocks far below
-    their row's largest one, a row of zeros, an infinity, and a weight row of zeros and of the format's largest scales among them."""
+    their row's largest one, a row of zeros, infinities and NaN in activations and weight scales, and a weight row of zeros among them."""
     import synth
     import torch_ggml_ops as tgo  # noqa: F401
     from torch_ggml_ops import _native
 
     qtype, lib = QTYPES[qname], _native.lib
-    if _native.forward_operand_for(qtype, rows, n) != "scaled":
-        pytest.skip("not a call with scaled operands")
+    assert _native.forward_operand_for(qtype, rows, n) == "scaled"
+    assert lib.tgo_forward_scratch_bytes_as(rows, k, n, qtype, _native.OPERANDS["scaled"]) > 0
     packed = synth.random_packed_weight(qtype, (n,), k, seed=qtype + n)
     packed[1] = 0
+    # fp16 scale fields of a row's last block: an infinity, a NaN, and both in one row
+    width, fields = synth.BLOCK_BYTES[qtype], synth._SCALE_FIELDS[qtype]
+    for row, (first, last) in ((2, (0x7C00, 0x7C00)), (4, (0x7E00, 0x7E00)), (n - 1, (0xFC00, 0x7E01))):
+        blocks = packed[row].view(-1, width)
+        for block, value in ((0, first), (-1, last)):
+            for field in fields:
+                blocks[block, field], blocks[block, field + 1] = value & 0xFF, value >> 8
+        if row == 4:
+            blocks[0] = 0
     packed = packed.cuda()
     x = random_bf16((rows, k), seed=rows)
     x[3] = 0
     x[5, 256:] *= 2.0**-20
     x[6, :32] *= 2.0**-30
+    x[8, 1] = float("nan")
+    x[9] = float("nan")
+    x[10, k - 1] = -float("inf")
+    x[10, 0] = float("nan")
     x[rows - 1, 7] = float("inf")
     workspace = torch.empty(lib.tgo_q8_workspace_bytes(rows, k), dtype=torch.uint8, device="cuda")
     outputs = []
@@ -130,8 +146,12 @@ def test_forward_has_the_bits_of_the_scaled_kernel(qname, rows, n, k):
                 rows, k, n, qtype, _native.stream_of(x.device),
             )
         )
-        outputs.append(output.view(torch.int16))
-    assert torch.equal(*outputs)
+        outputs.append(output)
+    scaled, unpacked = outputs
+    is_nan = scaled.isnan()
+    assert torch.equal(is_nan, unpacked.isnan()) and not is_nan[rows // 2, n // 2]
+    # (which of several NaN of a sum comes out is the instructions' business)
+    assert torch.equal(scaled.view(torch.int16).masked_fill(is_nan, 0), unpacked.view(torch.int16).masked_fill(is_nan, 0))
 
 
 @pytest.mark.parametrize("qname", ("Q5_K", "IQ2_S"))
