@@ -40,6 +40,7 @@ def problems(checker, lds, *lines):
     "lines",
     (
         (SOUND, SOUND),
+        (by_hand("s_mov_b32 m0, s9", "s_nop 0", SLAB, SLAB + " offset:1024"),),
         ("\ts_add_u32 s9, s8, 16", SOUND),   # scalar results are interlocked
         ("\tv_readfirstlane_b32 s2, v9", "\ts_nop 2", SOUND),   # 3 + 2 wait states
         ("\tv_readfirstlane_b32 s4, v9", SOUND),

@@ -80,10 +80,10 @@ def check(body, labels, lds: bool) -> tuple[int, list[str]]:
             for source in before(at, M0_STATES):
                 if re.match(r"m0\b", body[source][2]):
                     problems.append(f"line {number}: {mnemonic} follows a write of m0 without a wait state")
-            own = at - 1   # its own piece of assembly writes m0
-            while own >= 0 and body[own][1] == "s_nop" and body[own][3]:
+            own = at   # its own piece of assembly writes m0
+            while own >= 0 and body[own][3] == by_hand and not re.match(r"m0\b", body[own][2]):
                 own -= 1
-            if own < 0 or not body[own][3] or not re.match(r"m0\b", body[own][2]):
+            if own < 0 or body[own][3] != by_hand:
                 problems.append(f"line {number}: {mnemonic} takes m0 from elsewhere")
         elif lds:
             problems.append(f"line {number}: {mnemonic} does not go to LDS")

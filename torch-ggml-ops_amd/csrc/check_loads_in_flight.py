@@ -35,14 +35,15 @@ def _registers(operands: str) -> frozenset:
 
 
 def functions(text: str):
-    """(name, [(line number, mnemonic, operands, inside inline assembly)], {label: index}) of each function."""
-    name, body, labels, by_hand = None, [], {}, False
+    """(name, [(line number, mnemonic, operands, which piece of inline assembly, 0 for none)], {label: index}) of each function."""
+    name, body, labels, by_hand, pieces = None, [], {}, 0, 0
     for number, line in enumerate(text.splitlines(), 1):
         stripped = line.strip()
         if stripped.startswith(";;#ASMSTART"):
-            by_hand = True
+            pieces += 1
+            by_hand = pieces
         elif stripped.startswith(";;#ASMEND"):
-            by_hand = False
+            by_hand = 0
         code = stripped.split(";", 1)[0].strip()
         if not code:
             continue
@@ -65,7 +66,7 @@ def functions(text: str):
 
 def check(body, labels) -> tuple[int, list[str]]:
     """(hand-issued loads, violations) of one function."""
-    issued = sum(by_hand and _LOAD.match(mnemonic) is not None for _, mnemonic, _, by_hand in body)
+    issued = sum(by_hand != 0 and _LOAD.match(mnemonic) is not None for _, mnemonic, _, by_hand in body)
     problems, seen = {}, set()
     todo = [(0, ())]   # (instruction, outstanding loads: the registers of a hand-issued one, or None)
     while todo:
