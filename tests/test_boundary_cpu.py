@@ -481,7 +481,7 @@ def test_gradients_that_unpack_their_weights_once(package):
 
     for rows, widths, k in ((4096, [28672], 512), (3193, [15872], 768), (2048, [8192], 1536), (195, [832, 832], 2560), (2857, [5632, 5632], 1024)):
         assert not unpacks(rows, widths, k)
-    for rows, widths, k in ((4096, [4096], 2048), (2048, [4096, 1024, 1024], 4096), (8192, [15872], 512), (4096, [2048, 2048], 2048)):
+    for rows, widths, k in ((4096, [4096], 2048), (2048, [4096, 1024, 1024], 4096), (161, [2188, 547, 547], 1280), (8192, [15872], 512), (4096, [2048, 2048], 2048)):
         assert unpacks(rows, widths, k)
 
 

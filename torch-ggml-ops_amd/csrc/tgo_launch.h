@@ -661,7 +661,7 @@ static inline UnpackedGradWorkspace unpacked_grad_workspace(void * base, int64_t
 // 1536 93 us, 3193 x 15872 x 768 172, 4096 x 28672 x 512 302; the other kernels 85, 129 and 214).
 // Of the time of the kernels that unpack as they multiply, where this rule leaves them, inputs from memory, all formats: 246 of 460 calls of 96 to
 // 16384 rows, 256 to 28672 weight rows, K 512 to 8192: 0.83 on the mean, 1.17 at most (2 us of an IQ2_S call of 11); 31 of 68 pairs of one shape
-// 0.87, 1.11; 45 of 62 calls of three projections 0.67, 1.00.
+// 0.87, 1.11; 46 of 62 calls of three projections 0.67, 1.00.
 // 4096 x 2048, 4096 rows Q4_K 85.2 -> 76.2 us, Q6_K 87.4 -> 77.0; 8192 rows 164 -> 125, 168 -> 127.  On the other side of it, always unpacked:
 // 28672 x 8192, 300 rows Q4_K 211 -> 439 us; 4096 x 2048, 300 rows 27.6 -> 44.8; and the wrong one: 257 rows of 1260 x 4608 IQ2_S 24.7 -> 27.3.
 static inline bool grad_unpacks(int64_t rows, int64_t out_features, int64_t in_features, int calls = 1) {
@@ -679,18 +679,17 @@ static inline bool grad_unpacks(int64_t rows, int64_t out_features, int64_t in_f
     const float waiting = rows * out_features >= (1 << 24) ? 0.165f * static_cast<float>(steps) : 0.0f;
     return 1.05f * (unpack_microseconds(out_features, in_features) + std::max(product_plan(rows, in_features, steps).microseconds, waiting)) < together;
 }
-// Of several projections as one reduction: their sums in fp32.  (Below a million weights the terms keep being rounded one by one.)  Neighbours of
-// one width are a call otherwise (mmq_pair_grad_input, if their formats agree).
+// Of several projections as one reduction: their sums in fp32.  (Below a million weights the terms keep being rounded one by one, for the bits' sake and
+// not for speed.)  Two of one width are one call otherwise too (mmq_pair_grad_input, if their formats agree).  More than two count as a call each, also
+// where two of them are such a pair, for what the calls cost on the host: 161 rows of 2188 + 547 + 547 x 1280 Q5_K, forward and backward from Python,
+// 167 us, and 187 with the pair counted as one call.
 static inline bool multi_grad_unpacks(int64_t rows, int count, const int64_t * out_features, int64_t in_features) {
     int64_t total = 0;
-    int calls = 0;
-    for (int i = 0; i < count; ++i, ++calls) {
+    for (int i = 0; i < count; ++i) {
         total += out_features[i];
-        if (i + 1 < count && out_features[i + 1] == out_features[i]) {
-            total += out_features[++i];
-        }
     }
-    return (count == 1 || total * in_features >= (1 << 20)) && grad_unpacks(rows, total, in_features, calls);
+    const bool pair = count == 2 && out_features[0] == out_features[1];
+    return (count == 1 || total * in_features >= (1 << 20)) && grad_unpacks(rows, total, in_features, pair ? 1 : count);
 }
 // Grad-input of up to four projections of one input: the sum of their Jacobian products, rounded once.  `workspace`:
 // unpacked_grad_workspace().bytes.
@@ -760,7 +759,9 @@ struct MoeDecodeArgs {
 // 256 experts with power-law 0.3 routing 0.56 to 0.67 (50.5 -> 32.1), of 128 experts of 2048 x 768 with power-law 1.1 routing 0.66 to 0.90, five
 // of 64 of 4096 x 1024 0.83 to 0.94.  Beyond the lines: 8 tokens of 128 of 2048 x 768, 1.1: 0.71 to 1.05; 8 of 64 of 4096 x 1024: 0.98 to 1.29; 16 of
 // 256 of 2048 x 512: 0.77 to 0.92 at 0.3, 1.08 to 1.35 at 1.1.  Experts of less than half a million weights keep the operators, and with them
-// the operators' bits: those round every expert's row before they add it, and their sums have another order.
+// the operators' bits: those round every expert's row before they add it, and their sums have another order (a line of bits, not of speed: 1024 x 512,
+// on it, 17 such layers 0.40 to 0.75 of the time).  The sizes end where the kernels' instances do: a wave of the down projection holds its rows of eight experts in registers
+// (up to four super-blocks each), gate and up have instances of 8 and 16 super-blocks; larger layers have not been measured.
 static inline bool moe_decodes(int64_t tokens, int64_t top_k, int64_t experts, int64_t features, int64_t intermediate) {
     const int64_t slots = tokens * top_k;
     return top_k <= MOE_DECODE_TOP_K && slots <= MOE_DECODE_SLOTS && features % 256 == 0 && features <= 4096 && intermediate % 256 == 0 &&
