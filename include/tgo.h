@@ -98,9 +98,10 @@ int tgo_mmq_forward(const void * input_bf16, const void * packed, void * output_
  *   tgo_forward_scratch_bytes     what tgo_mmq_forward_scratch may use, under any setting of the operands
  *   tgo_forward_scratch_bytes_as  what a call on operands of that kind uses: TGO_OPERAND_SCALED the unpacked weights (which may be hundreds of
  *                                 MiB), TGO_OPERAND_INT8 and _HALF the ranges' sums, which are also all that the prepared entry points and
- *                                 tgo_mmq_multi_forward use, with operands of any kind
- *   tgo_mmq_forward_sized         tgo_mmq_forward_scratch with any number of bytes there: a call does without what does not fit, and so a
- *                                 caller may ask for what tgo_forward_operand_for's present kind uses */
+ *                                 tgo_mmq_multi_forward use, with operands of any kind; TGO_OPERAND_AUTO what tgo_mmq_forward_sized
+ *                                 uses under the present setting
+ *   tgo_mmq_forward_sized         tgo_mmq_forward_scratch with any number of bytes there: a call does without what does not fit, should
+ *                                 the setting change in between */
 int64_t tgo_forward_scratch_bytes(int64_t rows, int64_t in_features, int64_t out_features, int quant_type);
 int64_t tgo_forward_scratch_bytes_as(int64_t rows, int64_t in_features, int64_t out_features, int quant_type, int operand);
 int tgo_mmq_forward_sized(const void * input_bf16, const void * packed, void * output_bf16, void * workspace, void * scratch,

@@ -385,6 +385,13 @@ int64_t tgo_forward_scratch_bytes_as(int64_t rows, int64_t in_features, int64_t 
     if (rows <= 0 || in_features <= 0 || out_features <= 0 || tgo::use_gemv(rows, 0)) {
         return 0;
     }
+    if (operand == TGO_OPERAND_AUTO) {
+        const int setting = tgo::forward_operand_setting();
+        if (tgo::dense_takes_tiles(setting, rows, in_features, out_features, quant_type)) {
+            return 0;
+        }
+        operand = tgo::forward_operand_kind(setting, quant_type, rows, out_features, 1);
+    }
     if (operand == TGO_OPERAND_SCALED) {
         return tgo::forward_unpacks(quant_type, rows, in_features, out_features)
             ? tgo::unpacked_forward_bytes(quant_type, (out_features + 31) / 32, in_features) : 0;

@@ -109,13 +109,7 @@ PyObject * direct_mmq(PyObject *, PyObject * const * args, Py_ssize_t count) {
         shape.back() = out_features;
         output = at::detail::empty_cuda(shape, at::kBFloat16, input.device(), std::nullopt);
         const int64_t workspace_bytes = (tgo_q8_workspace_bytes(rows, in_features) + 255) / 256 * 256;
-        int64_t scratch_bytes = tgo_forward_scratch_bytes_as(rows, in_features, out_features, static_cast<int>(quant_type),
-                                                             tgo_forward_operand_for(static_cast<int>(quant_type), rows, out_features, 1));
-        if (scratch_bytes > 0) {
-            // (the decode kernel of up to 128 rows needs none; a call without it is as correct should the setting change in between)
-            const char * const kernels = tgo_forward_kernel_for(static_cast<int>(quant_type), rows, in_features, out_features, 0, 1);
-            scratch_bytes = kernels != nullptr && std::strcmp(kernels, "tiles") == 0 ? 0 : scratch_bytes;
-        }
+        const int64_t scratch_bytes = tgo_forward_scratch_bytes_as(rows, in_features, out_features, static_cast<int>(quant_type), TGO_OPERAND_AUTO);
         const c10::DataPtr workspace = c10::GetAllocator(c10::kCUDA)->allocate(workspace_bytes + scratch_bytes);
         void * const scratch = scratch_bytes > 0 ? static_cast<uint8_t *>(workspace.get()) + workspace_bytes : nullptr;
         status = tgo_mmq_forward_sized(input.data_ptr(), weight.data_ptr(), output.data_ptr(), workspace.get(), scratch, scratch_bytes, rows,

@@ -230,20 +230,19 @@ def stream_of(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
-def forward_scratch_bytes(rows: int, in_features: int, out_features: int, quant_type: int, kind: int) -> int:
-    """Scratch bytes worth allocating for a dense forward call on operands of this kind: none where the decode kernel takes it (a
-    call without scratch is as correct should the setting change in between)."""
-    size = lib.tgo_forward_scratch_bytes_as(rows, in_features, out_features, int(quant_type), kind)
+def ranges_scratch_bytes(rows: int, in_features: int, out_features: int, quant_type: int) -> int:
+    """Scratch bytes worth allocating for a dense forward call on a workspace: the sums of K's ranges, none where the decode kernel
+    takes the call (which is as correct without scratch should the setting change in between)."""
+    size = lib.tgo_forward_scratch_bytes_as(rows, in_features, out_features, int(quant_type), OPERANDS["int8"])
     return size if size == 0 or forward_kernel_for(int(quant_type), rows, in_features, out_features) != "tiles" else 0
 
 
-def forward_scratch(tensor: torch.Tensor, rows: int, in_features: int, out_features: int, quant_type: int, kind: int):
-    """(tensor that keeps it, pointer, bytes) of the scratch memory of a dense forward call; (None, None, 0) when it needs none."""
-    size = forward_scratch_bytes(rows, in_features, out_features, quant_type, kind)
+def scratch_of(tensor: torch.Tensor, size: int):
+    """(tensor that keeps it, pointer) of `size` bytes of scratch memory beside `tensor`; (None, None) for none."""
     if size == 0:
-        return None, None, 0
+        return None, None
     scratch = tensor.new_empty((size,), dtype=torch.uint8)
-    return scratch, scratch.data_ptr(), size
+    return scratch, scratch.data_ptr()
 
 
 def on_device(device: torch.device):

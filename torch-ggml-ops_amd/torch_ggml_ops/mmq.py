@@ -35,8 +35,10 @@ def _mmq_device(input: torch.Tensor, packed_weight: torch.Tensor, quant_type: in
         workspace = input.new_empty(
             (_native.lib.tgo_q8_workspace_bytes(rows, in_features),), dtype=torch.uint8
         )
-        kind = _native.lib.tgo_forward_operand_for(int(quant_type), rows, out_features, 1)
-        _scratch, scratch, scratch_bytes = _native.forward_scratch(input, rows, in_features, out_features, quant_type, kind)
+        scratch_bytes = _native.lib.tgo_forward_scratch_bytes_as(
+            rows, in_features, out_features, int(quant_type), _native.OPERANDS["auto"]
+        )
+        _scratch, scratch = _native.scratch_of(input, scratch_bytes)
         _native.check(
             _native.lib.tgo_mmq_forward_sized(
                 input.data_ptr(), packed_weight.data_ptr(), output.data_ptr(), workspace.data_ptr(), scratch, scratch_bytes,

@@ -96,10 +96,9 @@ def _mmq_prepared_device(
         )
     with _native.on_device(workspace.device):
         output = workspace.new_empty((rows, out_features), dtype=torch.bfloat16)
-        # (the ranges' sums of exact operands: weights are unpacked once per call only together with their activations)
-        _scratch, scratch, _ = _native.forward_scratch(
-            workspace, rows, in_features, out_features, quant_type, _native.OPERANDS["int8"]
-        )
+        # (weights are unpacked once per call only together with their activations)
+        scratch_bytes = _native.ranges_scratch_bytes(rows, in_features, out_features, quant_type)
+        _scratch, scratch = _native.scratch_of(workspace, scratch_bytes)
         _native.check(
             _native.lib.tgo_mmq_forward_prepared_scratch(
                 workspace.data_ptr(), packed_weight.data_ptr(), output.data_ptr(), scratch,
@@ -152,22 +151,18 @@ def _multi_device(input, packed_weights, quant_types, out_features, operand):
             _native.lib.tgo_multi_forward_scratch_bytes(count, widths, types, rows, in_features) if operand == "scaled" else 0
         )
         if unpacked_bytes > 0:
-            scratch = input.new_empty((unpacked_bytes,), dtype=torch.uint8)
+            _scratch, scratch = _native.scratch_of(input, unpacked_bytes)
             _native.check(
-                _native.lib.tgo_mmq_multi_forward_unpacked(
-                    *projections, scratch.data_ptr(), rows, in_features, _stream(input)
-                )
+                _native.lib.tgo_mmq_multi_forward_unpacked(*projections, scratch, rows, in_features, _stream(input))
             )
             return outputs
         scratch_bytes = max(
-            _native.forward_scratch_bytes(rows, in_features, features, quant_type, _native.OPERANDS["int8"])
+            _native.ranges_scratch_bytes(rows, in_features, features, quant_type)
             for quant_type, features in zip(quant_types, out_features)
         )
-        scratch = input.new_empty((scratch_bytes,), dtype=torch.uint8) if scratch_bytes > 0 else None
+        _scratch, scratch = _native.scratch_of(input, scratch_bytes)
         _native.check(
-            _native.lib.tgo_mmq_multi_forward(
-                *projections, None if scratch is None else scratch.data_ptr(), rows, in_features, kind, _stream(input)
-            )
+            _native.lib.tgo_mmq_multi_forward(*projections, scratch, rows, in_features, kind, _stream(input))
         )
     return outputs
 
