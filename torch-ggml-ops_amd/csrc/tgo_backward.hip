@@ -665,9 +665,10 @@ struct HalfBlockPieces {
 //
 // Measured, 256 rows of a 248320 x 2048 head (16 ranges): Q4_K 955 -> 316 us, Q6_K 655 -> 356, IQ2_S 527 -> 333 (820 TFLOP/s)
 // against the general kernel, whose waves dequantize and multiply in turn.  Then a lane decoded four values of eight weight rows, for a tile that
-// was stored transposed, after a stage for the block scales; with 32 values of a row per lane and the transposition in the reads (tile_granule) the
-// LDS is busy for 0.29 to 0.36 of the time instead of 0.43 to 0.6: 4096 tokens of eight choices among 256 experts with power-law 0.3 routing, 2 x
-// 512 x 2048 IQ2_S 276 -> 254 us, 512 x 2048 Q5_K 150 -> 138; dense calls of 33 to 900 rows 0.97 on the mean.  With the pieces of the column tile's
+// was stored transposed, after a stage for the block scales; with 32 values of a row per lane and the transposition in the reads (tile_granule) a
+// step has neither that stage nor its two waits: 4096 tokens of eight choices among 256 experts with power-law 0.3 routing, 2 x
+// 512 x 2048 IQ2_S 276 -> 254 us, 512 x 2048 Q5_K 150 -> 138; dense calls of 33 to 900 rows 0.97 on the mean.  (The LDS moves
+// data for 0.31 of the time instead of 0.46, a pair of 8192 tokens Q5_K; its instructions take 0.40 to 0.58 of it over the formats and 0.43 to 0.61 before.)  With the pieces of the column tile's
 // half block in place of the whole block (5 to 8 of 9 to 14) the head Q6_K 344 -> 317, IQ2_S 313 -> 305, Q5_K 319 -> 315; a pair of 8192 tokens
 // Q6_K 497 -> 478, IQ2_S 448 -> 439, Q5_K 458 -> 454.  What is left: the matrix pipe is busy
 // for 0.24 (tasks that half fill 256 rows, Q5_K) to 0.47 of the time (256 rows of the Q6_K head) at the clock that the card's power leaves (1.9 GHz with 256 rows of the head).
@@ -1288,7 +1289,7 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
 // Tasks of at most BACKWARD_SHORT_ROWS rows.  Dequantizing a step's 64 x 128 weights costs the same however few
 // rows multiply them, so here it is nearly all of the work and every wave does it: a wave owns 16 of the step's 64
 // weight rows from the global load to the bf16 tile (packed blocks DEPTH steps ahead in registers, parked in the
-// wave's own LDS slot, block scales, decode; LDS executes a wave's accesses in order, so these stages need no
+// wave's own LDS slot, decoded; LDS executes a wave's accesses in order, so these stages need no
 // workgroup barrier), one barrier per step publishes the tile, and then every wave multiplies the task's rows with
 // one 32-column slice of it (4 or 8 matrix instructions).  Small footprint: three workgroups share a CU, so one's
 // barrier and memory waits are covered by the others' decoding.  One workgroup per (task, column tile).
@@ -1299,8 +1300,9 @@ __global__ __launch_bounds__(BSP_THREADS, 2) void mmq_grad_input_split_kernel(co
 // scale per 16 values unpack four quants per operation as the role-split kernel does, instead of one by one: the whole gradient of 1024 tokens of
 // eight choices, 256 experts of 2 x 512 x 2048, IQ2_S 215 -> 175 us, Q3_K 205 -> 188, Q6_K 240 -> 227, and with pieces instead of the aligned units
 // that cover a block, and of those only what the tile needs, 155, 177 and 193 (Q5_K 187 -> 179, Q4_K 176 -> 162; 600 tokens of 128 experts of 2048 x
-// 768: IQ2_S 118 -> 90, Q3_K 104 -> 89, Q6_K 115 -> 91).  Four workgroups per CU, which Q3_K to Q5_K then have room for, are no faster.  Bound by the
-// vector unit (Q5_K 0.53 of the time at 2.7 waves per SIMD; LDS 0.42, of which a third bank conflicts, matrix cores 0.11).
+// 768: IQ2_S 118 -> 90, Q3_K 104 -> 89, Q6_K 115 -> 91).  Four workgroups per CU, which Q3_K to Q5_K then have room for, are no faster.  No unit
+// is full: the groups of 8192 tokens above have the LDS busy for 0.52 of the time (Q5_K), the vector unit for 0.45, the matrix cores for 0.10, and their
+// waves wait for a counter 0.30 of theirs.
 constexpr int BSH_THREADS = 256;
 constexpr int BSH_ROWS_PER_WAVE = BWD_NS / 4;
 constexpr int BSH_DEPTH = 2;

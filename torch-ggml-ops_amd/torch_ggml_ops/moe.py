@@ -448,6 +448,10 @@ def moe_layer(
     ``[tokens, top_k]``; ``gate_weight``/``up_weight`` packed ``[experts, intermediate, ...]`` and
     ``down_weight`` packed ``[experts, features, ...]``.  Differentiable with respect to ``hidden`` and
     ``slot_weights``.
+
+    A plain call without a gradient for a few tokens (up to 64 choices of experts of a decode step's sizes) is two launches
+    of their own and gives other bits than the same call with a gradient, or under a mode or a tracer: it rounds the sum over a token's
+    experts once, where the operators round every expert's row first.
     """
     if _direct is not None and not torch.compiler.is_compiling():
         output = _direct.moe_layer(
