@@ -45,8 +45,9 @@ def test_groups_whose_cotangent_is_longer_than_32_bits_reach(oracle, qname, shor
     ends = np.cumsum(sizes).tolist()
     host = synth.random_packed_weight(qtype, (experts, n), k, seed=qtype + short)
     grad = torch.empty((ends[-1], n), dtype=torch.bfloat16, device="cuda")
+    generator = torch.Generator(device="cuda").manual_seed(short)
     for first in range(0, ends[-1], 2**16):
-        grad[first : first + 2**16].normal_()
+        grad[first : first + 2**16].normal_(generator=generator)
     metadata = (torch.arange(experts, device="cuda"), torch.tensor(ends, device="cuda", dtype=torch.int32))
     actual = torch.ops.torch_ggml_ops.grouped_mmq_grad_input.default(grad, host.cuda(), *metadata, qtype, k)
     picked = np.r_[0:4, ends[0] - 4 : ends[-1]]
